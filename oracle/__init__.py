@@ -52,7 +52,7 @@ def build(quiet: bool = True) -> None:
     """Builds liboracle.so (and oracle/_ref when the reference tree exists)."""
     out = subprocess.DEVNULL if quiet else None
     subprocess.check_call(["make", "-s", "-C", HERE], stdout=out)
-    if os.path.isdir("/root/reference"):
+    if os.path.isdir("/root/reference/f77src"):
         subprocess.check_call(["make", "-s", "-C", os.path.join(HERE, "ref")], stdout=out)
 
 
