@@ -504,16 +504,47 @@ __global__ void k_mm16(const double *__restrict__ A, const double *__restrict__ 
 
 // ---------------------------------------------------------------------------
 // block Gram-Schmidt with delayed reorthogonalisation (block DCGS2): the
-// 16x16 tile algebra of one Arnoldi step, one block of 256 threads (one per
-// tile element; the first wave runs the Cholesky factorisations)
+// 16x16 tile algebra of one Arnoldi step, one block of 16 waves (a tile
+// product per wave; the first wave runs the Cholesky factorisations)
 // ---------------------------------------------------------------------------
-// c[e] = sum_l op(a)[i][l] b[l][k] for the thread's element e = (i, k)
-__device__ __forceinline__ double tdot(const double *a, const double *b, bool ta) {
-  const int i = threadIdx.x / kS, k = threadIdx.x % kS;
-  double s = 0.0;
+// 16x16 tile products on the FP64 matrix cores, one wave per product: the
+// operands in the input layout of v_mfma_f64_16x16x4f64 (k = 4 q + lane / 16),
+// the sum in its output layout (row lane / 16 + 4 r, column lane % 16)
+struct TileFrag {
+  double v[4];
+};
+template <bool TRANS = false>
+__device__ __forceinline__ TileFrag tile_a(const double *M) {
+  const int l = threadIdx.x & 63, r = l & 15, kk = l >> 4;
+  TileFrag f;
 #pragma unroll
-  for (int l = 0; l < kS; ++l) s += (ta ? a[l * kS + i] : a[i * kS + l]) * b[l * kS + k];
-  return s;
+  for (int q = 0; q < 4; ++q) f.v[q] = TRANS ? M[(4 * q + kk) * kS + r] : M[r * kS + 4 * q + kk];
+  return f;
+}
+__device__ __forceinline__ TileFrag tile_b(const double *M) {
+  const int l = threadIdx.x & 63, c = l & 15, kk = l >> 4;
+  TileFrag f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) f.v[q] = M[(4 * q + kk) * kS + c];
+  return f;
+}
+__device__ __forceinline__ f64x4 tile_load(const double *M) {
+  const int l = threadIdx.x & 63, c = l & 15, kk = l >> 4;
+  f64x4 a;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) a[r] = M[(kk + 4 * r) * kS + c];
+  return a;
+}
+__device__ __forceinline__ void tile_store(double *M, f64x4 a) {
+  const int l = threadIdx.x & 63, c = l & 15, kk = l >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) M[(kk + 4 * r) * kS + c] = a[r];
+}
+// acc + a b
+__device__ __forceinline__ f64x4 tile_mm(f64x4 acc, const TileFrag &a, const TileFrag &b) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a.v[q], b.v[q], acc, 0, 0, 0);
+  return acc;
 }
 
 // At step j the slots hold V_0..V_{j-1} (final), U_j = W1_{j-1} P^-1 (the
@@ -528,100 +559,136 @@ __device__ __forceinline__ double tdot(const double *a, const double *b, bool ta
 //   U_{j+1} = W M - sum_{k<=j} V_k D_k,  M = T^-1 P'^-1,  D_k = (G_k T^-1 + h_k) P'^-1
 // and (C, P) <- (h, P').  The update coefficients go to cV (V_j over slots
 // 0..j) and cU (U_{j+1} over slots 0..j+1).  FINAL (j = m): only T and column
-// m-1.  Work tiles: wk[0..7] scalars-like tiles, then G_k, p_j and h_k.
-constexpr int kWkTiles = 8 + 3 * (kMaxM + 2);
+// m-1.
+//
+// One block of 16 waves; wave 0 factorises while wave k + 1 (then k) carries
+// row k of the tile columns, so a phase costs a few dependent products and
+// one round trip through the L2, and the two Cholesky chains bound the step
+// (a mean of 44 us over the 12 steps of a cycle; one element per thread and one
+// tile after the other took 160 us).  Sums run over the
+// tiles in ascending order.
+// Work tiles (wk): S, T, T^-1, P', P'^-1, Q, two scratch, then G_k, p_j, h_k
+// and the per-row contributions to Q and to sum h_k^T h_k.
+constexpr int kWkRows = kMaxM + 2;
+constexpr int kWkTiles = 8 + 5 * kWkRows + 1;
+constexpr int kTileWaves = 16;
+static_assert(kMaxM <= kTileWaves, "one wave per basis block");
 template <bool FINAL>
-__global__ __launch_bounds__(256) void k_bdcgs_tiles(const double *__restrict__ G, const double *__restrict__ G2,
-                                                     double *__restrict__ Hbar, int m, int j, double *__restrict__ Cp,
-                                                     double *__restrict__ Pp, double *__restrict__ S0,
-                                                     double *__restrict__ cV, double *__restrict__ cU,
-                                                     double *__restrict__ wk, int *__restrict__ flag) {
+__global__ __launch_bounds__(64 * kTileWaves) void k_bdcgs_tiles(const double *__restrict__ G,
+                                                                 const double *__restrict__ G2, double *Hbar, int m,
+                                                                 int j, double *Cp, double *Pp, double *S0, double *cV,
+                                                                 double *cU, double *wk, int *flag) {
   __shared__ CholLds sh;
-  const int e = threadIdx.x;
+  const int wave = threadIdx.x >> 6;
   double *S = wk, *T = wk + kTile, *Ti = wk + 2 * kTile, *Pn = wk + 3 * kTile, *Pi = wk + 4 * kTile;
-  double *tmp = wk + 6 * kTile, *tmp2 = wk + 7 * kTile;
-  double *Gk = wk + 8 * kTile, *pj = Gk + (size_t)(kMaxM + 2) * kTile, *hk = pj + kTile;
+  double *Q = wk + 5 * kTile, *tmp = wk + 6 * kTile, *tmp2 = wk + 7 * kTile;
+  double *Gk = wk + 8 * kTile, *pj = Gk + kWkRows * kTile, *hk = pj + kTile, *qk = hk + kWkRows * kTile,
+         *hh = qk + kWkRows * kTile, *Ek = hh + kWkRows * kTile;
   auto At = [&](int b) { return G + (size_t)b * kTile; };
   auto Bt = [&](int b) { return G2 + (size_t)b * kTile; };
   auto Ht = [&](int r, int c) { return Hbar + ((size_t)r * m + c) * kTile; };
-  // T^T T = alpha - sum A_b^T A_b
-  {
-    double sv = At(j)[e];
-    for (int b = 0; b < j; ++b) sv -= tdot(At(b), At(b), true);
-    S[e] = sv;
+  const f64x4 zero = (f64x4){0.0, 0.0, 0.0, 0.0};
+  auto neg = [](TileFrag f) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) f.v[q] = -f.v[q];
+    return f;
+  };
+  if (wave == 0) {
+    // T^T T = alpha - sum A_b^T A_b
+    f64x4 s = tile_load(At(j));
+    for (int b = 0; b < j; ++b) s = tile_mm(s, neg(tile_a<true>(At(b))), tile_b(At(b)));
+    tile_store(S, s);
+  } else {
+    // row k < j: column j-1 of H (C_k + A_k P), then G_k = sum_{c<j} H_kc A_c
+    // (H_kc = 0 for k > c + 1)
+    for (int k = wave - 1; k < j; k += kTileWaves - 1) {
+      const f64x4 h = tile_mm(tile_load(Cp + (size_t)k * kTile), tile_a(At(k)), tile_b(Pp));
+      tile_store(Ht(k, j - 1), h);
+      if (FINAL) continue;
+      f64x4 g = zero;
+      for (int c = k > 0 ? k - 1 : 0; c < j - 1; ++c) g = tile_mm(g, tile_a(Ht(k, c)), tile_b(At(c)));
+      tile_store(Gk + (size_t)k * kTile, g);
+    }
+    if (!FINAL && wave == kTileWaves - 1) {
+      f64x4 s = tile_load(Bt(j));
+      for (int b = 0; b < j; ++b) s = tile_mm(s, neg(tile_a<true>(At(b))), tile_b(Bt(b)));
+      tile_store(tmp, s);
+    }
   }
   __syncthreads();
   chol16(S, T, Ti, flag, sh);
+  // the newest column's term of G_k, read back through the L2 meanwhile
+  if (!FINAL && wave > 0)
+    for (int k = wave - 1; k < j; k += kTileWaves - 1) {
+      double *g = Gk + (size_t)k * kTile;
+      tile_store(g, tile_mm(tile_load(g), tile_a(Ht(k, j - 1)), tile_b(At(j - 1))));
+    }
   __syncthreads();
-  if (j >= 1) {
-    for (int b = 0; b < j; ++b) Ht(b, j - 1)[e] = Cp[(size_t)b * kTile + e] + tdot(At(b), Pp, false);
-    Ht(j, j - 1)[e] = tdot(T, Pp, false);
-  } else {
-    tmp[e] = tdot(T, S0, false);
-    __syncthreads();
-    S0[e] = tmp[e];
+  if (wave == 0) {
+    if (j >= 1) {
+      tile_store(Ht(j, j - 1), tile_mm(zero, tile_a(T), tile_b(Pp)));
+    } else {
+      const f64x4 s0 = tile_mm(zero, tile_a(T), tile_b(S0));
+      tile_store(S0, s0);
+    }
   }
   if (FINAL) return;
+  if (wave == 1) tile_store(pj, tile_mm(zero, tile_a<true>(Ti), tile_b(tmp)));  // p_j = T^-T (beta - sum A_b^T B_b)
   __syncthreads();
-  // G_k = sum_{c<j} H_kc A_c (H_kc = 0 for k > c + 1)
-  for (int k = 0; k <= j; ++k) {
-    double sv = 0.0;
-    for (int c = k > 0 ? k - 1 : 0; c < j; ++c) sv += tdot(Ht(k, c), At(c), false);
-    Gk[(size_t)k * kTile + e] = sv;
-  }
-  // p_j = T^-T (beta - sum A_b^T B_b)
-  {
-    double sv = Bt(j)[e];
-    for (int b = 0; b < j; ++b) sv -= tdot(At(b), Bt(b), true);
-    tmp[e] = sv;
-  }
+  if (wave == 0)
+    tile_store(Gk + (size_t)j * kTile, j >= 1 ? tile_mm(zero, tile_a(Ht(j, j - 1)), tile_b(At(j - 1))) : zero);
   __syncthreads();
-  pj[e] = tdot(Ti, tmp, true);
-  __syncthreads();
-  auto pk = [&](int k) { return k < j ? Bt(k) : pj; };
-  // h_k = (p_k - G_k) T^-1, and Q = gamma - sum (G_k^T p_k + p_k^T G_k - G_k^T G_k)
-  {
-    double q = Bt(j + 1)[e];
-    for (int k = 0; k <= j; ++k) {
-      const double *g = Gk + (size_t)k * kTile, *pp = pk(k);
-      q -= tdot(g, pp, true) + tdot(pp, g, true) - tdot(g, g, true);
-    }
-    tmp[e] = q;
-  }
-  for (int k = 0; k <= j; ++k) {
-    const double *g = Gk + (size_t)k * kTile, *pp = pk(k);
-    const int i = e / kS, c = e % kS;
-    double sv = 0.0;
+  // row k <= j: h_k = (p_k - G_k) T^-1, its part of Q = gamma - sum (G_k^T p_k
+  // + p_k^T G_k - G_k^T G_k) and of sum h_k^T h_k, and E_k = G_k T^-1 + h_k
+  if (wave <= j) {
+    const double *g = Gk + (size_t)wave * kTile, *p = wave < j ? Bt(wave) : pj;
+    double *h = hk + (size_t)wave * kTile;
+    const TileFrag ti = tile_b(Ti), ga = tile_a(g);
+    TileFrag d = tile_a(p);
 #pragma unroll
-    for (int l = 0; l < kS; ++l) sv += (pp[i * kS + l] - g[i * kS + l]) * Ti[l * kS + c];
-    hk[(size_t)k * kTile + e] = sv;
+    for (int q = 0; q < 4; ++q) d.v[q] -= ga.v[q];
+    const f64x4 hv = tile_mm(zero, d, ti);
+    tile_store(h, hv);
+    tile_store(Ek + (size_t)wave * kTile, tile_mm(hv, ga, ti));
+    const TileFrag gt = tile_a<true>(g), pt = tile_a<true>(p), gb = tile_b(g), pb = tile_b(p);
+    tile_store(qk + (size_t)wave * kTile, tile_mm(tile_mm(tile_mm(zero, gt, pb), pt, gb), neg(gt), gb));
+    if (wave < j) {
+      TileFrag a = tile_a(At(wave));
+      tile_store(cV + (size_t)wave * kTile, tile_mm(zero, neg(a), ti));  // V_j = U_j T^-1 - sum V_b (A_b T^-1)
+    } else {
+      tile_store(cV + (size_t)j * kTile, tile_load(Ti));
+    }
+  }
+  __syncthreads();
+  if (wave <= j) {
+    const double *h = hk + (size_t)wave * kTile;
+    tile_store(hh + (size_t)wave * kTile, tile_mm(zero, tile_a<true>(h), tile_b(h)));
+    tile_store(Cp + (size_t)wave * kTile, tile_load(h));  // C <- h
+  }
+  if (threadIdx.x < kTile) {
+    double q = Bt(j + 1)[threadIdx.x];
+    for (int k = 0; k <= j; ++k) q -= qk[(size_t)k * kTile + threadIdx.x];
+    Q[threadIdx.x] = q;
   }
   __syncthreads();
   // Gram = T^-T Q T^-1 - sum h_k^T h_k
-  tmp2[e] = tdot(tmp, Ti, false);
-  __syncthreads();
-  {
-    double sv = tdot(Ti, tmp2, true);
-    for (int k = 0; k <= j; ++k) sv -= tdot(hk + (size_t)k * kTile, hk + (size_t)k * kTile, true);
-    S[e] = sv;
+  if (wave == 0) tile_store(tmp2, tile_mm(zero, tile_a(Q), tile_b(Ti)));
+  if (wave >= 4 && wave < 8) {
+    const int e = threadIdx.x - 256;
+    double s = 0.0;
+    for (int k = 0; k <= j; ++k) s += hh[(size_t)k * kTile + e];
+    tmp[e] = -s;
   }
+  __syncthreads();
+  if (wave == 0) tile_store(S, tile_mm(tile_load(tmp), tile_a<true>(Ti), tile_b(tmp2)));
   __syncthreads();
   chol16(S, Pn, Pi, flag, sh);
   __syncthreads();
-  // M = T^-1 P'^-1 -> cU[j+1]; D_k = (G_k T^-1 + h_k) P'^-1 -> cU[k] = -D_k
-  cU[(size_t)(j + 1) * kTile + e] = tdot(Ti, Pi, false);
-  for (int k = 0; k <= j; ++k) {
-    tmp[e] = tdot(Gk + (size_t)k * kTile, Ti, false) + hk[(size_t)k * kTile + e];
-    __syncthreads();
-    cU[(size_t)k * kTile + e] = -tdot(tmp, Pi, false);
-    __syncthreads();
-  }
-  // V_j = U_j T^-1 - sum V_b (A_b T^-1)
-  for (int b = 0; b < j; ++b) cV[(size_t)b * kTile + e] = -tdot(At(b), Ti, false);
-  cV[(size_t)j * kTile + e] = Ti[e];
-  // (C, P) <- (h, P')
-  for (int k = 0; k <= j; ++k) Cp[(size_t)k * kTile + e] = hk[(size_t)k * kTile + e];
-  Pp[e] = Pn[e];
+  // M = T^-1 P'^-1 -> cU[j+1]; D_k = E_k P'^-1 -> cU[k] = -D_k; P <- P'
+  if (wave <= j) tile_store(cU + (size_t)wave * kTile, tile_mm(zero, neg(tile_a(Ek + (size_t)wave * kTile)), tile_b(Pi)));
+  if (wave == (j + 1) % kTileWaves)
+    tile_store(cU + (size_t)(j + 1) * kTile, tile_mm(zero, tile_a(Ti), tile_b(Pi)));
+  if (threadIdx.x < kTile) Pp[threadIdx.x] = Pn[threadIdx.x];
 }
 
 // Y[:, c] = X[:, c] / d_c with d_c = sqrt(nrm2[c]) (1 for a zero column)
@@ -846,13 +913,13 @@ void enqueue_cycle(aerofx_ctx *c, BlockSolver *s, int prec) {
     else
       apply_ops64(c, s, Uj, Wn);
     tsg_dots(s, j + 2, s->V, Uj, s->G, Wn, s->G2);
-    hipLaunchKernelGGL((k_bdcgs_tiles<false>), dim3(1), dim3(256), 0, s->stream, s->G, s->G2, s->Hbar, s->m, j, s->Cp,
+    hipLaunchKernelGGL((k_bdcgs_tiles<false>), dim3(1), dim3(64 * kTileWaves), 0, s->stream, s->G, s->G2, s->Hbar, s->m, j, s->Cp,
                        s->Pp, s->S0, s->cV, s->cU, s->wk, s->flag);
     tsg_update2(s, j);
   }
   // the last block's reorthogonalisation completes column m-1
   tsg_dots(s, s->m + 1, s->V, s->V + (size_t)s->m * blk, s->G);
-  hipLaunchKernelGGL((k_bdcgs_tiles<true>), dim3(1), dim3(256), 0, s->stream, s->G, s->G2, s->Hbar, s->m, s->m, s->Cp,
+  hipLaunchKernelGGL((k_bdcgs_tiles<true>), dim3(1), dim3(64 * kTileWaves), 0, s->stream, s->G, s->G2, s->Hbar, s->m, s->m, s->Cp,
                      s->Pp, s->S0, s->cV, s->cU, s->wk, s->flag);
 }
 
