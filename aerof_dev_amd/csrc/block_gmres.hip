@@ -27,8 +27,8 @@
 // Gram-Schmidt and update stay FP64.
 //
 // Determinism: V^T W is summed over a fixed split of the rows into chunks
-// (one wave per chunk, rows in order), and the chunk partials in a fixed
-// tree, so the tuned launch shape changes which unit does the work, not the
+// (four waves per chunk, added in wave order), and the chunk partials in a
+// fixed tree, so the tuned launch shape changes which unit does the work, not the
 // arithmetic.  The autotuner times each candidate shape once per context
 // and keeps the fastest.
 #include <hip/hip_runtime.h>
@@ -230,25 +230,32 @@ __global__ void k_f64_to_f32(size_t len, const double *__restrict__ a, float *__
 // ---------------------------------------------------------------------------
 // tall-skinny GEMMs on the FP64 matrix cores
 // ---------------------------------------------------------------------------
-// partial[c][b] = sum over the rows of chunk c of V_b^T W (16x16 tiles).
+// partial[c][b] = sum over the rows of chunk c of V_b^T W (16x16 tiles), one
+// chunk per workgroup of four waves.
 // v_mfma_f64_16x16x4f64: lane l supplies A[l%16][l/16] and B[l/16][l%16] and
 // holds D[l/16 + 4r][l%16], r < 4 (checked on gfx950).  Here A = V_b^T over 4 rows, B = W over
 // the same rows: both are the 4x16 row slab [k0 + l/16][l%16].
 // With TWO, the same sweep also forms V_b^T W2 into partial2 (one read of
 // the V_b for two right-hand blocks).  NBMAX (>= nb) sizes the accumulators:
-// fewer registers, more waves per SIMD for the early steps of a cycle.  The
-// 12-block instance fits 254 VGPRs with no accumulation registers when asked
-// for two waves per SIMD (it used 254 + 16, one wave): 16-RHS mixed solve at
-// 128^3 3.92 -> 3.76 s.  The 17-block one would spill.
+// fewer registers, more waves per SIMD for the early steps of a cycle (up to
+// 12 blocks two waves per SIMD without spilling, 17 one).
+//
+// Memory-bound (a sweep reads each slot once); what it needs is loads in
+// flight.  The waves of a workgroup take every fourth 16-row group of the
+// chunk and their tiles are added through LDS in wave order, so the number of
+// waves does not set the number of partial tiles: kDotsChunks workgroups are
+// two per CU at two waves per SIMD.  (One wave per chunk of 512 rows left 686
+// waves for the 1024 SIMDs at 351k rows and read 1.9 TB/s.)
+constexpr int kDotsChunks = 512;
 template <bool TWO, int NBMAX>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBMAX == 12 ? 2 : 1))) void k_tsg_dots(size_t npad, size_t rows_per_chunk, int nchunks, int mp1, int nb,
-                           const double *__restrict__ V, size_t ldv, const double *__restrict__ W,
-                           const double *__restrict__ W2, double *__restrict__ partial,
-                           double *__restrict__ partial2) {
-  const int lane = threadIdx.x & 63;
-  const int chunk = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (chunk >= nchunks) return;
-  const size_t r0 = (size_t)chunk * rows_per_chunk;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBMAX <= 12 ? 2 : 1))) void k_tsg_dots(
+    size_t npad, size_t rows_per_chunk, int mp1, int nb, const double *__restrict__ V, size_t ldv,
+    const double *__restrict__ W, const double *__restrict__ W2, double *__restrict__ partial,
+    double *__restrict__ partial2) {
+  constexpr int NS = TWO ? 2 : 1, BB = 4;  // BB slots per LDS round
+  __shared__ double sh[4][BB * NS][kTile];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const size_t r0 = (size_t)blockIdx.x * rows_per_chunk;
   const size_t r1 = min(npad, r0 + rows_per_chunk);
   f64x4 acc[NBMAX], acc2[TWO ? NBMAX : 1];
 #pragma unroll
@@ -258,9 +265,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBMAX == 12
     for (int b = 0; b < NBMAX; ++b) acc2[TWO ? b : 0] = (f64x4){0.0, 0.0, 0.0, 0.0};
   }
   const int rr = lane >> 4, cc = lane & 15;
-  // rows_per_chunk is a multiple of 16: four MFMA steps per iteration, their
-  // loads issued together
-  for (size_t k0 = r0; k0 < r1; k0 += 16) {
+  // npad and rows_per_chunk are multiples of 64: four MFMA steps per
+  // iteration, their loads issued together
+  for (size_t k0 = r0 + 16 * wave; k0 < r1; k0 += 64) {
     double w[4], w2[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -280,40 +287,52 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBMAX == 12
         }
       }
   }
+  const int e = threadIdx.x;  // output element e = r * 64 + lane of a tile
+  const int pos = ((e & 63) / kS + 4 * (e >> 6)) * kS + (e & (kS - 1));
 #pragma unroll
-  for (int b = 0; b < NBMAX; ++b)
-    if (b < nb) {
-      double *dst = partial + ((size_t)chunk * mp1 + b) * kTile;
+  for (int b0 = 0; b0 < NBMAX; b0 += BB) {
+    if (b0 >= nb) break;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) dst[(rr + 4 * r) * kS + cc] = acc[b][r];
-      if (TWO) {
-        double *dst2 = partial2 + ((size_t)chunk * mp1 + b) * kTile;
+    for (int b = b0; b < b0 + BB && b < NBMAX; ++b)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) dst2[(rr + 4 * r) * kS + cc] = acc2[TWO ? b : 0][r];
+      for (int r = 0; r < 4; ++r) {
+        sh[wave][(b - b0) * NS][r * 64 + lane] = acc[b][r];
+        if (TWO) sh[wave][(b - b0) * NS + NS - 1][r * 64 + lane] = acc2[TWO ? b : 0][r];
       }
+    __syncthreads();
+    for (int b = b0; b < b0 + BB && b < nb; ++b) {
+      const size_t dst = ((size_t)blockIdx.x * mp1 + b) * kTile + pos;
+      const int q = (b - b0) * NS;
+      partial[dst] = ((sh[0][q][e] + sh[1][q][e]) + sh[2][q][e]) + sh[3][q][e];
+      if (TWO) partial2[dst] = ((sh[0][q + NS - 1][e] + sh[1][q + NS - 1][e]) + sh[2][q + NS - 1][e]) + sh[3][q + NS - 1][e];
     }
+    __syncthreads();
+  }
 }
 
-// Two-level fixed-order reduction of the chunk partials.  Level 1: block
-// (b, g) sums chunks [g*nc/G, (g+1)*nc/G) of tile b into part2[g][b] (lane e
-// owns element e); level 2: one block per tile sums the G group sums.
-constexpr int kRedGroups = 64;
-__global__ __launch_bounds__(256) void k_tsg_reduce1(const double *__restrict__ partial, int nchunks, int mp1,
-                                                     double *__restrict__ part2) {
-  const int b = blockIdx.x, g = blockIdx.y, e = threadIdx.x;
-  const int per = (nchunks + kRedGroups - 1) / kRedGroups;
-  const int c0 = g * per, c1 = min(nchunks, c0 + per);
+// out[b] = sum of the chunk partials of tile b (blockIdx.z = 1: partial2 ->
+// out2) in a fixed order: a block takes 32 elements of one tile, 32 groups of
+// lanes add equal runs of chunks in order, then the groups are added in order.
+// One launch for both sets (two launches per set before: 26 us a step).
+__global__ __launch_bounds__(1024) void k_tsg_reduce(const double *__restrict__ partial,
+                                                     const double *__restrict__ partial2, int nchunks, int mp1,
+                                                     double *__restrict__ out, double *__restrict__ out2) {
+  __shared__ double sh[32][32];
+  const int el = threadIdx.x & 31, g = threadIdx.x >> 5, b = blockIdx.x, e = blockIdx.y * 32 + el;
+  const double *src = blockIdx.z ? partial2 : partial;
+  const int per = (nchunks + 31) / 32;
+  const int c0 = min(nchunks, g * per), c1 = min(nchunks, c0 + per);
   double s = 0.0;
-  for (int c = c0; c < c1; ++c) s += partial[((size_t)c * mp1 + b) * kTile + e];
-  part2[((size_t)g * mp1 + b) * kTile + e] = s;
-}
-
-__global__ __launch_bounds__(256) void k_tsg_reduce2(const double *__restrict__ part2, int mp1,
-                                                     double *__restrict__ out) {
-  const int b = blockIdx.x, e = threadIdx.x;
-  double s = 0.0;
-  for (int g = 0; g < kRedGroups; ++g) s += part2[((size_t)g * mp1 + b) * kTile + e];
-  out[(size_t)b * kTile + e] = s;
+#pragma unroll 8
+  for (int c = c0; c < c1; ++c) s += src[((size_t)c * mp1 + b) * kTile + e];
+  sh[g][el] = s;
+  __syncthreads();
+  if (g == 0) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) t += sh[k][el];
+    (blockIdx.z ? out2 : out)[(size_t)b * kTile + e] = t;
+  }
 }
 
 // Out = beta Out + alpha sum_b V_b H_b over 16-row tiles, one wave per tile.
@@ -742,7 +761,7 @@ __global__ void k_colnorm_reduce(const double *__restrict__ partial, double *__r
 // host side
 // ---------------------------------------------------------------------------
 struct TsgShape {
-  int waves_dots = 4;    // waves per workgroup of k_tsg_dots
+  int waves_dots = 4;    // waves per workgroup of k_tsg_dots (fixed: they share LDS)
   int waves_update = 4;  // waves per workgroup of k_tsg_update
   bool tuned = false;
 };
@@ -752,10 +771,10 @@ struct BlockSolver {
   size_t n = 0, npad = 0;
   double *V = nullptr;        // [m+1][npad][16]
   double *W = nullptr, *Z = nullptr, *R = nullptr, *X = nullptr, *B = nullptr, *T = nullptr;
-  int nchunks = 0;            // row split of V^T W (fixed by npad)
+  int nchunks = 0;            // row split of V^T W (fixed by npad): chunks and
+  size_t chunk_rows = 0;      // rows of each, a multiple of 64
   double *partial = nullptr;  // [nchunks][m+1][256]
   double *partial2 = nullptr; // [nchunks][m+1][256], second right-hand block of a fused sweep
-  double *part2 = nullptr;    // [kRedGroups][m+1][256]
   double *Hbar = nullptr;     // [(m+1)][m] tiles: block (i, j) at (i * m + j)
   double *S0 = nullptr;       // tile
   double *G = nullptr;        // scratch tiles [kMaxM+1]
@@ -803,12 +822,9 @@ BlockSolver *get_block(aerofx_ctx *c, int m, int *rc);
 // out[b] = V_b^T W (and out2[b] = V_b^T W2 when W2 is given), b < nb
 void tsg_dots(BlockSolver *s, int nb, const double *V, const double *W, double *out, const double *W2 = nullptr,
               double *out2 = nullptr) {
-  // rows per chunk: a multiple of 16 (four MFMA steps), fixed by npad alone
-  const size_t rows = std::max<size_t>(16, ((s->npad + s->nchunks - 1) / s->nchunks + 15) / 16 * 16);
-  const int wpb = s->shape.waves_dots;
-  const dim3 grid((s->nchunks + wpb - 1) / wpb), block(64 * wpb);
+  const dim3 grid(s->nchunks), block(256);
 #define TSG_DOTS(TWO, NBM)                                                                                     \
-  hipLaunchKernelGGL((k_tsg_dots<TWO, NBM>), grid, block, 0, s->stream, s->npad, rows, s->nchunks, s->m + 1, nb, V, \
+  hipLaunchKernelGGL((k_tsg_dots<TWO, NBM>), grid, block, 0, s->stream, s->npad, s->chunk_rows, s->m + 1, nb, V, \
                      s->npad * kS, W, W2, s->partial, s->partial2)
   if (W2) {
     if (nb <= 4) TSG_DOTS(true, 4);
@@ -822,14 +838,8 @@ void tsg_dots(BlockSolver *s, int nb, const double *V, const double *W, double *
     else TSG_DOTS(false, kMaxM + 1);
   }
 #undef TSG_DOTS
-  hipLaunchKernelGGL(k_tsg_reduce1, dim3(nb, kRedGroups), dim3(256), 0, s->stream, s->partial, s->nchunks, s->m + 1,
-                     s->part2);
-  hipLaunchKernelGGL(k_tsg_reduce2, dim3(nb), dim3(256), 0, s->stream, s->part2, s->m + 1, out);
-  if (W2) {
-    hipLaunchKernelGGL(k_tsg_reduce1, dim3(nb, kRedGroups), dim3(256), 0, s->stream, s->partial2, s->nchunks,
-                       s->m + 1, s->part2);
-    hipLaunchKernelGGL(k_tsg_reduce2, dim3(nb), dim3(256), 0, s->stream, s->part2, s->m + 1, out2);
-  }
+  hipLaunchKernelGGL(k_tsg_reduce, dim3(nb, kTile / 32, W2 ? 2 : 1), dim3(1024), 0, s->stream, s->partial,
+                     s->partial2, s->nchunks, s->m + 1, out, out2);
 }
 
 // the step's two in-place updates (V_j, U_{j+1}) in one sweep
@@ -972,19 +982,16 @@ void host_lsq(int m, const std::vector<double> &Ht, const std::vector<double> &S
   }
 }
 
-// times each candidate launch shape on the current buffers; keeps the fastest
-// Times the candidate waves per workgroup of the two sweeps a step runs (the
-// two-right-hand-block Gram sweep and the fused update) at a mid-cycle
-// width; each candidate is timed twice over three launches and its best is
-// kept, so one noisy measurement does not decide.
+// Times the candidate waves per workgroup of the fused update sweep at a
+// mid-cycle width on the current buffers; each candidate is timed twice over
+// three launches and its best is kept, so one noisy measurement does not
+// decide.
 void autotune(aerofx_ctx *c, BlockSolver *s) {
   if (s->shape.tuned) return;
   hipEvent_t a, b;
   (void)hipEventCreate(&a);
   (void)hipEventCreate(&b);
   const int j = std::min(s->m, 8) - 1;  // step whose sweeps are timed
-  const size_t blk = s->npad * kS;
-  double *U = s->V + (size_t)j * blk, *W = s->V + (size_t)(j + 1) * blk;
   // defined coefficients for the update's timing runs (the slots are
   // rewritten by every cycle before they are read)
   (void)hipMemsetAsync(s->cV, 0, (size_t)(kMaxM + 2) * kTile * sizeof(double), s->stream);
@@ -999,27 +1006,17 @@ void autotune(aerofx_ctx *c, BlockSolver *s) {
     (void)hipEventElapsedTime(&ms, a, b);
     return ms;
   };
-  const int cand[] = {1, 2, 4};  // waves per workgroup (<= 256 threads)
-  float best[4] = {1e30f, 1e30f, 1e30f, 1e30f};
-  for (int pass = 0; pass < 2; ++pass)
-    for (int k = 0; k < 3; ++k) {
-      s->shape.waves_dots = cand[k];
-      best[k] = std::min(best[k], time3([&] { tsg_dots(s, j + 2, s->V, U, s->G, W, s->G2); }));
-    }
-  int kb = 0;
-  for (int k = 1; k < 3; ++k)
-    if (best[k] < best[kb]) kb = k;
-  c->blk_tune[0] = s->shape.waves_dots = cand[kb];
   const int cand_u[] = {1, 2, 4, 8};
-  for (float &x : best) x = 1e30f;
+  float best[4] = {1e30f, 1e30f, 1e30f, 1e30f};
   for (int pass = 0; pass < 2; ++pass)
     for (int k = 0; k < 4; ++k) {
       s->shape.waves_update = cand_u[k];
       best[k] = std::min(best[k], time3([&] { tsg_update2(s, j); }));
     }
-  kb = 0;
+  int kb = 0;
   for (int k = 1; k < 4; ++k)
     if (best[k] < best[kb]) kb = k;
+  c->blk_tune[0] = s->shape.waves_dots;
   c->blk_tune[1] = s->shape.waves_update = cand_u[kb];
   s->shape.tuned = true;
   (void)hipEventDestroy(a);
@@ -1034,15 +1031,14 @@ BlockSolver *get_block(aerofx_ctx *c, int m, int *rc) {
   s->m = m;
   s->n = 5 * (size_t)c->N;
   s->npad = (s->n + 63) / 64 * 64;  // also a multiple of 16 rows: whole MFMA row groups
-  // about 512 rows per wave of V^T W, between 64 and 8192 chunks
-  s->nchunks = (int)std::min<size_t>(8192, std::max<size_t>(64, s->npad / 512));
+  s->chunk_rows = ((s->npad + kDotsChunks - 1) / kDotsChunks + 63) / 64 * 64;
+  s->nchunks = (int)((s->npad + s->chunk_rows - 1) / s->chunk_rows);
   const size_t blk = s->npad * kS;
   int r = 0;
   if ((r = alloc_d(c, (size_t)(m + 1) * blk, &s->V)) || (r = alloc_d(c, blk, &s->W)) || (r = alloc_d(c, blk, &s->Z)) ||
       (r = alloc_d(c, blk, &s->R)) || (r = alloc_d(c, blk, &s->X)) || (r = alloc_d(c, blk, &s->B)) ||
       (r = alloc_d(c, blk, &s->T)) || (r = alloc_d(c, (size_t)s->nchunks * (m + 1) * kTile, &s->partial)) ||
       (r = alloc_d(c, (size_t)s->nchunks * (m + 1) * kTile, &s->partial2)) ||
-      (r = alloc_d(c, (size_t)kRedGroups * (m + 1) * kTile, &s->part2)) ||
       (r = alloc_d(c, (size_t)(m + 1) * m * kTile, &s->Hbar)) || (r = alloc_d(c, kTile, &s->S0)) ||
       (r = alloc_d(c, (size_t)(kMaxM + 1) * kTile, &s->G)) || (r = alloc_d(c, (size_t)(kMaxM + 1) * kTile, &s->G2)) ||
       (r = alloc_d(c, kTile, &s->Rt)) || (r = alloc_d(c, kTile, &s->Ri)) || (r = alloc_d(c, kTile, &s->Rt2)) ||
