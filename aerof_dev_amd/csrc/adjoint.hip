@@ -361,8 +361,8 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
   const double ici = t.invcv[i], icj = t.invcv[j];
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
-    Vi[k] = V[5 * (size_t)i + k];
-    Vj[k] = V[5 * (size_t)j + k];
+    Vi[k] = V[il<5>(i, k)];
+    Vj[k] = V[il<5>(j, k)];
     g[k] = lam[5 * (size_t)i + k] * ici - lam[5 * (size_t)j + k] * icj;
   }
   double dx[3] = {0.0, 0.0, 0.0}, gi[15], gj[15];
@@ -373,11 +373,8 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
     dx[0] = xj.x - xi.x;
     dx[1] = xj.y - xi.y;
     dx[2] = xj.z - xi.z;
-#pragma unroll
-    for (int q = 0; q < 15; ++q) {
-      gi[q] = grad[16 * (size_t)i + q];
-      gj[q] = grad[16 * (size_t)j + q];
-    }
+    load_il<15>(grad, i, gi);
+    load_il<15>(grad, j, gj);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       const double ddVij = dx[0] * gi[k] + dx[1] * gi[5 + k] + dx[2] * gi[10 + k];
@@ -530,7 +527,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       mu[k] = lam[5 * (size_t)n + k] * ic;
-      Vn[k] = V[5 * (size_t)n + k];
+      Vn[k] = V[il<5>(n, k)];
     }
     for (int q = f0; q < f1; ++q) {
       const int face = t.fidx[q];
@@ -573,7 +570,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
     vb[k] = Vb[5 * (size_t)n + k];
-    Vn[k] = V[5 * (size_t)n + k];
+    Vn[k] = V[il<5>(n, k)];
   }
   if (second) {
     double Ln[6], gn[15];
@@ -593,8 +590,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double
       for (int q = 0; q < 6; ++q) Lm[q] = t.lsq6[6 * (size_t)m + q];
 #pragma unroll
       for (int q = 0; q < 15; ++q) gm[q] = Gb[16 * (size_t)m + q];
-#pragma unroll
-      for (int k = 0; k < 5; ++k) Vm[k] = V[5 * (size_t)m + k];
+      load_il<5>(V, m, Vm);
       double wn[3], wm[3];
       lsq_weights(Ln, dx0, dx1, dx2, wn);      // row n, neighbour m
       lsq_weights(Lm, -dx0, -dx1, -dx2, wm);   // row m, neighbour n (dx_mn = X_n - X_m)
@@ -784,7 +780,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_faces(int F, const int *__res
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       mu[k] = lam[5 * (size_t)n + k] * ic;
-      vv[k] = Dual(V[5 * (size_t)n + k]);
+      vv[k] = Dual(V[il<5>(n, k)]);
     }
 #pragma unroll 1
     for (int dir = 0; dir < 3; ++dir) {
@@ -1052,7 +1048,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_lift_faces(int F, const int *__re
 #pragma unroll
   for (int v = 0; v < 3; ++v) {
     nd[v] = faces[3 * (size_t)f + v];
-    psum += V[5 * (size_t)nd[v] + 4];
+    psum += V[il<5>(nd[v], 4)];
   }
   if (!wall) psum = 0.0;
   const double *nv = fnorm3 + 3 * (size_t)f;
@@ -1163,7 +1159,7 @@ extern "C" int aerofx_wall_force(aerofx_ctx *ctx, const double *U, const double 
   if (rc) return rc;
   Adjoint *a = ctx->adj;
   const DevTables &t = ctx->tab;
-  if ((rc = launch_primitive(ctx, U, ctx->d_V))) return rc;
+  if ((rc = launch_primitive_il(ctx, U))) return rc;
   if (ctx->F > 0) {
     hipLaunchKernelGGL(k_lift_faces, grid_for(ctx->F), dim3(kAdjBlock), 0, ctx->stream, ctx->F, a->faces, t.fcode,
                        t.fnorm3, t.X4, ctx->d_V, dir[0], dir[1], dir[2], a->Jf, dJdX ? a->FX : nullptr);

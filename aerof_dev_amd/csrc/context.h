@@ -15,13 +15,9 @@ namespace aerofx {
 constexpr int kBlock = 256;       // threads per block of the edge/entry kernels
 constexpr int kMaxRows = 64;      // node rows per block (LDS staging bound)
 constexpr int kNumXcd = 8;        // MI355X: 8 XCDs, blocks dealt round-robin
+constexpr int kNumCu = 256;
+constexpr size_t kLdsPerCu = 160 * 1024;
 constexpr int kPad = kBlock + 1;  // LDS row stride (odd: conflict-free)
-// threads (= edges) per block of the flux pass; also the largest number of
-// upper edges one node may have (measured at 128^3: 256 -> 0.645 ms,
-// 128 -> 0.629 ms, 64 -> 0.618 ms for the edge-flux kernel).  A mesh whose
-// nodes all have at most kFluxBlockSmall upper edges gets the small blocks.
-constexpr int kFluxBlock = 128;
-constexpr int kFluxBlockSmall = 64;
 // LDS-staged residual passes: strips of consecutive nodes (gradients) or
 // rows (fluxes) whose touched nodes are loaded into LDS once per block.
 //   gradient strip: <= kGradStrip nodes (one lane each), <= kGradHalo staged
@@ -55,11 +51,71 @@ __host__ __device__ inline size_t blk64_base(size_t e) { return (e >> 6) * (64 *
 constexpr int kBlkStride = 64;
 inline size_t blk64_count(size_t nblocks) { return (nblocks + 63) / 64 * 64 * 25; }
 
+// Node and edge data of W doubles per item that the passes gather (primitive
+// state, gradients, coordinates, fluxes): groups of 64 items, the fields of a
+// group in planes of two (the last of an odd W alone), so a lane loads 16 B
+// and 64 lanes reading neighbouring items touch a contiguous piece of each
+// plane.  The vector cache takes one access per clock, each up to 64 B of four
+// consecutive lanes: with records of 40 to 128 B a gather costs 43 to 64
+// accesses per load and wave, which took 85 % of the flux pass's clocks; from
+// the planes it takes about 28 over the neighbours of 64 consecutive nodes in
+// RCM order (flux and node pass at 2.1M nodes 864 -> 727 us).
+template <int W>
+__host__ __device__ __forceinline__ size_t il(size_t n, int k) {
+  const size_t g = (n >> 6) * (64 * W), l = n & 63;
+  return k < (W & ~1) ? g + (k >> 1) * 128 + 2 * l + (k & 1) : g + (W - 1) * 64 + l;
+}
+template <int W>
+inline size_t il_count(size_t n) {
+  return (n + 63) / 64 * 64 * W;
+}
+template <int W>
+__device__ __forceinline__ void load_il(const double *__restrict__ p, int n, double v[W]) {
+  const double *q = p + ((size_t)n >> 6) * (64 * W);
+  const int l = n & 63;
+#pragma unroll
+  for (int k = 0; k < W / 2; ++k) {
+    const double2 a = *reinterpret_cast<const double2 *>(q + k * 128 + 2 * l);
+    v[2 * k] = a.x;
+    v[2 * k + 1] = a.y;
+  }
+  if (W & 1) v[W - 1] = q[(W - 1) * 64 + l];
+}
+template <int W>
+__device__ __forceinline__ void store_il(double *__restrict__ p, int n, const double v[W]) {
+  double *q = p + ((size_t)n >> 6) * (64 * W);
+  const int l = n & 63;
+#pragma unroll
+  for (int k = 0; k < W / 2; ++k) *reinterpret_cast<double2 *>(q + k * 128 + 2 * l) = make_double2(v[2 * k], v[2 * k + 1]);
+  if (W & 1) q[(W - 1) * 64 + l] = v[W - 1];
+}
+
+// Rows of a CSR table regrouped for one wave per 64 consecutive rows (a
+// slice): entry k of all rows of slice s that have one, consecutively from
+// koff[kptr[s] + k], in row order.  Lane r finds its entry by counting the
+// lanes below it that have one, so nothing is padded whatever the degrees.
+struct RowSlices {
+  const int *kptr;  // [slices + 1] first (slice, k) pair of each slice
+  const int *koff;  // per (slice, k): its first entry
+  const int *idx;   // the entries
+};
+
+__device__ __forceinline__ int lanes_below(bool active) {
+  const unsigned long long b = __ballot(active);
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u));
+}
+
+// 64 B of LDS per halo node: five workgroups per CU at 512 nodes
+constexpr int kHaloCap = 1024;
+constexpr int kHaloRow = 64;  // bounds the padding of the places
+
 // Device-resident mesh tables.  All arrays are laid out for the kernel that
 // streams them: contiguous per node row or per edge.
 struct DevTables {
   int N, E, F;
+  int ns;                // 64-node slices
   const double *X4;      // [N][4] coordinates padded to 32 B
+  const double *X3;      // il<3>: coordinates
   const int *fs_mask;    // [N] failsafe first-order nodes (gradients zeroed), or null
   const double *lsq6;    // [N][6] (1/r11, 1/r22, 1/r33, r12/r11, r23/r22, psi)
   const double *invcv;   // [N] 1/ctrlVol
@@ -73,11 +129,23 @@ struct DevTables {
   const int *adj;        // [2E]
   const int *eidx;       // [2E] edge id of each adjacency entry
   const int *mirror;     // [2E] entry (m, n) of the entry (n, m)
-  // flux pass A: edges grouped by their lower node i (edge order)
-  int nfchunks;
-  int fblock;            // edges per flux block: kFluxBlockSmall or kFluxBlock
-  const int4 *fchunk4;   // [nfchunks] (first row, end row, first edge, end edge) of each chunk;
-                         // a row of more than fblock upper edges is cut into row-less pieces
+  // residual passes: all neighbours, upper neighbours (the edge storage order
+  // of the flux pass: an edge's position is its place in up.idx) and, per
+  // lower neighbour, the position of that edge
+  RowSlices nb, up, lo;
+  // gradient pass through LDS: the different neighbours of each slice
+  // (halo_cap per slice, in the order its entries first name them, the last
+  // repeated), and the places among them of the entries 2 p (low half) and
+  // 2 p + 1 of row r of a slice at [(slice * halo_pairs + p) * 64 + r];
+  // halo_cap = 0: a slice has more than kHaloCap or a row more than kHaloRow,
+  // the pass gathers per entry
+  int halo_cap, halo_pairs;
+  const int *halo;
+  const uint32_t *hloc;
+  int nup;               // (slice, k) pairs of up
+  const int *upslice;    // [nup] their slices
+  const int *pedge;      // [E] edge id at each position
+  const double *pnormal; // il<3> over positions: dual-face area vectors
   const int *eup;        // [N+1] first edge whose lower node is i
   const int2 *eij;       // [E] edge endpoints (i, j), i < j
 
@@ -87,6 +155,7 @@ struct DevTables {
   const int *ledge;      // [E] edges (m, n), m < n, of node n, ascending m
   const int *frow;       // [N+1] face-list pointers
   const int *fidx;       // [3F] faces touching each node, ascending
+  const int *fnode;      // [3F] node of each face slot
   const int *fcode;      // [F] boundary code
   const double *fnorm3;  // [F][3] (1/3) face normal
   const double *fnorm;   // [F][3] face normal
@@ -101,6 +170,7 @@ struct DevTables {
   const int2 *fbh;       // [nfb] (first halo entry, end halo entry)
   const int *fhalo;      // staged node ids, ascending within each strip
   const uint32_t *floc;  // [E] halo position of i | halo position of j << 16
+  const int *epos;       // [E] position of each edge in the flux storage
 };
 
 struct FluxConsts {
@@ -149,11 +219,13 @@ struct aerofx_ctx {
   // device
   aerofx::DevTables tab{};
   std::vector<void *> allocs;
-  double *d_V = nullptr;     // [N][5] primitive state of the last residual
-  double *d_grad = nullptr;  // [N][16] LSQ gradients, [d*5+k]
-  double *d_Fm = nullptr;    // [E][5] edge fluxes in edge order
-  double *d_P = nullptr;     // [N][5] per-node sums over upper edges
+  double *d_V = nullptr;     // il<5>: primitive state of the last residual
+  double *d_grad = nullptr;  // il<15>: LSQ gradients, field d*5+k
+  double *d_Fm = nullptr;    // il<5> over positions: edge fluxes
+  double *d_P = nullptr;     // il<5>: per-node sums over upper edges
+  double *d_Ff = nullptr;    // [3F][5] boundary-face fluxes, per node face slot
   int *d_err = nullptr;      // [0] reconstruction errors, [1] singular blocks, [2] bad states
+  bool staged_tried = false;  // the staged family's tables were built, or do not fit
   int residual_kernels = AEROFX_RESIDUAL_PER_LANE;  // AEROFX_RESIDUAL_PER_LANE or _STAGED
   // Newton.FailSafe: 0 off, 1 on, 2 always on; d_fs [3N] = tag0, tag1, mask
   // (DistSVec<int,2> tag of Domain and the node tags of DistNodalGrad)
@@ -171,6 +243,8 @@ struct aerofx_ctx {
   int2 *d_wall = nullptr;
   double *d_idtv = nullptr;
   double *d_visc_c = nullptr;  // [4T][5] element contributions of the Galerkin term, in node-slot order
+                               // (the residual's, whose density row is zero: [4T][4])
+  double *d_visc_g = nullptr;  // il<4>: their node sums
   double *d_adj_tmp = nullptr;  // [N][5] the adjoint with the wall rows masked
   // viscous wall force: element of each face, per node the wall-face element
   // slots (4 f + k), per slot the derivatives [4F][5] / [4F][3]
@@ -252,6 +326,8 @@ int launch_visc_residual(aerofx_ctx *c, const double *V, double *R, bool scale, 
 // the element pass alone into the contribution buffer (the node pass of the
 // residual sums it)
 int launch_visc_elements(aerofx_ctx *c, const double *V, const int *done);
+// their node sums into d_visc_g
+int launch_visc_sum(aerofx_ctx *c, const int *done);
 int launch_visc_jacobian(aerofx_ctx *c, const double *U, int precision);
 int launch_bcs_residual(aerofx_ctx *c, const double *U, double *F, const int *done);
 int launch_visc_idtv(aerofx_ctx *c, double **idtv);
@@ -278,9 +354,10 @@ int refuse_viscous(aerofx_ctx *c, const char *who);
 // returns at once when done != nullptr and *done != 0 (device-resident
 // Krylov loops with a matrix-free operator)
 int launch_residual(aerofx_ctx *c, const double *U, double *R, bool scale, const int *done = nullptr);
-// the same passes with their scratch (primitive state V [N][5], gradients
-// [N][16], upper-edge sums P [N][5], edge fluxes Fm [E][5]) given explicitly;
-// the error count still goes to c->d_err[0]
+// the same passes with their scratch (primitive state V, gradients, edge
+// fluxes Fm and upper-edge sums P, laid out as d_V, d_grad, d_Fm and d_P of
+// the context) given explicitly; the error count still goes to c->d_err[0],
+// and to host_err (pinned) when that is given
 struct ResidualBufs {
   double *V, *grad, *Fm, *P;
   int *tag0 = nullptr;  // failsafe: sides of non-physical reconstructions are tagged here
@@ -295,9 +372,12 @@ int residual_failsafe(aerofx_ctx *c, const ResidualBufs &b, const double *U, dou
 // passes differentiate the full second-order residual)
 int refuse_failsafe_nodes(aerofx_ctx *c, const char *who);
 int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, double *R, bool scale,
-                         const int *done = nullptr);
+                         const int *done = nullptr, int *host_err = nullptr);
+// tables of the LDS-staged family, built when it is first selected
+int ensure_staged(aerofx_ctx *c);
 int launch_gradients_v(aerofx_ctx *c, const double *V, double *ddx, double *ddy, double *ddz);
-int launch_primitive(aerofx_ctx *c, const double *U, double *V);
+int launch_primitive(aerofx_ctx *c, const double *U, double *V);  // V [N][5]
+int launch_primitive_il(aerofx_ctx *c, const double *U);          // c->d_V
 
 // implicit operators (jacobian.hip)
 int launch_timestep(aerofx_ctx *c, double cfl, double *dt);

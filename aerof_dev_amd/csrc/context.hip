@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cstring>
 #include <exception>
+#include <future>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -43,13 +44,16 @@ namespace {
 
 // ---------------------------------------------------------------------------
 // Scratch of aerofx_residual_noalloc: one static array per GPU, holding the
-// residual passes' V [N][5], gradients [N][16], upper-edge sums P [N][5] and
-// edge fluxes Fm [E][5], each part at a 256-byte boundary.  Host code never
+// residual passes' V, gradients, upper-edge sums P and edge fluxes Fm (laid
+// out as the context's own), each part at a 256-byte boundary.  Host code never
 // passes the array's name to a kernel: it uses the device address that
 // hipGetSymbolAddress returns for the current GPU, looked up once per GPU.
 // ---------------------------------------------------------------------------
 constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
-static __device__ __align__(256) double scratch[kNoAllocScratchBytes / sizeof(double)];
+// (the interleaved arrays end on whole groups of 64 items: up to 63 items more
+// in each of the four than the documented size counts, 15 KB together)
+constexpr size_t kNoAllocSlackBytes = size_t(64) << 10;
+static __device__ __align__(256) double scratch[(kNoAllocScratchBytes + kNoAllocSlackBytes) / sizeof(double)];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -163,34 +167,161 @@ std::vector<int> chunk_rows(const std::vector<int> &rowptr, int N, int limit, st
   return ch;
 }
 
-// Flux chunks (first row, end row, first edge, end edge): whole rows with at
-// most `limit` upper edges and kMaxRows rows; a row with more upper edges is
-// cut into pieces of `limit` edges with no rows (first row = end row): its
-// flux sum is then formed by the node pass, in the same edge order.
-std::vector<int4> flux_chunks(const std::vector<int> &eup, int N, int limit) {
-  std::vector<int4> out;
-  int r0 = 0, acc = 0;
-  auto close = [&](int r1) {
-    if (r1 > r0) out.push_back(make_int4(r0, r1, eup[r0], eup[r1]));
-    r0 = r1;
-    acc = 0;
-  };
-  for (int n = 0; n < N; ++n) {
-    const int cnt = eup[n + 1] - eup[n];
-    if (cnt > limit) {
-      close(n);
-      for (int l = eup[n]; l < eup[n + 1]; l += limit) out.push_back(make_int4(n, n, l, std::min(l + limit, eup[n + 1])));
-      r0 = n + 1;
-      continue;
+// A CSR table's rows regrouped per 64 (RowSlices); src[e] gives the entry
+// stored for CSR entry e, and at (or null) receives each entry's place.
+struct HostSlices {
+  std::vector<int> kptr, koff, idx;
+};
+HostSlices slice_rows(int N, const std::vector<int> &rowptr, const std::vector<int> &src, std::vector<int> *at) {
+  HostSlices h;
+  const int ns = (N + 63) / 64;
+  h.kptr.assign(ns + 1, 0);
+  h.idx.resize(src.size());
+  if (at) at->resize(src.size());
+  int cur = 0;
+  for (int s = 0; s < ns; ++s) {
+    const int n0 = 64 * s, n1 = std::min(N, n0 + 64);
+    int most = 0;
+    for (int n = n0; n < n1; ++n) most = std::max(most, rowptr[n + 1] - rowptr[n]);
+    for (int k = 0; k < most; ++k) {
+      h.koff.push_back(cur);
+      for (int n = n0; n < n1; ++n) {
+        const int e = rowptr[n] + k;
+        if (e >= rowptr[n + 1]) continue;
+        h.idx[cur] = src[e];
+        if (at) (*at)[e] = cur;
+        ++cur;
+      }
     }
-    if (acc + cnt > limit || n - r0 == kMaxRows) close(n);
-    acc += cnt;
+    h.kptr[s + 1] = (int)h.koff.size();
   }
-  close(N);
-  return out;
+  return h;
+}
+
+// The different entries of each slice in first-named order, padded to the most
+// of a slice (rounded up to 8) with the last one, and every entry's place
+// among them, padded to the longest row; returns that most, or 0 if it is
+// above kHaloCap or the longest row above kHaloRow.
+int slice_halos(int N, const HostSlices &h, const std::vector<int> &rowptr, int longest, std::vector<int> &halo,
+                std::vector<uint32_t> &loc) {
+  const int ns = (int)h.kptr.size() - 1;
+  if (longest > kHaloRow) return 0;
+  std::vector<int> stamp(N, -1), pos(N), list, start(1, 0);
+  list.reserve(8 * (size_t)N);
+  const int pairs = (longest + 1) / 2;
+  loc.assign((size_t)ns * pairs * 64, 0);
+  int most = 1;
+  for (int s = 0; s < ns; ++s) {
+    const int base = (int)list.size(), n0 = 64 * s, n1 = std::min(N, n0 + 64);
+    int e = h.kptr[s] < (int)h.koff.size() ? h.koff[h.kptr[s]] : 0;
+    for (int k = 0; k < h.kptr[s + 1] - h.kptr[s]; ++k)
+      for (int n = n0; n < n1; ++n) {
+        if (rowptr[n] + k >= rowptr[n + 1]) continue;
+        const int m = h.idx[e++];
+        if (stamp[m] != s) {
+          stamp[m] = s;
+          pos[m] = (int)list.size() - base;
+          list.push_back(m);
+        }
+        loc[((size_t)s * pairs + k / 2) * 64 + (n - n0)] |= (uint32_t)pos[m] << (k & 1 ? 16 : 0);
+      }
+    start.push_back((int)list.size());
+    most = std::max(most, (int)list.size() - base);
+    if (most > kHaloCap) return 0;
+  }
+  most = (most + 7) & ~7;
+  halo.resize((size_t)ns * most);
+  for (int s = 0; s < ns; ++s) {
+    const int cnt = start[s + 1] - start[s];
+    for (int q = 0; q < most; ++q)
+      halo[(size_t)s * most + q] = cnt ? list[start[s] + std::min(q, cnt - 1)] : 64 * s;
+  }
+  return most;
+}
+
+int upload_slices(aerofx_ctx *c, const HostSlices &h, RowSlices *r) {
+  int rc;
+  if ((rc = upload(c, h.kptr, &r->kptr)) || (rc = upload(c, h.koff, &r->koff)) ||
+      (rc = upload(c, h.idx, &r->idx)))
+    return rc;
+  return 0;
+}
+
+// interleaved copy of a table of three doubles per item (items taken at
+// perm, or in order), rows of `ld` doubles
+__global__ __launch_bounds__(kBlock) void k_interleave3(int n, const int *__restrict__ perm,
+                                                        const double *__restrict__ src, int ld,
+                                                        double *__restrict__ dst) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const size_t q = (size_t)(perm ? perm[i] : i) * ld;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) dst[il<3>(i, d)] = src[q + d];
+}
+
+int interleave3(aerofx_ctx *c, int n, const int *perm, const double *src, int ld, const double **out) {
+  void *p = nullptr;
+  int rc = ctx_alloc(c, sizeof(double) * il_count<3>(n), &p);
+  if (rc) return rc;
+  if (n > 0)
+    hipLaunchKernelGGL(k_interleave3, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, 0, n, perm, src, ld,
+                       static_cast<double *>(p));
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_hip_error(e, "interleave launch");
+  *out = static_cast<const double *>(p);
+  return 0;
 }
 
 }  // namespace
+
+// LDS-staged strips (both passes or neither; ngb stays 0 when the mesh does
+// not fit them)
+int ensure_staged(aerofx_ctx *c) {
+  DevTables &t = c->tab;
+  if (c->staged_tried) return 0;
+  const int N = c->N, E = c->E;
+  const int *ptr = c->ptr.data();
+  try {
+    std::vector<int> rowptr, adj, eid, eup(N + 1, 0), jcol(E);
+    node_csr(N, E, ptr, rowptr, adj, eid);
+    for (int l = 0; l < E; ++l) {
+      eup[ptr[2 * (size_t)l] + 1]++;
+      jcol[l] = ptr[2 * (size_t)l + 1];
+    }
+    for (int n = 0; n < N; ++n) eup[n + 1] += eup[n];
+    HaloStrips gs, fs;
+    if (halo_strips(N, rowptr.data(), adj.data(), kGradStrip, 1 << 30, kGradHalo, gs) &&
+        halo_strips(N, eup.data(), jcol.data(), kFluxStrip, kFluxStrip, kFluxHalo, fs)) {
+      const int ngb = (int)gs.own.size(), nfb = (int)fs.own.size();
+      std::vector<int4> gb4(ngb), fb4(nfb);
+      std::vector<int2> fbh(nfb);
+      for (int b = 0; b < ngb; ++b) gb4[b] = make_int4(gs.start[b], gs.start[b + 1], gs.hptr[b], gs.hptr[b + 1]);
+      for (int b = 0; b < nfb; ++b) {
+        fb4[b] = make_int4(fs.start[b], fs.start[b + 1], eup[fs.start[b]], eup[fs.start[b + 1]]);
+        fbh[b] = make_int2(fs.hptr[b], fs.hptr[b + 1]);
+      }
+      // position of each edge's lower node: rows are consecutive from own[b]
+      std::vector<uint32_t> floc(E);
+      for (int b = 0; b < nfb; ++b)
+        for (int r = fs.start[b]; r < fs.start[b + 1]; ++r)
+          for (int l = eup[r]; l < eup[r + 1]; ++l)
+            floc[l] = (uint32_t)(fs.own[b] + (r - fs.start[b])) | ((uint32_t)fs.loc[l] << 16);
+      std::vector<int> epos;
+      (void)slice_rows(N, eup, jcol, &epos);
+      int rc;
+      if ((rc = upload(c, gb4, &t.gb4)) || (rc = upload(c, gs.own, &t.gown)) || (rc = upload(c, gs.halo, &t.ghalo)) ||
+          (rc = upload(c, gs.loc, &t.gloc)) || (rc = upload(c, fb4, &t.fb4)) || (rc = upload(c, fbh, &t.fbh)) ||
+          (rc = upload(c, fs.halo, &t.fhalo)) || (rc = upload(c, floc, &t.floc)) || (rc = upload(c, epos, &t.epos)))
+        return rc;
+      t.nfb = nfb;
+      t.ngb = ngb;
+    }
+  } catch (std::exception &ex) {
+    return set_error(AEROFX_ERR_MESH, ex.what());
+  }
+  c->staged_tried = true;
+  return 0;
+}
 
 ProfScope::ProfScope(aerofx_ctx *ctx, int b) : c(ctx), bucket(b) {
   if (c->prof && (a = take_event(c))) (void)hipEventRecord(a, c->stream);
@@ -313,11 +444,29 @@ int aerofx_ctx_create(const aerofx_mesh *m, const aerofx_params *p, aerofx_ctx *
     std::vector<int> glong;
     std::vector<int> gchunk = chunk_rows(rowptr, N, kBlock, &glong);
     for (int n = 0; n < N; ++n) c->max_degree = std::max(c->max_degree, rowptr[n + 1] - rowptr[n]);
-    int maxup = 0;
-    for (int n = 0; n < N; ++n) maxup = std::max(maxup, eup[n + 1] - eup[n]);
-    const int fblock = maxup <= kFluxBlockSmall ? kFluxBlockSmall : kFluxBlock;
-    // one 16-B record per flux chunk: a block reads its rows and edges at once
-    std::vector<int4> fchunk4 = flux_chunks(eup, N, fblock);
+    // the residual passes' row slices: edges are stored in the order of up
+    std::vector<int> jcol(E), epos, lpos(E), fnode(3 * (size_t)F);
+    for (int l = 0; l < E; ++l) jcol[l] = eij[l].y;
+    // (the neighbour tables on a second host thread)
+    std::vector<int> halo;
+    std::vector<uint32_t> hloc;
+    int halo_cap = 0;
+    std::future<HostSlices> nb_task = std::async(std::launch::async, [&] {
+      HostSlices h = slice_rows(N, rowptr, adj, nullptr);
+      halo_cap = slice_halos(N, h, rowptr, c->max_degree, halo, hloc);
+      return h;
+    });
+    const HostSlices hup = slice_rows(N, eup, jcol, &epos);
+    for (int q = 0; q < E; ++q) lpos[q] = epos[ledge[q]];
+    const HostSlices hlo = slice_rows(N, lrow, lpos, nullptr);
+    std::vector<int> upslice(hup.koff.size());
+    for (int sl = 0; sl + 1 < (int)hup.kptr.size(); ++sl)
+      std::fill(upslice.begin() + hup.kptr[sl], upslice.begin() + hup.kptr[sl + 1], sl);
+    std::vector<int> pedge(E);
+    for (int l = 0; l < E; ++l) pedge[epos[l]] = l;
+    for (int n = 0; n < N; ++n)
+      for (int q = frow[n]; q < frow[n + 1]; ++q) fnode[q] = n;
+    const HostSlices hnb = nb_task.get();
     // node-derived tables
     std::vector<double> X4(4 * (size_t)N), lsq6(6 * (size_t)N), invcv(N), fnorm3(3 * (size_t)F);
     for (int n = 0; n < N; ++n) {
@@ -343,61 +492,39 @@ int aerofx_ctx_create(const aerofx_mesh *m, const aerofx_params *p, aerofx_ctx *
     t.F = F;
     if ((rc = upload(c, X4, &t.X4)) || (rc = upload(c, lsq6, &t.lsq6)) || (rc = upload(c, invcv, &t.invcv)) || (rc = upload(c, c->cv, &t.cv)) ||
         (rc = upload(c, gchunk, &t.gchunk)) || (rc = upload(c, glong, &t.glong)) || (rc = upload(c, rowptr, &t.rowptr)) ||
-        (rc = upload(c, adj, &t.adj)) || (rc = upload(c, eid, &t.eidx)) || (rc = upload(c, mirror, &t.mirror)) || (rc = upload(c, fchunk4, &t.fchunk4)) || (rc = upload(c, eup, &t.eup)) ||
+        (rc = upload(c, adj, &t.adj)) || (rc = upload(c, eid, &t.eidx)) || (rc = upload(c, mirror, &t.mirror)) || (rc = upload(c, eup, &t.eup)) ||
         (rc = upload(c, eij, &t.eij)) || (rc = upload(c, ledge, &t.ledge)) ||
         (rc = upload(c, c->normals, &t.normal)) || (rc = upload(c, lrow, &t.lrow)) ||
         (rc = upload(c, frow, &t.frow)) || (rc = upload(c, fidx, &t.fidx)) || (rc = upload(c, fcode, &t.fcode)) ||
-        (rc = upload(c, fnorm3, &t.fnorm3)) || (rc = upload(c, c->fnorm, &t.fnorm))) {
+        (rc = upload(c, fnorm3, &t.fnorm3)) || (rc = upload(c, c->fnorm, &t.fnorm)) ||
+        (rc = upload(c, fnode, &t.fnode)) || (rc = upload(c, pedge, &t.pedge)) ||
+        (rc = upload(c, upslice, &t.upslice)) ||
+        (halo_cap && ((rc = upload(c, halo, &t.halo)) || (rc = upload(c, hloc, &t.hloc)))) ||
+        (rc = upload_slices(c, hup, &t.up)) || (rc = upload_slices(c, hlo, &t.lo)) ||
+        (rc = upload_slices(c, hnb, &t.nb)) || (rc = interleave3(c, N, nullptr, t.X4, 4, &t.X3)) ||
+        (rc = interleave3(c, E, t.pedge, t.normal, 3, &t.pnormal))) {
       destroy(c);
       return rc;
     }
     t.ngchunks = (int)gchunk.size() - 1;
     t.nglong = (int)glong.size();
-    t.nfchunks = (int)fchunk4.size();
-    t.fblock = fblock;
-    // LDS-staged strips (both passes or neither)
     {
-      HaloStrips gs, fs;
-      std::vector<int> jcol(E);
-      for (int l = 0; l < E; ++l) jcol[l] = ptr[2 * (size_t)l + 1];
-      if (halo_strips(N, rowptr.data(), adj.data(), kGradStrip, 1 << 30, kGradHalo, gs) &&
-          halo_strips(N, eup.data(), jcol.data(), kFluxStrip, kFluxStrip, kFluxHalo, fs)) {
-        const int ngb = (int)gs.own.size(), nfb = (int)fs.own.size();
-        std::vector<int4> gb4(ngb), fb4(nfb);
-        std::vector<int2> fbh(nfb);
-        for (int b = 0; b < ngb; ++b) gb4[b] = make_int4(gs.start[b], gs.start[b + 1], gs.hptr[b], gs.hptr[b + 1]);
-        for (int b = 0; b < nfb; ++b) {
-          fb4[b] = make_int4(fs.start[b], fs.start[b + 1], eup[fs.start[b]], eup[fs.start[b + 1]]);
-          fbh[b] = make_int2(fs.hptr[b], fs.hptr[b + 1]);
-        }
-        // position of each edge's lower node: rows are consecutive from own[b]
-        std::vector<uint32_t> floc(E);
-        for (int b = 0; b < nfb; ++b)
-          for (int r = fs.start[b]; r < fs.start[b + 1]; ++r)
-            for (int l = eup[r]; l < eup[r + 1]; ++l)
-              floc[l] = (uint32_t)(fs.own[b] + (r - fs.start[b])) | ((uint32_t)fs.loc[l] << 16);
-        if ((rc = upload(c, gb4, &t.gb4)) || (rc = upload(c, gs.own, &t.gown)) ||
-            (rc = upload(c, gs.halo, &t.ghalo)) || (rc = upload(c, gs.loc, &t.gloc)) ||
-            (rc = upload(c, fb4, &t.fb4)) || (rc = upload(c, fbh, &t.fbh)) || (rc = upload(c, fs.halo, &t.fhalo)) ||
-            (rc = upload(c, floc, &t.floc))) {
-          destroy(c);
-          return rc;
-        }
-        t.ngb = ngb;
-        t.nfb = nfb;
-      }
+      // the interleaving kernels ran on the null stream
+      hipError_t es = hipStreamSynchronize(nullptr);
+      if (es != hipSuccess) { destroy(c); return set_hip_error(es, "interleaved tables"); }
     }
+    t.ns = (N + 63) / 64;
+    t.halo_cap = halo_cap;
+    t.halo_pairs = (c->max_degree + 1) / 2;
+    t.nup = (int)hup.koff.size();
     void *pv = nullptr;
-    if ((rc = ctx_alloc(c, 5 * sizeof(double) * (size_t)N, &pv))) { destroy(c); return rc; }
-    c->d_V = static_cast<double *>(pv);
-    if ((rc = ctx_alloc(c, 16 * sizeof(double) * (size_t)N, &pv))) { destroy(c); return rc; }
-    c->d_grad = static_cast<double *>(pv);
-    if ((rc = ctx_alloc(c, 5 * sizeof(double) * (size_t)E, &pv))) { destroy(c); return rc; }
-    c->d_Fm = static_cast<double *>(pv);
-    if ((rc = ctx_alloc(c, 5 * sizeof(double) * (size_t)N, &pv))) { destroy(c); return rc; }
-    c->d_P = static_cast<double *>(pv);
-    if ((rc = ctx_alloc(c, 5 * sizeof(double) * (size_t)N, &pv))) { destroy(c); return rc; }
-    c->d_dt = static_cast<double *>(pv);
+    const std::pair<double **, size_t> bufs[] = {{&c->d_V, il_count<5>(N)},     {&c->d_grad, il_count<15>(N)},
+                                                 {&c->d_Fm, il_count<5>(E)},    {&c->d_P, il_count<5>(N)},
+                                                 {&c->d_Ff, 15 * (size_t)F},    {&c->d_dt, 5 * (size_t)N}};
+    for (const auto &b : bufs) {
+      if ((rc = ctx_alloc(c, sizeof(double) * b.second, &pv))) { destroy(c); return rc; }
+      *b.first = static_cast<double *>(pv);
+    }
     if ((rc = ctx_alloc(c, 4 * sizeof(int), &pv))) { destroy(c); return rc; }
     c->d_err = static_cast<int *>(pv);
     hipError_t e = hipMemset(c->d_err, 0, 4 * sizeof(int));
@@ -444,6 +571,8 @@ int aerofx_ctx_set_residual_kernels(aerofx_ctx *c, int family) {
   if (family != AEROFX_RESIDUAL_AUTO && family != AEROFX_RESIDUAL_PER_LANE && family != AEROFX_RESIDUAL_STAGED)
     return set_error(AEROFX_ERR_ARG,
                      "set_residual_kernels: AEROFX_RESIDUAL_AUTO, AEROFX_RESIDUAL_PER_LANE or AEROFX_RESIDUAL_STAGED");
+  if (family == AEROFX_RESIDUAL_STAGED)
+    if (int rc = ensure_staged(c)) return rc;
   c->residual_kernels = family == AEROFX_RESIDUAL_STAGED && c->tab.ngb > 0 ? AEROFX_RESIDUAL_STAGED
                                                                             : AEROFX_RESIDUAL_PER_LANE;
   return c->residual_kernels;
@@ -571,10 +700,13 @@ int aerofx_residual_noalloc(aerofx_ctx *c, const double *U, double *R, int flags
   if (!c || !U || !R) return set_error(AEROFX_ERR_ARG, "residual_noalloc: null argument");
   if (!c->noalloc_scratch)
     return set_error(AEROFX_ERR_STATE, "residual_noalloc: no scratch address on this GPU: " + c->noalloc_err);
-  const size_t oV = 0, oG = align256(5 * sizeof(double) * (size_t)c->N);
-  const size_t oP = oG + align256(16 * sizeof(double) * (size_t)c->N);
-  const size_t oF = oP + align256(5 * sizeof(double) * (size_t)c->N);
-  const size_t need = oF + align256(5 * sizeof(double) * (size_t)c->E);
+  // the documented rule (which meshes are taken); the arrays' own layout is
+  // never more than kNoAllocSlackBytes beyond it
+  const size_t need = 2 * align256(5 * sizeof(double) * (size_t)c->N) + align256(16 * sizeof(double) * (size_t)c->N) +
+                      align256(5 * sizeof(double) * (size_t)c->E);
+  const size_t oV = 0, oG = align256(sizeof(double) * il_count<5>(c->N));
+  const size_t oP = oG + align256(sizeof(double) * il_count<15>(c->N));
+  const size_t oF = oP + align256(sizeof(double) * il_count<5>(c->N));
   if (need > kNoAllocScratchBytes)
     return set_error(AEROFX_ERR_ARG, "residual_noalloc: the mesh (" + std::to_string(c->N) + " nodes, " +
                                          std::to_string(c->E) + " edges) needs " + std::to_string(need) +

@@ -39,8 +39,7 @@ __global__ __launch_bounds__(kBlock) void k_timestep(DevTables t, const double *
   const int n = blockIdx.x * kBlock + threadIdx.x;
   if (n >= t.N) return;
   double Vn[5];
-#pragma unroll
-  for (int k = 0; k < 5; ++k) Vn[k] = V[5 * (size_t)n + k];
+  load_il<5>(V, n, Vn);
   const double beta2 = 1.0;
   double idti = 0.0;
   for (int e = t.rowptr[n]; e < t.rowptr[n + 1]; ++e) {
@@ -51,12 +50,10 @@ __global__ __launch_bounds__(kBlock) void k_timestep(DevTables t, const double *
     double invS = 1.0 / S;
     double nn0 = invS * nl[0], nn1 = invS * nl[1], nn2 = invS * nl[2];
     double ndot = invS * 0.0;
-    double Vmid[5];
+    double Vm[5], Vmid[5];
+    load_il<5>(V, m, Vm);
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      const double vm = V[5 * (size_t)m + k];
-      Vmid[k] = 0.5 * (nlow ? Vn[k] + vm : vm + Vn[k]);
-    }
+    for (int k = 0; k < 5; ++k) Vmid[k] = 0.5 * (nlow ? Vn[k] + Vm[k] : Vm[k] + Vn[k]);
     double a = sound_speed(g, Vmid);
     double un = Vmid[1] * nn0 + Vmid[2] * nn1 + Vmid[3] * nn2 - ndot;
     double coeff1 = (1.0 + beta2) * un;
@@ -118,11 +115,8 @@ __device__ __forceinline__ void jac_entry(const DevTables &t, const double *__re
     return;
   }
   double Vn[5], Vm[5];
-#pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    Vn[k] = V[5 * (size_t)n + k];
-    Vm[k] = V[5 * (size_t)m + k];
-  }
+  load_il<5>(V, n, Vn);
+  load_il<5>(V, m, Vm);
   const double voln = t.invcv[n];
   double length = 1.0;
   if (LM) {
@@ -159,8 +153,7 @@ __device__ __forceinline__ void jac_face(const DevTables &t, const double *__res
   const int code = t.fcode[face];
   const double nv[3] = {t.fnorm3[3 * (size_t)face], t.fnorm3[3 * (size_t)face + 1], t.fnorm3[3 * (size_t)face + 2]};
   double Vn[5], jac[25];
-#pragma unroll
-  for (int k = 0; k < 5; ++k) Vn[k] = V[5 * (size_t)n + k];
+  load_il<5>(V, n, Vn);
   if (is_wall_code(code)) {
     wall_jac(fc.gas, nv, 0.0, Vn, jac);
   } else {

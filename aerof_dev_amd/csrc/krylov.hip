@@ -1109,7 +1109,7 @@ constexpr int kDerivRestart = 20;
 // inverse in `precision`; the zero-pivot count is checked.
 static int derivative_operators(aerofx_ctx *c, const double *U, double cfl, int precision, const char *who) {
   int rc;
-  if ((rc = launch_primitive(c, U, c->d_V))) return rc;
+  if ((rc = launch_primitive_il(c, U))) return rc;
   if (cfl > 0.0 && (rc = launch_timestep(c, cfl, c->d_dt))) return rc;
   if ((rc = launch_jacobian(c, cfl > 0.0 ? c->d_dt : nullptr, precision, U))) return rc;
   hipError_t e = hipMemcpyAsync(c->h_err + 1, c->d_err + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream);
@@ -1297,14 +1297,14 @@ int aerofx_gmres_transpose(aerofx_ctx *c, const double *b, double *x, int m, dou
 
 int aerofx_timestep(aerofx_ctx *c, const double *U, double cfl, double *dt) {
   if (!c || !U || !dt) return set_error(AEROFX_ERR_ARG, "timestep: null argument");
-  int rc = launch_primitive(c, U, c->d_V);
+  int rc = launch_primitive_il(c, U);
   return rc ? rc : launch_timestep(c, cfl, dt);
 }
 
 int aerofx_jacobian_setup(aerofx_ctx *c, const double *U, const double *dt, int precision) {
   if (!c || !U) return set_error(AEROFX_ERR_ARG, "jacobian_setup: null argument");
   if (precision != 0 && precision != 1) return set_error(AEROFX_ERR_ARG, "jacobian_setup: precision 0 or 1");
-  int rc = launch_primitive(c, U, c->d_V);
+  int rc = launch_primitive_il(c, U);
   if (rc) return rc;
   if ((rc = launch_jacobian(c, dt, precision, U))) return rc;
   hipError_t e = hipMemcpyAsync(c->h_err + 1, c->d_err + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream);

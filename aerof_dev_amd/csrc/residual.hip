@@ -1,131 +1,175 @@
 // residual.hip -- the FP64 edge residual on gfx950.
 //
-// SpaceOperator<5>::computeResidual (SpaceOperator.C:524-634) in three
-// kernels, all deterministic (no atomics on floating-point data):
+// SpaceOperator<5>::computeResidual (SpaceOperator.C:524-634), all
+// deterministic (no atomics on floating-point data):
 //
-//  1. k_gradients  one lane per node n walks its neighbours m in ascending
+//  1. k_gradients_halo (k_gradients for meshes whose neighbourhoods do not fit
+//     it)  one lane per node n walks its neighbours m in ascending
 //     order (= ascending edge id) accumulating W(R_n, X_m - X_n) (V_m - V_n):
 //     the reference's LSQ edge loop (SubDomain.C:137-159, 297-374) with the
-//     same per-node addition order.  The pass also writes V = V(U).
-//  2. k_flux_edges edge-parallel, edges grouped by their lower node i (the
-//     reference's edge order, EdgeCore.C:92-119): each edge flux is computed
-//     once (MUSCL + Van Albada + ROEFLUX7, Edge.C:372-439); the block sums the
-//     +f contributions of each of its rows in edge order (P_i) and writes f
-//     contiguously in edge order (Fm).
+//     same per-node addition order.  The pass also writes V = V(U), which
+//     later passes gather, interleaved.
+//  2. k_flux_edges each edge flux once (MUSCL + Van Albada + ROEFLUX7,
+//     Edge.C:372-439), a wave per 64 lower nodes i: lane r takes the edges of
+//     node i in turn, so its state, coordinates and gradients stay in
+//     registers and the +f contributions P_i are summed in edge order (large
+//     meshes), or a wave per (64 nodes, k-th upper edge) (small ones).
+//     Boundary-face fluxes (Face.C:356-389) per face slot by further blocks.
 //  3. k_flux_nodes node-parallel: R_n = (sum over lower edges (m, n), m
-//     ascending, of -f, gathered from Fm) + P_n + boundary-face fluxes in face order (Face.C:356-389), times
-//     1/V_n (SpaceOperator.C:599-624).
+//     ascending, of -f, gathered from Fm) + P_n + boundary-face fluxes in face
+//     order, times 1/V_n (SpaceOperator.C:599-624).
 //
-// Node data are gathered through L2 (the RCM neighbour window is small).  blockIdx is remapped so that each XCD sweeps one
-// contiguous node range, keeping the RCM neighbour window in its L2.
+// Layouts: il and RowSlices (context.h).  blockIdx is remapped so that each XCD
+// sweeps one contiguous node range, keeping the RCM neighbour window in its
+// L2.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "context.h"
 #include "host_internal.h"
 
 namespace aerofx {
 
-// neighbours per load batch of the gradient pass (measured at 128^3: 2 ->
-// 0.317 ms, 4 -> 0.310, 6 -> 0.307, 8 -> 0.301; from 10 on the batch no
-// longer stays in registers)
+// neighbours per load batch of the per-entry gradient pass (measured at 128^3
+// with record gathers: 2 -> 0.317 ms, 4 -> 0.310, 6 -> 0.307, 8 -> 0.301; from
+// 10 on the batch no longer stays in registers)
 constexpr int kGradChunk = 8;
 
+constexpr int kWave = 64;
+__device__ __forceinline__ int lane_id() { return (int)threadIdx.x & (kWave - 1); }
+// slice of this wave: blocks of four slices, one contiguous range per XCD
+__device__ __forceinline__ int wave_slice(const DevTables &t) {
+  const int nb = (t.ns + kBlock / kWave - 1) / (kBlock / kWave);
+  return xcd_chunk(blockIdx.x, nb) * (kBlock / kWave) + (int)(threadIdx.x / kWave);
+}
+static dim3 slice_grid(int ns) { return dim3((unsigned)((ns + kBlock / kWave - 1) / (kBlock / kWave))); }
+
 // ---------------------------------------------------------------------------
-// 1. gradients (+ primitive state): one lane per node, neighbours in
-//    ascending order (= the reference's edge order), so every node's sums are
-//    formed exactly as in the reference's sequential edge loop.
+// 1. gradients: one lane per node, neighbours in ascending order (= the
+//    reference's edge order), so every node's sums are formed exactly as in
+//    the reference's sequential edge loop.
 // ---------------------------------------------------------------------------
-template <bool FROM_U>
-__device__ __forceinline__ void load_prim(const double *__restrict__ W, int n, const Gas &gas, double v[5]) {
-  double w[5];
-#pragma unroll
-  for (int k = 0; k < 5; ++k) w[k] = W[5 * (size_t)n + k];
-  if (FROM_U) {
-    prim_from_cons(w, gas, v);
+// where a state comes from: U or V as [N][5], or the interleaved V
+enum { kFromU = 0, kFromV = 1, kFromVil = 2 };
+template <int FROM>
+__device__ __forceinline__ void load_state(const double *__restrict__ W, int n, double w[5]) {
+  if (FROM == kFromVil) {
+    load_il<5>(W, n, w);
   } else {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) v[k] = w[k];
+    for (int k = 0; k < 5; ++k) w[k] = W[5 * (size_t)n + k];
+  }
+}
+__device__ __forceinline__ void load_x(const DevTables &t, int n, double x[3]) {
+  load_il<3>(t.X3, n, x);
+}
+
+__device__ __forceinline__ void load_lsq(const DevTables &t, int n, double L[6]) {
+#pragma unroll
+  for (int q = 0; q < 6; ++q) L[q] = t.lsq6[6 * (size_t)n + q];
+}
+
+// acc += W(L, X_m - X_n) (V_m - V_n) (SubDomain.C:137-159, 297-374),
+// variables V0 <= q < V1
+template <int V0 = 0, int V1 = 5>
+__device__ __forceinline__ void lsq_add(const double L[6], const double xm[3], const double xn[3],
+                                        const double Vm[5], const double Vn[5], double acc[15]) {
+  const double or11 = L[0], or22 = L[1], or33 = L[2], r12or11 = L[3], r23or22 = L[4], psi = L[5];
+  const double dx0 = xm[0] - xn[0], dx1 = xm[1] - xn[1], dx2 = xm[2] - xn[2];
+  const double alpha1 = dx0 * or11 * or11;
+  const double alpha2 = (dx1 - r12or11 * dx0) * or22 * or22;
+  const double alpha3 = (dx2 - r23or22 * dx1 + psi * dx0) * or33 * or33;
+  const double w0 = alpha1 - r12or11 * alpha2 + psi * alpha3;
+  const double w1 = alpha2 - r23or22 * alpha3;
+  const double w2 = alpha3;
+#pragma unroll
+  for (int q = V0; q < V1; ++q) {
+    const double d = Vm[q] - Vn[q];
+    acc[q] += w0 * d;
+    acc[5 + q] += w1 * d;
+    acc[10 + q] += w2 * d;
   }
 }
 
-template <bool FROM_U, bool OUT3>
+// kFromU also writes V (Vout); OUT3: gradients to ddx, ddy, ddz [N][5]
+template <int FROM, bool OUT3>
 __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double *__restrict__ W, Gas gas,
                                                       double *__restrict__ Vout, double *__restrict__ grad,
                                                       double *__restrict__ ddx, double *__restrict__ ddy,
                                                       double *__restrict__ ddz, int *__restrict__ err,
                                                       const int *__restrict__ done) {
   if (done && *done) return;
-  const int nb = (t.N + kBlock - 1) / kBlock;
-  const int n = xcd_chunk(blockIdx.x, nb) * kBlock + (int)threadIdx.x;
   if (err && blockIdx.x == 0 && threadIdx.x == 0) *err = 0;  // the flux pass follows in stream order
-  if (n >= t.N) return;
-  double Vn[5];
-  load_prim<FROM_U>(W, n, gas, Vn);
-  if (Vout) {
+  const int sl = wave_slice(t);
+  if (sl >= t.ns) return;
+  const int lane = lane_id();
+  const int n = sl * kWave + lane;
+  const bool live = n < t.N;
+  const int nn = live ? n : t.N - 1;
+  double Vn[5], xn[3];
+  {
+    double w[5];
+    load_state<FROM>(W, nn, w);
+    if (FROM == kFromU) {
+      prim_from_cons(w, gas, Vn);
+    } else {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) Vout[5 * (size_t)n + k] = Vn[k];
+      for (int k = 0; k < 5; ++k) Vn[k] = w[k];
+    }
   }
-  const double4 xn = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)n);
-  const double *L = t.lsq6 + 6 * (size_t)n;
-  const double or11 = L[0], or22 = L[1], or33 = L[2], r12or11 = L[3], r23or22 = L[4], psi = L[5];
-  double acc[15];
+  if (Vout && live) store_il<5>(Vout, n, Vn);
+  load_x(t, nn, xn);
+  double L[6], acc[15];
+  load_lsq(t, nn, L);
 #pragma unroll
   for (int q = 0; q < 15; ++q) acc[q] = 0.0;
   // Neighbours in chunks of kGradChunk: the chunk's states and coordinates
   // are requested together and the next chunk's indices are prefetched, so a
   // row costs about one memory latency per chunk.  The sums are still formed
   // one neighbour at a time in ascending order.
-  const int e0 = t.rowptr[n], e1 = t.rowptr[n + 1];
+  const int deg = live ? t.rowptr[n + 1] - t.rowptr[n] : 0;
+  const int k0 = t.nb.kptr[sl], kn = t.nb.kptr[sl + 1] - k0;
   int mi[kGradChunk];
-#pragma unroll
-  for (int k = 0; k < kGradChunk; ++k) mi[k] = e0 + k < e1 ? t.adj[e0 + k] : n;
-  for (int e = e0; e < e1; e += kGradChunk) {
-    double Wm[kGradChunk][5];
-    double4 xm[kGradChunk];
+  auto fetch = [&](int base) {
 #pragma unroll
     for (int k = 0; k < kGradChunk; ++k) {
-#pragma unroll
-      for (int q = 0; q < 5; ++q) Wm[k][q] = W[5 * (size_t)mi[k] + q];
-      xm[k] = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)mi[k]);
+      const bool act = base + k < deg;
+      const int off = base + k < kn ? t.nb.koff[k0 + base + k] : 0;
+      const int rank = lanes_below(act);
+      mi[k] = act ? t.nb.idx[off + rank] : nn;
     }
-#pragma unroll
-    for (int k = 0; k < kGradChunk; ++k) mi[k] = e + kGradChunk + k < e1 ? t.adj[e + kGradChunk + k] : n;
+  };
+  if (kn > 0) fetch(0);
+  for (int e = 0; e < kn; e += kGradChunk) {
+    double Wm[kGradChunk][5], xm[kGradChunk][3];
 #pragma unroll
     for (int k = 0; k < kGradChunk; ++k) {
-      if (e + k >= e1) break;
+      load_state<FROM>(W, mi[k], Wm[k]);
+      load_x(t, mi[k], xm[k]);
+    }
+    if (e + kGradChunk < kn) fetch(e + kGradChunk);
+#pragma unroll
+    for (int k = 0; k < kGradChunk; ++k) {
+      if (e + k >= deg) break;
       double Vm[5];
-      if (FROM_U) {
+      if (FROM == kFromU) {
         prim_from_cons(Wm[k], gas, Vm);
       } else {
 #pragma unroll
         for (int q = 0; q < 5; ++q) Vm[q] = Wm[k][q];
       }
-      const double dx0 = xm[k].x - xn.x, dx1 = xm[k].y - xn.y, dx2 = xm[k].z - xn.z;
-      const double alpha1 = dx0 * or11 * or11;
-      const double alpha2 = (dx1 - r12or11 * dx0) * or22 * or22;
-      const double alpha3 = (dx2 - r23or22 * dx1 + psi * dx0) * or33 * or33;
-      const double w0 = alpha1 - r12or11 * alpha2 + psi * alpha3;
-      const double w1 = alpha2 - r23or22 * alpha3;
-      const double w2 = alpha3;
-#pragma unroll
-      for (int q = 0; q < 5; ++q) {
-        const double d = Vm[q] - Vn[q];
-        acc[q] += w0 * d;
-        acc[5 + q] += w1 * d;
-        acc[10 + q] += w2 * d;
-      }
+      lsq_add(L, xm[k], xn, Vm, Vn, acc);
     }
   }
+  if (!live) return;
   if (!OUT3 && t.fs_mask && t.fs_mask[n]) {
     // DistNodalGrad::limit with failsafe tags (DistNodalGrad.C:1083-1104)
 #pragma unroll
     for (int q = 0; q < 15; ++q) acc[q] = 0.0;
   }
   if (!OUT3) {
-    double2 *g2 = reinterpret_cast<double2 *>(grad + 16 * (size_t)n);
-#pragma unroll
-    for (int q = 0; q < 7; ++q) g2[q] = make_double2(acc[2 * q], acc[2 * q + 1]);
-    g2[7] = make_double2(acc[14], 0.0);
+    store_il<15>(grad, n, acc);
   } else {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -136,110 +180,325 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
   }
 }
 
-// ---------------------------------------------------------------------------
-// 2. edge fluxes, computed once per edge.  A block covers whole rows (all
-//    edges whose lower node lies in [r0, r1), <= FB edges); lane k of the
-//    block takes edge l0 + k.  Node i data are read directly (the ~7 lanes of
-//    a row hit the same lines); only the fluxes go through LDS, for the
-//    per-row sums P_i in edge order.
-// ---------------------------------------------------------------------------
-//    LM: the spatial low-Mach flux (ROEFLUX5) with the edge length
-//    |X_j - X_i| in Turkel's beta.
-template <bool SECOND, int FB, bool LM>
-__global__ __launch_bounds__(FB) void k_flux_edges(DevTables t, const double *__restrict__ V,
-                                                       const double *__restrict__ grad, FluxConsts fc,
-                                                       double *__restrict__ Fm, double *__restrict__ P,
-                                                       int *__restrict__ err, int *__restrict__ tag0,
-                                                       const int *__restrict__ done) {
+// The same through LDS, a slice at a time per workgroup: the slice's
+// neighbours overlap (about 14 * 64 adjacency entries are 480 different nodes
+// in RCM or row order, runs of consecutive ids).  Each node of the halo is
+// loaded once, by consecutive lanes, and the entries read LDS: 16-B pairs,
+// consecutive lanes on consecutive nodes.  The pass is bound by the loads in
+// flight, which LDS limits (64 B a halo node: five workgroups per CU): two
+// waves share the halo and split the variables, the workgroups stay for
+// several slices and request the next one's data before they compute, and the
+// tables are padded to one length per slice, so those requests depend on one
+// earlier load only.  The sums are k_gradients', term for term.  At 2.1M nodes
+// 245 us, 275k nodes 35 us (k_gradients with record gathers 296 and 46;
+// without the overlap 266 + 28 for a pass that converts U first, with one wave
+// per slice 366 + 28).
+constexpr int kHaloWaves = 2;
+constexpr int kHaloThreads = kWave * kHaloWaves;
+constexpr int kHaloBatch = 4;   // halo nodes a lane has in flight
+constexpr int kHaloPairs = 8;   // place pairs (two entries) requested together
+
+struct HaloLoad {
+  double w[kHaloBatch][5], x[kHaloBatch][3];
+  __device__ __forceinline__ void request(const DevTables &t, const double *__restrict__ U,
+                                          const int m[kHaloBatch]) {
+#pragma unroll
+    for (int r = 0; r < kHaloBatch; ++r) {
+      load_state<kFromU>(U, m[r], w[r]);
+      load_x(t, m[r], x[r]);
+    }
+  }
+  // pair q of halo node h to sp[q * cap + h]: (V0, V1) (V2, V3) (V4, X0) (X1, X2)
+  __device__ __forceinline__ void put(const Gas &gas, double2 *sp, int cap, int r0) {
+#pragma unroll
+    for (int r = 0; r < kHaloBatch; ++r) {
+      const int h = r0 + r * kHaloThreads + (int)threadIdx.x;
+      if (h >= cap) break;
+      double v[5];
+      prim_from_cons(w[r], gas, v);
+      sp[h] = make_double2(v[0], v[1]);
+      sp[cap + h] = make_double2(v[2], v[3]);
+      sp[2 * cap + h] = make_double2(v[4], x[r][0]);
+      sp[3 * cap + h] = make_double2(x[r][1], x[r][2]);
+    }
+  }
+};
+
+__device__ __forceinline__ void halo_ids(const DevTables &t, int sl, int r0, int m[kHaloBatch]) {
+  const int *halo = t.halo + (size_t)sl * t.halo_cap;
+#pragma unroll
+  for (int r = 0; r < kHaloBatch; ++r) m[r] = halo[min(r0 + r * kHaloThreads + (int)threadIdx.x, t.halo_cap - 1)];
+}
+
+// this lane's node: state, coordinates, factors, degree and the places of its
+// first entries
+struct HaloRow {
+  double w[5], xn[3], L[6];
+  int deg;
+  uint32_t loc[kHaloPairs];
+  __device__ __forceinline__ void request(const DevTables &t, const double *__restrict__ U, int sl) {
+    const int nn = min(sl * kWave + lane_id(), t.N - 1);
+    load_state<kFromU>(U, nn, w);
+    load_x(t, nn, xn);
+    load_lsq(t, nn, L);
+    deg = t.rowptr[nn + 1] - t.rowptr[nn];
+    places(t, sl, 0);
+  }
+  __device__ __forceinline__ void places(const DevTables &t, int sl, int p0) {
+    const uint32_t *q = t.hloc + (size_t)sl * t.halo_pairs * kWave + lane_id();
+#pragma unroll
+    for (int p = 0; p < kHaloPairs; ++p) loc[p] = p0 + p < t.halo_pairs ? q[(p0 + p) * kWave] : 0;
+  }
+};
+
+// variables V0 <= q < V1 of this lane's gradients
+template <int V0, int V1>
+__device__ __forceinline__ void halo_sums(const DevTables &t, const double2 *sp, HaloRow &row, const double Vn[5],
+                                          int sl, int n, double *__restrict__ grad) {
+  const int cap = t.halo_cap;
+  double acc[15];
+#pragma unroll
+  for (int q = 0; q < 15; ++q) acc[q] = 0.0;
+  for (int p0 = 0; p0 < t.halo_pairs; p0 += kHaloPairs) {
+    if (p0) row.places(t, sl, p0);
+#pragma unroll
+    for (int k = 0; k < 2 * kHaloPairs; ++k) {
+      if (2 * p0 + k >= 2 * t.halo_pairs) break;
+      const int hm = k & 1 ? row.loc[k >> 1] >> 16 : row.loc[k >> 1] & 0xffffu;
+      const double2 b = sp[cap + hm], c = sp[2 * cap + hm], d = sp[3 * cap + hm];
+      const double2 a = V0 < 2 ? sp[hm] : make_double2(0.0, 0.0);
+      const double Vm[5] = {a.x, a.y, b.x, b.y, c.x}, xm[3] = {c.y, d.x, d.y};
+      if (2 * p0 + k < row.deg) lsq_add<V0, V1>(row.L, xm, row.xn, Vm, Vn, acc);
+    }
+  }
+  if (t.fs_mask && t.fs_mask[n]) {
+    // DistNodalGrad::limit with failsafe tags (DistNodalGrad.C:1083-1104)
+#pragma unroll
+    for (int q = 0; q < 15; ++q) acc[q] = 0.0;
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int q = V0; q < V1; ++q) grad[il<15>(n, 5 * d + q)] = acc[5 * d + q];
+}
+
+// The workgroups b, b + 8, ... take turns over the b % 8-th part of the slices
+// (the XCD they run on).
+__global__ __launch_bounds__(kHaloThreads) void k_gradients_halo(DevTables t, const double *__restrict__ U, Gas gas,
+                                                                 double *__restrict__ Vout,
+                                                                 double *__restrict__ grad, int *__restrict__ err,
+                                                                 const int *__restrict__ done) {
   if (done && *done) return;
-  __shared__ double sf[5 * (FB + 1)];
-  const int4 ch = t.fchunk4[xcd_chunk(blockIdx.x, t.nfchunks)];
-  const int r0 = ch.x, r1 = ch.y, l0 = ch.z, l1 = ch.w;
-  const int tid = threadIdx.x;
+  extern __shared__ double2 sp[];
+  const int cap = t.halo_cap;
+  if (err && blockIdx.x == 0 && threadIdx.x == 0) *err = 0;  // the flux pass follows in stream order
+  const int xcd = blockIdx.x % kNumXcd, turn = blockIdx.x / kNumXcd;
+  const int step = ((int)gridDim.x - xcd + kNumXcd - 1) / kNumXcd;  // workgroups of this part
+  const int s0 = (int)((long long)t.ns * xcd / kNumXcd), s1 = (int)((long long)t.ns * (xcd + 1) / kNumXcd);
+  int sl = s0 + turn;
+  if (sl >= s1) return;
+  HaloLoad load;
+  HaloRow row;
+  int m[kHaloBatch];
+  halo_ids(t, sl, 0, m);
+  row.request(t, U, sl);
+  load.request(t, U, m);
+  int next = sl + step;
+  if (next < s1) halo_ids(t, next, 0, m);
+  while (true) {
+    load.put(gas, sp, cap, 0);
+    for (int r0 = kHaloBatch * kHaloThreads; r0 < cap; r0 += kHaloBatch * kHaloThreads) {
+      // a halo beyond one batch: its remainder without the overlap
+      int mr[kHaloBatch];
+      halo_ids(t, sl, r0, mr);
+      load.request(t, U, mr);
+      load.put(gas, sp, cap, r0);
+    }
+    HaloRow cur = row;
+    double Vn[5];
+    prim_from_cons(cur.w, gas, Vn);
+    __syncthreads();
+    const bool more = next < s1;
+    if (more) {
+      load.request(t, U, m);
+      row.request(t, U, next);
+    }
+    const int n = sl * kWave + lane_id();
+    if (n < t.N) {
+      if ((int)threadIdx.x < kWave) {
+        store_il<5>(Vout, n, Vn);
+        halo_sums<0, 3>(t, sp, cur, Vn, sl, n, grad);
+      } else {
+        halo_sums<3, 5>(t, sp, cur, Vn, sl, n, grad);
+      }
+    }
+    if (!more) return;
+    sl = next;
+    next += step;
+    if (next < s1) halo_ids(t, next, 0, m);
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 2. edge fluxes, computed once per edge
+// ---------------------------------------------------------------------------
+// the passes' streamed data of large meshes: past the caches, which then keep
+// the gathered node data (flux pass at 2.1M nodes 492 -> 468 us, the node pass
+// after it 212 -> 205; at 275k nodes the fluxes would miss the cache instead:
+// 106 -> 109 us)
+typedef double nt_double2 __attribute__((ext_vector_type(2)));
+template <int W, bool NT>
+__device__ __forceinline__ void stream_load(const double *__restrict__ p, int n, double v[W]) {
+  if (!NT) return load_il<W>(p, n, v);
+  const double *q = p + ((size_t)n >> 6) * (64 * W);
+  const int l = n & 63;
+#pragma unroll
+  for (int k = 0; k < W / 2; ++k) {
+    const nt_double2 a = __builtin_nontemporal_load(reinterpret_cast<const nt_double2 *>(q + k * 128 + 2 * l));
+    v[2 * k] = a.x;
+    v[2 * k + 1] = a.y;
+  }
+  if (W & 1) v[W - 1] = __builtin_nontemporal_load(q + (W - 1) * 64 + l);
+}
+template <int W, bool NT>
+__device__ __forceinline__ void stream_store(double *__restrict__ p, int n, const double v[W]) {
+  if (!NT) return store_il<W>(p, n, v);
+  double *q = p + ((size_t)n >> 6) * (64 * W);
+  const int l = n & 63;
+#pragma unroll
+  for (int k = 0; k < W / 2; ++k) {
+    const nt_double2 a = {v[2 * k], v[2 * k + 1]};
+    __builtin_nontemporal_store(a, reinterpret_cast<nt_double2 *>(q + k * 128 + 2 * l));
+  }
+  if (W & 1) __builtin_nontemporal_store(v[W - 1], q + (W - 1) * 64 + l);
+}
+
+// One edge: reconstruction, check and flux.  LM: the spatial low-Mach flux
+// (ROEFLUX5) with the edge length |X_j - X_i| in Turkel's beta.  bi, bj: the
+// sides whose reconstruction is non-physical (checkReconstructedValues,
+// EdgeCore.C:137-166, VarFcnSGEuler.h:90-110).
+template <bool SECOND, bool LM>
+__device__ __forceinline__ void edge_flux(const FluxConsts &fc, const double Vi[5], const double xi[3],
+                                          const double *gi, const double Vj[5], const double xj[3],
+                                          const double *gj, const double nv[3], double f[5], bool &bi, bool &bj) {
   const Gas &g = fc.gas;
-  if (tid < l1 - l0) {
-    const int l = l0 + tid;
-    const int2 ij = t.eij[l];
-    const int i = ij.x, j = ij.y;
-    double Vi[5], Vj[5];
+  double Vij[5], Vji[5];
+  double length = 1.0, dx0 = 0.0, dx1 = 0.0, dx2 = 0.0;
+  if (SECOND || LM) {
+    dx0 = xj[0] - xi[0];
+    dx1 = xj[1] - xi[1];
+    dx2 = xj[2] - xi[2];
+  }
+  if (LM) length = sqrt(dx0 * dx0 + dx1 * dx1 + dx2 * dx2);
+  if (SECOND) {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-      Vi[k] = V[5 * (size_t)i + k];
-      Vj[k] = V[5 * (size_t)j + k];
+      const double ddVij = dx0 * gi[k] + dx1 * gi[5 + k] + dx2 * gi[10 + k];
+      const double ddVji = dx0 * gj[k] + dx1 * gj[5 + k] + dx2 * gj[10 + k];
+      reconstruct(fc.beta, Vi[k], ddVij, Vj[k], ddVji, Vij[k], Vji[k]);
     }
-    double Vij[5], Vji[5];
-    double length = 1.0;
-    if (LM) {
-      const double4 xi = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)i);
-      const double4 xj = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)j);
-      const double dx0 = xj.x - xi.x, dx1 = xj.y - xi.y, dx2 = xj.z - xi.z;
-      length = sqrt(dx0 * dx0 + dx1 * dx1 + dx2 * dx2);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      Vij[k] = Vi[k];
+      Vji[k] = Vj[k];
     }
-    if (SECOND) {
-      const double4 xi = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)i);
-      const double4 xj = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)j);
-      const double dx0 = xj.x - xi.x, dx1 = xj.y - xi.y, dx2 = xj.z - xi.z;
-      const double2 *gi2 = reinterpret_cast<const double2 *>(grad + 16 * (size_t)i);
-      const double2 *gj2 = reinterpret_cast<const double2 *>(grad + 16 * (size_t)j);
-      double gi[16], gj[16];
+  }
+  bi = Vij[0] <= 0.0 || Vij[4] + g.pstiff <= 0.0;
+  bj = Vji[0] <= 0.0 || Vji[4] + g.pstiff <= 0.0;
+  if (nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2] < 1e-36) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const double2 a = gi2[q], b = gj2[q];
-        gi[2 * q] = a.x;
-        gi[2 * q + 1] = a.y;
-        gj[2 * q] = b.x;
-        gj[2 * q + 1] = b.y;
-      }
+    for (int k = 0; k < 5; ++k) f[k] = 0.0;
+  } else if (LM) {
+    roe_turkel_flux(g, fc.lm, true, nv, length, Vij, Vji, f);
+  } else {
+    roe_flux(g, nv, Vij, Vji, f);
+  }
+}
+
+// flux of boundary-face slot q (a face of node fnode[q]) into Ff[q]
+__device__ __forceinline__ void face_slot_flux(const DevTables &t, const double *__restrict__ V, const FluxConsts &fc,
+                                               int q, double *__restrict__ Ff) {
+  const int n = t.fnode[q], face = t.fidx[q];
+  const int code = t.fcode[face];
+  const double nv[3] = {t.fnorm3[3 * (size_t)face], t.fnorm3[3 * (size_t)face + 1], t.fnorm3[3 * (size_t)face + 2]};
+  double Vn[5], fl[5];
+  load_state<kFromVil>(V, n, Vn);
+  if (is_wall_code(code)) {
+    wallflux(nv, 0.0, Vn, fl);
+  } else {
+    const double *ub = (code == AEROFX_BC_INLET || code == -AEROFX_BC_INLET) ? fc.ub_in : fc.ub_out;
+    boundflux5(fc.gas, nv, 0.0, Vn, ub, fl);
+  }
 #pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        const double ddVij = dx0 * gi[k] + dx1 * gi[5 + k] + dx2 * gi[10 + k];
-        const double ddVji = dx0 * gj[k] + dx1 * gj[5 + k] + dx2 * gj[10 + k];
-        vanalbada(fc.beta, Vi[k], ddVij, Vj[k], ddVji, Vij[k], Vji[k]);
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        Vij[k] = Vi[k];
-        Vji[k] = Vj[k];
-      }
-    }
-    // checkReconstructedValues (EdgeCore.C:137-166, VarFcnSGEuler.h:90-110);
-    // with the failsafe the failing sides are tagged
-    const bool bi = Vij[0] <= 0.0 || Vij[4] + g.pstiff <= 0.0, bj = Vji[0] <= 0.0 || Vji[4] + g.pstiff <= 0.0;
+  for (int k = 0; k < 5; ++k) Ff[5 * (size_t)q + k] = fl[k];
+}
+
+// ALL: a wave per slice, lane r takes the upper edges of its node in turn
+// (node data in registers, P summed here); otherwise a wave per (slice, k)
+// pair.  The first nfb blocks take the boundary-face slots.
+template <bool SECOND, bool LM, bool ALL>
+__global__ __launch_bounds__(kBlock) void k_flux_edges(DevTables t, int nfb, const double *__restrict__ V,
+                                                       const double *__restrict__ grad, FluxConsts fc,
+                                                       double *__restrict__ Fm, double *__restrict__ P,
+                                                       double *__restrict__ Ff, int *__restrict__ err,
+                                                       int *__restrict__ tag0, const int *__restrict__ done) {
+  if (done && *done) return;
+  if ((int)blockIdx.x < nfb) {
+    const int q = blockIdx.x * kBlock + (int)threadIdx.x;
+    if (q < 3 * t.F) face_slot_flux(t, V, fc, q, Ff);
+    return;
+  }
+  const int nw = ALL ? t.ns : t.nup;
+  const int nb = (nw + kBlock / kWave - 1) / (kBlock / kWave);
+  const int w = xcd_chunk(blockIdx.x - nfb, nb) * (kBlock / kWave) + (int)(threadIdx.x / kWave);
+  if (w >= nw) return;
+  const int sl = ALL ? w : t.upslice[w];
+  const int kb = t.up.kptr[sl], ke = t.up.kptr[sl + 1];
+  const int lane = lane_id();
+  const int i = sl * kWave + lane;
+  const bool live = i < t.N;
+  const int ii = live ? i : t.N - 1;
+  const int deg = live ? t.eup[i + 1] - t.eup[i] : 0;
+  double Vi[5], xi[3] = {0.0, 0.0, 0.0}, gi[15];
+  load_state<kFromVil>(V, ii, Vi);
+  if (SECOND || LM) load_x(t, ii, xi);
+  if (SECOND) load_il<15>(grad, ii, gi);
+  double p[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int kk = ALL ? kb : w; kk < (ALL ? ke : w + 1); ++kk) {
+    const bool act = kk - kb < deg;
+    const int pos = t.up.koff[kk] + lanes_below(act);
+    if (!act) continue;
+    const int j = t.up.idx[pos];
+    double Vj[5], xj[3] = {0.0, 0.0, 0.0}, gj[15];
+    load_state<kFromVil>(V, j, Vj);
+    if (SECOND || LM) load_x(t, j, xj);
+    if (SECOND) load_il<15>(grad, j, gj);
+    double nv[3];
+    stream_load<3, ALL>(t.pnormal, pos, nv);
+    double f[5];
+    bool bi, bj;
+    edge_flux<SECOND, LM>(fc, Vi, xi, gi, Vj, xj, gj, nv, f, bi, bj);
     if (bi || bj) {
       atomicAdd(err, (int)bi + (int)bj);
-      if (tag0) {
+      if (tag0) {  // with the failsafe the failing sides are tagged
         if (bi) tag0[i] = 1;
         if (bj) tag0[j] = 1;
       }
     }
-    const double nv[3] = {t.normal[3 * (size_t)l], t.normal[3 * (size_t)l + 1], t.normal[3 * (size_t)l + 2]};
-    double f[5];
-    if (sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]) < 1e-18) {
+    stream_store<5, ALL>(Fm, pos, f);
 #pragma unroll
-      for (int k = 0; k < 5; ++k) f[k] = 0.0;
-    } else if (LM) {
-      roe_turkel_flux(g, fc.lm, true, nv, length, Vij, Vji, f);
-    } else {
-      roeflux7(g, nv, 0.0, Vij, Vji, f);
-    }
-    double *dst = Fm + 5 * (size_t)l;  // contiguous in edge order
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      sf[k * (FB + 1) + tid] = f[k];
-      dst[k] = f[k];
-    }
+    for (int k = 0; k < 5; ++k) p[k] += f[k];
   }
-  __syncthreads();
-  const int nr = r1 - r0;
-  for (int idx = tid; idx < nr * 5; idx += FB) {
-    const int rr = idx / 5, q = idx - 5 * rr;
-    const int r = r0 + rr;
-    const int b = t.eup[r] - l0, eend = t.eup[r + 1] - l0;
-    double s = 0.0;
-    for (int e = b; e < eend; ++e) s += sf[q * (FB + 1) + e];
-    P[5 * (size_t)r + q] = s;
-  }
+  if (ALL && live) store_il<5>(P, i, p);
+}
+
+__global__ __launch_bounds__(kBlock) void k_face_flux(DevTables t, const double *__restrict__ V, FluxConsts fc,
+                                                      double *__restrict__ Ff, const int *__restrict__ done) {
+  if (done && *done) return;
+  const int q = blockIdx.x * kBlock + (int)threadIdx.x;
+  if (q < 3 * t.F) face_slot_flux(t, V, fc, q, Ff);
 }
 
 // ---------------------------------------------------------------------------
@@ -295,37 +554,23 @@ __global__ __launch_bounds__(kGradStrip) void k_gradients_staged(DevTables t, co
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
     Vn[k] = sv[k * kGradHalo + hn];
-    Vout[5 * (size_t)n + k] = Vn[k];
+    Vout[il<5>(n, k)] = Vn[k];
   }
-  const double xn0 = sv[5 * kGradHalo + hn], xn1 = sv[6 * kGradHalo + hn], xn2 = sv[7 * kGradHalo + hn];
-  const double *L = t.lsq6 + 6 * (size_t)n;
-  const double or11 = L[0], or22 = L[1], or33 = L[2], r12or11 = L[3], r23or22 = L[4], psi = L[5];
-  double acc[15];
+  const double xn[3] = {sv[5 * kGradHalo + hn], sv[6 * kGradHalo + hn], sv[7 * kGradHalo + hn]};
+  double L[6], acc[15];
+  load_lsq(t, n, L);
 #pragma unroll
   for (int q = 0; q < 15; ++q) acc[q] = 0.0;
   const int e0 = t.rowptr[n], e1 = t.rowptr[n + 1];
   for (int e = e0; e < e1; ++e) {
     const int hm = t.gloc[e];
-    const double dx0 = sv[5 * kGradHalo + hm] - xn0, dx1 = sv[6 * kGradHalo + hm] - xn1,
-                 dx2 = sv[7 * kGradHalo + hm] - xn2;
-    const double alpha1 = dx0 * or11 * or11;
-    const double alpha2 = (dx1 - r12or11 * dx0) * or22 * or22;
-    const double alpha3 = (dx2 - r23or22 * dx1 + psi * dx0) * or33 * or33;
-    const double w0 = alpha1 - r12or11 * alpha2 + psi * alpha3;
-    const double w1 = alpha2 - r23or22 * alpha3;
-    const double w2 = alpha3;
+    const double xm[3] = {sv[5 * kGradHalo + hm], sv[6 * kGradHalo + hm], sv[7 * kGradHalo + hm]};
+    double Vm[5];
 #pragma unroll
-    for (int q = 0; q < 5; ++q) {
-      const double d = sv[q * kGradHalo + hm] - Vn[q];
-      acc[q] += w0 * d;
-      acc[5 + q] += w1 * d;
-      acc[10 + q] += w2 * d;
-    }
+    for (int q = 0; q < 5; ++q) Vm[q] = sv[q * kGradHalo + hm];
+    lsq_add(L, xm, xn, Vm, Vn, acc);
   }
-  double2 *g2 = reinterpret_cast<double2 *>(grad + 16 * (size_t)n);
-#pragma unroll
-  for (int q = 0; q < 7; ++q) g2[q] = make_double2(acc[2 * q], acc[2 * q + 1]);
-  g2[7] = make_double2(acc[14], 0.0);
+  store_il<15>(grad, n, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -335,8 +580,7 @@ __global__ __launch_bounds__(kGradStrip) void k_gradients_staged(DevTables t, co
 //     field with consecutive lanes on consecutive doubles of a record
 //     (V: 5, X: 3 of 4, gradients: 15 of 16), so the loads coalesce.  Lane k
 //     computes edge l0 + k from LDS exactly as the per-lane kernel does; the
-//     fluxes go back through the same LDS for coalesced Fm stores and the
-//     per-row sums P.
+//     fluxes go through the same LDS for the per-row sums P.
 // ---------------------------------------------------------------------------
 template <bool SECOND>
 __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const double *__restrict__ V,
@@ -360,7 +604,6 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
   const int r0 = ch.x, r1 = ch.y, l0 = ch.z, l1 = ch.w;
   const int H = hr.y - hr.x;
   const int tid = threadIdx.x;
-  const Gas &g = fc.gas;
   for (int h = tid; h < H; h += kFluxStrip) sidx[h] = t.fhalo[hr.x + h];
   __syncthreads();
   // all of a lane's staging loads are in flight together: consecutive lanes
@@ -374,7 +617,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
   for (int r = 0; r < PV; ++r) {
     const int q = tid + r * kFluxStrip;
     const int h = q / 5, f = q - 5 * h;
-    rv[r] = q < 5 * H ? V[5 * (size_t)sidx[min(h, H - 1)] + f] : 0.0;
+    rv[r] = q < 5 * H ? V[il<5>(sidx[min(h, H - 1)], f)] : 0.0;
   }
   if (SECOND) {
 #pragma unroll
@@ -385,7 +628,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
 #pragma unroll
     for (int r = 0; r < PG; ++r) {
       const int q = tid + r * kFluxStrip;
-      rg[r] = q < 16 * H ? grad[16 * (size_t)sidx[min(q >> 4, H - 1)] + (q & 15)] : 0.0;
+      rg[r] = q < 16 * H && (q & 15) < 15 ? grad[il<15>(sidx[min(q >> 4, H - 1)], q & 15)] : 0.0;
     }
   }
 #pragma unroll
@@ -419,37 +662,18 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
       Vi[k] = si[k];
       Vj[k] = sj[k];
     }
-    double Vij[5], Vji[5];
-    if (SECOND) {
-      const double dx0 = sj[5] - si[5], dx1 = sj[6] - si[6], dx2 = sj[7] - si[7];
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        const double ddVij = dx0 * si[8 + k] + dx1 * si[13 + k] + dx2 * si[18 + k];
-        const double ddVji = dx0 * sj[8 + k] + dx1 * sj[13 + k] + dx2 * sj[18 + k];
-        vanalbada(fc.beta, Vi[k], ddVij, Vj[k], ddVji, Vij[k], Vji[k]);
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        Vij[k] = Vi[k];
-        Vji[k] = Vj[k];
-      }
-    }
-    // checkReconstructedValues (EdgeCore.C:137-166, VarFcnSGEuler.h:90-110)
-    const int bad = (Vij[0] <= 0.0 || Vij[4] + g.pstiff <= 0.0) + (Vji[0] <= 0.0 || Vji[4] + g.pstiff <= 0.0);
-    if (bad) atomicAdd(err, bad);
-    const double nv[3] = {t.normal[3 * (size_t)l], t.normal[3 * (size_t)l + 1], t.normal[3 * (size_t)l + 2]};
-    if (sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]) >= 1e-18) roeflux7(g, nv, 0.0, Vij, Vji, f);
+    double nv[3];
+    load_il<3>(t.pnormal, t.epos[l], nv);
+    bool bi, bj;
+    edge_flux<SECOND, false>(fc, Vi, si + 5, si + 8, Vj, sj + 5, sj + 8, nv, f, bi, bj);
+    if (bi || bj) atomicAdd(err, (int)bi + (int)bj);
   }
   __syncthreads();  // the node staging is dead: reuse it for the fluxes
   double *sf = sh;
 #pragma unroll
   for (int k = 0; k < 5; ++k) sf[k * FS + tid] = f[k];
   __syncthreads();
-  for (int q = tid; q < 5 * ne; q += kFluxStrip) {
-    const int e = q / 5, k = q - 5 * e;
-    Fm[5 * (size_t)l0 + q] = sf[k * FS + e];
-  }
+  if (tid < ne) store_il<5>(Fm, t.epos[l0 + tid], f);
   const int nr = r1 - r0;
   for (int idx = tid; idx < nr * 5; idx += kFluxStrip) {
     const int rr = idx / 5, q = idx - 5 * rr;
@@ -457,92 +681,105 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
     const int eb = t.eup[r] - l0, eend = t.eup[r + 1] - l0;
     double s = 0.0;
     for (int e = eb; e < eend; ++e) s += sf[q * FS + e];
-    P[5 * (size_t)r + q] = s;
+    P[il<5>(r, q)] = s;
   }
 }
 
 // ---------------------------------------------------------------------------
-// 3. node assembly: lower edges, upper-edge partial sum (formed here from the
-//    edge fluxes for a row of more than fblock upper edges), faces, 1/V
+// 3. node assembly: lower edges, upper-edge sum, faces, 1/V
 // ---------------------------------------------------------------------------
-// vrow / vc (or null): the Navier-Stokes Galerkin contributions of the
-// node's elements, one contiguous run per node in element order, added
-// before the 1/V scaling
-__global__ __launch_bounds__(kBlock) void k_flux_nodes(DevTables t, const double *__restrict__ V,
-                                                       const double *__restrict__ Fm,
-                                                       const double *__restrict__ P, FluxConsts fc, int scale,
-                                                       const int *__restrict__ vrow, const double *__restrict__ vc,
+// s -= (LOWER: edge positions in rows.idx) or += (upper edges: the entries'
+// own places) the fluxes of this lane's row, in row order; four entries'
+// loads in flight together.
+template <bool LOWER>
+__device__ __forceinline__ void add_slots(const RowSlices &rows, int sl, int deg, const double *__restrict__ Fm,
+                                          double s[5]) {
+  constexpr int B = 4;
+  const int kb = rows.kptr[sl], kn = rows.kptr[sl + 1] - kb;
+  for (int k0 = 0; k0 < kn; k0 += B) {
+    int pos[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int off = k0 + u < kn ? rows.koff[kb + k0 + u] : 0;
+      const bool act = k0 + u < deg;
+      const int e = off + lanes_below(act);
+      pos[u] = act ? (LOWER ? rows.idx[e] : e) : 0;
+    }
+    double v[B][5];
+#pragma unroll
+    for (int u = 0; u < B; ++u) load_il<5>(Fm, pos[u], v[u]);
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (k0 + u < deg) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) s[k] = LOWER ? s[k] - v[u][k] : s[k] + v[u][k];
+      }
+  }
+}
+
+// P null: the upper-edge sum is formed here from the edge fluxes, in edge
+// order.  vg (or null): the node sums of the Navier-Stokes Galerkin
+// contributions (momentum and energy), added before the 1/V scaling.
+// host_err (or null): pinned copy of the error count of the finished flux
+// pass, so a synchronous caller needs no copy of its own.
+__global__ __launch_bounds__(kBlock) void k_flux_nodes(DevTables t, const double *__restrict__ Fm,
+                                                       const double *__restrict__ P, const double *__restrict__ Ff,
+                                                       int scale, const double *__restrict__ vg,
+                                                       const int *__restrict__ err, int *__restrict__ host_err,
                                                        double *__restrict__ R, const int *__restrict__ done) {
   if (done && *done) return;
-  const int nb = (t.N + kBlock - 1) / kBlock;
-  const int n = xcd_chunk(blockIdx.x, nb) * kBlock + (int)threadIdx.x;
-  if (n >= t.N) return;
+  if (host_err && blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(host_err, *err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  const int sl = wave_slice(t);
+  if (sl >= t.ns) return;
+  const int lane = lane_id();
+  const int n = sl * kWave + lane;
+  const bool live = n < t.N;
   double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  const int q0 = t.lrow[n], q1 = t.lrow[n + 1];
-#pragma unroll 4
-  for (int q = q0; q < q1; ++q) {
-    const size_t base = 5 * (size_t)t.ledge[q];
+  add_slots<true>(t.lo, sl, live ? t.lrow[n + 1] - t.lrow[n] : 0, Fm, s);
+  if (P) {
+    if (live) {
+      double p[5];
+      load_il<5>(P, n, p);
 #pragma unroll
-    for (int k = 0; k < 5; ++k) s[k] -= Fm[base + k];
-  }
-  const int u0 = t.eup[n], u1 = t.eup[n + 1];
-  if (u1 - u0 > t.fblock) {
-    // a row cut over several flux blocks: its upper-edge sum, in edge order
+      for (int k = 0; k < 5; ++k) s[k] += p[k];
+    }
+  } else {
     double p[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int l = u0; l < u1; ++l)
-#pragma unroll
-      for (int k = 0; k < 5; ++k) p[k] += Fm[5 * (size_t)l + k];
+    add_slots<false>(t.up, sl, live ? t.eup[n + 1] - t.eup[n] : 0, Fm, p);
 #pragma unroll
     for (int k = 0; k < 5; ++k) s[k] += p[k];
-  } else {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) s[k] += P[5 * (size_t)n + k];
   }
-  const int f0 = t.frow[n], f1 = t.frow[n + 1];
-  if (f0 < f1) {
-    double Vn[5];
+  if (!live) return;
+  for (int q = t.frow[n]; q < t.frow[n + 1]; ++q)
 #pragma unroll
-    for (int k = 0; k < 5; ++k) Vn[k] = V[5 * (size_t)n + k];
-    for (int q = f0; q < f1; ++q) {
-      const int face = t.fidx[q];
-      const int code = t.fcode[face];
-      const double nv[3] = {t.fnorm3[3 * (size_t)face], t.fnorm3[3 * (size_t)face + 1],
-                            t.fnorm3[3 * (size_t)face + 2]};
-      double fl[5];
-      if (is_wall_code(code)) {
-        wallflux(nv, 0.0, Vn, fl);
-      } else {
-        const double *ub = (code == AEROFX_BC_INLET || code == -AEROFX_BC_INLET) ? fc.ub_in : fc.ub_out;
-        boundflux5(fc.gas, nv, 0.0, Vn, ub, fl);
-      }
+    for (int k = 0; k < 5; ++k) s[k] += Ff[5 * (size_t)q + k];
+  if (vg) {
+    double g[4];
+    load_il<4>(vg, n, g);
 #pragma unroll
-      for (int k = 0; k < 5; ++k) s[k] += fl[k];
-    }
-  }
-  if (vc) {
-    double g[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int q = vrow[n]; q < vrow[n + 1]; ++q)
-#pragma unroll
-      for (int k = 0; k < 5; ++k) g[k] += vc[5 * (size_t)q + k];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) s[k] += g[k];
+    for (int k = 0; k < 4; ++k) s[1 + k] += g[k];
   }
   const double ic = t.invcv[n];
 #pragma unroll
   for (int k = 0; k < 5; ++k) R[5 * (size_t)n + k] = scale ? s[k] * ic : s[k];
 }
 
-__global__ void k_primitive(int N, const double *__restrict__ U, Gas g, double *__restrict__ V,
-                            const int *__restrict__ done) {
+// V = V(U), as [N][5] (IL false) or interleaved; clears *err (or null)
+template <bool IL>
+__global__ __launch_bounds__(kBlock) void k_primitive(int N, const double *__restrict__ U, Gas g,
+                                                      double *__restrict__ V, int *__restrict__ err,
+                                                      const int *__restrict__ done) {
   if (done && *done) return;
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  const int n = blockIdx.x * kBlock + threadIdx.x;
+  if (err && n == 0) *err = 0;
   if (n >= N) return;
   double u[5], v[5];
 #pragma unroll
   for (int k = 0; k < 5; ++k) u[k] = U[5 * (size_t)n + k];
   prim_from_cons(u, g, v);
 #pragma unroll
-  for (int k = 0; k < 5; ++k) V[5 * (size_t)n + k] = v[k];
+  for (int k = 0; k < 5; ++k) V[IL ? il<5>(n, k) : 5 * (size_t)n + k] = v[k];
 }
 
 __global__ void k_zero_int(int *p, int n, const int *done) {
@@ -554,64 +791,91 @@ __global__ void k_zero_int(int *p, int n, const int *done) {
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-template <bool SECOND, int FB>
-static void launch_flux_edges(aerofx_ctx *c, const ResidualBufs &b, const int *done) {
+// Slices from which a wave takes whole rows of edges and the streamed data
+// bypass the caches; below, one edge per lane keeps more waves busy and the
+// fluxes (40 B an edge) are still cached when the node pass reads them.  Flux
+// and node pass, rows against edges: 106 / 104 us at 275k nodes (4291
+// slices), 192 / 202 at 531k (8304), 672 / 757 at 2.1M.
+constexpr int kRowWaveSlices = 6144;
+
+static size_t halo_lds(const DevTables &t) { return 4 * sizeof(double2) * (size_t)t.halo_cap; }
+// as many workgroups as fit all CUs (by LDS, and four by the registers)
+static dim3 halo_grid(const DevTables &t) {
+  const int fit = (int)std::max<size_t>(1, std::min<size_t>(4, kLdsPerCu / halo_lds(t)));
+  return dim3((unsigned)std::min((t.ns + kNumXcd - 1) / kNumXcd * kNumXcd, kNumCu * fit));
+}
+
+template <bool SECOND, bool LM>
+static void launch_flux_edges(aerofx_ctx *c, const ResidualBufs &b, bool all, const int *done) {
   const DevTables &t = c->tab;
-  if (c->fc.low_mach)
-    hipLaunchKernelGGL((k_flux_edges<SECOND, FB, true>), dim3(t.nfchunks), dim3(FB), 0, c->stream, t, b.V, b.grad,
-                       c->fc, b.Fm, b.P, c->d_err, b.tag0, done);
+  const int nfb = (3 * t.F + kBlock - 1) / kBlock;
+  const dim3 grid(nfb + slice_grid(all ? t.ns : t.nup).x);
+  if (grid.x == 0) return;
+  if (all)
+    hipLaunchKernelGGL((k_flux_edges<SECOND, LM, true>), grid, dim3(kBlock), 0, c->stream, t, nfb, b.V, b.grad, c->fc,
+                       b.Fm, b.P, c->d_Ff, c->d_err, b.tag0, done);
   else
-    hipLaunchKernelGGL((k_flux_edges<SECOND, FB, false>), dim3(t.nfchunks), dim3(FB), 0, c->stream, t, b.V, b.grad,
-                       c->fc, b.Fm, b.P, c->d_err, b.tag0, done);
+    hipLaunchKernelGGL((k_flux_edges<SECOND, LM, false>), grid, dim3(kBlock), 0, c->stream, t, nfb, b.V, b.grad,
+                       c->fc, b.Fm, b.P, c->d_Ff, c->d_err, b.tag0, done);
 }
 
 int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, double *R, bool scale,
-                         const int *done) {
+                         const int *done, int *host_err) {
   const DevTables &t = c->tab;
   // the staged kernels evaluate ROEFLUX7 only, without the failsafe
   const bool staged = t.ngb > 0 && c->residual_kernels == AEROFX_RESIDUAL_STAGED && !c->fc.low_mach && !c->failsafe;
+  const bool rows = t.ns >= kRowWaveSlices;
+  const bool all = staged || rows;  // P formed by the flux pass
+  const dim3 ngrid((t.N + kBlock - 1) / kBlock), blk(kBlock);
   if (c->p.second_order) {
     ProfScope ps(c, AEROFX_TIMER_NODAL_GRAD);
-    if (staged)
+    if (staged) {
       hipLaunchKernelGGL(k_gradients_staged, dim3(t.ngb), dim3(kGradStrip), 0, c->stream, t, U, c->gas, b.V,
                          b.grad, c->d_err, done);
-    else
-      hipLaunchKernelGGL((k_gradients<true, false>), dim3((t.N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream,
-                         t, U, c->gas, b.V, b.grad, nullptr, nullptr, nullptr, c->d_err, done);
+    } else if (t.halo_cap) {
+      hipLaunchKernelGGL(k_gradients_halo, halo_grid(t), dim3(kHaloThreads), halo_lds(t), c->stream, t, U, c->gas,
+                         b.V, b.grad, c->d_err, done);
+    } else {
+      hipLaunchKernelGGL((k_gradients<kFromU, false>), slice_grid(t.ns), blk, 0, c->stream, t, U, c->gas, b.V,
+                         b.grad, nullptr, nullptr, nullptr, c->d_err, done);
+    }
   } else {
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, c->stream, c->d_err, 1, done);
-    hipLaunchKernelGGL(k_primitive, dim3((t.N + 255) / 256), dim3(256), 0, c->stream, t.N, U, c->gas, b.V, done);
+    hipLaunchKernelGGL(k_primitive<true>, ngrid, blk, 0, c->stream, t.N, U, c->gas, b.V, c->d_err, done);
   }
   {
     ProfScope ps(c, AEROFX_TIMER_FV_TERM);
-    if (staged && c->p.second_order)
-      hipLaunchKernelGGL(k_flux_staged<true>, dim3(t.nfb), dim3(kFluxStrip), 0, c->stream, t, b.V, b.grad,
-                         c->fc, b.Fm, b.P, c->d_err, done);
-    else if (staged)
-      hipLaunchKernelGGL(k_flux_staged<false>, dim3(t.nfb), dim3(kFluxStrip), 0, c->stream, t, b.V, b.grad,
-                         c->fc, b.Fm, b.P, c->d_err, done);
-    else if (c->p.second_order && t.fblock == kFluxBlockSmall)
-      launch_flux_edges<true, kFluxBlockSmall>(c, b, done);
-    else if (c->p.second_order)
-      launch_flux_edges<true, kFluxBlock>(c, b, done);
-    else if (t.fblock == kFluxBlockSmall)
-      launch_flux_edges<false, kFluxBlockSmall>(c, b, done);
-    else
-      launch_flux_edges<false, kFluxBlock>(c, b, done);
+    if (staged) {
+      if (t.F > 0)
+        hipLaunchKernelGGL(k_face_flux, dim3((3 * t.F + kBlock - 1) / kBlock), blk, 0, c->stream, t, b.V, c->fc,
+                           c->d_Ff, done);
+      if (c->p.second_order)
+        hipLaunchKernelGGL(k_flux_staged<true>, dim3(t.nfb), dim3(kFluxStrip), 0, c->stream, t, b.V, b.grad,
+                           c->fc, b.Fm, b.P, c->d_err, done);
+      else
+        hipLaunchKernelGGL(k_flux_staged<false>, dim3(t.nfb), dim3(kFluxStrip), 0, c->stream, t, b.V, b.grad,
+                           c->fc, b.Fm, b.P, c->d_err, done);
+    } else if (c->p.second_order && c->fc.low_mach) {
+      launch_flux_edges<true, true>(c, b, rows, done);
+    } else if (c->p.second_order) {
+      launch_flux_edges<true, false>(c, b, rows, done);
+    } else if (c->fc.low_mach) {
+      launch_flux_edges<false, true>(c, b, rows, done);
+    } else {
+      launch_flux_edges<false, false>(c, b, rows, done);
+    }
   }
   // the Navier-Stokes Galerkin term (SpaceOperator.C:570-573): its element
-  // pass, summed by the node pass with the fluxes (or, without the
-  // contribution buffer, the per-node kernel after it)
+  // pass and node sums, added by the node pass (or, without the contribution
+  // buffer, the per-node kernel after it)
   const bool fold = c->viscous && c->d_visc_c;
   if (fold) {
     int rc = launch_visc_elements(c, b.V, done);
-    if (rc) return rc;
+    if (rc || (rc = launch_visc_sum(c, done))) return rc;
   }
   {
     ProfScope ps(c, AEROFX_TIMER_FV_NODES);
-    hipLaunchKernelGGL(k_flux_nodes, dim3((t.N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, t, b.V,
-                       b.Fm, b.P, c->fc, scale ? 1 : 0, fold ? c->elem->ntrow : nullptr,
-                       fold ? c->d_visc_c : nullptr, R, done);
+    hipLaunchKernelGGL(k_flux_nodes, slice_grid(t.ns), blk, 0, c->stream, t, b.Fm, all ? b.P : nullptr, c->d_Ff,
+                       scale ? 1 : 0, fold ? c->d_visc_g : nullptr, c->d_err, host_err, R, done);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_hip_error(e, "residual launch");
@@ -637,9 +901,9 @@ __global__ void k_fs_finalize(DevTables t, const int *__restrict__ tag0, int *__
   if (tag1[n]) mask[n] = 1;
 }
 
+// the count that the residual's node pass left in h_err[0]
 static int read_error_count(aerofx_ctx *c, int *count) {
-  hipError_t e = hipMemcpyAsync(c->h_err, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  hipError_t e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) return set_hip_error(e, "residual error count");
   *count = c->h_err[0];
   return 0;
@@ -650,14 +914,14 @@ int residual_failsafe(aerofx_ctx *c, const ResidualBufs &b, const double *U, dou
   ResidualBufs b1 = b;
   const int N = c->N;
   b1.tag0 = fs ? c->d_fs : nullptr;
-  int rc = launch_residual_with(c, b1, U, R, scale);
+  int rc = launch_residual_with(c, b1, U, R, scale, nullptr, c->h_err);
   if (rc || (rc = read_error_count(c, count))) return rc;
   if (!fs || *count == 0) return 0;
   // Domain::computeFiniteVolumeTerm with failsafe (Domain.C:884-917)
   hipLaunchKernelGGL(k_fs_finalize, dim3((N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->tab, c->d_fs,
                      c->d_fs + N, c->d_fs + 2 * (size_t)N);
   c->fs_any = true;
-  if ((rc = launch_residual_with(c, b, U, R, scale)) || (rc = read_error_count(c, count))) return rc;
+  if ((rc = launch_residual_with(c, b, U, R, scale, nullptr, c->h_err)) || (rc = read_error_count(c, count))) return rc;
   // FailSafe = On clears the tags after the fix; AlwaysOn keeps them
   if (c->failsafe == 1) hipLaunchKernelGGL(k_zero_int, dim3((2 * N + 63) / 64), dim3(64), 0, c->stream, c->d_fs,
                                            2 * N, nullptr);
@@ -672,14 +936,22 @@ int refuse_failsafe_nodes(aerofx_ctx *c, const char *who) {
 }
 
 int launch_gradients_v(aerofx_ctx *c, const double *V, double *ddx, double *ddy, double *ddz) {
-  hipLaunchKernelGGL((k_gradients<false, true>), dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->tab, V,
+  hipLaunchKernelGGL((k_gradients<kFromV, true>), slice_grid(c->tab.ns), dim3(kBlock), 0, c->stream, c->tab, V,
                      c->gas, nullptr, nullptr, ddx, ddy, ddz, nullptr, nullptr);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_hip_error(e, "gradients launch");
 }
 
 int launch_primitive(aerofx_ctx *c, const double *U, double *V) {
-  hipLaunchKernelGGL(k_primitive, dim3((c->N + 255) / 256), dim3(256), 0, c->stream, c->N, U, c->gas, V, nullptr);
+  hipLaunchKernelGGL(k_primitive<false>, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N, U,
+                     c->gas, V, nullptr, nullptr);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : set_hip_error(e, "primitive launch");
+}
+
+int launch_primitive_il(aerofx_ctx *c, const double *U) {
+  hipLaunchKernelGGL(k_primitive<true>, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N, U,
+                     c->gas, c->d_V, nullptr, nullptr);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_hip_error(e, "primitive launch");
 }

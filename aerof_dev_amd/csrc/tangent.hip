@@ -40,7 +40,8 @@ struct Tangent {
   double *dfn = nullptr;  // [F][3] full face normal
   double *dF = nullptr;   // [E][5]
   // the state part of the exact product operator (MatVecProdH2), kept from
-  // its selection: primitive state [N][5] and LSQ gradients [N][16]
+  // its selection: primitive state and LSQ gradients,
+  // interleaved as d_V and d_grad
   double *V0 = nullptr, *G0 = nullptr;
 };
 
@@ -266,14 +267,16 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_flux(DevTables t, const doubl
   Dual Vi[5], Vj[5], Vij[5], Vji[5];
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
-    Vi[k] = Dual(V[5 * (size_t)i + k], dV[5 * (size_t)i + k]);
-    Vj[k] = Dual(V[5 * (size_t)j + k], dV[5 * (size_t)j + k]);
+    Vi[k] = Dual(V[il<5>(i, k)], dV[5 * (size_t)i + k]);
+    Vj[k] = Dual(V[il<5>(j, k)], dV[5 * (size_t)j + k]);
   }
   if (SECOND) {
     const Dual dx0 = coord(t.X4, dX, j, 0) - coord(t.X4, dX, i, 0);
     const Dual dx1 = coord(t.X4, dX, j, 1) - coord(t.X4, dX, i, 1);
     const Dual dx2 = coord(t.X4, dX, j, 2) - coord(t.X4, dX, i, 2);
-    const double *gi = grad + 16 * (size_t)i, *gj = grad + 16 * (size_t)j;
+    double gi[15], gj[15];
+    load_il<15>(grad, i, gi);
+    load_il<15>(grad, j, gj);
     const double *hi = dG + 16 * (size_t)i, *hj = dG + 16 * (size_t)j;
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -325,7 +328,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_nodes(DevTables t, const doub
   if (f0 < f1) {
     Dual Vn[5];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) Vn[k] = Dual(V[5 * (size_t)n + k], dV[5 * (size_t)n + k]);
+    for (int k = 0; k < 5; ++k) Vn[k] = Dual(V[il<5>(n, k)], dV[5 * (size_t)n + k]);
     const double third = 1.0 / 3.0;
     for (int q = f0; q < f1; ++q) {
       const int face = t.fidx[q];
@@ -436,12 +439,12 @@ int launch_h2_select(aerofx_ctx *c, const double *Q) {
   if (rc) return rc;
   Tangent *g = c->tan;
   const DevTables &t = c->tab;
-  if (!g->V0 && ((rc = alloc_n(c, 5 * (size_t)t.N, &g->V0)) || (rc = alloc_n(c, 16 * (size_t)t.N, &g->G0))))
+  if (!g->V0 && ((rc = alloc_n(c, il_count<5>(t.N), &g->V0)) || (rc = alloc_n(c, il_count<15>(t.N), &g->G0))))
     return rc;
   if ((rc = launch_residual(c, Q, g->S, false))) return rc;
-  hipError_t e = hipMemcpyAsync(g->V0, c->d_V, 5 * sizeof(double) * (size_t)t.N, hipMemcpyDeviceToDevice, c->stream);
+  hipError_t e = hipMemcpyAsync(g->V0, c->d_V, sizeof(double) * il_count<5>(t.N), hipMemcpyDeviceToDevice, c->stream);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(g->G0, c->d_grad, 16 * sizeof(double) * (size_t)t.N, hipMemcpyDeviceToDevice, c->stream);
+    e = hipMemcpyAsync(g->G0, c->d_grad, sizeof(double) * il_count<15>(t.N), hipMemcpyDeviceToDevice, c->stream);
   if (e != hipSuccess) return set_hip_error(e, "h2 select copy");
   hipLaunchKernelGGL(k_fill0, grid_for(3LL * t.E), dim3(kTanBlock), 0, c->stream, 3 * (size_t)t.E, g->dn);
   hipLaunchKernelGGL(k_fill0, grid_for(t.N), dim3(kTanBlock), 0, c->stream, (size_t)t.N, g->dcv);

@@ -37,8 +37,7 @@ __device__ __forceinline__ void load_element(const int4 *__restrict__ tets, cons
     x[k][0] = p.x;
     x[k][1] = p.y;
     x[k][2] = p.z;
-#pragma unroll
-    for (int q = 0; q < 5; ++q) v[k][q] = V[5 * (size_t)id[k] + q];
+    load_il<5>(V, id[k], v[k]);
   }
 }
 
@@ -90,8 +89,8 @@ __global__ __launch_bounds__(kBlock) void k_visc_residual(int N, const int *__re
 }
 
 // Element pass of the residual: each element once, its four vertex
-// contributions vol (r . g_j) to C[pos[4 t + j]][5], pos the place of slot
-// (t, j) in the node->element slot list, so that the node pass below reads
+// contributions vol (r . g_j) to C[pos[4 t + j]][4], pos the place of slot
+// (t, j) in the node->element slot list, so that the node sums below read
 // each node's contributions as one contiguous run (in element order: the
 // sums of k_visc_residual, term for term) and consecutive nodes read
 // consecutive runs.
@@ -118,10 +117,28 @@ __global__ __launch_bounds__(kBlock) void k_visc_elements(int T, const int4 *__r
   for (int j = 0; j < 4; ++j) {
     double c[5];
     ns_node_residual(e, g[j], vol, c);
-    double *out = C + 5 * (size_t)pj[j];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) out[k] = c[k];
+    // the density row is zero: four values, one 32-B piece
+    *reinterpret_cast<double4 *>(C + 4 * (size_t)pj[j]) = make_double4(c[1], c[2], c[3], c[4]);
   }
+}
+
+// Node sums of those contributions, four lanes per node (one per component),
+// in element order: a wave's load touches the runs of 16 nodes, and four
+// slots share a line.  One lane per node and five records per slot touched a
+// line per lane and load: the node pass of the residual took 85 us at 179k
+// nodes.
+__global__ __launch_bounds__(kBlock) void k_visc_sum(int N, const int *__restrict__ ntrow,
+                                                     const double *__restrict__ C, double *__restrict__ G,
+                                                     const int *__restrict__ done) {
+  if (done && *done) return;
+  const int idx = blockIdx.x * kBlock + threadIdx.x;
+  const int n = idx >> 2, k = idx & 3;
+  if (n >= N) return;
+  const int s1 = ntrow[n + 1];
+  double acc = 0.0;
+#pragma unroll 8
+  for (int s = ntrow[n]; s < s1; ++s) acc += C[4 * (size_t)s + k];
+  G[il<4>(n, k)] = acc;
 }
 
 // Transposed element pass: each element once, C[pos[4 t + k]] = vol (d r /
@@ -764,20 +781,21 @@ int launch_visc_elements(aerofx_ctx *c, const double *V, const int *done) {
   return check("viscous element launch");
 }
 
+int launch_visc_sum(aerofx_ctx *c, const int *done) {
+  ProfScope ps(c, AEROFX_TIMER_FE_TERM);
+  hipLaunchKernelGGL(k_visc_sum, dim3((unsigned)((4 * (size_t)c->N + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->stream, c->N,
+                     c->elem->ntrow, c->d_visc_c, c->d_visc_g, done);
+  return check("viscous sum launch");
+}
+
+// without the contribution buffer: each element evaluated once per vertex
 int launch_visc_residual(aerofx_ctx *c, const double *V, double *R, bool scale, const int *done) {
   if (!c->viscous) return 0;
   const ElemTables *el = c->elem;
   ProfScope ps(c, AEROFX_TIMER_FE_TERM);
-  if (c->d_visc_c) {
-    hipLaunchKernelGGL(k_visc_elements, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                       (const int4 *)el->tets, c->tab.X4, V, c->ns, (const int4 *)c->d_visc_pos, c->d_visc_c, done);
-    hipLaunchKernelGGL(k_visc_gather, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
-                       el->ntrow, c->d_visc_c, c->tab.invcv, scale ? 1 : 0, R, done);
-  } else {
-    hipLaunchKernelGGL(k_visc_residual, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
-                       el->ntrow, el->ntslot, (const int4 *)el->tets, c->tab.X4, V, c->tab.invcv, c->ns,
-                       scale ? 1 : 0, R, done);
-  }
+  hipLaunchKernelGGL(k_visc_residual, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
+                     el->ntrow, el->ntslot, (const int4 *)el->tets, c->tab.X4, V, c->tab.invcv, c->ns,
+                     scale ? 1 : 0, R, done);
   return check("viscous residual launch");
 }
 
@@ -934,11 +952,14 @@ int aerofx_ctx_set_viscous(aerofx_ctx *c, const aerofx_viscous *v) {
   // set-up, so that no residual call allocates); without the memory the
   // per-node kernel evaluates each element once per vertex instead
   if (!c->d_visc_c) {
-    void *p = nullptr, *q = nullptr;
+    void *p = nullptr, *q = nullptr, *g = nullptr;
     if (hipMalloc(&p, sizeof(double) * 20 * (size_t)c->T) == hipSuccess &&
-        hipMalloc(&q, sizeof(int) * 4 * (size_t)c->T) == hipSuccess) {
+        hipMalloc(&q, sizeof(int) * 4 * (size_t)c->T) == hipSuccess &&
+        hipMalloc(&g, sizeof(double) * il_count<4>(c->N)) == hipSuccess) {
       c->allocs.push_back(p);
       c->allocs.push_back(q);
+      c->allocs.push_back(g);
+      c->d_visc_g = (double *)g;
       c->d_visc_c = (double *)p;
       c->d_visc_pos = (int *)q;
       const int ns4 = 4 * c->T;
@@ -948,6 +969,7 @@ int aerofx_ctx_set_viscous(aerofx_ctx *c, const aerofx_viscous *v) {
     } else {
       (void)hipGetLastError();
       if (p) (void)hipFree(p);
+      if (q) (void)hipFree(q);
     }
   }
   NsConsts ns{};
