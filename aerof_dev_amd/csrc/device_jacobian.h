@@ -141,6 +141,84 @@ __device__ __forceinline__ void roejac6(double gamma_diss, const Gas &g, const d
   for (int k = 0; k < 25; ++k) jac[k] = 0.5 * H[k] * rnorm;
 }
 
+// Both Jacobian blocks of an edge seen from node n with neighbour m, through
+// the area vector en (not normalised, outward from n), without low-Mach
+// preconditioning:
+//   own = dF/dU_n = 0.5 |en| (A(Vn) + |A_roe|),  off = dF/dU_m = 0.5 |en| (A(Vm) - |A_roe|)
+// -- the matrices of roejac6 (sw = 1 and 2), from their structure instead of
+// its products: A = u_n I + (1, u, H) (x) rho d(u.n)/dU + (0, n, u_n) (x) dp/dU, and
+// |A| = |u_n| I + sum of (|lambda| - |u_n|) r (x) l over the two acoustic waves,
+// so each matrix is a diagonal and two rank-one terms, |A| is formed once for
+// both, and nothing is divided by the eigenvector norms (about 330 vector
+// instructions for the pair, two calls of roejac6 take 2200).
+__device__ __forceinline__ void euler_rank(const Gas &g, const double V[5], double n0, double n1, double n2,
+                                           double &un, double col[5], double dun[4], double dp[5]) {
+#pragma clang fp contract(on)
+  const double q = 0.5 * (V[1] * V[1] + V[2] * V[2] + V[3] * V[3]);
+  un = V[1] * n0 + V[2] * n1 + V[3] * n2;
+  col[0] = 1.0;
+  col[1] = V[1];
+  col[2] = V[2];
+  col[3] = V[3];
+  col[4] = g.gam * g.invgam1 * (V[4] + g.pstiff) * frcp(V[0]) + q;
+  dun[0] = -un;
+  dun[1] = n0;
+  dun[2] = n1;
+  dun[3] = n2;
+  dp[0] = g.gam1 * q;
+  dp[1] = -g.gam1 * V[1];
+  dp[2] = -g.gam1 * V[2];
+  dp[3] = -g.gam1 * V[3];
+  dp[4] = g.gam1;
+}
+
+__device__ __forceinline__ void roe_jac_pair(const Gas &g, const double en[3], const double Vn[5], const double Vm[5],
+                                             double own[25], double off[25]) {
+#pragma clang fp contract(on)
+  const double rn2 = en[0] * en[0] + en[1] * en[1] + en[2] * en[2];
+  const double irn = frsq(rn2), hrn = 0.5 * sqrt_from_rsq(rn2, irn);
+  const double n0 = en[0] * irn, n1 = en[1] * irn, n2 = en[2] * irn;
+  double unn, cn[5], dn[4], pn[5], unm, cm[5], dm[4], pm[5];
+  euler_rank(g, Vn, n0, n1, n2, unn, cn, dn, pn);
+  euler_rank(g, Vm, n0, n1, n2, unm, cm, dm, pm);
+  const double sn = sqrt_from_rsq(Vn[0], frsq(Vn[0])), sm = sqrt_from_rsq(Vm[0], frsq(Vm[0]));
+  const double w = frcp(sn + sm), wn = sn * w, wm = sm * w;
+  const double u = wn * Vn[1] + wm * Vm[1], v = wn * Vn[2] + wm * Vm[2], z = wn * Vn[3] + wm * Vm[3];
+  const double H = wn * cn[4] + wm * cm[4];
+  const double q = 0.5 * (u * u + v * v + z * z);
+  const double c2 = g.gam1 * (H - q);
+  const double ic = frsq(c2), c = sqrt_from_rsq(c2, ic);
+  const double un = n0 * u + n1 * v + n2 * z, an = fabs(un);
+  // (|lambda| - |u_n|) / (2 c^2) of the two waves; r = (1, u + s n, H + s u_n),
+  // l = (dp - s d(u.n) rho) of the average with s = +-c
+  const double hic2 = 0.5 * ic * ic;
+  const double ap = (fabs(un + c) - an) * hic2, am = (fabs(un - c) - an) * hic2;
+  const double cun = c * un, c0 = c * n0, c1 = c * n1, cz = c * n2;
+  const double l0 = g.gam1 * q, l1 = -g.gam1 * u, l2 = -g.gam1 * v, l3 = -g.gam1 * z;
+  const double lp[5] = {ap * (l0 - cun), ap * (l1 + c0), ap * (l2 + c1), ap * (l3 + cz), ap * g.gam1};
+  const double lm[5] = {am * (l0 + cun), am * (l1 - c0), am * (l2 - c1), am * (l3 - cz), am * g.gam1};
+  const double rp[5] = {1.0, u + c0, v + c1, z + cz, H + cun}, rm[5] = {1.0, u - c0, v - c1, z - cz, H - cun};
+  const double nn[5] = {0.0, n0, n1, n2, unn}, nm[5] = {0.0, n0, n1, n2, unm};
+#pragma unroll
+  for (int i = 0; i < 5; ++i)
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      double a = rp[i] * lp[j] + rm[i] * lm[j];
+      double x = nn[i] * pn[j], y = nm[i] * pm[j];
+      if (j < 4) {
+        x += cn[i] * dn[j];
+        y += cm[i] * dm[j];
+      }
+      if (i == j) {
+        a += an;
+        x += unn;
+        y += unm;
+      }
+      own[5 * i + j] = hrn * (x + a);
+      off[5 * i + j] = hrn * (y - a);
+    }
+}
+
 __device__ __forceinline__ void post_dVdU(const Gas &g, const double V[5], const double m[25], double res[25]) {
   const double gam1 = g.gam1;
   double invrho = 1.0 / V[0];
@@ -198,12 +276,22 @@ __device__ __forceinline__ void farfield_jac(const Gas &g, const double n[3], do
 // column-major LINPACK routines and transposes back; that is the same
 // arithmetic as running them on M(i,j) = blk[5i+j] directly, which is what
 // A_(i,j) addresses.  Returns 0 or the 1-based zero-pivot column.
+// Every index is a constant after unrolling (the row and column swaps are
+// selects), so the block stays in registers: with ipvt-indexed accesses it
+// went through scratch memory (inverting 105k FP64 blocks 35 us, now 11).
+template <class T>
+__device__ __forceinline__ void swap_if(bool p, T &a, T &b) {
+  const T x = p ? b : a, y = p ? a : b;
+  a = x;
+  b = y;
+}
 template <class T>
 __device__ __forceinline__ int invert5(T blk[25]) {
   T *a = blk;
   int ipvt[5];
   T work[5];
 #define A_(i, j) a[5 * (i) + (j)]
+#pragma unroll
   for (int k = 0; k < 4; ++k) {
     // pivot: largest |a| in column k, rows k..4, first on ties
     int l = k;
@@ -214,39 +302,52 @@ __device__ __forceinline__ int invert5(T blk[25]) {
       if (t2 > mx) { mx = t2; l = i; }
     }
     ipvt[k] = l;
-    if (A_(l, k) == (T)0) return k + 1;
-    if (l != k) { T t = A_(l, k); A_(l, k) = A_(k, k); A_(k, k) = t; }
+#pragma unroll
+    for (int i = k + 1; i < 5; ++i)
+#pragma unroll
+      for (int j = k; j < 5; ++j) swap_if(l == i, A_(k, j), A_(i, j));
+    if (A_(k, k) == (T)0) return k + 1;
     T t = (T)(-1. / A_(k, k));
+#pragma unroll
     for (int i = k + 1; i < 5; ++i) A_(i, k) *= t;
+#pragma unroll
     for (int j = k + 1; j < 5; ++j) {
-      t = A_(l, j);
-      if (l != k) { A_(l, j) = A_(k, j); A_(k, j) = t; }
+      t = A_(k, j);
+#pragma unroll
       for (int i = k + 1; i < 5; ++i) A_(i, j) += t * A_(i, k);
     }
   }
-  ipvt[4] = 4;
   if (A_(4, 4) == (T)0) return 5;
   // inverse(U)
+#pragma unroll
   for (int k = 0; k < 5; ++k) {
     A_(k, k) = (T)(1.0 / A_(k, k));
     T t = -A_(k, k);
+#pragma unroll
     for (int i = 0; i < k; ++i) A_(i, k) *= t;
+#pragma unroll
     for (int j = k + 1; j < 5; ++j) {
       t = A_(k, j);
       A_(k, j) = (T)0;
+#pragma unroll
       for (int i = 0; i <= k; ++i) A_(i, j) += t * A_(i, k);
     }
   }
   // inverse(U) * inverse(L)
+#pragma unroll
   for (int k = 3; k >= 0; --k) {
+#pragma unroll
     for (int i = k + 1; i < 5; ++i) { work[i] = A_(i, k); A_(i, k) = (T)0; }
+#pragma unroll
     for (int j = k + 1; j < 5; ++j) {
       T t = work[j];
+#pragma unroll
       for (int i = 0; i < 5; ++i) A_(i, k) += t * A_(i, j);
     }
-    int l = ipvt[k];
-    if (l != k)
-      for (int i = 0; i < 5; ++i) { T t3 = A_(i, k); A_(i, k) = A_(i, l); A_(i, l) = t3; }
+#pragma unroll
+    for (int l = k + 1; l < 5; ++l)
+#pragma unroll
+      for (int i = 0; i < 5; ++i) swap_if(ipvt[k] == l, A_(i, k), A_(i, l));
   }
 #undef A_
   return 0;

@@ -29,54 +29,95 @@ namespace aerofx {
 // ---------------------------------------------------------------------------
 // local time step (Edge.C:87-143, Face.C:242-290, Domain.C:32-100), beta = 1
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double sound_speed(const Gas &g, const double V[5]) {
-  return sqrt(g.gam * (V[4] + g.pstiff) / V[0]);
+// min(u.n - c, 0) S through the area vector nv outward from the node: with
+// beta = 1 the wave speed 0.5 (2 u_n - 2 c) of the reference
+__device__ __forceinline__ double inflow_speed(const Gas &g, const double V[5], const double nv[3]) {
+#pragma clang fp contract(on)
+  const double s2 = nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2];
+  const double S = s2 > 0.0 ? sqrt_from_rsq(s2, frsq(s2)) : 0.0;
+  const double c2 = g.gam * (V[4] + g.pstiff) * frcp(V[0]);
+  const double w = (V[1] * nv[0] + V[2] * nv[1] + V[3] * nv[2]) - sqrt_from_rsq(c2, frsq(c2)) * S;
+  return w < 0.0 ? w : 0.0;
 }
 
+// Entry e = (n, m): the part of edge (n, m) in the sum of node n.
+__device__ __forceinline__ double timestep_entry(const DevTables &t, const double *__restrict__ V, const Gas &g,
+                                                 int n, int e) {
+  const int m = t.adj[e];
+  const double *nl = t.normal + 3 * (size_t)t.eidx[e];
+  const double sg = n < m ? 1.0 : -1.0;
+  const double nv[3] = {sg * nl[0], sg * nl[1], sg * nl[2]};
+  double Vn[5], Vm[5], Vmid[5];
+  load_il<5>(V, n, Vn);
+  load_il<5>(V, m, Vm);
+#pragma unroll
+  for (int k = 0; k < 5; ++k) Vmid[k] = 0.5 * (Vn[k] + Vm[k]);
+  return inflow_speed(g, Vmid, nv);
+}
+
+// sum: the edges' part of node n; adds the faces and writes dt (Face::
+// computeTimeStep: full face normal, 1/3 of the face per node; Domain.C:91
+// with the viscous term weighted by Time.ViscosityParameter)
+__device__ __forceinline__ void timestep_node(const DevTables &t, const double *__restrict__ V, const Gas &g,
+                                              double cfl, const double *__restrict__ idtv, double viscous, int n,
+                                              double sum, double *__restrict__ dt) {
+  const int q0 = t.frow[n], q1 = t.frow[n + 1];
+  if (q0 < q1) {
+    double Vn[5];
+    load_il<5>(V, n, Vn);
+    for (int q = q0; q < q1; ++q) {
+      const double *nf = t.fnorm + 3 * (size_t)t.fidx[q];
+      const double nv[3] = {nf[0], nf[1], nf[2]};
+      sum += inflow_speed(g, Vn, nv) / 3;
+    }
+  }
+  dt[n] = cfl * t.cv[n] / (-1.0 * sum + (idtv ? viscous * idtv[n] : 0.0 * 0.0));
+}
+
+// The row of entry `tid` of a chunk: the last row start <= tid.
+__device__ __forceinline__ int chunk_row(const int *srow, int nr, int tid) {
+  int lo = 0, hi = nr;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (srow[mid] <= tid) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
+// Entry-parallel over the whole-row chunks: a lane per adjacency entry, the
+// rows summed through LDS in entry order, so an entry's gathers are not a
+// chain of 14 (34 -> 21 us at 105k nodes).
 __global__ __launch_bounds__(kBlock) void k_timestep(DevTables t, const double *__restrict__ V, Gas g, double cfl,
                                                      const double *__restrict__ idtv, double viscous,
                                                      double *__restrict__ dt) {
-  const int n = blockIdx.x * kBlock + threadIdx.x;
-  if (n >= t.N) return;
-  double Vn[5];
-  load_il<5>(V, n, Vn);
-  const double beta2 = 1.0;
-  double idti = 0.0;
-  for (int e = t.rowptr[n]; e < t.rowptr[n + 1]; ++e) {
-    const int m = t.adj[e], l = t.eidx[e];
-    const bool nlow = n < m;
-    const double *nl = t.normal + 3 * (size_t)l;
-    double S = sqrt(nl[0] * nl[0] + nl[1] * nl[1] + nl[2] * nl[2]);
-    double invS = 1.0 / S;
-    double nn0 = invS * nl[0], nn1 = invS * nl[1], nn2 = invS * nl[2];
-    double ndot = invS * 0.0;
-    double Vm[5], Vmid[5];
-    load_il<5>(V, m, Vm);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) Vmid[k] = 0.5 * (nlow ? Vn[k] + Vm[k] : Vm[k] + Vn[k]);
-    double a = sound_speed(g, Vmid);
-    double un = Vmid[1] * nn0 + Vmid[2] * nn1 + Vmid[3] * nn2 - ndot;
-    double coeff1 = (1.0 + beta2) * un;
-    double q = (1.0 - beta2) * un, r = 2.0 * a;
-    double coeff2 = sqrt(q * q + r * r);
-    double c = nlow ? 0.5 * (coeff1 - coeff2) : 0.5 * (-coeff1 - coeff2);
-    idti += (c < 0.0 ? c : 0.0) * S;
+  __shared__ double sc[kBlock];
+  __shared__ int srow[kMaxRows + 1];
+  const int c = xcd_chunk(blockIdx.x, t.ngchunks);
+  const int r0 = t.gchunk[c], r1 = t.gchunk[c + 1];
+  const int e0 = t.rowptr[r0], e1 = t.rowptr[r1];
+  const int tid = threadIdx.x, nr = r1 - r0;
+  if (e1 - e0 > kBlock) {
+    // one long row: its entries in passes, the sum carried in entry order
+    double s = 0.0;
+    for (int base = e0; base < e1; base += kBlock) {
+      if (base + tid < e1) sc[tid] = timestep_entry(t, V, g, r0, base + tid);
+      __syncthreads();
+      if (tid == 0)
+        for (int q = 0; q < min(kBlock, e1 - base); ++q) s += sc[q];
+      __syncthreads();
+    }
+    if (tid == 0) timestep_node(t, V, g, cfl, idtv, viscous, r0, s, dt);
+    return;
   }
-  for (int q = t.frow[n]; q < t.frow[n + 1]; ++q) {
-    // Face::computeTimeStep: full face normal, 1/3 of the face per node
-    const double *nf = t.fnorm + 3 * (size_t)t.fidx[q];
-    double S = sqrt(nf[0] * nf[0] + nf[1] * nf[1] + nf[2] * nf[2]);
-    double invS = 1.0 / S;
-    double un = Vn[1] * (invS * nf[0]) + Vn[2] * (invS * nf[1]) + Vn[3] * (invS * nf[2]) - invS * 0.0;
-    double a = sound_speed(g, Vn);
-    double coeff1 = (1.0 + beta2) * un;
-    double qq = (1.0 - beta2) * un, r = 2.0 * a;
-    double coeff2 = sqrt(qq * qq + r * r);
-    double c = 0.5 * (coeff1 - coeff2);
-    idti += (c < 0.0 ? c : 0.0) * S / 3;
+  if (tid <= nr) srow[tid] = t.rowptr[r0 + tid] - e0;
+  __syncthreads();
+  if (tid < e1 - e0) sc[tid] = timestep_entry(t, V, g, r0 + chunk_row(srow, nr, tid), e0 + tid);
+  __syncthreads();
+  if (tid < nr) {
+    double s = 0.0;
+    for (int q = srow[tid]; q < srow[tid + 1]; ++q) s += sc[q];
+    timestep_node(t, V, g, cfl, idtv, viscous, r0 + tid, s, dt);
   }
-  // Domain.C:91 with the viscous term weighted by Time.ViscosityParameter
-  dt[n] = cfl * t.cv[n] / (-1.0 * idti + (idtv ? viscous * idtv[n] : 0.0 * 0.0));
 }
 
 // ---------------------------------------------------------------------------
@@ -84,17 +125,13 @@ __global__ __launch_bounds__(kBlock) void k_timestep(DevTables t, const double *
 // SubDomain.C:1744-1767, TimeState.C:731-756)
 // ---------------------------------------------------------------------------
 // Entry-parallel: a block covers whole rows (<= 256 adjacency entries, <= 64
-// rows).  Phase 1: lane k evaluates the two ROEJAC6 blocks of entry e0 + k,
+// rows).  Phase 1: lane k evaluates the two Jacobian blocks of entry e0 + k,
 // stores the off-diagonal block (64 consecutive entries -> contiguous
 // segments) and its diagonal contribution in LDS; lanes also take the rows'
 // boundary-face slots and store each face Jacobian in a per-slot buffer.
 // Phase 2: one lane per (row, element) adds the entries in entry order, then
 // the faces in face order, scales by 1/V and adds 1/dt -- the reference's
 // per-node order.
-// Two roejac6 evaluations inline take 256 VGPRs + 18 AGPRs, one wave per
-// SIMD; asking for two waves spills ~18 registers to scratch and is faster
-// (assembly 50 -> 38 ms over a 96x32x32 FP64 steady solve; three waves spill
-// 116 and are slower).
 // Adjacency entry e = (n, m) of H1: its off-diagonal block A_nm (scaled by
 // 1/V_n) into B, and its contribution to the diagonal block of n into dg
 // (dF/dU_i for n = i, -dF/dU_j for n = j).  LM: the low-Mach (Roe-Turkel)
@@ -125,6 +162,17 @@ __device__ __forceinline__ void jac_entry(const DevTables &t, const double *__re
     const double d0 = n < m ? xm.x - xn.x : xn.x - xm.x, d1 = n < m ? xm.y - xn.y : xn.y - xm.y,
                  d2 = n < m ? xm.z - xn.z : xn.z - xm.z;
     length = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+  }
+  if (!LM) {
+    // outward from n: A_ii += dF/dU_i, A_ij = dF/dU_j / V_i, and with the
+    // normal reversed A_jj -= dF/dU_j, A_ji = -dF/dU_i / V_j
+    const double sg = n < m ? 1.0 : -1.0;
+    const double en[3] = {sg * nl[0], sg * nl[1], sg * nl[2]};
+    double off[25];
+    roe_jac_pair(g, en, Vn, Vm, dg, off);
+#pragma unroll
+    for (int k = 0; k < 25; ++k) Be[k * kBlkStride] = (T)(off[k] * voln);
+    return;
   }
   double blk[25];
   if (n < m) {
@@ -164,13 +212,13 @@ __device__ __forceinline__ void jac_face(const DevTables &t, const double *__res
   for (int k = 0; k < 25; ++k) fjac[25 * (size_t)q + k] = jac[k];
 }
 
-// Two roejac6 evaluations inline take 256 VGPRs + 18 AGPRs, one wave per
-// SIMD; asking for two waves spills ~18 registers to scratch and is faster
-// (assembly 50 -> 38 ms over a 96x32x32 FP64 steady solve; three waves spill
-// 116 and are slower).  A chunk that is one row of more than kBlock entries
-// is left to k_jacobian_long.
+// The low-Mach edges evaluate roejac6 twice inline (two waves per SIMD with ~18
+// registers spilled beat one without); the others are bound by the blocks
+// they write (assembly at 105k nodes 367 -> 137 us in FP64, 88k nodes 236 -> 88
+// in FP32 with roe_jac_pair; three waves per SIMD are what the LDS admits).  A chunk that is one row of more than kBlock entries is left to
+// k_jacobian_long.
 template <class T, bool LM>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_jacobian(DevTables t, const double *__restrict__ V, FluxConsts fc,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(LM ? 2 : 3, LM ? 2 : 3))) void k_jacobian(DevTables t, const double *__restrict__ V, FluxConsts fc,
                                                      const double *__restrict__ dt, double *__restrict__ fjac,
                                                      T *__restrict__ D, T *__restrict__ B) {
   __shared__ double sd[25 * kPad];
@@ -184,26 +232,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   __syncthreads();
   if (tid < e1 - e0) {
     const int e = e0 + tid;
-    // row of entry tid: the last row start <= tid
-    int lo = 0, hi = nr;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (srow[mid] <= tid) lo = mid; else hi = mid;
-    }
     double dg[25];
-    jac_entry<T, LM>(t, V, fc, r0 + lo, e, B, dg);
+    jac_entry<T, LM>(t, V, fc, r0 + chunk_row(srow, nr, tid), e, B, dg);
 #pragma unroll
     for (int k = 0; k < 25; ++k) sd[k * kPad + tid] = dg[k];
   }
   // boundary-face Jacobians of the block's rows, one per face slot
   const int q0 = t.frow[r0], q1 = t.frow[r1];
   for (int q = q0 + tid; q < q1; q += kBlock) {
-    int lo = 0, hi = nr;  // row owning slot q
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (t.frow[r0 + mid] <= q) lo = mid; else hi = mid;
-    }
-    jac_face(t, V, fc, r0 + lo, q, fjac);
+    jac_face(t, V, fc, t.fnode[q], q, fjac);
   }
   __syncthreads();
   for (int idx = tid; idx < nr * 25; idx += kBlock) {
@@ -576,11 +613,10 @@ int ensure_jacobian_storage(aerofx_ctx *c, int precision) {
 }
 
 int launch_timestep(aerofx_ctx *c, double cfl, double *dt) {
-  const int nb = (c->N + kBlock - 1) / kBlock;
   double *idtv = nullptr;
   int rc = launch_visc_idtv(c, &idtv);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_timestep, dim3(nb), dim3(kBlock), 0, c->stream, c->tab, c->d_V, c->gas, cfl, idtv,
+  hipLaunchKernelGGL(k_timestep, dim3(c->tab.ngchunks), dim3(kBlock), 0, c->stream, c->tab, c->d_V, c->gas, cfl, idtv,
                      c->ns.viscous_cst, dt);
   return check_launch("timestep launch");
 }
