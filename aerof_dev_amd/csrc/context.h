@@ -245,6 +245,8 @@ struct aerofx_ctx {
   double *d_visc_c = nullptr;  // [4T][5] element contributions of the Galerkin term, in node-slot order
                                // (the residual's, whose density row is zero: [4T][4])
   double *d_visc_g = nullptr;  // il<4>: their node sums
+  int *d_visc_chunk = nullptr; // row chunks of the Galerkin Jacobian pass; visc_chunks of them (0: a row is too long)
+  int visc_chunks = 0;
   double *d_adj_tmp = nullptr;  // [N][5] the adjoint with the wall rows masked
   // viscous wall force: element of each face, per node the wall-face element
   // slots (4 f + k), per slot the derivatives [4F][5] / [4F][3]
