@@ -173,6 +173,44 @@ struct DevTables {
   const int *epos;       // [E] position of each edge in the flux storage
 };
 
+constexpr int kWave = 64;
+__device__ __forceinline__ int lane_id() { return (int)threadIdx.x & (kWave - 1); }
+// slice of this wave: blocks of four slices, one contiguous range per XCD
+__device__ __forceinline__ int wave_slice(const DevTables &t) {
+  const int nb = (t.ns + kBlock / kWave - 1) / (kBlock / kWave);
+  return xcd_chunk(blockIdx.x, nb) * (kBlock / kWave) + (int)(threadIdx.x / kWave);
+}
+inline dim3 slice_grid(int ns) { return dim3((unsigned)((ns + kBlock / kWave - 1) / (kBlock / kWave))); }
+
+// s -= (LOWER: edge positions in rows.idx) or += (upper edges: the entries'
+// own places) the fluxes of this lane's row, in row order; four entries'
+// loads in flight together.
+template <bool LOWER>
+__device__ __forceinline__ void add_slots(const RowSlices &rows, int sl, int deg, const double *__restrict__ Fm,
+                                          double s[5]) {
+  constexpr int B = 4;
+  const int kb = rows.kptr[sl], kn = rows.kptr[sl + 1] - kb;
+  for (int k0 = 0; k0 < kn; k0 += B) {
+    int pos[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int off = k0 + u < kn ? rows.koff[kb + k0 + u] : 0;
+      const bool act = k0 + u < deg;
+      const int e = off + lanes_below(act);
+      pos[u] = act ? (LOWER ? rows.idx[e] : e) : 0;
+    }
+    double v[B][5];
+#pragma unroll
+    for (int u = 0; u < B; ++u) load_il<5>(Fm, pos[u], v[u]);
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (k0 + u < deg) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) s[k] = LOWER ? s[k] - v[u][k] : s[k] + v[u][k];
+      }
+  }
+}
+
 struct FluxConsts {
   Gas gas;
   double beta;
@@ -377,6 +415,8 @@ int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, 
                          const int *done = nullptr, int *host_err = nullptr);
 // tables of the LDS-staged family, built when it is first selected
 int ensure_staged(aerofx_ctx *c);
+// LSQ gradients (il<15>) of a field laid out as d_V
+int launch_gradients_il(aerofx_ctx *c, const double *W, double *grad, const int *done);
 int launch_gradients_v(aerofx_ctx *c, const double *V, double *ddx, double *ddy, double *ddz);
 int launch_primitive(aerofx_ctx *c, const double *U, double *V);  // V [N][5]
 int launch_primitive_il(aerofx_ctx *c, const double *U);          // c->d_V

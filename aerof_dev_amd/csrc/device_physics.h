@@ -164,9 +164,28 @@ __device__ __forceinline__ double sqrt_from_rsq(double x, double y) {
   return fma(0.5 * y, fma(-s, s, x), s);
 }
 
+__device__ __forceinline__ double neg_part(double x) { return fmin(x, 0.0); }
+__device__ __forceinline__ double pos_part(double x) { return fmax(x, 0.0); }
+__device__ __forceinline__ double gabs(double x) { return fabs(x); }
+// ... and of Duals
+__device__ __forceinline__ Dual frcp(Dual x) {
+  const double y = frcp(x.v);
+  return Dual(y, -(y * y) * x.d);
+}
+__device__ __forceinline__ Dual frsq(Dual x) {
+  const double y = frsq(x.v);
+  return Dual(y, -0.5 * (y * y * y) * x.d);
+}
+__device__ __forceinline__ Dual sqrt_from_rsq(Dual x, Dual y) {
+  return Dual(sqrt_from_rsq(x.v, y.v), 0.5 * y.v * x.d);
+}
+__device__ __forceinline__ Dual neg_part(Dual x) { return x.v < 0.0 ? x : Dual(0.0); }
+__device__ __forceinline__ Dual pos_part(Dual x) { return x.v > 0.0 ? x : Dual(0.0); }
+__device__ __forceinline__ Dual gabs(Dual x) { return x.v < 0.0 ? -x : x; }
+
 // The residual's Van Albada reconstruction and Roe flux: the functions of
-// vanalbada and roeflux7 (which the derivative passes differentiate) with the
-// fewest FP64 operations (805 -> 530 vector instructions an edge with the
+// vanalbada and roeflux7 (which the reverse pass differentiates; the forward
+// one takes these with T = Dual) with the fewest FP64 operations (805 -> 530 vector instructions an edge with the
 // edge pass's loads and addressing, 60 % -> 40 % of its clocks at 2.1M nodes):
 //  * the flux's sums contracted to fused multiply-adds (the gradients' and the
 //    projected slopes' keep their order), the divisions through frcp;
@@ -176,56 +195,58 @@ __device__ __forceinline__ double sqrt_from_rsq(double x, double y) {
 //    n.dm - u_n drho = sqrt(rho_l rho_r) n.du exactly, also with pstiff.
 // The last replaces differences of conservative variables, which lose digits
 // in smooth flow.
-__device__ __forceinline__ double va_slope(double a, double b) {
+template <class T>
+__device__ __forceinline__ T va_slope(T a, T b) {
 #pragma clang fp contract(on)
   const double eps = 1.e-16;
-  const double a2 = a * a, b2 = b * b, ab = a * b;
-  const double den = a2 + (b2 + 2.0 * eps);
-  const double num = ab > 0.0 ? ab * (a + b) + eps * (a + b) : (ab == 0.0 ? 0.5 * eps * (a + b) : 0.0);
+  const T a2 = a * a, b2 = b * b, ab = a * b;
+  const T den = a2 + (b2 + 2.0 * eps);
+  const T num = ab > 0.0 ? ab * (a + b) + eps * (a + b) : (ab == 0.0 ? 0.5 * eps * (a + b) : T(0.0));
   return num * frcp(den);
 }
 
-__device__ __forceinline__ void reconstruct(double beta, double Vi, double ddVij, double Vj, double ddVji, double &Vij,
-                                            double &Vji) {
+template <class T>
+__device__ __forceinline__ void reconstruct(double beta, T Vi, T ddVij, T Vj, T ddVji, T &Vij, T &Vji) {
 #pragma clang fp contract(on)
   const double beta2 = 1.0 - 2.0 * beta, tb = 2.0 * beta;
-  const double dVji = Vj - Vi;
-  const double dV = beta2 * dVji;
+  const T dVji = Vj - Vi;
+  const T dV = beta2 * dVji;
   Vij = Vi + 0.5 * va_slope(dV + tb * ddVij, dVji);
   Vji = Vj - 0.5 * va_slope(dV + tb * ddVji, dVji);
 }
 
-__device__ __forceinline__ void roe_flux(const Gas &g, const double en[3], const double L[5], const double R[5],
-                                         double f[5]) {
+template <class T>
+__device__ __forceinline__ void roe_flux(const Gas &g, const T en[3], const T L[5], const T R[5], T f[5]) {
 #pragma clang fp contract(on)
-  const double rn2 = en[0] * en[0] + en[1] * en[1] + en[2] * en[2];
-  const double irn = frsq(rn2), rn = sqrt_from_rsq(rn2, irn);
-  const double n0 = en[0] * irn, n1 = en[1] * irn, n2 = en[2] * irn;
-  const double il = frsq(L[0]), ir = frsq(R[0]);  // 1 / sqrt(rho)
-  const double sl = sqrt_from_rsq(L[0], il), sr = sqrt_from_rsq(R[0], ir);
-  const double gg = g.gam * g.invgam1, irl = frcp(L[0]), irr = frcp(R[0]);
-  const double hl = gg * (L[4] + g.pstiff) * irl + 0.5 * (L[1] * L[1] + L[2] * L[2] + L[3] * L[3]);
-  const double hr = gg * (R[4] + g.pstiff) * irr + 0.5 * (R[1] * R[1] + R[2] * R[2] + R[3] * R[3]);
-  const double w = frcp(sl + sr), wl = sl * w, wr = sr * w;
-  const double u = wl * L[1] + wr * R[1], v = wl * L[2] + wr * R[2], z = wl * L[3] + wr * R[3];
-  const double H = wl * hl + wr * hr;
-  const double q = 0.5 * (u * u + v * v + z * z);
-  const double c2 = g.gam1 * (H - q);
-  const double ic = frsq(c2), c = sqrt_from_rsq(c2, ic);
-  const double ml = L[1] * en[0] + L[2] * en[1] + L[3] * en[2], mr = R[1] * en[0] + R[2] * en[1] + R[3] * en[2];
-  const double un = n0 * u + n1 * v + n2 * z;
+  const T rn2 = en[0] * en[0] + en[1] * en[1] + en[2] * en[2];
+  const T irn = frsq(rn2), rn = sqrt_from_rsq(rn2, irn);
+  const T n0 = en[0] * irn, n1 = en[1] * irn, n2 = en[2] * irn;
+  const T il = frsq(L[0]), ir = frsq(R[0]);  // 1 / sqrt(rho)
+  const T sl = sqrt_from_rsq(L[0], il), sr = sqrt_from_rsq(R[0], ir);
+  const double gg = g.gam * g.invgam1;
+  const T irl = frcp(L[0]), irr = frcp(R[0]);
+  const T hl = gg * (L[4] + g.pstiff) * irl + 0.5 * (L[1] * L[1] + L[2] * L[2] + L[3] * L[3]);
+  const T hr = gg * (R[4] + g.pstiff) * irr + 0.5 * (R[1] * R[1] + R[2] * R[2] + R[3] * R[3]);
+  const T w = frcp(sl + sr), wl = sl * w, wr = sr * w;
+  const T u = wl * L[1] + wr * R[1], v = wl * L[2] + wr * R[2], z = wl * L[3] + wr * R[3];
+  const T H = wl * hl + wr * hr;
+  const T q = 0.5 * (u * u + v * v + z * z);
+  const T c2 = g.gam1 * (H - q);
+  const T ic = frsq(c2), c = sqrt_from_rsq(c2, ic);
+  const T ml = L[1] * en[0] + L[2] * en[1] + L[3] * en[2], mr = R[1] * en[0] + R[2] * en[1] + R[3] * en[2];
+  const T un = n0 * u + n1 * v + n2 * z;
   // upwind side by the Roe normal velocity, and the acoustic wave running
   // against it
   const bool left = un > 0.0;
-  const double *S = left ? L : R;
-  const double hs = left ? hl : hr;
-  const double cs = left ? -c : c;
-  const double lam = left ? fmin(un - c, 0.0) : fmax(un + c, 0.0);  // its speed, 0 if it runs with the flow
+  const T *S = left ? L : R;
+  const T hs = left ? hl : hr;
+  const T cs = left ? -c : c;
+  const T lam = left ? neg_part(un - c) : pos_part(un + c);  // its speed, 0 if it runs with the flow
   // dp + (+-c) sqrt(rho_l rho_r) dun, over 2 c^2, times |lam|
-  const double a = 0.5 * (ic * ic) * fabs(lam) * (rn * (R[4] - L[4]) + cs * (sl * sr) * (mr - ml));
-  const double m = S[0] * (left ? ml : mr);
+  const T a = 0.5 * (ic * ic) * gabs(lam) * (rn * (R[4] - L[4]) + cs * (sl * sr) * (mr - ml));
+  const T m = S[0] * (left ? ml : mr);
   f[0] = m - a;
-  const double pn = S[4] - a * cs * irn;
+  const T pn = S[4] - a * cs * irn;
   f[1] = m * S[1] + pn * en[0] - a * u;
   f[2] = m * S[2] + pn * en[1] - a * v;
   f[3] = m * S[3] + pn * en[2] - a * z;

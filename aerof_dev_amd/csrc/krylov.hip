@@ -41,7 +41,6 @@ constexpr int kDotBlocks = 1024;  // fixed: the reduction order never depends on
 constexpr int kSweepBlocks = 256;  // blocks of the basis sweeps: one per CU
 constexpr int kMaxBasis = 32;     // basis vectors handled by one sweep (m <= 31)
 static_assert(kMaxBasis == kMaxBasisCoef, "coefficient layout shared with the update kernel");
-constexpr int kWave = 64;
 
 // Device-resident GMRES state (one per right-hand side).
 // Coefficients of the Gram-Schmidt update kernel, in GmresState::coef:

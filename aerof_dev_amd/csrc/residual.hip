@@ -36,15 +36,6 @@ namespace aerofx {
 // 10 on the batch no longer stays in registers)
 constexpr int kGradChunk = 8;
 
-constexpr int kWave = 64;
-__device__ __forceinline__ int lane_id() { return (int)threadIdx.x & (kWave - 1); }
-// slice of this wave: blocks of four slices, one contiguous range per XCD
-__device__ __forceinline__ int wave_slice(const DevTables &t) {
-  const int nb = (t.ns + kBlock / kWave - 1) / (kBlock / kWave);
-  return xcd_chunk(blockIdx.x, nb) * (kBlock / kWave) + (int)(threadIdx.x / kWave);
-}
-static dim3 slice_grid(int ns) { return dim3((unsigned)((ns + kBlock / kWave - 1) / (kBlock / kWave))); }
-
 // ---------------------------------------------------------------------------
 // 1. gradients: one lane per node, neighbours in ascending order (= the
 //    reference's edge order), so every node's sums are formed exactly as in
@@ -59,6 +50,15 @@ __device__ __forceinline__ void load_state(const double *__restrict__ W, int n, 
   } else {
 #pragma unroll
     for (int k = 0; k < 5; ++k) w[k] = W[5 * (size_t)n + k];
+  }
+}
+template <int FROM>
+__device__ __forceinline__ void to_prim(const double w[5], const Gas &gas, double v[5]) {
+  if (FROM == kFromU) {
+    prim_from_cons(w, gas, v);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) v[k] = w[k];
   }
 }
 __device__ __forceinline__ void load_x(const DevTables &t, int n, double x[3]) {
@@ -111,12 +111,7 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
   {
     double w[5];
     load_state<FROM>(W, nn, w);
-    if (FROM == kFromU) {
-      prim_from_cons(w, gas, Vn);
-    } else {
-#pragma unroll
-      for (int k = 0; k < 5; ++k) Vn[k] = w[k];
-    }
+    to_prim<FROM>(w, gas, Vn);
   }
   if (Vout && live) store_il<5>(Vout, n, Vn);
   load_x(t, nn, xn);
@@ -153,12 +148,7 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
     for (int k = 0; k < kGradChunk; ++k) {
       if (e + k >= deg) break;
       double Vm[5];
-      if (FROM == kFromU) {
-        prim_from_cons(Wm[k], gas, Vm);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 5; ++q) Vm[q] = Wm[k][q];
-      }
+      to_prim<FROM>(Wm[k], gas, Vm);
       lsq_add(L, xm[k], xn, Vm, Vn, acc);
     }
   }
@@ -198,13 +188,14 @@ constexpr int kHaloThreads = kWave * kHaloWaves;
 constexpr int kHaloBatch = 4;   // halo nodes a lane has in flight
 constexpr int kHaloPairs = 8;   // place pairs (two entries) requested together
 
+template <int FROM>
 struct HaloLoad {
   double w[kHaloBatch][5], x[kHaloBatch][3];
   __device__ __forceinline__ void request(const DevTables &t, const double *__restrict__ U,
                                           const int m[kHaloBatch]) {
 #pragma unroll
     for (int r = 0; r < kHaloBatch; ++r) {
-      load_state<kFromU>(U, m[r], w[r]);
+      load_state<FROM>(U, m[r], w[r]);
       load_x(t, m[r], x[r]);
     }
   }
@@ -215,7 +206,7 @@ struct HaloLoad {
       const int h = r0 + r * kHaloThreads + (int)threadIdx.x;
       if (h >= cap) break;
       double v[5];
-      prim_from_cons(w[r], gas, v);
+      to_prim<FROM>(w[r], gas, v);
       sp[h] = make_double2(v[0], v[1]);
       sp[cap + h] = make_double2(v[2], v[3]);
       sp[2 * cap + h] = make_double2(v[4], x[r][0]);
@@ -236,9 +227,10 @@ struct HaloRow {
   double w[5], xn[3], L[6];
   int deg;
   uint32_t loc[kHaloPairs];
+  template <int FROM>
   __device__ __forceinline__ void request(const DevTables &t, const double *__restrict__ U, int sl) {
     const int nn = min(sl * kWave + lane_id(), t.N - 1);
-    load_state<kFromU>(U, nn, w);
+    load_state<FROM>(U, nn, w);
     load_x(t, nn, xn);
     load_lsq(t, nn, L);
     deg = t.rowptr[nn + 1] - t.rowptr[nn];
@@ -284,6 +276,7 @@ __device__ __forceinline__ void halo_sums(const DevTables &t, const double2 *sp,
 
 // The workgroups b, b + 8, ... take turns over the b % 8-th part of the slices
 // (the XCD they run on).
+template <int FROM>
 __global__ __launch_bounds__(kHaloThreads) void k_gradients_halo(DevTables t, const double *__restrict__ U, Gas gas,
                                                                  double *__restrict__ Vout,
                                                                  double *__restrict__ grad, int *__restrict__ err,
@@ -297,11 +290,11 @@ __global__ __launch_bounds__(kHaloThreads) void k_gradients_halo(DevTables t, co
   const int s0 = (int)((long long)t.ns * xcd / kNumXcd), s1 = (int)((long long)t.ns * (xcd + 1) / kNumXcd);
   int sl = s0 + turn;
   if (sl >= s1) return;
-  HaloLoad load;
+  HaloLoad<FROM> load;
   HaloRow row;
   int m[kHaloBatch];
   halo_ids(t, sl, 0, m);
-  row.request(t, U, sl);
+  row.request<FROM>(t, U, sl);
   load.request(t, U, m);
   int next = sl + step;
   if (next < s1) halo_ids(t, next, 0, m);
@@ -316,17 +309,17 @@ __global__ __launch_bounds__(kHaloThreads) void k_gradients_halo(DevTables t, co
     }
     HaloRow cur = row;
     double Vn[5];
-    prim_from_cons(cur.w, gas, Vn);
+    to_prim<FROM>(cur.w, gas, Vn);
     __syncthreads();
     const bool more = next < s1;
     if (more) {
       load.request(t, U, m);
-      row.request(t, U, next);
+      row.request<FROM>(t, U, next);
     }
     const int n = sl * kWave + lane_id();
     if (n < t.N) {
       if ((int)threadIdx.x < kWave) {
-        store_il<5>(Vout, n, Vn);
+        if (Vout) store_il<5>(Vout, n, Vn);
         halo_sums<0, 3>(t, sp, cur, Vn, sl, n, grad);
       } else {
         halo_sums<3, 5>(t, sp, cur, Vn, sl, n, grad);
@@ -688,35 +681,6 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
 // ---------------------------------------------------------------------------
 // 3. node assembly: lower edges, upper-edge sum, faces, 1/V
 // ---------------------------------------------------------------------------
-// s -= (LOWER: edge positions in rows.idx) or += (upper edges: the entries'
-// own places) the fluxes of this lane's row, in row order; four entries'
-// loads in flight together.
-template <bool LOWER>
-__device__ __forceinline__ void add_slots(const RowSlices &rows, int sl, int deg, const double *__restrict__ Fm,
-                                          double s[5]) {
-  constexpr int B = 4;
-  const int kb = rows.kptr[sl], kn = rows.kptr[sl + 1] - kb;
-  for (int k0 = 0; k0 < kn; k0 += B) {
-    int pos[B];
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const int off = k0 + u < kn ? rows.koff[kb + k0 + u] : 0;
-      const bool act = k0 + u < deg;
-      const int e = off + lanes_below(act);
-      pos[u] = act ? (LOWER ? rows.idx[e] : e) : 0;
-    }
-    double v[B][5];
-#pragma unroll
-    for (int u = 0; u < B; ++u) load_il<5>(Fm, pos[u], v[u]);
-#pragma unroll
-    for (int u = 0; u < B; ++u)
-      if (k0 + u < deg) {
-#pragma unroll
-        for (int k = 0; k < 5; ++k) s[k] = LOWER ? s[k] - v[u][k] : s[k] + v[u][k];
-      }
-  }
-}
-
 // P null: the upper-edge sum is formed here from the edge fluxes, in edge
 // order.  vg (or null): the node sums of the Navier-Stokes Galerkin
 // contributions (momentum and energy), added before the 1/V scaling.
@@ -833,7 +797,7 @@ int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, 
       hipLaunchKernelGGL(k_gradients_staged, dim3(t.ngb), dim3(kGradStrip), 0, c->stream, t, U, c->gas, b.V,
                          b.grad, c->d_err, done);
     } else if (t.halo_cap) {
-      hipLaunchKernelGGL(k_gradients_halo, halo_grid(t), dim3(kHaloThreads), halo_lds(t), c->stream, t, U, c->gas,
+      hipLaunchKernelGGL(k_gradients_halo<kFromU>, halo_grid(t), dim3(kHaloThreads), halo_lds(t), c->stream, t, U, c->gas,
                          b.V, b.grad, c->d_err, done);
     } else {
       hipLaunchKernelGGL((k_gradients<kFromU, false>), slice_grid(t.ns), blk, 0, c->stream, t, U, c->gas, b.V,
@@ -933,6 +897,18 @@ int refuse_failsafe_nodes(aerofx_ctx *c, const char *who) {
   if (!c->fs_any) return 0;
   return set_error(AEROFX_ERR_STATE, std::string(who) +
                                          ": failsafe first-order nodes are set (aerofx_ctx_reset_failsafe clears them)");
+}
+
+int launch_gradients_il(aerofx_ctx *c, const double *W, double *grad, const int *done) {
+  const DevTables &t = c->tab;
+  if (t.halo_cap)
+    hipLaunchKernelGGL(k_gradients_halo<kFromVil>, halo_grid(t), dim3(kHaloThreads), halo_lds(t), c->stream, t, W,
+                       c->gas, nullptr, grad, nullptr, done);
+  else
+    hipLaunchKernelGGL((k_gradients<kFromVil, false>), slice_grid(t.ns), dim3(kBlock), 0, c->stream, t, W, c->gas,
+                       nullptr, grad, nullptr, nullptr, nullptr, nullptr, done);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : set_hip_error(e, "gradients launch");
 }
 
 int launch_gradients_v(aerofx_ctx *c, const double *V, double *ddx, double *ddy, double *ddz) {
