@@ -11,19 +11,22 @@
 //
 // Stages (all deterministic: per-edge, per-tet and per-face results go to
 // their own slots and each node sums its slots in a fixed order):
-//   1. forward residual: V, LSQ gradients, R (scaled)
-//   2. k_adj_edges_u / _x  one thread per edge: mu = lambda/V, g = mu_i - mu_j;
-//      g^T dF/d(V_ij, V_ji, n) by the reverse mode of the Roe flux,
-//      then reverse through the Van Albada reconstruction by hand
-//      -> per edge: Vbar_i, Vbar_j, Gbar_i, Gbar_j, dxbar, nbar
-//   3. k_adj_nodes  one thread per node: sums the edge slots, adds the
-//      boundary-face terms -> Vbar, Gbar, the dx part of Xbar
-//   4. k_adj_lsq    one thread per node: reverse of the LSQ gradients
-//      (grad_i = sum_j W_ij (V_j - V_i)), then Ubar = (dV/dU)^T Vbar; for X
-//      also the weight and Cholesky-factor terms -> S_i = d/dM_i, symmetric
+//   1. forward residual: V, LSQ gradients g, R (scaled); mu = lambda/V
+//   2. k_adj_edges  one lane per edge: w = mu_i - mu_j; w^T dF/d(V_ij, V_ji, n)
+//      by the reverse mode of the Roe flux, then reverse through the Van Albada
+//      reconstruction by hand -> per edge: Vbar_i, c_i, Vbar_j, c_j, dxbar,
+//      nbar; its first blocks: the same per boundary-face slot
+//   3. k_adj_nodes  one lane per node: sums its slots -> Vbar, Gbar, the dx
+//      part of Xbar; then the reverse of the LSQ gradients' own node.  With
+//      M g = sum_j dx_ij (V_j - V_i), M = sum_j dx_ij dx_ij^T and H = M^-1 Gbar,
+//        d(Gbar . g) = sum_j d[dx_ij . H (V_j - V_i)] - H . (dM g),
+//      so H and the symmetric S = -(H g^T + g H^T) are all that is passed on
+//   4. k_adj_lsq    one lane per node, with K = H_i + H_j:
+//      Vbar_i -= K dx_ij, Xbar_i -= K (V_j - V_i) + (S_i + S_j) dx_ij, then
+//      Ubar = (dV/dU)^T Vbar
 //   5. k_adj_tets / k_adj_faces: control-volume, dual-normal and face-normal
 //      geometry, reverse over each element's coordinates
-//   6. k_adj_xgather: Xbar_i = slots of 3-5 and -sum_j (S_i + S_j) dx_ij
+//   6. k_adj_xgather: Xbar_i plus its tet and face slots
 #include <hip/hip_runtime.h>
 
 #include "context.h"
@@ -34,19 +37,25 @@
 namespace aerofx {
 
 struct Adjoint {
-  double *EV = nullptr;   // [E][20] Vbar_i, c_i, Vbar_j, c_j (Gbar_i[d*5+k] = c_i[k] dx[d])
-  double *EX = nullptr;   // [E][6]  dxbar, nbar (coordinate derivatives only)
-  double *Vb = nullptr;   // [N][5]
-  double *Gb = nullptr;   // [N][16]
-  double *Xb = nullptr;   // [N][4]
-  double *S = nullptr;    // [N][6]
+  double *EVi = nullptr;  // il<10> (first order il<5>) over edge positions: Vbar_i, c_i (Gbar_i[d*5+k] = c_i[k] dx[d])
+  double *EVj = nullptr;  // the same of the upper end
+  double *EXd = nullptr;  // il<3> over edge positions: dxbar
+  double *EXn = nullptr;  // il<3> over edge positions: nbar
+  double *FV = nullptr;   // [3F][5] Vbar of each node face slot
+  double *FN = nullptr;   // [3F][3] its share of the face normal's, at 3 f + local vertex
+  double *mu = nullptr;   // il<5>: lambda / V
+  double *cvb = nullptr;  // [N] -mu . R
+  double *Vb = nullptr;   // il<5>
+  double *H = nullptr;    // il<15>
+  double *S = nullptr;    // il<6>
+  double *Xb = nullptr;   // il<3>
   double *R = nullptr;    // [N][5] forward residual (scaled)
   double *TX = nullptr;   // [T][12]
   double *FX = nullptr;   // [F][9]
   double *Jf = nullptr;   // [F] per-face objective values, then the sum at [F]
   double *h_J = nullptr;  // pinned
   int *tets = nullptr;    // [T][4]
-  int *tedge = nullptr;   // [T][6]
+  int *tpos = nullptr;    // [T][6] edge positions
   int *faces = nullptr;   // [F][3]
   int *ntrow = nullptr;   // [N+1]
   int *ntslot = nullptr;  // [4T] 4*t + local vertex
@@ -56,72 +65,39 @@ struct Adjoint {
 namespace {
 
 constexpr int kAdjBlock = 256;
-// ElemTet edge -> (end, end) and edge -> (face, face) tables (ElemTetCore.C:19-21)
-__constant__ int cEdgeEnd[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
-__constant__ int cEdgeFace[6][2] = {{0, 1}, {2, 0}, {1, 2}, {0, 3}, {3, 1}, {2, 3}};
-
-// LSQ weights W(dx; L) as the gradient pass evaluates them.
-__device__ __forceinline__ void lsq_weights(const double L[6], double dx0, double dx1, double dx2, double w[3]) {
-  const double or11 = L[0], or22 = L[1], or33 = L[2], r12or11 = L[3], r23or22 = L[4], psi = L[5];
-  const double alpha1 = dx0 * or11 * or11;
-  const double alpha2 = (dx1 - r12or11 * dx0) * or22 * or22;
-  const double alpha3 = (dx2 - r23or22 * dx1 + psi * dx0) * or33 * or33;
-  w[0] = alpha1 - r12or11 * alpha2 + psi * alpha3;
-  w[1] = alpha2 - r23or22 * alpha3;
-  w[2] = alpha3;
-}
-
-// Reverse of lsq_weights: given Wbar, accumulate dxbar and (optionally) Lbar.
-__device__ __forceinline__ void lsq_weights_rev(const double L[6], double dx0, double dx1, double dx2,
-                                                const double wb[3], double dxb[3], double *Lb) {
-  const double or11 = L[0], or22 = L[1], or33 = L[2], r12or11 = L[3], r23or22 = L[4], psi = L[5];
-  const double a3b = wb[2] + psi * wb[0] - r23or22 * wb[1];
-  const double a2b = wb[1] - r12or11 * wb[0];
-  const double a1b = wb[0];
-  const double s11 = or11 * or11, s22 = or22 * or22, s33 = or33 * or33;
-  const double c3 = a3b * s33, c2 = a2b * s22;
-  dxb[0] += a1b * s11 - c2 * r12or11 + c3 * psi;
-  dxb[1] += c2 - c3 * r23or22;
-  dxb[2] += c3;
-  if (Lb) {
-    const double alpha2 = (dx1 - r12or11 * dx0) * s22;
-    const double alpha3 = (dx2 - r23or22 * dx1 + psi * dx0) * s33;
-    const double t2 = dx1 - r12or11 * dx0;
-    const double t3 = dx2 - r23or22 * dx1 + psi * dx0;
-    Lb[0] += a1b * dx0 * 2.0 * or11;
-    Lb[1] += a2b * t2 * 2.0 * or22;
-    Lb[2] += a3b * t3 * 2.0 * or33;
-    Lb[3] += -alpha2 * wb[0] - c2 * dx0;
-    Lb[4] += -alpha3 * wb[1] - c3 * dx1;
-    Lb[5] += alpha3 * wb[0] + c3 * dx0;
-  }
-}
+// ElemTet edge -> (end, end) table (ElemTetCore.C:19-21) and the edge's opposite
+// vertices (c, d): in a tet the median dual face of edge (a, b), from a to b, is
+// (c - d) x (a + b - c - d) / 24
+constexpr int kEnd[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
+constexpr int kOpp[6][2] = {{3, 2}, {1, 3}, {2, 1}, {3, 0}, {0, 2}, {1, 0}};
 
 __device__ __forceinline__ double seed(int dir, int k) { return dir == k ? 1.0 : 0.0; }
 
 // Reverse mode of roeflux7 (device_physics.h) with evitno = 0, the edge
 // call: given the weights g on the five flux components, returns
 // bL = g^T dphi/dUg, bR = g^T dphi/dUd and be = g^T dphi/den.  The forward
-// statements are repeated as written (one rounding each, the same upwind
-// branch), then each is reversed in the opposite order; one forward and one
-// reverse sweep replace the 13 directional passes of the Dual form.
+// statements are repeated in their order (the same upwind branch), then each is
+// reversed in the opposite order: one forward and one reverse sweep, with each
+// reciprocal and root formed once.
 __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], const double L[5], const double R[5],
                                              const double g[5], double bL[5], double bR[5], double be[3]) {
+#pragma clang fp contract(on)
   const double gam = gs.gam, gam1 = gs.gam1, invgam1 = gs.invgam1, ps = gs.pstiff;
   // ---- forward
   const double rn2 = e[0] * e[0] + e[1] * e[1] + e[2] * e[2];
-  const double rnorm = sqrt(rn2);
-  const double invnorm = 1.0 / rnorm;
+  const double invnorm = frsq(rn2);
+  const double rnorm = sqrt_from_rsq(rn2, invnorm);
   const double n0 = e[0] * invnorm, n1 = e[1] * invnorm, n2 = e[2] * invnorm;
   const double vitg2 = L[1] * L[1] + L[2] * L[2] + L[3] * L[3];
   const double vitd2 = R[1] * R[1] + R[2] * R[2] + R[3] * R[3];
-  const double s1 = sqrt(L[0]), s2 = sqrt(R[0]);
+  const double is1 = frsq(L[0]), is2 = frsq(R[0]);
+  const double s1 = sqrt_from_rsq(L[0], is1), s2 = sqrt_from_rsq(R[0], is2);
   const double ener1 = (L[4] + gam * ps) * invgam1 + 0.5 * L[0] * vitg2;
   const double ener2 = (R[4] + gam * ps) * invgam1 + 0.5 * R[0] * vitd2;
-  const double usro = 1.0 / (s1 + s2);
+  const double usro = frcp(s1 + s2);
   const double m2 = s1 * L[1] + s2 * R[1], m3 = s1 * L[2] + s2 * R[2], m4n = s1 * L[3] + s2 * R[3];
   const double u2 = m2 * usro, u3 = m3 * usro, u4 = m4n * usro;
-  const double A1 = (ener1 + L[4]) / s1, A2 = (ener2 + R[4]) / s2;
+  const double A1 = (ener1 + L[4]) * is1, A2 = (ener2 + R[4]) * is2;
   const double u5 = (A1 + A2) * usro;
   const double VdotNt = n0 * u2 + n1 * u3 + n2 * u4;
   const bool left = VdotNt > 0.0;
@@ -129,16 +105,18 @@ __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], c
   const double vit2 = left ? vitg2 : vitd2;
   const double VdotN = S[1] * n0 + S[2] * n1 + S[3] * n2;
   const double H0 = gam * (S[4] + ps) + 0.5 * gam1 * S[0] * vit2;
-  const double H = H0 / (gam1 * S[0]);
+  const double iS0 = left ? is1 * is1 : is2 * is2;
+  const double H = H0 * invgam1 * iS0;
   const double p0 = S[0] * VdotN;
   const double p1 = p0 * S[1] + S[4] * n0, p2 = p0 * S[2] + S[4] * n1, p3 = p0 * S[3] + S[4] * n2;
   const double p4 = p0 * H;
   const double qir = 0.5 * (u2 * u2 + u3 * u3 + u4 * u4);
   const double cr2 = gam1 * (u5 - qir);
-  const double cr = sqrt(cr2);
-  const double icr2 = 1.0 / cr2;
+  const double icr = frsq(cr2);
+  const double cr = sqrt_from_rsq(cr2, icr);
+  const double icr2 = icr * icr;
   const double vp4 = VdotNt + cr, vp5 = VdotNt - cr;
-  const double r = cr, sm = -cr, cb = -cr, itb = -1.0 / cr;
+  const double r = cr, sm = -cr, cb = -cr, itb = -icr;
   const double d1 = -L[0] + R[0];
   const double d2 = -L[0] * L[1] + R[0] * R[1];
   const double d3 = -L[0] * L[2] + R[0] * R[2];
@@ -231,10 +209,10 @@ __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], c
   bRr[2] += R[0] * b_d3;
   bRr[3] += R[0] * b_d4;
   // r = cr, sm = -cr, cb = -cr, itb = -1/cr; vp4 = VdotNt + cr, vp5 = VdotNt - cr
-  double b_cr = b_r - b_sm - b_cb + b_itb / (cr * cr) + b_vp4 - b_vp5;
+  double b_cr = b_r - b_sm - b_cb + b_itb * icr2 + b_vp4 - b_vp5;
   b_VdotNt += b_vp4 + b_vp5;
   // icr2 = 1/cr2, cr = sqrt(cr2), cr2 = gam1 (u5 - qir)
-  const double b_cr2 = -icr2 * icr2 * b_icr2 + 0.5 * b_cr / cr;
+  const double b_cr2 = -icr2 * icr2 * b_icr2 + 0.5 * b_cr * icr;
   b_u5 += gam1 * b_cr2;
   b_qir += -gam1 * b_cr2;
   // qir = (u2^2 + u3^2 + u4^2) / 2
@@ -256,8 +234,8 @@ __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], c
   bS[0] = VdotN * b_p0;
   const double b_VdotN = S[0] * b_p0;
   // H = H0 / (gam1 S0), H0 = gam (S4 + ps) + gam1 S0 vit2 / 2
-  const double b_H0 = b_H / (gam1 * S[0]);
-  bS[0] += -H * b_H / S[0] + 0.5 * gam1 * vit2 * b_H0;
+  const double b_H0 = b_H * invgam1 * iS0;
+  bS[0] += -H * b_H * iS0 + 0.5 * gam1 * vit2 * b_H0;
   bS[4] += gam * b_H0;
   const double b_vit2 = 0.5 * gam1 * S[0] * b_H0;
   // VdotN = S1 n0 + S2 n1 + S3 n2
@@ -287,12 +265,12 @@ __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], c
   // u5 = (A1 + A2) usro, A1 = (ener1 + L4) / s1, A2 = (ener2 + R4) / s2
   double b_usro = (A1 + A2) * b_u5;
   const double b_A1 = usro * b_u5, b_A2 = usro * b_u5;
-  b_ener1 += b_A1 / s1;
-  bLl[4] += b_A1 / s1;
-  double b_s1 = -A1 / s1 * b_A1;
-  b_ener2 += b_A2 / s2;
-  bRr[4] += b_A2 / s2;
-  double b_s2 = -A2 / s2 * b_A2;
+  b_ener1 += b_A1 * is1;
+  bLl[4] += b_A1 * is1;
+  double b_s1 = -A1 * is1 * b_A1;
+  b_ener2 += b_A2 * is2;
+  bRr[4] += b_A2 * is2;
+  double b_s2 = -A2 * is2 * b_A2;
   // u_c = m_c usro, m_c = s1 L_c + s2 R_c
   b_usro += m2 * b_u2 + m3 * b_u3 + m4n * b_u4;
   const double b_m2 = usro * b_u2, b_m3 = usro * b_u3, b_m4 = usro * b_u4;
@@ -315,8 +293,8 @@ __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], c
   bRr[0] += 0.5 * vitd2 * b_ener2;
   b_vitd2 += 0.5 * R[0] * b_ener2;
   // s = sqrt(rho)
-  bLl[0] += 0.5 * b_s1 / s1;
-  bRr[0] += 0.5 * b_s2 / s2;
+  bLl[0] += 0.5 * b_s1 * is1;
+  bRr[0] += 0.5 * b_s2 * is2;
   // vit2 = |u|^2
 #pragma unroll
   for (int k = 1; k < 4; ++k) {
@@ -326,7 +304,7 @@ __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], c
   // n = e invnorm, invnorm = 1/rnorm, rnorm = sqrt(rn2)
   const double b_invnorm = e[0] * b_n0 + e[1] * b_n1 + e[2] * b_n2;
   b_rnorm += -invnorm * invnorm * b_invnorm;
-  const double b_rn2 = 0.5 * b_rnorm / rnorm;
+  const double b_rn2 = 0.5 * b_rnorm * invnorm;
   be[0] = invnorm * b_n0 + 2.0 * e[0] * b_rn2;
   be[1] = invnorm * b_n1 + 2.0 * e[1] * b_rn2;
   be[2] = invnorm * b_n2 + 2.0 * e[2] * b_rn2;
@@ -337,333 +315,384 @@ __device__ __forceinline__ void roeflux7_vjp(const Gas &gs, const double e[3], c
   }
 }
 
-// d VA(a, b) / da and / db of the Van Albada function (RecFcn.h:269-281)
+// d VA(a, b) / da and / db of the Van Albada function q = num / den (RecFcn.h:269-281)
 __device__ __forceinline__ void va_partials(double a, double b, double &da, double &db) {
-  const double eps0 = 1.e-16;
-  da = va_fcn(eps0, Dual(a, 1.0), Dual(b, 0.0)).d;
-  db = va_fcn(eps0, Dual(a, 0.0), Dual(b, 1.0)).d;
+#pragma clang fp contract(on)
+  const double eps = 1.e-16;
+  const double a2 = a * a, b2 = b * b, ab = a * b;
+  const double id = frcp(a2 + b2 + 2.0 * eps);
+  const bool pos = ab > 0.0, zero = ab == 0.0;
+  const double num = pos ? ab * (a + b) + eps * (a + b) : (zero ? 0.5 * eps * (a + b) : 0.0);
+  const double q2 = 2.0 * (num * id);
+  const double na = pos ? 2.0 * ab + (b2 + eps) : (zero ? 0.5 * eps : 0.0);
+  const double nb = pos ? 2.0 * ab + (a2 + eps) : (zero ? 0.5 * eps : 0.0);
+  da = (na - q2 * a) * id;
+  db = (nb - q2 * b) * id;
 }
 
 }  // namespace
 
+// mu = lambda / V, and what each control volume's derivative weighs:
+// R_i = F_i / V_i, so d/dV_i (lambda_i . R_i) = -mu_i . R_i
+__global__ __launch_bounds__(kAdjBlock) void k_adj_mu(DevTables t, const double *__restrict__ lam,
+                                                      const double *__restrict__ R, double *__restrict__ mu,
+                                                      double *__restrict__ cvb) {
+  const int n = blockIdx.x * kAdjBlock + threadIdx.x;
+  if (n >= t.N) return;
+  const double ic = t.invcv[n];
+  double m[5], s = 0.0;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    m[k] = lam[5 * (size_t)n + k] * ic;
+    s += m[k] * R[5 * (size_t)n + k];
+  }
+  store_il<5>(mu, n, m);
+  cvb[n] = -s;
+}
+
 // ---------------------------------------------------------------------------
 // 2. per edge
 // ---------------------------------------------------------------------------
-template <bool SECOND, bool WANTX>
-__device__ __forceinline__ void adj_edge(const DevTables &t, const double *__restrict__ V,
-                                         const double *__restrict__ grad, const double *__restrict__ lam,
-                                         const FluxConsts &fc, double *__restrict__ EV, double *__restrict__ EX) {
-  const long long l = (long long)blockIdx.x * kAdjBlock + threadIdx.x;
-  if (l >= t.E) return;
-  const int2 ij = t.eij[l];
-  const int i = ij.x, j = ij.y;
-  double Vi[5], Vj[5], g[5];
-  const double ici = t.invcv[i], icj = t.invcv[j];
+// A boundary-face slot: mu^T d(face flux) / d(V, face normal / 3).
+template <bool WANTX>
+__device__ __forceinline__ void adj_face_slot(const DevTables &t, const double *__restrict__ V,
+                                              const double *__restrict__ mu, const FluxConsts &fc,
+                                              const int *__restrict__ nfslot, int q, double *__restrict__ FV,
+                                              double *__restrict__ FN) {
+  const int n = t.fnode[q], face = t.fidx[q];
+  const int code = t.fcode[face];
+  double Vn[5], m[5], nf[3];
+  load_il<5>(V, n, Vn);
+  load_il<5>(mu, n, m);
 #pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    Vi[k] = V[il<5>(i, k)];
-    Vj[k] = V[il<5>(j, k)];
-    g[k] = lam[5 * (size_t)i + k] * ici - lam[5 * (size_t)j + k] * icj;
+  for (int a = 0; a < 3; ++a) nf[a] = t.fnorm3[3 * (size_t)face + a];
+#pragma unroll 1
+  for (int dir = 0; dir < (WANTX ? 8 : 5); ++dir) {
+    Dual nv[3], vv[5], fl[5];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) nv[a] = Dual(nf[a], seed(dir, 5 + a));
+#pragma unroll
+    for (int k = 0; k < 5; ++k) vv[k] = Dual(Vn[k], seed(dir, k));
+    face_flux(fc, code, nv, vv, fl);
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) s += m[k] * fl[k].d;
+    if (dir < 5)
+      FV[5 * (size_t)q + dir] = s;
+    else
+      FN[3 * (size_t)nfslot[q] + dir - 5] = s;
   }
-  double dx[3] = {0.0, 0.0, 0.0}, gi[15], gj[15];
-  double VL[5], VR[5];
+}
+
+// A wave per (64 nodes, k-th upper edge), as the residual's flux pass on small
+// meshes; the first nfb blocks take the boundary-face slots.  Everything is read
+// and written by position, so what is not gathered is contiguous.  Two waves per
+// SIMD (256 registers): the gradients are read again after the flux for dxbar
+// rather than held across it (1013 -> 619 us at 815k nodes, 5.6M edges).
+template <bool SECOND, bool WANTX>
+__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_edges(
+    DevTables t, int nfb, const double *__restrict__ V, const double *__restrict__ grad,
+    const double *__restrict__ mu, FluxConsts fc, const int *__restrict__ nfslot, double *__restrict__ EVi,
+    double *__restrict__ EVj, double *__restrict__ EXd, double *__restrict__ EXn, double *__restrict__ FV,
+    double *__restrict__ FN) {
+  if ((int)blockIdx.x < nfb) {
+    const int q = blockIdx.x * kAdjBlock + threadIdx.x;
+    if (q < 3 * t.F) adj_face_slot<WANTX>(t, V, mu, fc, nfslot, q, FV, FN);
+    return;
+  }
+  const int nb = (t.nup + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
+  const int w = xcd_chunk(blockIdx.x - nfb, nb) * (kAdjBlock / kWave) + (int)(threadIdx.x / kWave);
+  if (w >= t.nup) return;
+  const int sl = t.upslice[w];
+  const int i = sl * kWave + lane_id();
+  const bool act = i < t.N && w - t.up.kptr[sl] < t.eup[min(i, t.N - 1) + 1] - t.eup[min(i, t.N - 1)];
+  const int pos = t.up.koff[w] + lanes_below(act);
+  if (!act) return;
+  const int j = t.up.idx[pos];
+  double VL[5], VR[5], dV[5], g[5], dx[3], di[5], dj[5];
+  {
+    double mj[5];
+    load_il<5>(mu, i, g);
+    load_il<5>(mu, j, mj);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) g[k] -= mj[k];
+  }
+  load_il<5>(V, i, VL);
+  load_il<5>(V, j, VR);
   if (SECOND) {
-    const double4 xi = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)i);
-    const double4 xj = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)j);
-    dx[0] = xj.x - xi.x;
-    dx[1] = xj.y - xi.y;
-    dx[2] = xj.z - xi.z;
+    double xi[3], gi[15], gj[15];
+    load_il<3>(t.X3, i, xi);
+    load_il<3>(t.X3, j, dx);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) dx[a] -= xi[a];
     load_il<15>(grad, i, gi);
     load_il<15>(grad, j, gj);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-      const double ddVij = dx[0] * gi[k] + dx[1] * gi[5 + k] + dx[2] * gi[10 + k];
-      const double ddVji = dx[0] * gj[k] + dx[1] * gj[5 + k] + dx[2] * gj[10 + k];
-      vanalbada(fc.beta, Vi[k], ddVij, Vj[k], ddVji, VL[k], VR[k]);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      VL[k] = Vi[k];
-      VR[k] = Vj[k];
+      di[k] = dx[0] * gi[k] + dx[1] * gi[5 + k] + dx[2] * gi[10 + k];
+      dj[k] = dx[0] * gj[k] + dx[1] * gj[5 + k] + dx[2] * gj[10 + k];
+      const double a = VL[k], b = VR[k];
+      dV[k] = b - a;
+      reconstruct(fc.beta, a, di[k], b, dj[k], VL[k], VR[k]);
     }
   }
-  const double nv[3] = {t.normal[3 * (size_t)l], t.normal[3 * (size_t)l + 1], t.normal[3 * (size_t)l + 2]};
-  double fb[13];
+  double nv[3], fb[13];
+  load_il<3>(t.pnormal, pos, nv);
 #pragma unroll
   for (int d = 0; d < 13; ++d) fb[d] = 0.0;
-  if (!(sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]) < 1e-18))
+  if (!(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2] < 1e-36))
     roeflux7_vjp(fc.gas, nv, VL, VR, g, fb, fb + 5, fb + 10);
-  double vbi[5], vbj[5], ci[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, cj[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  double dxb[3] = {0.0, 0.0, 0.0};
-  if (SECOND) {
-    const double beta = fc.beta, beta2 = 1.0 - 2.0 * beta;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      const double ddVij = dx[0] * gi[k] + dx[1] * gi[5 + k] + dx[2] * gi[10 + k];
-      const double ddVji = dx[0] * gj[k] + dx[1] * gj[5 + k] + dx[2] * gj[10 + k];
-      const double dVji = Vj[k] - Vi[k];
-      const double dV = beta2 * dVji;
-      const double dVi = dV + 2.0 * beta * ddVij;
-      const double dVj = dV + 2.0 * beta * ddVji;
-      double da_i, db_i, da_j, db_j;
-      va_partials(dVi, dVji, da_i, db_i);
-      va_partials(dVj, dVji, da_j, db_j);
-      const double Lb = fb[k], Rb = fb[5 + k];
-      const double A = 0.5 * Lb * da_i, B = 0.5 * Lb * db_i;
-      const double A2 = -0.5 * Rb * da_j, B2 = -0.5 * Rb * db_j;
-      const double dVjib = B + B2 + beta2 * (A + A2);
-      const double ddVijb = 2.0 * beta * A, ddVjib = 2.0 * beta * A2;
-      vbi[k] = Lb - dVjib;
-      vbj[k] = Rb + dVjib;
-      // Gbar_i[5a+k] = ddVijb dx[a]: the node pass forms the products
-      ci[k] = ddVijb;
-      cj[k] = ddVjib;
-      if (WANTX) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) dxb[a] += ddVijb * gi[5 * a + k] + ddVjib * gj[5 * a + k];
-      }
+  if (WANTX) store_il<3>(EXn, pos, fb + 10);
+  if (!SECOND) {
+    store_il<5>(EVi, pos, fb);
+    store_il<5>(EVj, pos, fb + 5);
+    if (WANTX) {
+      const double z[3] = {0.0, 0.0, 0.0};
+      store_il<3>(EXd, pos, z);
     }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      vbi[k] = fb[k];
-      vbj[k] = fb[5 + k];
-    }
+    return;
   }
-  double2 *ev = reinterpret_cast<double2 *>(EV + 20 * (size_t)l);
-  ev[0] = make_double2(vbi[0], vbi[1]);
-  ev[1] = make_double2(vbi[2], vbi[3]);
-  ev[2] = make_double2(vbi[4], ci[0]);
-  ev[3] = make_double2(ci[1], ci[2]);
-  ev[4] = make_double2(ci[3], ci[4]);
-  ev[5] = make_double2(vbj[0], vbj[1]);
-  ev[6] = make_double2(vbj[2], vbj[3]);
-  ev[7] = make_double2(vbj[4], cj[0]);
-  ev[8] = make_double2(cj[1], cj[2]);
-  ev[9] = make_double2(cj[3], cj[4]);
+  const double beta = fc.beta, beta2 = 1.0 - 2.0 * beta;
+  double ei[10], ej[10];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    const double d = beta2 * dV[k];
+    double da_i, db_i, da_j, db_j;
+    va_partials(d + 2.0 * beta * di[k], dV[k], da_i, db_i);
+    va_partials(d + 2.0 * beta * dj[k], dV[k], da_j, db_j);
+    const double Lb = fb[k], Rb = fb[5 + k];
+    const double A = 0.5 * Lb * da_i, B = 0.5 * Lb * db_i;
+    const double A2 = -0.5 * Rb * da_j, B2 = -0.5 * Rb * db_j;
+    const double dVb = B + B2 + beta2 * (A + A2);
+    ei[k] = Lb - dVb;
+    ej[k] = Rb + dVb;
+    // Gbar_i[5a+k] = c_i dx[a]: the node pass forms the products
+    ei[5 + k] = 2.0 * beta * A;
+    ej[5 + k] = 2.0 * beta * A2;
+  }
+  store_il<10>(EVi, pos, ei);
+  store_il<10>(EVj, pos, ej);
   if (WANTX) {
-    double *ex = EX + 6 * (size_t)l;
+    const double *g2 = grad;
+    asm volatile("" : "+s"(g2));
+    double h[15], dxb[3] = {0.0, 0.0, 0.0};
+    load_il<15>(g2, i, h);
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      ex[a] = dxb[a];
-      ex[3 + a] = fb[10 + a];
-    }
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int k = 0; k < 5; ++k) dxb[a] += ei[5 + k] * h[5 * a + k];
+    load_il<15>(g2, j, h);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int k = 0; k < 5; ++k) dxb[a] += ej[5 + k] * h[5 * a + k];
+    store_il<3>(EXd, pos, dxb);
   }
-}
-
-// The (dR/dU)^T-only edge pass fits two waves per SIMD without spilling
-// (256 VGPRs; 2.10 -> 1.83 ms at 815k nodes); with the coordinate slots it
-// would spill 68 registers and is left at the compiler's choice.
-template <bool SECOND>
-__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_edges_u(
-    DevTables t, const double *__restrict__ V, const double *__restrict__ grad, const double *__restrict__ lam,
-    FluxConsts fc, double *__restrict__ EV, double *__restrict__ EX) {
-  adj_edge<SECOND, false>(t, V, grad, lam, fc, EV, EX);
-}
-template <bool SECOND>
-__global__ __launch_bounds__(kAdjBlock) void k_adj_edges_x(DevTables t, const double *__restrict__ V,
-                                                           const double *__restrict__ grad,
-                                                           const double *__restrict__ lam, FluxConsts fc,
-                                                           double *__restrict__ EV, double *__restrict__ EX) {
-  adj_edge<SECOND, true>(t, V, grad, lam, fc, EV, EX);
 }
 
 // ---------------------------------------------------------------------------
 // 3. per node: edge slots in edge order, then faces
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const double *__restrict__ V,
-                                                         const double *__restrict__ lam, FluxConsts fc,
-                                                         const double *__restrict__ EV,
-                                                         const double *__restrict__ EX, int second, int want_x,
-                                                         double *__restrict__ Vb, double *__restrict__ Gb,
+// one edge slot: Vbar, and Gbar += c dx^T with dx = X_j - X_i of the edge (i, j)
+template <bool SECOND>
+__device__ __forceinline__ void add_slot(const double *ev, const double dx[3], double vb[5], double gb[15]) {
+#pragma unroll
+  for (int k = 0; k < 5; ++k) vb[k] += ev[k];
+  if (SECOND) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int k = 0; k < 5; ++k) gb[5 * a + k] += ev[5 + k] * dx[a];
+  }
+}
+
+// A wave per 64 nodes: the slots of the upper edges are contiguous, those of the
+// lower ones are gathered, and both ends' coordinates follow from the adjacency
+// rows, whose first entries are the lower neighbours.  Bound by the slots' bytes
+// (624 -> 342 us at 815k nodes, 3.9 TB/s).
+template <bool SECOND, bool WANTX>
+__global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const double *__restrict__ grad,
+                                                         const double *__restrict__ EVi,
+                                                         const double *__restrict__ EVj,
+                                                         const double *__restrict__ EXd,
+                                                         const double *__restrict__ FV, double *__restrict__ Vb,
+                                                         double *__restrict__ H, double *__restrict__ S,
                                                          double *__restrict__ Xb) {
-  const int n = blockIdx.x * kAdjBlock + threadIdx.x;
-  if (n >= t.N) return;
-  double vb[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, gb[15], xb[3] = {0.0, 0.0, 0.0};
+  constexpr int W = SECOND ? 10 : 5;
+  const int sl = wave_slice(t);
+  if (sl >= t.ns) return;
+  const int n = sl * kWave + lane_id();
+  const bool live = n < t.N;
+  double vb[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, gb[15], xb[3] = {0.0, 0.0, 0.0}, xn[3] = {0.0, 0.0, 0.0};
 #pragma unroll
   for (int q = 0; q < 15; ++q) gb[q] = 0.0;
-  const double4 xn = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)n);
-  // one edge slot: Vbar, and Gbar = c dx^T with dx = X_j - X_i as the edge
-  // pass formed it (the same products, added in the same order)
-  auto add_slot = [&](const double *ev, int m, bool upper) {
-    double c[5];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      vb[k] += ev[k];
-      c[k] = ev[5 + k];
-    }
-    if (second) {
-      const double4 xm = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)m);
-      const double dx[3] = {upper ? xm.x - xn.x : xn.x - xm.x, upper ? xm.y - xn.y : xn.y - xm.y,
-                            upper ? xm.z - xn.z : xn.z - xm.z};
-#pragma unroll
-      for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int k = 0; k < 5; ++k) gb[5 * a + k] += c[k] * dx[a];
-    }
-  };
+  if (SECOND) load_il<3>(t.X3, min(n, t.N - 1), xn);
   // edges (m, n), m < n: the j-side slots
-  for (int q = t.lrow[n]; q < t.lrow[n + 1]; ++q) {
-    const size_t l = t.ledge[q];
-    add_slot(EV + 20 * l + 10, t.eij[l].x, false);
-    if (want_x) {
+  {
+    const int deg = live ? t.lrow[n + 1] - t.lrow[n] : 0, all = live ? t.rowptr[n + 1] - t.rowptr[n] : 0;
+    const int kb = t.lo.kptr[sl], ke = t.lo.kptr[sl + 1], ab = t.nb.kptr[sl];
+    for (int k = 0; k < ke - kb; ++k) {
+      const bool act = k < deg;
+      const int q = t.lo.koff[kb + k] + lanes_below(act), e = t.nb.koff[ab + k] + lanes_below(k < all);
+      if (!act) continue;
+      const int pos = t.lo.idx[q];
+      double ev[W], dx[3] = {0.0, 0.0, 0.0}, d[3];
+      load_il<W>(EVj, pos, ev);
+      if (SECOND) {
+        load_il<3>(t.X3, t.nb.idx[e], dx);
 #pragma unroll
-      for (int a = 0; a < 3; ++a) xb[a] += EX[6 * l + a];
+        for (int a = 0; a < 3; ++a) dx[a] = xn[a] - dx[a];
+      }
+      if (SECOND && WANTX) {
+        load_il<3>(EXd, pos, d);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) xb[a] += d[a];
+      }
+      add_slot<SECOND>(ev, dx, vb, gb);
     }
   }
   // edges (n, m), n < m: the i-side slots
-  for (int l = t.eup[n]; l < t.eup[n + 1]; ++l) {
-    add_slot(EV + 20 * (size_t)l, t.eij[l].y, true);
-    if (want_x) {
+  {
+    const int deg = live ? t.eup[n + 1] - t.eup[n] : 0;
+    const int kb = t.up.kptr[sl], ke = t.up.kptr[sl + 1];
+    for (int k = 0; k < ke - kb; ++k) {
+      const bool act = k < deg;
+      const int pos = t.up.koff[kb + k] + lanes_below(act);
+      if (!act) continue;
+      double ev[W], dx[3] = {0.0, 0.0, 0.0}, d[3];
+      load_il<W>(EVi, pos, ev);
+      if (SECOND) {
+        load_il<3>(t.X3, t.up.idx[pos], dx);
 #pragma unroll
-      for (int a = 0; a < 3; ++a) xb[a] -= EX[6 * (size_t)l + a];
-    }
-  }
-  const int f0 = t.frow[n], f1 = t.frow[n + 1];
-  if (f0 < f1) {
-    const double ic = t.invcv[n];
-    double mu[5], Vn[5];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      mu[k] = lam[5 * (size_t)n + k] * ic;
-      Vn[k] = V[il<5>(n, k)];
-    }
-    for (int q = f0; q < f1; ++q) {
-      const int face = t.fidx[q];
-      const int code = t.fcode[face];
-#pragma unroll 1
-      for (int dir = 0; dir < 5; ++dir) {
-        Dual nv[3], vv[5], fl[5];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) nv[a] = Dual(t.fnorm3[3 * (size_t)face + a]);
-#pragma unroll
-        for (int k = 0; k < 5; ++k) vv[k] = Dual(Vn[k], seed(dir, k));
-        face_flux(fc, code, nv, vv, fl);
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < 5; ++k) s += mu[k] * fl[k].d;
-        vb[dir] += s;
+        for (int a = 0; a < 3; ++a) dx[a] -= xn[a];
       }
+      if (SECOND && WANTX) {
+        load_il<3>(EXd, pos, d);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) xb[a] -= d[a];
+      }
+      add_slot<SECOND>(ev, dx, vb, gb);
     }
   }
+  if (!live) return;
+  for (int q = t.frow[n]; q < t.frow[n + 1]; ++q)
 #pragma unroll
-  for (int k = 0; k < 5; ++k) Vb[5 * (size_t)n + k] = vb[k];
+    for (int k = 0; k < 5; ++k) vb[k] += FV[5 * (size_t)q + k];
+  store_il<5>(Vb, n, vb);
+  if (WANTX) store_il<3>(Xb, n, xb);
+  if (!SECOND) return;
+  double L[6];
 #pragma unroll
-  for (int r = 0; r < 15; ++r) Gb[16 * (size_t)n + r] = gb[r];
+  for (int q = 0; q < 6; ++q) L[q] = t.lsq6[6 * (size_t)n + q];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) Xb[4 * (size_t)n + a] = xb[a];
+  for (int k = 0; k < 5; ++k) {
+    double w[3];
+    lsq_weights(L, gb[k], gb[5 + k], gb[10 + k], w);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) gb[5 * a + k] = w[a];
+  }
+  store_il<15>(H, n, gb);
+  if (WANTX) {
+    double gn[15], s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    load_il<15>(grad, n, gn);
+    int e = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = a; b < 3; ++b, ++e)
+#pragma unroll
+        for (int k = 0; k < 5; ++k) s[e] -= gb[5 * a + k] * gn[5 * b + k] + gb[5 * b + k] * gn[5 * a + k];
+    store_il<6>(S, n, s);
+  }
 }
 
 // ---------------------------------------------------------------------------
 // 4. per node: reverse of the LSQ gradients, then U
 // ---------------------------------------------------------------------------
+// Bound by the gathers of H, S, V and X (29 values an entry, where the weights of
+// both ends were formed per entry from their factors; 376 -> 229 us at 815k nodes).
+template <bool SECOND, bool WANTX>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double *__restrict__ V,
                                                        const double *__restrict__ U, Gas gas,
-                                                       const double *__restrict__ Vb,
-                                                       const double *__restrict__ Gb, int second, int want_x,
-                                                       double *__restrict__ Ub, double *__restrict__ Xb,
-                                                       double *__restrict__ S) {
-  const int n = blockIdx.x * kAdjBlock + threadIdx.x;
-  if (n >= t.N) return;
-  double vb[5], Vn[5];
+                                                       const double *__restrict__ Vb, const double *__restrict__ H,
+                                                       const double *__restrict__ S, double *__restrict__ Ub,
+                                                       double *__restrict__ Xb) {
+  const int sl = wave_slice(t);
+  if (sl >= t.ns) return;
+  const int n = sl * kWave + lane_id();
+  const bool live = n < t.N;
+  const int nn = min(n, t.N - 1);
+  double vb[5], Vn[5], xb[3] = {0.0, 0.0, 0.0};
+  load_il<5>(Vb, nn, vb);
+  load_il<5>(V, nn, Vn);
+  if (SECOND) {
+    // sum over j of dx and of V_j - V_i: what the node's own H and S multiply
+    double xn[3], sx[3] = {0.0, 0.0, 0.0}, sv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    load_il<3>(t.X3, nn, xn);
+    const int deg = live ? t.rowptr[n + 1] - t.rowptr[n] : 0;
+    const int kb = t.nb.kptr[sl], ke = t.nb.kptr[sl + 1];
+    auto add = [&](const double h[15], const double s[6], const double dx[3], const double dV[5]) {
 #pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    vb[k] = Vb[5 * (size_t)n + k];
-    Vn[k] = V[il<5>(n, k)];
-  }
-  if (second) {
-    double Ln[6], gn[15];
+      for (int k = 0; k < 5; ++k) vb[k] -= h[k] * dx[0] + h[5 + k] * dx[1] + h[10 + k] * dx[2];
+      if (WANTX) {
 #pragma unroll
-    for (int q = 0; q < 6; ++q) Ln[q] = t.lsq6[6 * (size_t)n + q];
+        for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int q = 0; q < 15; ++q) gn[q] = Gb[16 * (size_t)n + q];
-    const double4 xn = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)n);
-    double xacc[3] = {0.0, 0.0, 0.0}, Lb[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double M[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int e = t.rowptr[n]; e < t.rowptr[n + 1]; ++e) {
-      const int m = t.adj[e];
-      const double4 xm = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)m);
-      const double dx0 = xm.x - xn.x, dx1 = xm.y - xn.y, dx2 = xm.z - xn.z;
-      double Lm[6], gm[15], Vm[5];
+          for (int k = 0; k < 5; ++k) xb[a] -= h[5 * a + k] * dV[k];
+        xb[0] -= s[0] * dx[0] + s[1] * dx[1] + s[2] * dx[2];
+        xb[1] -= s[1] * dx[0] + s[3] * dx[1] + s[4] * dx[2];
+        xb[2] -= s[2] * dx[0] + s[4] * dx[1] + s[5] * dx[2];
+      }
+    };
+    for (int k = 0; k < ke - kb; ++k) {
+      const bool act = k < deg;
+      const int pos = t.nb.koff[kb + k] + lanes_below(act);
+      if (!act) continue;
+      const int m = t.nb.idx[pos];
+      double h[15], s[6], dx[3], dV[5];
+      load_il<3>(t.X3, m, dx);
+      load_il<15>(H, m, h);
+      if (WANTX) {
+        load_il<5>(V, m, dV);
+        load_il<6>(S, m, s);
 #pragma unroll
-      for (int q = 0; q < 6; ++q) Lm[q] = t.lsq6[6 * (size_t)m + q];
-#pragma unroll
-      for (int q = 0; q < 15; ++q) gm[q] = Gb[16 * (size_t)m + q];
-      load_il<5>(V, m, Vm);
-      double wn[3], wm[3];
-      lsq_weights(Ln, dx0, dx1, dx2, wn);      // row n, neighbour m
-      lsq_weights(Lm, -dx0, -dx1, -dx2, wm);   // row m, neighbour n (dx_mn = X_n - X_m)
-#pragma unroll
-      for (int k = 0; k < 5; ++k)
-        vb[k] += (wm[0] * gm[k] + wm[1] * gm[5 + k] + wm[2] * gm[10 + k]) -
-                 (wn[0] * gn[k] + wn[1] * gn[5 + k] + wn[2] * gn[10 + k]);
-      if (want_x) {
-        double wbn[3], wbm[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          double s1 = 0.0, s2 = 0.0;
-#pragma unroll
-          for (int k = 0; k < 5; ++k) {
-            s1 += gn[5 * a + k] * (Vm[k] - Vn[k]);
-            s2 += gm[5 * a + k] * (Vn[k] - Vm[k]);
-          }
-          wbn[a] = s1;
-          wbm[a] = s2;
+        for (int q = 0; q < 5; ++q) {
+          dV[q] -= Vn[q];
+          sv[q] += dV[q];
         }
-        double dxn[3] = {0.0, 0.0, 0.0}, dxm[3] = {0.0, 0.0, 0.0};
-        lsq_weights_rev(Ln, dx0, dx1, dx2, wbn, dxn, Lb);
-        lsq_weights_rev(Lm, -dx0, -dx1, -dx2, wbm, dxm, nullptr);
-#pragma unroll
-        for (int a = 0; a < 3; ++a) xacc[a] += dxm[a] - dxn[a];
-        // LSQ moments in edge order (rows are in ascending edge id)
-        M[0] += dx0 * dx0;
-        M[1] += dx0 * dx1;
-        M[2] += dx0 * dx2;
-        M[3] += dx1 * dx1;
-        M[4] += dx1 * dx2;
-        M[5] += dx2 * dx2;
       }
-    }
-    if (want_x) {
-      double Mb[6];
-#pragma unroll 1
-      for (int dir = 0; dir < 6; ++dir) {
-        Dual Md[6], Ld[6];
 #pragma unroll
-        for (int q = 0; q < 6; ++q) Md[q] = Dual(M[q], seed(dir, q));
-        lsq_params(Md, Ld);
-        double s = 0.0;
-#pragma unroll
-        for (int q = 0; q < 6; ++q) s += Lb[q] * Ld[q].d;
-        Mb[dir] = s;
+      for (int a = 0; a < 3; ++a) {
+        dx[a] -= xn[a];
+        sx[a] += dx[a];
       }
-      double *sn = S + 6 * (size_t)n;
-      sn[0] = 2.0 * Mb[0];
-      sn[1] = Mb[1];
-      sn[2] = Mb[2];
-      sn[3] = 2.0 * Mb[3];
-      sn[4] = Mb[4];
-      sn[5] = 2.0 * Mb[5];
-#pragma unroll
-      for (int a = 0; a < 3; ++a) Xb[4 * (size_t)n + a] += xacc[a];
+      add(h, s, dx, dV);
     }
+    double h[15], s[6];
+    load_il<15>(H, nn, h);
+    if (WANTX) load_il<6>(S, nn, s);
+    add(h, s, sx, sv);
+  }
+  if (!live) return;
+  if (WANTX) {
+    double x[3];
+    load_il<3>(Xb, n, x);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) x[a] += xb[a];
+    store_il<3>(Xb, n, x);
   }
   if (Ub) {
-    double u[5], ub[5];
+    // V = (rho, u / rho, (gam - 1) (E - rho |u|^2 / 2) - gam pstiff)
+    const double ir = 1.0 / U[5 * (size_t)n], gp = gas.gam1 * vb[4];
+    double q = 0.0, r = 0.0, ub[5];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) u[k] = U[5 * (size_t)n + k];
-#pragma unroll 1
-    for (int dir = 0; dir < 5; ++dir) {
-      Dual ud[5], vd[5];
-#pragma unroll
-      for (int k = 0; k < 5; ++k) ud[k] = Dual(u[k], seed(dir, k));
-      prim_from_cons(ud, gas, vd);
-      double s = 0.0;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) s += vb[k] * vd[k].d;
-      ub[dir] = s;
+    for (int k = 1; k < 4; ++k) {
+      ub[k] = vb[k] * ir - gp * Vn[k];
+      q += Vn[k] * Vn[k];
+      r += Vn[k] * vb[k];
     }
+    ub[0] = vb[0] - r * ir + 0.5 * gp * q;
+    ub[4] = gp;
 #pragma unroll
     for (int k = 0; k < 5; ++k) Ub[5 * (size_t)n + k] = ub[k];
   }
@@ -672,207 +701,173 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double
 // ---------------------------------------------------------------------------
 // 5. geometry: per tet (control volumes, dual normals), per boundary face
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kAdjBlock) void k_adj_tets(int T, const int *__restrict__ tets,
-                                                        const int *__restrict__ tedge,
+__device__ __forceinline__ void load_x4(const double *__restrict__ X4, int n, double x[3]) {
+  const double4 p = *reinterpret_cast<const double4 *>(X4 + 4 * (size_t)n);
+  x[0] = p.x;
+  x[1] = p.y;
+  x[2] = p.z;
+}
+// z += s (x x y)
+__device__ __forceinline__ void add_cross(double s, const double x[3], const double y[3], double z[3]) {
+  z[0] += s * (x[1] * y[2] - x[2] * y[1]);
+  z[1] += s * (x[2] * y[0] - x[0] * y[2]);
+  z[2] += s * (x[0] * y[1] - x[1] * y[0]);
+}
+
+// The tet's share of each quantity is a product of coordinate differences, so
+// its reverse is a few cross products: with p = c - d, r = (a - c) + (b - d) and
+// w the weight of an edge, d(w . p x r) = dp . r x w + dr . w x p.  Bound by the
+// gathers of six nbar and the stores (659 -> 282 us for 4.7M tets; 12 passes in
+// dual numbers before).
+__global__ __launch_bounds__(kAdjBlock) void k_adj_tets(int T, const int4 *__restrict__ tets,
+                                                        const int *__restrict__ tpos,
                                                         const double *__restrict__ X4,
-                                                        const double *__restrict__ invcv,
-                                                        const double *__restrict__ lam,
-                                                        const double *__restrict__ R,
-                                                        const double *__restrict__ EX, double *__restrict__ TX) {
-  const long long t = (long long)blockIdx.x * kAdjBlock + threadIdx.x;
+                                                        const double *__restrict__ cvb,
+                                                        const double *__restrict__ EXn, double *__restrict__ TX) {
+#pragma clang fp contract(on)
+  const int nblk = (T + kAdjBlock - 1) / kAdjBlock;
+  const int t = xcd_chunk(blockIdx.x, nblk) * kAdjBlock + (int)threadIdx.x;
   if (t >= T) return;
-  int nd[4];
-  double x[4][3], cvb = 0.0;
+  const int4 d4 = tets[t];
+  const int nd[4] = {d4.x, d4.y, d4.z, d4.w};
+  int ps[6];
+#pragma unroll
+  for (int e = 0; e < 6; e += 2) {
+    const int2 q = *reinterpret_cast<const int2 *>(tpos + 6 * (size_t)t + e);
+    ps[e] = q.x;
+    ps[e + 1] = q.y;
+  }
+  double x[4][3], z[4][3], cv = 0.0;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
-    nd[v] = tets[4 * t + v];
-    const double4 xv = *reinterpret_cast<const double4 *>(X4 + 4 * (size_t)nd[v]);
-    x[v][0] = xv.x;
-    x[v][1] = xv.y;
-    x[v][2] = xv.z;
-    // R_i = F_i / cv_i: d/dcv_i (lambda_i . R_i) = -lambda_i . R_i / cv_i
-    double s = 0.0;
+    load_x4(X4, nd[v], x[v]);
+    cv += cvb[nd[v]];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) s += lam[5 * (size_t)nd[v] + k] * R[5 * (size_t)nd[v] + k];
-    cvb += -s * invcv[nd[v]];
+    for (int a = 0; a < 3; ++a) z[v][a] = 0.0;
   }
-  double nb[6][3], sg[6];
+  // ElemTet::computeVolume (ElemTetCore.C:31-44): v3 . (v1 x v2) / 6, a quarter
+  // of it to each vertex
+  {
+    double e[3][3];
+#pragma unroll
+    for (int v = 0; v < 3; ++v)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) e[v][a] = x[v + 1][a] - x[0][a];
+    const double s = cv * (1.0 / 24.0);
+    add_cross(s, e[1], e[2], z[1]);
+    add_cross(s, e[2], e[0], z[2]);
+    add_cross(s, e[0], e[1], z[3]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) z[0][a] -= z[1][a] + z[2][a] + z[3][a];
+  }
+  // dual-face normals (ElemTetCore.C:281-330)
 #pragma unroll
   for (int e = 0; e < 6; ++e) {
-    const size_t l = tedge[6 * t + e];
-    sg[e] = nd[cEdgeEnd[e][0]] < nd[cEdgeEnd[e][1]] ? 1.0 : -1.0;
+    const int a = kEnd[e][0], b = kEnd[e][1], c = kOpp[e][0], d = kOpp[e][1];
+    double w[3], p[3], r[3], gp[3] = {0.0, 0.0, 0.0}, gr[3] = {0.0, 0.0, 0.0};
+    load_il<3>(EXn, ps[e], w);
+    const double s = nd[a] < nd[b] ? 1.0 / 24.0 : -1.0 / 24.0;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) nb[e][a] = EX[6 * l + 3 + a];
+    for (int k = 0; k < 3; ++k) {
+      p[k] = x[c][k] - x[d][k];
+      r[k] = (x[a][k] - x[c][k]) + (x[b][k] - x[d][k]);
+    }
+    add_cross(s, r, w, gp);
+    add_cross(s, w, p, gr);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      z[a][k] += gr[k];
+      z[b][k] += gr[k];
+      z[c][k] += gp[k] - gr[k];
+      z[d][k] -= gp[k] + gr[k];
+    }
   }
-  const double third = 1.0 / 3.0, sixth = 1.0 / 6.0;
-#pragma unroll 1
-  for (int dir = 0; dir < 12; ++dir) {
-    Dual xd[4][3];
+  double2 *o = reinterpret_cast<double2 *>(TX + 12 * (size_t)t);
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-#pragma unroll
-      for (int a = 0; a < 3; ++a) xd[v][a] = Dual(x[v][a], seed(dir, 3 * v + a));
-    // ElemTet::computeVolume (ElemTetCore.C:31-44)
-    Dual v1[3], v2[3], v3[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      v1[a] = xd[1][a] - xd[0][a];
-      v2[a] = xd[2][a] - xd[0][a];
-      v3[a] = xd[3][a] - xd[0][a];
-    }
-    Dual c0 = v1[1] * v2[2] - v1[2] * v2[1];
-    Dual c1 = v1[2] * v2[0] - v1[0] * v2[2];
-    Dual c2 = v1[0] * v2[1] - v1[1] * v2[0];
-    Dual vol = sixth * (v3[0] * c0 + v3[1] * c1 + v3[2] * c2);
-    double acc = 0.25 * vol.d * cvb;
-    // dual-face normals (ElemTetCore.C:281-330)
-    Dual f[4][3], gc[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      f[0][a] = third * ((xd[0][a] + xd[1][a]) + xd[2][a]);
-      f[1][a] = third * ((xd[0][a] + xd[1][a]) + xd[3][a]);
-      f[2][a] = third * ((xd[0][a] + xd[2][a]) + xd[3][a]);
-      f[3][a] = third * ((xd[1][a] + xd[2][a]) + xd[3][a]);
-      gc[a] = 0.25 * (((xd[0][a] + xd[1][a]) + xd[2][a]) + xd[3][a]);
-    }
-#pragma unroll
-    for (int e = 0; e < 6; ++e) {
-      Dual p[3], q[3];
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        p[a] = f[cEdgeFace[e][1]][a] - gc[a];
-        q[a] = f[cEdgeFace[e][0]][a] - gc[a];
-      }
-      Dual A[3] = {p[1] * q[2] - p[2] * q[1], p[2] * q[0] - p[0] * q[2], p[0] * q[1] - p[1] * q[0]};
-      double s = 0.0;
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        Dual nn = 0.5 * (A[a] + A[a]) + 0.25 * (A[a] + A[a]);
-        s += nb[e][a] * nn.d;
-      }
-      acc += sg[e] * s;
-    }
-    TX[12 * t + dir] = acc;
+  for (int v = 0; v < 4; v += 2) {
+    o[3 * v / 2] = make_double2(z[v][0], z[v][1]);
+    o[3 * v / 2 + 1] = make_double2(z[v][2], z[v + 1][0]);
+    o[3 * v / 2 + 2] = make_double2(z[v + 1][1], z[v + 1][2]);
   }
 }
 
 __global__ __launch_bounds__(kAdjBlock) void k_adj_faces(int F, const int *__restrict__ faces,
-                                                         const int *__restrict__ fcode,
-                                                         const double *__restrict__ fnorm3,
                                                          const double *__restrict__ X4,
-                                                         const double *__restrict__ invcv,
-                                                         const double *__restrict__ V,
-                                                         const double *__restrict__ lam, FluxConsts fc,
-                                                         double *__restrict__ FX) {
+                                                         const double *__restrict__ FN, double *__restrict__ FX) {
   const int f = blockIdx.x * kAdjBlock + threadIdx.x;
   if (f >= F) return;
-  const int code = fcode[f];
-  double nb[3] = {0.0, 0.0, 0.0};
-  int nd[3];
-#pragma unroll
-  for (int v = 0; v < 3; ++v) nd[v] = faces[3 * (size_t)f + v];
-#pragma unroll 1
-  for (int v = 0; v < 3; ++v) {
-    const int n = nd[v];
-    const double ic = invcv[n];
-    double mu[5];
-    Dual vv[5];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      mu[k] = lam[5 * (size_t)n + k] * ic;
-      vv[k] = Dual(V[il<5>(n, k)]);
-    }
-#pragma unroll 1
-    for (int dir = 0; dir < 3; ++dir) {
-      Dual nv[3], fl[5];
-#pragma unroll
-      for (int a = 0; a < 3; ++a) nv[a] = Dual(fnorm3[3 * (size_t)f + a], seed(dir, a));
-      face_flux(fc, code, nv, vv, fl);
-      double s = 0.0;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) s += mu[k] * fl[k].d;
-      nb[dir] += s;
-    }
-  }
-  // nv = (1/3) n_f (FaceTriaCore.C:288-292)
-  const double third = 1.0 / 3.0;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) nb[a] *= third;
-  double x[3][3];
+  double x[3][3], nb[3] = {0.0, 0.0, 0.0};
 #pragma unroll
   for (int v = 0; v < 3; ++v) {
-    const double4 xv = *reinterpret_cast<const double4 *>(X4 + 4 * (size_t)nd[v]);
-    x[v][0] = xv.x;
-    x[v][1] = xv.y;
-    x[v][2] = xv.z;
+    load_x4(X4, faces[3 * (size_t)f + v], x[v]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) nb[a] += FN[9 * (size_t)f + 3 * v + a];
   }
-#pragma unroll 1
-  for (int dir = 0; dir < 9; ++dir) {
-    Dual xd[3][3];
+  // a third of FaceTria::computeNormal (FaceTriaCore.C:31-37, 288-292):
+  // (x2 - x0) x (x1 - x0) / 6
+  double p[3], q[3], gp[3] = {0.0, 0.0, 0.0}, gq[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int v = 0; v < 3; ++v)
+  for (int a = 0; a < 3; ++a) {
+    p[a] = x[2][a] - x[0][a];
+    q[a] = x[1][a] - x[0][a];
+  }
+  add_cross(1.0 / 6.0, q, nb, gp);
+  add_cross(1.0 / 6.0, nb, p, gq);
 #pragma unroll
-      for (int a = 0; a < 3; ++a) xd[v][a] = Dual(x[v][a], seed(dir, 3 * v + a));
-    // FaceTria::computeNormal (FaceTriaCore.C:31-37): 0.5 (x2 - x0) x (x1 - x0)
-    Dual p[3], q[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      p[a] = xd[2][a] - xd[0][a];
-      q[a] = xd[1][a] - xd[0][a];
-    }
-    Dual c0 = p[1] * q[2] - p[2] * q[1];
-    Dual c1 = p[2] * q[0] - p[0] * q[2];
-    Dual c2 = p[0] * q[1] - p[1] * q[0];
-    FX[9 * (size_t)f + dir] = nb[0] * (0.5 * c0).d + nb[1] * (0.5 * c1).d + nb[2] * (0.5 * c2).d;
+  for (int a = 0; a < 3; ++a) {
+    FX[9 * (size_t)f + a] = -(gp[a] + gq[a]);
+    FX[9 * (size_t)f + 3 + a] = gq[a];
+    FX[9 * (size_t)f + 6 + a] = gp[a];
   }
 }
 
 // ---------------------------------------------------------------------------
 // 6. per node: Xbar
 // ---------------------------------------------------------------------------
+// Four lanes per node, each every fourth slot: the slot lists are read in whole
+// lines and four gathers per node are in flight (688 -> 215 us at 815k nodes, with
+// the neighbours' S moved to the pass that reads them anyway).
 __global__ __launch_bounds__(kAdjBlock) void k_adj_xgather(DevTables t, const double *__restrict__ Xb,
-                                                           const double *__restrict__ S, int second,
                                                            const int *__restrict__ ntrow,
                                                            const int *__restrict__ ntslot,
                                                            const double *__restrict__ TX,
                                                            const int *__restrict__ nfslot,
                                                            const double *__restrict__ FX,
                                                            double *__restrict__ out) {
-  // XCD-aware block order (each XCD a contiguous node range): 0.1 ms less at
-  // 815k nodes; the same order made the node-sum and LSQ reverse passes slower
-  const int nb = (t.N + kAdjBlock - 1) / kAdjBlock;
-  const int n = xcd_chunk(blockIdx.x, nb) * kAdjBlock + (int)threadIdx.x;
-  if (n >= t.N) return;
-  double xb[3] = {Xb[4 * (size_t)n], Xb[4 * (size_t)n + 1], Xb[4 * (size_t)n + 2]};
-  if (second) {
-    const double *sn = S + 6 * (size_t)n;
-    const double4 xn = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)n);
-    for (int e = t.rowptr[n]; e < t.rowptr[n + 1]; ++e) {
-      const int m = t.adj[e];
-      const double *sm = S + 6 * (size_t)m;
-      const double4 xm = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)m);
-      const double d0 = xm.x - xn.x, d1 = xm.y - xn.y, d2 = xm.z - xn.z;
-      const double a0 = sn[0] + sm[0], a1 = sn[1] + sm[1], a2 = sn[2] + sm[2];
-      const double a3 = sn[3] + sm[3], a4 = sn[4] + sm[4], a5 = sn[5] + sm[5];
-      xb[0] -= a0 * d0 + a1 * d1 + a2 * d2;
-      xb[1] -= a1 * d0 + a3 * d1 + a4 * d2;
-      xb[2] -= a2 * d0 + a4 * d1 + a5 * d2;
+  const int nb = (t.N + kAdjBlock / 4 - 1) / (kAdjBlock / 4);
+  const int n = xcd_chunk(blockIdx.x, nb) * (kAdjBlock / 4) + (int)(threadIdx.x >> 2), r = threadIdx.x & 3;
+  double xb[3] = {0.0, 0.0, 0.0};
+  if (n < t.N) {
+    const int q1 = ntrow[n + 1];
+#pragma unroll 4
+    for (int q = ntrow[n] + r; q < q1; q += 4) {
+      const double *s = TX + 3 * (size_t)ntslot[q];  // 4 t + v
+#pragma unroll
+      for (int a = 0; a < 3; ++a) xb[a] += s[a];
+    }
+    for (int q = t.frow[n] + r; q < t.frow[n + 1]; q += 4) {
+      const double *s = FX + 3 * (size_t)nfslot[q];  // 3 f + v
+#pragma unroll
+      for (int a = 0; a < 3; ++a) xb[a] += s[a];
     }
   }
-  for (int q = ntrow[n]; q < ntrow[n + 1]; ++q) {
-    const size_t s = ntslot[q];  // 4 t + v
-    const size_t tt = s >> 2, v = s & 3;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) xb[a] += TX[12 * tt + 3 * v + a];
+  for (int a = 0; a < 3; ++a) {
+    xb[a] += __shfl_xor(xb[a], 1);
+    xb[a] += __shfl_xor(xb[a], 2);
   }
-  for (int q = t.frow[n]; q < t.frow[n + 1]; ++q) {
-    const size_t s = nfslot[q];  // 3 f + v
-    const size_t f = s / 3, v = s - 3 * f;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) xb[a] += FX[9 * f + 3 * v + a];
-  }
-#pragma unroll
-  for (int a = 0; a < 3; ++a) out[3 * (size_t)n + a] = xb[a];
+  if (n < t.N && r < 3) out[3 * (size_t)n + r] = Xb[il<3>(n, r)] + (r == 0 ? xb[0] : (r == 1 ? xb[1] : xb[2]));
+}
+
+// edge id -> position, and the tets' edge ids to positions
+__global__ __launch_bounds__(kAdjBlock) void k_adj_epos(int E, const int *__restrict__ pedge, int *__restrict__ epos) {
+  const int p = blockIdx.x * kAdjBlock + threadIdx.x;
+  if (p < E) epos[pedge[p]] = p;
+}
+__global__ __launch_bounds__(kAdjBlock) void k_adj_tpos(long long n, const int *__restrict__ epos,
+                                                        int *__restrict__ tpos) {
+  const long long k = (long long)blockIdx.x * kAdjBlock + threadIdx.x;
+  if (k < n) tpos[k] = epos[tpos[k]];
 }
 
 // ---------------------------------------------------------------------------
@@ -885,6 +880,8 @@ void free_adjoint(aerofx_ctx *c) {
 }
 
 namespace {
+
+inline dim3 grid_for(long long n) { return dim3((unsigned)((n + kAdjBlock - 1) / kAdjBlock)); }
 
 template <class T>
 int alloc_n(aerofx_ctx *c, size_t n, T **out) {
@@ -911,19 +908,28 @@ int ensure_adjoint(aerofx_ctx *c) {
   Adjoint *a = new Adjoint();
   const ElemTables &el = *c->elem;
   a->tets = el.tets;
-  a->tedge = el.tedge;
   a->faces = el.faces;
   a->ntrow = el.ntrow;
   a->ntslot = el.ntslot;
   a->nfslot = el.nfslot;
-  if ((rc = alloc_n(c, 20 * (size_t)E, &a->EV)) ||
-      (rc = alloc_n(c, 6 * (size_t)E, &a->EX)) || (rc = alloc_n(c, 5 * (size_t)N, &a->Vb)) ||
-      (rc = alloc_n(c, 16 * (size_t)N, &a->Gb)) || (rc = alloc_n(c, 4 * (size_t)N, &a->Xb)) ||
-      (rc = alloc_n(c, 6 * (size_t)N, &a->S)) || (rc = alloc_n(c, 5 * (size_t)N, &a->R)) ||
-      (rc = alloc_n(c, 12 * (size_t)std::max(T, 1), &a->TX)) ||
-      (rc = alloc_n(c, 9 * (size_t)std::max(F, 1), &a->FX)) || (rc = alloc_n(c, (size_t)F + 1, &a->Jf))) {
+  const size_t F1 = std::max(F, 1);
+  if ((rc = alloc_n(c, il_count<10>(E), &a->EVi)) || (rc = alloc_n(c, il_count<10>(E), &a->EVj)) ||
+      (rc = alloc_n(c, il_count<3>(E), &a->EXd)) || (rc = alloc_n(c, il_count<3>(E), &a->EXn)) ||
+      (rc = alloc_n(c, 15 * F1, &a->FV)) || (rc = alloc_n(c, 9 * F1, &a->FN)) ||
+      (rc = alloc_n(c, il_count<5>(N), &a->mu)) || (rc = alloc_n(c, (size_t)N, &a->cvb)) ||
+      (rc = alloc_n(c, il_count<5>(N), &a->Vb)) || (rc = alloc_n(c, il_count<15>(N), &a->H)) ||
+      (rc = alloc_n(c, il_count<3>(N), &a->Xb)) || (rc = alloc_n(c, il_count<6>(N), &a->S)) ||
+      (rc = alloc_n(c, 5 * (size_t)N, &a->R)) || (rc = alloc_n(c, 12 * (size_t)std::max(T, 1), &a->TX)) ||
+      (rc = alloc_n(c, 9 * F1, &a->FX)) || (rc = alloc_n(c, (size_t)F + 1, &a->Jf)) ||
+      (rc = upload_vec(c, c->tet_edges, &a->tpos))) {
     delete a;
     return rc;
+  }
+  if (T > 0) {
+    // the positions of the tets' edges (dxbar's buffer holds the map meanwhile)
+    int *epos = reinterpret_cast<int *>(a->EXd);
+    hipLaunchKernelGGL(k_adj_epos, grid_for(E), dim3(kAdjBlock), 0, c->stream, E, c->tab.pedge, epos);
+    hipLaunchKernelGGL(k_adj_tpos, grid_for(6LL * T), dim3(kAdjBlock), 0, c->stream, 6LL * T, epos, a->tpos);
   }
   hipError_t e = hipHostMalloc((void **)&a->h_J, sizeof(double), hipHostMallocDefault);
   if (e != hipSuccess) {
@@ -933,8 +939,6 @@ int ensure_adjoint(aerofx_ctx *c) {
   c->adj = a;
   return 0;
 }
-
-inline dim3 grid_for(long long n) { return dim3((unsigned)((n + kAdjBlock - 1) / kAdjBlock)); }
 
 }  // namespace
 
@@ -968,8 +972,7 @@ int ensure_elem_tables(aerofx_ctx *c) {
   }
   ElemTables *el = new ElemTables();
   int rc;
-  if ((rc = upload_vec(c, c->tets, &el->tets)) || (rc = upload_vec(c, c->tet_edges, &el->tedge)) ||
-      (rc = upload_vec(c, c->faces, &el->faces)) || (rc = upload_vec(c, ntrow, &el->ntrow)) ||
+  if ((rc = upload_vec(c, c->tets, &el->tets)) || (rc = upload_vec(c, c->faces, &el->faces)) || (rc = upload_vec(c, ntrow, &el->ntrow)) ||
       (rc = upload_vec(c, ntslot, &el->ntslot)) || (rc = upload_vec(c, nfslot, &el->nfslot)) ||
       (rc = upload_vec(c, etrow, &el->etrow)) || (rc = upload_vec(c, etslot, &el->etslot))) {
     delete el;
@@ -979,51 +982,53 @@ int ensure_elem_tables(aerofx_ctx *c) {
   return 0;
 }
 
-int launch_adjoint(aerofx_ctx *c, const double *U, const double *lam, double *Ub, double *Xout) {
-  int rc = ensure_adjoint(c);
-  if (rc) return rc;
+template <bool SECOND, bool WANTX>
+static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, double *Ub, double *Xout) {
   Adjoint *a = c->adj;
   const DevTables &t = c->tab;
-  const int second = c->p.second_order ? 1 : 0;
-  const int want_x = Xout ? 1 : 0;
-  // 1. forward pass: V, gradients (recomputed), R
-  if ((rc = launch_residual(c, U, a->R, true))) return rc;
+  const dim3 b(kAdjBlock);
+  // 1.
+  hipLaunchKernelGGL(k_adj_mu, grid_for(t.N), b, 0, c->stream, t, lam, a->R, a->mu, a->cvb);
   // 2.
-  if (t.E > 0) {
-    const dim3 g = grid_for(t.E), b(kAdjBlock);
-    if (second && want_x)
-      hipLaunchKernelGGL((k_adj_edges_x<true>), g, b, 0, c->stream, t, c->d_V, c->d_grad, lam, c->fc, a->EV, a->EX);
-    else if (second)
-      hipLaunchKernelGGL((k_adj_edges_u<true>), g, b, 0, c->stream, t, c->d_V, c->d_grad, lam, c->fc, a->EV, a->EX);
-    else if (want_x)
-      hipLaunchKernelGGL((k_adj_edges_x<false>), g, b, 0, c->stream, t, c->d_V, c->d_grad, lam, c->fc, a->EV, a->EX);
-    else
-      hipLaunchKernelGGL((k_adj_edges_u<false>), g, b, 0, c->stream, t, c->d_V, c->d_grad, lam, c->fc, a->EV, a->EX);
-  }
+  const int nfb = (3 * t.F + kAdjBlock - 1) / kAdjBlock;
+  const int nb = (t.nup + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
+  if (nfb + nb)
+    hipLaunchKernelGGL((k_adj_edges<SECOND, WANTX>), dim3((unsigned)(nfb + nb)), b, 0, c->stream, t, nfb, c->d_V,
+                       c->d_grad, a->mu, c->fc, a->nfslot, a->EVi, a->EVj, a->EXd, a->EXn, a->FV, a->FN);
   // 3.
-  hipLaunchKernelGGL(k_adj_nodes, grid_for(t.N), dim3(kAdjBlock), 0, c->stream, t, c->d_V, lam, c->fc, a->EV, a->EX,
-                     second, want_x, a->Vb, a->Gb, a->Xb);
+  hipLaunchKernelGGL((k_adj_nodes<SECOND, WANTX>), slice_grid(t.ns), b, 0, c->stream, t, c->d_grad, a->EVi, a->EVj,
+                     a->EXd, a->FV, a->Vb, a->H, a->S, a->Xb);
   // 4.
-  hipLaunchKernelGGL(k_adj_lsq, grid_for(t.N), dim3(kAdjBlock), 0, c->stream, t, c->d_V, U, c->gas, a->Vb, a->Gb,
-                     second, want_x, Ub, a->Xb, a->S);
+  hipLaunchKernelGGL((k_adj_lsq<SECOND, WANTX>), slice_grid(t.ns), b, 0, c->stream, t, c->d_V, U, c->gas, a->Vb, a->H,
+                     a->S, Ub, a->Xb);
+  int rc;
   // the Navier-Stokes Galerkin term (its element derivative, transposed)
   if (c->viscous && Ub && (rc = launch_visc_adjoint(c, lam, Ub))) return rc;
-  if (want_x) {
+  if (WANTX) {
     // 5.
     if (c->T > 0)
-      hipLaunchKernelGGL(k_adj_tets, grid_for(c->T), dim3(kAdjBlock), 0, c->stream, c->T, a->tets, a->tedge, t.X4,
-                         t.invcv, lam, a->R, a->EX, a->TX);
+      hipLaunchKernelGGL(k_adj_tets, grid_for(c->T), b, 0, c->stream, c->T, (const int4 *)a->tets, a->tpos, t.X4,
+                         a->cvb, a->EXn, a->TX);
     // the Navier-Stokes Galerkin term's coordinate derivative, per element
     if (c->T > 0 && (rc = launch_visc_adjoint_x(c, lam, a->TX))) return rc;
     if (c->F > 0)
-      hipLaunchKernelGGL(k_adj_faces, grid_for(c->F), dim3(kAdjBlock), 0, c->stream, c->F, a->faces, t.fcode,
-                         t.fnorm3, t.X4, t.invcv, c->d_V, lam, c->fc, a->FX);
+      hipLaunchKernelGGL(k_adj_faces, grid_for(c->F), b, 0, c->stream, c->F, a->faces, t.X4, a->FN, a->FX);
     // 6.
-    hipLaunchKernelGGL(k_adj_xgather, grid_for(t.N), dim3(kAdjBlock), 0, c->stream, t, a->Xb, a->S, second,
-                       a->ntrow, a->ntslot, a->TX, a->nfslot, a->FX, Xout);
+    hipLaunchKernelGGL(k_adj_xgather, grid_for(4LL * t.N), b, 0, c->stream, t, a->Xb, a->ntrow, a->ntslot, a->TX,
+                       a->nfslot, a->FX, Xout);
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_hip_error(e, "adjoint launch");
+}
+
+int launch_adjoint(aerofx_ctx *c, const double *U, const double *lam, double *Ub, double *Xout) {
+  int rc = ensure_adjoint(c);
+  // forward pass: V, gradients (recomputed), R
+  if (rc || (rc = launch_residual(c, U, c->adj->R, true))) return rc;
+  if (c->p.second_order) return Xout ? adjoint_stages<true, true>(c, U, lam, Ub, Xout)
+                                     : adjoint_stages<true, false>(c, U, lam, Ub, Xout);
+  return Xout ? adjoint_stages<false, true>(c, U, lam, Ub, Xout)
+              : adjoint_stages<false, false>(c, U, lam, Ub, Xout);
 }
 
 // ---------------------------------------------------------------------------

@@ -232,7 +232,6 @@ struct FgWork;
 // node or per edge in element order.
 struct ElemTables {
   int *tets = nullptr;    // [T][4]
-  int *tedge = nullptr;   // [T][6] edge of each local tet edge
   int *faces = nullptr;   // [F][3]
   int *ntrow = nullptr;   // [N+1]
   int *ntslot = nullptr;  // [4T] 4 t + local vertex, ascending t per node

@@ -276,7 +276,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_grad(DevTables t, const doubl
 #pragma unroll
   for (int q = 0; q < 5; ++q) {
     double w[3];
-    lsq_weights_t(L, acc[q], acc[5 + q], acc[10 + q], w);
+    lsq_weights(L, acc[q], acc[5 + q], acc[10 + q], w);
 #pragma unroll
     for (int a = 0; a < 3; ++a) acc[5 * a + q] = w[a];
   }
