@@ -384,32 +384,15 @@ __device__ __forceinline__ void adj_face_slot(const DevTables &t, const double *
   }
 }
 
-// A wave per (64 nodes, k-th upper edge), as the residual's flux pass on small
-// meshes; the first nfb blocks take the boundary-face slots.  Everything is read
-// and written by position, so what is not gathered is contiguous.  Two waves per
-// SIMD (256 registers): the gradients are read again after the flux for dxbar
-// rather than held across it (1013 -> 619 us at 815k nodes, 5.6M edges).
+// One edge (i, j) at position pos: e[0..5) = Vbar and e[5..10) = c of each end
+// (Gbar[5a+k] = c_k dx[a]: the sums form the products), dxbar, and nbar to its
+// place.
 template <bool SECOND, bool WANTX>
-__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_edges(
-    DevTables t, int nfb, const double *__restrict__ V, const double *__restrict__ grad,
-    const double *__restrict__ mu, FluxConsts fc, const int *__restrict__ nfslot, double *__restrict__ EVi,
-    double *__restrict__ EVj, double *__restrict__ EXd, double *__restrict__ EXn, double *__restrict__ FV,
-    double *__restrict__ FN) {
-  if ((int)blockIdx.x < nfb) {
-    const int q = blockIdx.x * kAdjBlock + threadIdx.x;
-    if (q < 3 * t.F) adj_face_slot<WANTX>(t, V, mu, fc, nfslot, q, FV, FN);
-    return;
-  }
-  const int nb = (t.nup + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
-  const int w = xcd_chunk(blockIdx.x - nfb, nb) * (kAdjBlock / kWave) + (int)(threadIdx.x / kWave);
-  if (w >= t.nup) return;
-  const int sl = t.upslice[w];
-  const int i = sl * kWave + lane_id();
-  const bool act = i < t.N && w - t.up.kptr[sl] < t.eup[min(i, t.N - 1) + 1] - t.eup[min(i, t.N - 1)];
-  const int pos = t.up.koff[w] + lanes_below(act);
-  if (!act) return;
-  const int j = t.up.idx[pos];
-  double VL[5], VR[5], dV[5], g[5], dx[3], di[5], dj[5];
+__device__ __forceinline__ void adj_edge(const DevTables &t, const double *__restrict__ V,
+                                         const double *__restrict__ grad, const double *__restrict__ mu,
+                                         const FluxConsts &fc, int i, int j, int pos, double *__restrict__ EXn,
+                                         double ei[10], double ej[10], double dxb[3]) {
+  double VL[5], VR[5], dV[5], g[5], di[5], dj[5];
   {
     double mj[5];
     load_il<5>(mu, i, g);
@@ -420,7 +403,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
   load_il<5>(V, i, VL);
   load_il<5>(V, j, VR);
   if (SECOND) {
-    double xi[3], gi[15], gj[15];
+    double xi[3], dx[3], gi[15], gj[15];
     load_il<3>(t.X3, i, xi);
     load_il<3>(t.X3, j, dx);
 #pragma unroll
@@ -444,16 +427,14 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
     roeflux7_vjp(fc.gas, nv, VL, VR, g, fb, fb + 5, fb + 10);
   if (WANTX) store_il<3>(EXn, pos, fb + 10);
   if (!SECOND) {
-    store_il<5>(EVi, pos, fb);
-    store_il<5>(EVj, pos, fb + 5);
-    if (WANTX) {
-      const double z[3] = {0.0, 0.0, 0.0};
-      store_il<3>(EXd, pos, z);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      ei[k] = fb[k];
+      ej[k] = fb[5 + k];
     }
     return;
   }
   const double beta = fc.beta, beta2 = 1.0 - 2.0 * beta;
-  double ei[10], ej[10];
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
     const double d = beta2 * dV[k];
@@ -466,16 +447,15 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
     const double dVb = B + B2 + beta2 * (A + A2);
     ei[k] = Lb - dVb;
     ej[k] = Rb + dVb;
-    // Gbar_i[5a+k] = c_i dx[a]: the node pass forms the products
     ei[5 + k] = 2.0 * beta * A;
     ej[5 + k] = 2.0 * beta * A2;
   }
-  store_il<10>(EVi, pos, ei);
-  store_il<10>(EVj, pos, ej);
   if (WANTX) {
     const double *g2 = grad;
     asm volatile("" : "+s"(g2));
-    double h[15], dxb[3] = {0.0, 0.0, 0.0};
+    double h[15];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) dxb[a] = 0.0;
     load_il<15>(g2, i, h);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
@@ -486,7 +466,94 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
     for (int a = 0; a < 3; ++a)
 #pragma unroll
       for (int k = 0; k < 5; ++k) dxb[a] += ej[5 + k] * h[5 * a + k];
-    store_il<3>(EXd, pos, dxb);
+  }
+}
+
+// A boundary-face slot in the first nfb blocks, then ROWS: a wave per 64 nodes,
+// lane r takes the upper edges of its node in turn and sums the node's own side
+// in LDS (23 values a lane; registers are short: two waves per SIMD need all
+// 256, and what the sums need of an edge is read again), so half of the records
+// are neither written nor read again; otherwise a wave per (64 nodes, k-th upper
+// edge).  Everything is read and written by
+// position, so what is not gathered is contiguous.  The gradients are read again
+// after the flux for dxbar rather than held across it (1013 -> 568 us at
+// 815k nodes, 5.6M edges, and 342 -> 260 us in the node pass by ROWS; bound by the
+// latency of the gathers at two waves per SIMD).
+template <bool SECOND, bool WANTX, bool ROWS>
+__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_edges(
+    DevTables t, int nfb, const double *__restrict__ V, const double *__restrict__ grad,
+    const double *__restrict__ mu, FluxConsts fc, const int *__restrict__ nfslot, double *__restrict__ EVi,
+    double *__restrict__ EVj, double *__restrict__ EXd, double *__restrict__ EXn, double *__restrict__ FV,
+    double *__restrict__ FN, double *__restrict__ Vb, double *__restrict__ Gb, double *__restrict__ Xb) {
+  constexpr int W = SECOND ? 10 : 5;
+  if ((int)blockIdx.x < nfb) {
+    const int q = blockIdx.x * kAdjBlock + threadIdx.x;
+    if (q < 3 * t.F) adj_face_slot<WANTX>(t, V, mu, fc, nfslot, q, FV, FN);
+    return;
+  }
+  const int nw = ROWS ? t.ns : t.nup;
+  const int nb = (nw + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
+  const int w = xcd_chunk(blockIdx.x - nfb, nb) * (kAdjBlock / kWave) + (int)(threadIdx.x / kWave);
+  if (w >= nw) return;
+  const int sl = ROWS ? w : t.upslice[w];
+  const int kb = t.up.kptr[sl], i = sl * kWave + lane_id();
+  const int deg = i < t.N ? t.eup[i + 1] - t.eup[i] : 0;
+  double ei[10], ej[10], dxb[3];
+  if (!ROWS) {
+    const bool act = w - kb < deg;
+    const int pos = t.up.koff[w] + lanes_below(act);
+    if (!act) return;
+    adj_edge<SECOND, WANTX>(t, V, grad, mu, fc, i, t.up.idx[pos], pos, EXn, ei, ej, dxb);
+    store_il<W>(EVi, pos, ei);
+    store_il<W>(EVj, pos, ej);
+    if (SECOND && WANTX) store_il<3>(EXd, pos, dxb);
+    return;
+  }
+  __shared__ double sums[kAdjBlock / kWave][23][kWave];
+  double(*sum)[kWave] = sums[threadIdx.x / kWave];
+  const int lane = lane_id(), ke = t.up.kptr[sl + 1];
+#pragma unroll
+  for (int q = 0; q < 23; ++q) sum[q][lane] = 0.0;
+  for (int k = kb; k < ke; ++k) {
+    const bool act = k - kb < deg;
+    const int pos = t.up.koff[k] + lanes_below(act);
+    if (!act) continue;
+    int own = i;
+    asm volatile("" : "+v"(own));  // the own side is read anew for each edge
+    const int j = t.up.idx[pos];
+    adj_edge<SECOND, WANTX>(t, V, grad, mu, fc, own, j, pos, EXn, ei, ej, dxb);
+    store_il<W>(EVj, pos, ej);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) sum[q][lane] += ei[q];
+    const double *X = t.X3;
+    asm volatile("" : "+s"(X));
+    double x[3], dx[3];
+    load_il<3>(X, own, x);
+    load_il<3>(X, j, dx);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) dx[a] -= x[a];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int q = 0; q < 5; ++q) sum[5 + 5 * a + q][lane] += ei[5 + q] * dx[a];
+    if (WANTX) {
+      store_il<3>(EXd, pos, dxb);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) sum[20 + a][lane] -= dxb[a];
+    }
+  }
+  if (i >= t.N) return;
+  double o[15];
+#pragma unroll
+  for (int q = 0; q < 5; ++q) o[q] = sum[q][lane];
+  store_il<5>(Vb, i, o);
+#pragma unroll
+  for (int q = 0; q < 15; ++q) o[q] = sum[5 + q][lane];
+  store_il<15>(Gb, i, o);
+  if (WANTX) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) o[a] = sum[20 + a][lane];
+    store_il<3>(Xb, i, o);
   }
 }
 
@@ -506,11 +573,12 @@ __device__ __forceinline__ void add_slot(const double *ev, const double dx[3], d
   }
 }
 
-// A wave per 64 nodes: the slots of the upper edges are contiguous, those of the
-// lower ones are gathered, and both ends' coordinates follow from the adjacency
+// A wave per 64 nodes: the slots of the upper edges are contiguous (ROWS: the
+// edge pass left their sums in Vb, H and Xb), those of the lower ones are
+// gathered, and both ends' coordinates follow from the adjacency
 // rows, whose first entries are the lower neighbours.  Bound by the slots' bytes
-// (624 -> 342 us at 815k nodes, 3.9 TB/s).
-template <bool SECOND, bool WANTX>
+// (624 -> 260 us at 815k nodes, 342 with both ends' slots; 3.5 TB/s).
+template <bool SECOND, bool WANTX, bool ROWS>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const double *__restrict__ grad,
                                                          const double *__restrict__ EVi,
                                                          const double *__restrict__ EVj,
@@ -527,6 +595,11 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
 #pragma unroll
   for (int q = 0; q < 15; ++q) gb[q] = 0.0;
   if (SECOND) load_il<3>(t.X3, min(n, t.N - 1), xn);
+  if (ROWS && live) {
+    load_il<5>(Vb, n, vb);
+    load_il<15>(H, n, gb);
+    if (WANTX) load_il<3>(Xb, n, xb);
+  }
   // edges (m, n), m < n: the j-side slots
   {
     const int deg = live ? t.lrow[n + 1] - t.lrow[n] : 0, all = live ? t.rowptr[n + 1] - t.rowptr[n] : 0;
@@ -552,7 +625,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
     }
   }
   // edges (n, m), n < m: the i-side slots
-  {
+  if (!ROWS) {
     const int deg = live ? t.eup[n + 1] - t.eup[n] : 0;
     const int kb = t.up.kptr[sl], ke = t.up.kptr[sl + 1];
     for (int k = 0; k < ke - kb; ++k) {
@@ -824,6 +897,8 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_faces(int F, const int *__res
 // ---------------------------------------------------------------------------
 // 6. per node: Xbar
 // ---------------------------------------------------------------------------
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte access at 8-byte alignment
+
 // Four lanes per node, each every fourth slot: the slot lists are read in whole
 // lines and four gathers per node are in flight (688 -> 215 us at 815k nodes, with
 // the neighbours' S moved to the pass that reads them anyway).
@@ -842,8 +917,10 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_xgather(DevTables t, const do
 #pragma unroll 4
     for (int q = ntrow[n] + r; q < q1; q += 4) {
       const double *s = TX + 3 * (size_t)ntslot[q];  // 4 t + v
-#pragma unroll
-      for (int a = 0; a < 3; ++a) xb[a] += s[a];
+      const double2u p = *reinterpret_cast<const double2u *>(s);
+      xb[0] += p.x;
+      xb[1] += p.y;
+      xb[2] += s[2];
     }
     for (int q = t.frow[n] + r; q < t.frow[n + 1]; q += 4) {
       const double *s = FX + 3 * (size_t)nfslot[q];  // 3 f + v
@@ -982,7 +1059,12 @@ int ensure_elem_tables(aerofx_ctx *c) {
   return 0;
 }
 
-template <bool SECOND, bool WANTX>
+// From this many 64-node slices the edge pass takes whole rows (at 562 slices
+// both products 157 us by entries, 169 by rows; 1839: 364, 352; 4292: 867, 822;
+// 14261: 2683, 2547): below that there are too few waves for the 1024 SIMDs.
+constexpr int kAdjRowSlices = 1536;
+
+template <bool SECOND, bool WANTX, bool ROWS>
 static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, double *Ub, double *Xout) {
   Adjoint *a = c->adj;
   const DevTables &t = c->tab;
@@ -991,12 +1073,13 @@ static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, dou
   hipLaunchKernelGGL(k_adj_mu, grid_for(t.N), b, 0, c->stream, t, lam, a->R, a->mu, a->cvb);
   // 2.
   const int nfb = (3 * t.F + kAdjBlock - 1) / kAdjBlock;
-  const int nb = (t.nup + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
+  const int nb = ((ROWS ? t.ns : t.nup) + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
   if (nfb + nb)
-    hipLaunchKernelGGL((k_adj_edges<SECOND, WANTX>), dim3((unsigned)(nfb + nb)), b, 0, c->stream, t, nfb, c->d_V,
-                       c->d_grad, a->mu, c->fc, a->nfslot, a->EVi, a->EVj, a->EXd, a->EXn, a->FV, a->FN);
+    hipLaunchKernelGGL((k_adj_edges<SECOND, WANTX, ROWS>), dim3((unsigned)(nfb + nb)), b, 0, c->stream, t, nfb, c->d_V,
+                       c->d_grad, a->mu, c->fc, a->nfslot, a->EVi, a->EVj, a->EXd, a->EXn, a->FV, a->FN,
+                       a->Vb, a->H, a->Xb);
   // 3.
-  hipLaunchKernelGGL((k_adj_nodes<SECOND, WANTX>), slice_grid(t.ns), b, 0, c->stream, t, c->d_grad, a->EVi, a->EVj,
+  hipLaunchKernelGGL((k_adj_nodes<SECOND, WANTX, ROWS>), slice_grid(t.ns), b, 0, c->stream, t, c->d_grad, a->EVi, a->EVj,
                      a->EXd, a->FV, a->Vb, a->H, a->S, a->Xb);
   // 4.
   hipLaunchKernelGGL((k_adj_lsq<SECOND, WANTX>), slice_grid(t.ns), b, 0, c->stream, t, c->d_V, U, c->gas, a->Vb, a->H,
@@ -1025,10 +1108,15 @@ int launch_adjoint(aerofx_ctx *c, const double *U, const double *lam, double *Ub
   int rc = ensure_adjoint(c);
   // forward pass: V, gradients (recomputed), R
   if (rc || (rc = launch_residual(c, U, c->adj->R, true))) return rc;
-  if (c->p.second_order) return Xout ? adjoint_stages<true, true>(c, U, lam, Ub, Xout)
-                                     : adjoint_stages<true, false>(c, U, lam, Ub, Xout);
-  return Xout ? adjoint_stages<false, true>(c, U, lam, Ub, Xout)
-              : adjoint_stages<false, false>(c, U, lam, Ub, Xout);
+  const bool rows = c->tab.ns >= kAdjRowSlices;
+  if (c->p.second_order && rows)
+    return Xout ? adjoint_stages<true, true, true>(c, U, lam, Ub, Xout)
+                : adjoint_stages<true, false, true>(c, U, lam, Ub, Xout);
+  if (c->p.second_order)
+    return Xout ? adjoint_stages<true, true, false>(c, U, lam, Ub, Xout)
+                : adjoint_stages<true, false, false>(c, U, lam, Ub, Xout);
+  return Xout ? adjoint_stages<false, true, false>(c, U, lam, Ub, Xout)
+              : adjoint_stages<false, false, false>(c, U, lam, Ub, Xout);
 }
 
 // ---------------------------------------------------------------------------
