@@ -61,46 +61,36 @@ struct GmresState {
 // ---------------------------------------------------------------------------
 // deterministic block reductions
 // ---------------------------------------------------------------------------
-// K = kMaxBasis values per lane: a transposing butterfly halves the values a
-// lane carries at each of the first five exchange steps (a lane keeps the
-// half selected by its lane bit and adds the partner's copy of that half),
-// so after steps 32..2 lane l holds one index, summed over the lanes that
-// share bit 0, and the step 1 exchange completes the wave sum: 32 shuffles
-// instead of 6 per value.  The fixed pattern keeps the sums deterministic.
-template <int HALF, int OFF>
-__device__ __forceinline__ void halve_step(double (&v)[kMaxBasis], int lane) {
-  const bool up = (lane & OFF) != 0;
+// K (a power of two) values per lane: a transposing butterfly halves the values
+// a lane carries at each exchange step (a lane keeps the half selected by its
+// lane bit and adds the partner's copy of that half) until one is left, and the
+// remaining steps complete the wave sum: K - 1 + log2(64 / K) shuffles instead
+// of 6 K.  The pattern of each value's sum is the plain butterfly's (32, 16, ..,
+// 1), whatever K.
+template <int K, int OFF>
+__device__ __forceinline__ void halve_steps(double *v, int lane) {
+  if constexpr (K > 1) {
+    const bool up = (lane & OFF) != 0;
 #pragma unroll
-  for (int i = 0; i < HALF; ++i) {
-    const double keep = up ? v[HALF + i] : v[i];
-    const double give = up ? v[i] : v[HALF + i];
-    v[i] = keep + __shfl_xor(give, OFF, kWave);
+    for (int i = 0; i < K / 2; ++i) {
+      const double keep = up ? v[K / 2 + i] : v[i];
+      const double give = up ? v[i] : v[K / 2 + i];
+      v[i] = keep + __shfl_xor(give, OFF, kWave);
+    }
+    halve_steps<K / 2, OFF / 2>(v, lane);
+  } else {
+#pragma unroll
+    for (int off = OFF; off > 0; off >>= 1) v[0] += __shfl_xor(v[0], off, kWave);
   }
 }
 
-__device__ __forceinline__ void block_reduce_store_k(double (&v)[kMaxBasis], int nk, int nparts,
-                                                     double *__restrict__ partial) {
-  static_assert(kMaxBasis == 32 && kWave == 64, "the butterfly below is written for 32 values, 64 lanes");
-  __shared__ double sh[kBlock / kWave][kMaxBasis];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  halve_step<16, 32>(v, lane);
-  halve_step<8, 16>(v, lane);
-  halve_step<4, 8>(v, lane);
-  halve_step<2, 4>(v, lane);
-  halve_step<1, 2>(v, lane);
-  const double tot = v[0] + __shfl_xor(v[0], 1, kWave);
-  // index held by this lane: bits 5..1 of the lane select halves 16, 8, 4, 2, 1
-  const int idx = ((lane >> 5) & 1) * 16 + ((lane >> 4) & 1) * 8 + ((lane >> 3) & 1) * 4 + ((lane >> 2) & 1) * 2 +
-                  ((lane >> 1) & 1);
-  if ((lane & 1) == 0) sh[wave][idx] = tot;
-  __syncthreads();
-  if ((int)threadIdx.x < nk) {
-    double s = 0.0;
-#pragma unroll
-    for (int w = 0; w < kBlock / kWave; ++w) s += sh[w][threadIdx.x];
-    partial[(size_t)threadIdx.x * kDotBlocks + blockIdx.x] = s;
-  }
-  (void)nparts;
+// the wave's sums of v[0..K) to out[0..K)
+template <int K>
+__device__ __forceinline__ void wave_sums(double (&v)[K], double *out) {
+  const int lane = threadIdx.x % kWave;
+  halve_steps<K, kWave / 2>(v, lane);
+  // the lane's top log2(K) bits are its value's index
+  if (lane % (kWave / K) == 0) out[lane / (kWave / K)] = v[0];
 }
 
 // sum over lanes 0..31 (the values of lanes 32..63 are summed separately),
@@ -127,53 +117,38 @@ __device__ __forceinline__ void block_reduce_store_1(double v, double *__restric
 }
 
 // Givens update of Hessenberg column jc (KspSolver.C:404-447, 919-962):
-// rotations, residual estimate, stop flag.  The column (jc + 2 entries, the
-// last one the subdiagonal) is in LDS; the block's threads stage the stored
-// rotations and g[jc] in LDS in one parallel round, then thread 0 runs the
-// rotation recurrence from LDS with unconditional loads.  Every thread of the
-// block must call it (it synchronises).
+// rotations, residual estimate, stop flag, by one thread.  The column (jc + 2
+// entries, the last one the subdiagonal) and what the update reads of the state
+// are in LDS.
 struct GivensStage {
   double rot[2 * kMaxBasis];
-  double gj;
-  int done;
+  double gj, target;
+  int iter, maxits, done;
 };
 
-// Loads what the update reads into the stage (the caller may do this early,
-// overlapping it with its own loads, and must synchronise before the update).
+// Loads what the update reads (early, with the caller's own loads; the caller
+// synchronises before the update).
 __device__ __forceinline__ void givens_stage(const GmresState *s, int jc, GivensStage &g) {
   const int t = threadIdx.x;
   if (t < 2 * kMaxBasis) g.rot[t] = s->cs[t];
-  if (t == 0) g.gj = s->g[jc];
+  if (t == 0) {
+    g.gj = s->g[jc];
+    g.target = s->target;
+    g.iter = s->iter;
+    g.maxits = s->maxits;
+    g.done = 0;
+  }
 }
 
-__device__ void givens_col(GmresState *s, int jc, const double *col, GivensStage &g, bool staged = false) {
-  const int t = threadIdx.x;
-  if (!staged) givens_stage(s, jc, g);
-  if (t == 0) g.done = s->done;
-  __syncthreads();
-  if (t != 0 || g.done) return;
+__device__ __forceinline__ void givens_col(GmresState *s, int jc, const double *col, GivensStage &g) {
   const int M = kMaxBasis;
-  double h[kMaxBasis + 1];
-#pragma unroll
-  for (int i = 0; i <= kMaxBasis; ++i) h[i] = i <= jc + 1 ? col[i] : 0.0;
-  const double hn = col[jc + 1];
-#pragma unroll
-  for (int i = 0; i < kMaxBasis - 1; ++i) {
-    const double sn = g.rot[2 * i], cs = g.rot[2 * i + 1];
-    const double hj = cs * h[i] + sn * h[i + 1];
-    const double hjp1 = -sn * h[i] + cs * h[i + 1];
-    if (i < jc) {
-      h[i] = hj;
-      h[i + 1] = hjp1;
-    }
+  double hjj = col[0];
+  const double hj1 = col[jc + 1];
+  for (int i = 0; i < jc; ++i) {
+    const double sn = g.rot[2 * i], cs = g.rot[2 * i + 1], hn = col[i + 1];
+    s->H[i * M + jc] = cs * hjj + sn * hn;
+    hjj = -sn * hjj + cs * hn;
   }
-  double hjj = 0.0, hj1 = 0.0;
-#pragma unroll
-  for (int i = 0; i < kMaxBasis; ++i)
-    if (i == jc) {
-      hjj = h[i];
-      hj1 = h[i + 1];
-    }
   double sn, cs;
   if (hjj * hjj == 0.0) {
     cs = 0.0;
@@ -185,23 +160,20 @@ __device__ void givens_col(GmresState *s, int jc, const double *col, GivensStage
   }
   s->cs[2 * jc + 1] = cs;
   s->cs[2 * jc] = sn;
-#pragma unroll
-  for (int i = 0; i < kMaxBasis; ++i)
-    if (i < jc) s->H[i * M + jc] = h[i];
   s->H[jc * M + jc] = cs * hjj + sn * hj1;
   s->H[(jc + 1) * M + jc] = 0.0;
   const double gj = g.gj;
   const double gj1 = -sn * gj;
   s->g[jc + 1] = gj1;
   s->g[jc] = cs * gj;
-  s->iter += 1;
+  s->iter = g.iter + 1;
   s->jlast = jc;
-  if (hn == 0.0) {
-    s->done = 1;
-    return;
+  bool stop = true;
+  if (hj1 != 0.0) {
+    s->l2res = fabs(gj1);
+    stop = fabs(gj1) <= g.target || g.iter + 1 >= g.maxits;
   }
-  s->l2res = fabs(gj1);
-  if (s->l2res <= s->target || s->iter >= s->maxits) s->done = 1;
+  if (stop) s->done = g.done = 1;
 }
 
 // Row pairs of a block's slice: the grid has nparts blocks (fixed by n, at
@@ -243,19 +215,22 @@ __global__ __launch_bounds__(kBlock) void k_sumsq(size_t n, const double *__rest
 //   a = V_{j-1}^T u_j,  b = V_{j-1}^T w,  alpha = u.u,  beta = u.w,  gamma = w.w
 // (partial rows 0.., 32.., 64, 65, 66).  The final sweep of a cycle (FINAL)
 // needs a and alpha only.
-template <bool FINAL>
+// K: the basis size rounded up to 8, 16 or 32, so that a short basis pays for
+// its own sums only (over a cycle of 30 at 105k nodes 20.5 us a sweep with one
+// instance, 9, 15 and 25 with three; at 1900 nodes 7.4, and 3.6, 4.7 and 7.2).
+template <bool FINAL, int K>
 __global__ __launch_bounds__(kBlock) void k_dots2(size_t n, const double *__restrict__ V, size_t ldv, int j,
                                                   const double *__restrict__ w, double *__restrict__ partial,
                                                   const int *__restrict__ done) {
   if (*done) return;
   const RowPairs rp(n);
   const double *u = V + (size_t)j * ldv;
-  double aa[kMaxBasis], bb[kMaxBasis], al = 0.0, be = 0.0, ga = 0.0;
+  double aa[K], bb[K], al = 0.0, be = 0.0, ga = 0.0;
 #pragma unroll
-  for (int k = 0; k < kMaxBasis; ++k) aa[k] = bb[k] = 0.0;
+  for (int k = 0; k < K; ++k) aa[k] = bb[k] = 0.0;
   auto row = [&](double ui, double wi, const double *vk) {
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k) {
+    for (int k = 0; k < K; ++k) {
       aa[k] += vk[k] * ui;
       if (!FINAL) bb[k] += vk[k] * wi;
     }
@@ -267,50 +242,58 @@ __global__ __launch_bounds__(kBlock) void k_dots2(size_t n, const double *__rest
   };
   // software-pipelined: the next row pair's loads are in flight while the
   // current pair is added (one wave per SIMD: nothing else hides latency)
-  auto load = [&](size_t i, double2 (&v)[kMaxBasis], double2 &u2, double2 &w2) {
+  auto load = [&](size_t i, double2 (&v)[K], double2 &u2, double2 &w2) {
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k)
+    for (int k = 0; k < K; ++k)
       v[k] = k < j ? *reinterpret_cast<const double2 *>(V + (size_t)k * ldv + i) : make_double2(0.0, 0.0);
     u2 = *reinterpret_cast<const double2 *>(u + i);
     w2 = FINAL ? make_double2(0.0, 0.0) : *reinterpret_cast<const double2 *>(w + i);
   };
   size_t i = rp.b0 + 2 * threadIdx.x;
-  double2 v[kMaxBasis], u2, w2;
+  double2 v[K], u2, w2;
   if (i < rp.even_end) load(i, v, u2, w2);
   while (i < rp.even_end) {
     const size_t inext = i + 2 * kBlock;
-    double2 vn[kMaxBasis], un2, wn2;
+    double2 vn[K], un2, wn2;
     if (inext < rp.even_end) load(inext, vn, un2, wn2);
-    double vk[kMaxBasis];
+    double vk[K];
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k) vk[k] = v[k].x;
+    for (int k = 0; k < K; ++k) vk[k] = v[k].x;
     row(u2.x, w2.x, vk);
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k) vk[k] = v[k].y;
+    for (int k = 0; k < K; ++k) vk[k] = v[k].y;
     row(u2.y, w2.y, vk);
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k) v[k] = vn[k];
+    for (int k = 0; k < K; ++k) v[k] = vn[k];
     u2 = un2;
     w2 = wn2;
     i = inext;
   }
   if (rp.has_tail()) {
     const size_t i = rp.b1 - 1;
-    double vk[kMaxBasis];
+    double vk[K];
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k) vk[k] = k < j ? V[(size_t)k * ldv + i] : 0.0;
+    for (int k = 0; k < K; ++k) vk[k] = k < j ? V[(size_t)k * ldv + i] : 0.0;
     row(u[i], FINAL ? 0.0 : w[i], vk);
   }
-  block_reduce_store_k(aa, j, gridDim.x, partial);
-  __syncthreads();  // the reduction's LDS is reused
-  if (!FINAL) {
-    block_reduce_store_k(bb, j, gridDim.x, partial + (size_t)kMaxBasis * kDotBlocks);
-    __syncthreads();
-  }
-  double sc[kMaxBasis];
+  // per wave, then over the waves: rows a, b and (alpha, beta, gamma)
+  __shared__ double sh[kBlock / kWave][2 * K + 4];
+  double *out = sh[threadIdx.x / kWave];
+  double sc[4] = {al, be, ga, 0.0};
+  wave_sums<K>(aa, out);
+  if (!FINAL) wave_sums<K>(bb, out + K);
+  wave_sums<4>(sc, out + 2 * K);
+  __syncthreads();
+  const int q = threadIdx.x;
+  if (q < 2 * K + 3) {
+    const int row = q < K ? q : (q < 2 * K ? kMaxBasis + q - K : 2 * kMaxBasis + q - 2 * K);
+    if (q < j || (!FINAL && q >= K && q < K + j) || q >= 2 * K) {
+      double t = 0.0;
 #pragma unroll
-  for (int k = 0; k < kMaxBasis; ++k) sc[k] = k == 0 ? al : k == 1 ? be : k == 2 ? ga : 0.0;
-  block_reduce_store_k(sc, 3, gridDim.x, partial + (size_t)2 * kMaxBasis * kDotBlocks);
+      for (int w = 0; w < kBlock / kWave; ++w) t += sh[w][q];
+      partial[(size_t)row * kDotBlocks + blockIdx.x] = t;
+    }
+  }
 }
 
 // out[k] = sum_b partial[k][b] in a fixed tree, one block per k
@@ -345,20 +328,26 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(const double *__rest
 //     ||A' v_j||^2 the Krylov space is exhausted: column j is final as it
 //     is, and the cycle stops.
 // coef (a, d, 1/tau, 1/(tau rho')) feeds k_dcgs_update.
+// Nothing but a serial chain of latencies: all loads go out at once, the
+// rotations and the coefficients run in two waves side by side, and the stop
+// flag stays in LDS (8.9 -> 4.7 us a step at 1900 nodes, 11.5 -> 6.2 at 105k).
 constexpr int kReduceThreads = 1024;
 template <bool FINAL>
 __global__ __launch_bounds__(kReduceThreads) void k_dcgs_reduce(const double *__restrict__ partial, int nparts,
                                                                 GmresState *st, int j) {
-  if (st->done) return;
-  __shared__ double sa[kMaxBasis], sb[kMaxBasis], ssc[3], col[kMaxBasis + 2], sg[kMaxBasis + 1];
+  __shared__ double sa[kMaxBasis], sb[kMaxBasis], ssc[3], col[kMaxBasis + 2], hcol[kMaxBasis + 2];
   __shared__ double sH[(kMaxBasis + 1) * kMaxBasis];  // Hbar_{j-1}, rows 0..j
   __shared__ double stau;
   __shared__ int sbreak;
+  // everything the step reads is requested at once, the stop flag included
+  const int done = st->done;
+  const double rho1 = st->rho;
   __shared__ GivensStage gstage;
   const int t = threadIdx.x, grp = t / 16, sub = t % 16;
-  // the Givens inputs of column j-1, loaded with the partials
-  if (j >= 1) givens_stage(st, j - 1, gstage);
-  // columns 0..j-2 of the Hessenberg matrix (final), loaded with the partials
+  const double cp = t < j ? st->cpart[t] : 0.0;
+  // the Givens inputs of column j-1
+  givens_stage(st, j >= 1 ? j - 1 : 0, gstage);
+  // columns 0..j-2 of the Hessenberg matrix (final)
   if (!FINAL)
     for (int e = t; e < (j + 1) * kMaxBasis; e += kReduceThreads)
       if (e % kMaxBasis + 1 < j) sH[e] = st->Hh[e];
@@ -387,6 +376,7 @@ __global__ __launch_bounds__(kReduceThreads) void k_dcgs_reduce(const double *__
       else ssc[grp - (FINAL ? j : 2 * j)] = s;
     }
   }
+  if (done) return;
   __syncthreads();
   if (t < 32) {
     // a.a over one half-wave, fixed butterfly
@@ -400,11 +390,10 @@ __global__ __launch_bounds__(kReduceThreads) void k_dcgs_reduce(const double *__
   const double tau = stau;
   if (j >= 1) {
     // column j-1, complete now
-    const double rho = st->rho;
     if (t <= kMaxBasis + 1) {
       double v = 0.0;
-      if (t < j) v = st->cpart[t] + rho * sa[t];
-      if (t == j) v = rho * tau;
+      if (t < j) v = cp + rho1 * sa[t];
+      if (t == j) v = rho1 * tau;
       col[t] = v;
       if (t <= j) {
         st->Hh[t * kMaxBasis + (j - 1)] = v;
@@ -412,33 +401,30 @@ __global__ __launch_bounds__(kReduceThreads) void k_dcgs_reduce(const double *__
       }
     }
     __syncthreads();
-    givens_col(st, j - 1, col, gstage, true);
-    __syncthreads();
-    if (FINAL || st->done) return;
+    // the rotations of column j-1, by the first wave ...
+    if (t == 0) givens_col(st, j - 1, col, gstage);
   } else if (t == 0) {
-    st->g[0] *= tau;
+    st->g[0] = gstage.gj * tau;
   }
   if (FINAL) return;
-  // g = Hbar_{j-1} a (rows 0..j), in ascending column order
-  if (t <= j) {
-    double gt = 0.0;
-    for (int cc = 0; cc < j; ++cc) gt += sH[t * kMaxBasis + cc] * sa[cc];
-    sg[t] = gt;
-  }
-  __syncthreads();
-  if (t < 32) {
-    // one lane per basis index k <= j; sums over the half-wave, fixed butterfly
-    const int k = t;
+  // ... while the second takes the coefficients of the next vector (not read if
+  // the rotations stop the cycle), one lane per basis index k <= j; sums over
+  // the half-wave, fixed butterfly
+  if (t >= kWave && t < kWave + 32) {
+    const int k = t - kWave;
+    // g = Hbar_{j-1} a (rows 0..j), in ascending column order
+    double gk = 0.0;
+    if (k <= j)
+      for (int cc = 0; cc < j; ++cc) gk += sH[k * kMaxBasis + cc] * sa[cc];
     const double ab = wsum32(k < j ? sa[k] * sb[k] : 0.0);
     const double inv_tau = 1.0 / tau;
-    double p = 0.0, h = 0.0, gk = 0.0;
+    double p = 0.0, h = 0.0;
     if (k <= j) {
-      gk = sg[k];
       p = k < j ? sb[k] : (ssc[1] - ab) * inv_tau;
       h = (p - gk) * inv_tau;
       st->cpart[k] = h;
       st->coef[kCoefD + k] = gk + tau * h;
-      col[k] = h;
+      hcol[k] = h;
       if (k < j) st->coef[k] = sa[k];
     }
     const double gp = wsum32(gk * p), gg = wsum32(gk * gk), hh = wsum32(h * h);
@@ -457,13 +443,16 @@ __global__ __launch_bounds__(kReduceThreads) void k_dcgs_reduce(const double *__
     }
   }
   __syncthreads();
-  if (sbreak && t <= j + 1) {
-    // exhausted Krylov space: column j is h with a zero subdiagonal
-    if (t == j + 1) col[t] = 0.0;
-    st->Hh[t * kMaxBasis + j] = t <= j ? col[t] : 0.0;
+  if (!sbreak || gstage.done) return;
+  // exhausted Krylov space: column j is h with a zero subdiagonal, which sets the
+  // stop flag
+  if (t <= j + 1) {
+    if (t == j + 1) hcol[t] = 0.0;
+    st->Hh[t * kMaxBasis + j] = t <= j ? hcol[t] : 0.0;
   }
+  givens_stage(st, j, gstage);
   __syncthreads();
-  if (sbreak) givens_col(st, j, col, gstage);  // sets the stop flag (zero subdiagonal)
+  if (t == 0) givens_col(st, j, hcol, gstage);
 }
 
 // y = a x + b y, a possibly scaled by a device scalar (*as).  With b = 0, y
@@ -483,14 +472,22 @@ __global__ __launch_bounds__(kBlock) void k_fill(size_t n, double v, double *__r
   if (i < n) y[i] = v;
 }
 
-// w = sum_{k <= jlast} y_k V_k
+// w = sum_{k <= jlast} y_k V_k, eight rows' loads in flight (26 -> 21 us at
+// 105k nodes, 9.4 -> 5.1 at 1900; one at a time before)
 __global__ __launch_bounds__(kBlock) void k_combine(size_t n, double *__restrict__ w, const double *__restrict__ V,
                                                     size_t ldv, const GmresState *__restrict__ s) {
   const size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x;
   if (i >= n) return;
   const int nk = s->jlast + 1;
   double acc = 0.0;
-  for (int k = 0; k < nk; ++k) acc += s->y[k] * V[(size_t)k * ldv + i];
+  for (int k0 = 0; k0 < nk; k0 += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = k0 + u < nk ? V[(size_t)(k0 + u) * ldv + i] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k0 + u < nk) acc += s->y[k0 + u] * v[u];
+  }
   w[i] = acc;
 }
 
@@ -510,25 +507,27 @@ __global__ void k_gmres_start(GmresState *s, const double *__restrict__ nrm2, in
   s->jlast = -1;
 }
 
-// back-substitution (KspSolver.C:968-982)
-// (the triangle and g are staged in LDS by the block first, then one lane
-// runs the recurrence in the reference's order)
-__global__ __launch_bounds__(256) void k_gmres_backsolve(GmresState *s) {
+// back-substitution (KspSolver.C:968-982) by one wave: lane i holds row i and
+// takes off each y_k as it is found, in the reference's order for its row
+// (26 -> 6 us; one thread over the triangle in LDS before)
+__global__ __launch_bounds__(kWave) void k_gmres_backsolve(GmresState *s) {
   constexpr int M = kMaxBasis;
-  __shared__ double sH[M * M], sg[M], sy[M];
+  const int i = threadIdx.x % M;
   const int j = s->jlast;
-  for (int e = threadIdx.x; e < M * M; e += blockDim.x) sH[e] = s->H[e];
-  if (threadIdx.x < M) sg[threadIdx.x] = s->g[threadIdx.x];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = j; i >= 0; --i) {
-      double yi = sg[i];
-      for (int k = j; k >= i + 1; --k) yi -= sH[i * M + k] * sy[k];
-      sy[i] = yi / sH[i * M + i];
-    }
+  double row[M], x = s->g[i], diag = 1.0;
+#pragma unroll
+  for (int k = 0; k < M; ++k) row[k] = s->H[i * M + k];
+#pragma unroll
+  for (int k = 0; k < M; ++k)
+    if (k == i) diag = row[k];
+#pragma unroll
+  for (int k = M - 1; k >= 0; --k) {
+    if (k > j) continue;
+    const double yk = __shfl(x / diag, k, M);
+    if (i == k) x = yk;
+    if (i < k) x -= row[k] * yk;
   }
-  __syncthreads();
-  if ((int)threadIdx.x <= j) s->y[threadIdx.x] = sy[threadIdx.x];
+  if ((int)threadIdx.x <= j) s->y[threadIdx.x] = x;
 }
 
 // count nodes whose density or pressure is not positive
@@ -876,8 +875,8 @@ static int enqueue_arnoldi(aerofx_ctx *c, int m, bool trans) {
     }
     {
       ProfScope ps(c, AEROFX_TIMER_GRAM_SCHMIDT);
-      hipLaunchKernelGGL((k_dots2<false>), dim3(k->nparts), dim3(kBlock), 0, c->stream, n, k->V, k->ldv, j, k->w,
-                         k->partial, done);
+      const auto dots = j <= 8 ? k_dots2<false, 8> : (j <= 16 ? k_dots2<false, 16> : k_dots2<false, kMaxBasis>);
+      hipLaunchKernelGGL(dots, dim3(k->nparts), dim3(kBlock), 0, c->stream, n, k->V, k->ldv, j, k->w, k->partial, done);
       hipLaunchKernelGGL((k_dcgs_reduce<false>), dim3(1), dim3(kReduceThreads), 0, c->stream, k->partial,
                          k->nparts, k->st, j);
     }
@@ -893,8 +892,9 @@ static int enqueue_arnoldi(aerofx_ctx *c, int m, bool trans) {
   }
   {
     ProfScope ps(c, AEROFX_TIMER_GRAM_SCHMIDT);
-    hipLaunchKernelGGL((k_dots2<true>), dim3(k->nparts), dim3(kBlock), 0, c->stream, n, k->V, k->ldv, m, nullptr,
-                       k->partial, done);
+    const auto dots = m <= 8 ? k_dots2<true, 8> : (m <= 16 ? k_dots2<true, 16> : k_dots2<true, kMaxBasis>);
+    hipLaunchKernelGGL(dots, dim3(k->nparts), dim3(kBlock), 0, c->stream, n, k->V, k->ldv, m, nullptr, k->partial,
+                       done);
     hipLaunchKernelGGL((k_dcgs_reduce<true>), dim3(1), dim3(kReduceThreads), 0, c->stream, k->partial, k->nparts,
                        k->st, m);
   }
@@ -994,7 +994,7 @@ static int gmres(aerofx_ctx *c, const double *b, double *x, int m, double eps, i
     if ((rc = fetch_state(c))) return rc;
     const GmresState &hs = *k->h_st;
     if (hs.jlast >= 0) {
-      hipLaunchKernelGGL(k_gmres_backsolve, dim3(1), dim3(256), 0, c->stream, k->st);
+      hipLaunchKernelGGL(k_gmres_backsolve, dim3(1), dim3(kWave), 0, c->stream, k->st);
       hipLaunchKernelGGL(k_combine, grid_for(n), dim3(kBlock), 0, c->stream, n, k->w, k->V, k->ldv, k->st);
       if ((rc = launch_prec_apply(c, k->w, k->r, trans))) return rc;
       hipLaunchKernelGGL(k_axpby, grid_for(n), dim3(kBlock), 0, c->stream, n, 1.0, nullptr, k->r, 1.0, x, nullptr);
