@@ -790,8 +790,10 @@ __device__ __forceinline__ void add_cross(double s, const double x[3], const dou
 // The tet's share of each quantity is a product of coordinate differences, so
 // its reverse is a few cross products: with p = c - d, r = (a - c) + (b - d) and
 // w the weight of an edge, d(w . p x r) = dp . r x w + dr . w x p.  Bound by the
-// gathers of six nbar and the stores (659 -> 282 us for 4.7M tets; 12 passes in
-// dual numbers before).
+// gathers of six nbar (659 -> 215 us for 4.7M tets; 12 passes in dual numbers
+// before, and 282 us with each lane storing its own 96 bytes: the vector cache
+// takes a store of 64 scattered pieces one piece at a time, so they go out
+// through LDS as whole lines).
 __global__ __launch_bounds__(kAdjBlock) void k_adj_tets(int T, const int4 *__restrict__ tets,
                                                         const int *__restrict__ tpos,
                                                         const double *__restrict__ X4,
@@ -799,8 +801,9 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_tets(int T, const int4 *__res
                                                         const double *__restrict__ EXn, double *__restrict__ TX) {
 #pragma clang fp contract(on)
   const int nblk = (T + kAdjBlock - 1) / kAdjBlock;
-  const int t = xcd_chunk(blockIdx.x, nblk) * kAdjBlock + (int)threadIdx.x;
-  if (t >= T) return;
+  __shared__ double2 out[6 * kAdjBlock];
+  const int t0 = xcd_chunk(blockIdx.x, nblk) * kAdjBlock, t1 = t0 + (int)threadIdx.x;
+  const int t = min(t1, T - 1);  // the lanes past the last tet repeat it and store nothing
   const int4 d4 = tets[t];
   const int nd[4] = {d4.x, d4.y, d4.z, d4.w};
   int ps[6];
@@ -855,12 +858,20 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_tets(int T, const int4 *__res
       z[d][k] -= gp[k] + gr[k];
     }
   }
-  double2 *o = reinterpret_cast<double2 *>(TX + 12 * (size_t)t);
+  double2 *o = out + 6 * threadIdx.x;
 #pragma unroll
   for (int v = 0; v < 4; v += 2) {
     o[3 * v / 2] = make_double2(z[v][0], z[v][1]);
     o[3 * v / 2 + 1] = make_double2(z[v][2], z[v + 1][0]);
     o[3 * v / 2 + 2] = make_double2(z[v + 1][1], z[v + 1][2]);
+  }
+  __syncthreads();
+  double2 *g = reinterpret_cast<double2 *>(TX) + 6 * (size_t)t0;
+  const int n = 6 * min(kAdjBlock, T - t0);
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    const int q = (int)threadIdx.x + r * kAdjBlock;
+    if (q < n) g[q] = out[q];
   }
 }
 
