@@ -91,7 +91,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_edge_normals(DevTables t, con
                                                                 const double *__restrict__ dX,
                                                                 double *__restrict__ dn) {
 #pragma clang fp contract(on)
-  const int pos = blockIdx.x * kTanBlock + threadIdx.x;
+  const int pos = xcd_chunk(blockIdx.x, (t.E + kTanBlock - 1) / kTanBlock) * kTanBlock + (int)threadIdx.x;
   if (pos >= t.E) return;
   const int l = t.pedge[pos];
   const int2 ij = t.eij[l];

@@ -99,13 +99,22 @@ __global__ void k_slot_positions(int n, const int *__restrict__ ntslot, int *__r
   if (s < n) pos[ntslot[s]] = s;
 }
 
+// the value of the other lane of a pair (2 i, 2 i + 1)
+__device__ __forceinline__ int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true); }
+__device__ __forceinline__ double pair_swap(double v) {
+  return __hiloint2double(pair_swap(__double2hiint(v)), pair_swap(__double2loint(v)));
+}
+
+// Bound by the vector cache, which takes the scattered 32-B pieces one quarter
+// wave's line at a time: the two lanes of a pair write both halves of one tet's
+// piece together, then of the other's (VISCFIG).
 __global__ __launch_bounds__(kBlock) void k_visc_elements(int T, const int4 *__restrict__ tets,
                                                           const double *__restrict__ X4, const double *__restrict__ V,
                                                           NsConsts ns, const int4 *__restrict__ pos,
                                                           double *__restrict__ C, const int *__restrict__ done) {
   if (done && *done) return;
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= T) return;
+  const int ti = xcd_chunk(blockIdx.x, (T + kBlock - 1) / kBlock) * kBlock + (int)threadIdx.x;
+  const int t = min(ti, T - 1);  // a lane past the last tet only helps its pair
   double x[4][3], v[4][5], g[4][3];
   load_element(tets, X4, V, t, x, v);
   const double vol = p1_gradients(x, g);
@@ -113,12 +122,19 @@ __global__ __launch_bounds__(kBlock) void k_visc_elements(int T, const int4 *__r
   ns_element(ns, g, v, e);
   const int4 p4 = pos[t];
   const int pj[4] = {p4.x, p4.y, p4.z, p4.w};
+  const bool odd = threadIdx.x & 1;
+  const bool first = (ti & ~1) < T, second = (ti | 1) < T;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     double c[5];
     ns_node_residual(e, g[j], vol, c);
     // the density row is zero: four values, one 32-B piece
-    *reinterpret_cast<double4 *>(C + 4 * (size_t)pj[j]) = make_double4(c[1], c[2], c[3], c[4]);
+    const double o0 = pair_swap(odd ? c[1] : c[3]), o1 = pair_swap(odd ? c[2] : c[4]);
+    const int po = pair_swap(pj[j]);
+    double *a = C + 4 * (size_t)(odd ? po : pj[j]) + (odd ? 2 : 0);
+    double *b = C + 4 * (size_t)(odd ? pj[j] : po) + (odd ? 2 : 0);
+    if (first) *reinterpret_cast<double2 *>(a) = odd ? make_double2(o0, o1) : make_double2(c[1], c[2]);
+    if (second) *reinterpret_cast<double2 *>(b) = odd ? make_double2(c[3], c[4]) : make_double2(o0, o1);
   }
 }
 
@@ -131,7 +147,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_sum(int N, const int *__restric
                                                      const double *__restrict__ C, double *__restrict__ G,
                                                      const int *__restrict__ done) {
   if (done && *done) return;
-  const int idx = blockIdx.x * kBlock + threadIdx.x;
+  const int idx = xcd_chunk(blockIdx.x, (4 * N + kBlock - 1) / kBlock) * kBlock + (int)threadIdx.x;
   const int n = idx >> 2, k = idx & 3;
   if (n >= N) return;
   const int s1 = ntrow[n + 1];
