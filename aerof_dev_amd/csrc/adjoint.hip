@@ -387,7 +387,7 @@ __device__ __forceinline__ void adj_face_slot(const DevTables &t, const double *
 // One edge (i, j) at position pos: e[0..5) = Vbar and e[5..10) = c of each end
 // (Gbar[5a+k] = c_k dx[a]: the sums form the products), dxbar, and nbar to its
 // place.
-template <bool SECOND, bool WANTX>
+template <bool SECOND, bool WANTX, bool NT>
 __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__restrict__ V,
                                          const double *__restrict__ grad, const double *__restrict__ mu,
                                          const FluxConsts &fc, int i, int j, int pos, double *__restrict__ EXn,
@@ -420,12 +420,12 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
     }
   }
   double nv[3], fb[13];
-  load_il<3>(t.pnormal, pos, nv);
+  stream_load<3, NT>(t.pnormal, pos, nv);
 #pragma unroll
   for (int d = 0; d < 13; ++d) fb[d] = 0.0;
   if (!(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2] < 1e-36))
     roeflux7_vjp(fc.gas, nv, VL, VR, g, fb, fb + 5, fb + 10);
-  if (WANTX) store_il<3>(EXn, pos, fb + 10);
+  if (WANTX) stream_store<3, NT>(EXn, pos, fb + 10);
   if (!SECOND) {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -476,10 +476,10 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
 // are neither written nor read again; otherwise a wave per (64 nodes, k-th upper
 // edge).  Everything is read and written by
 // position, so what is not gathered is contiguous.  The gradients are read again
-// after the flux for dxbar rather than held across it (1013 -> 568 us at
-// 815k nodes, 5.6M edges, and 342 -> 260 us in the node pass by ROWS; bound by the
-// latency of the gathers at two waves per SIMD).
-template <bool SECOND, bool WANTX, bool ROWS>
+// after the flux for dxbar rather than held across it.  ROWS 2: streams past the
+// caches, which keep the gathered node data (815k nodes, 5.6M edges: 1013 -> 530
+// us, 619 by entries, 568 by rows; the node pass 342 -> 241; 5 TB/s counted).
+template <bool SECOND, bool WANTX, int ROWS>
 __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_edges(
     DevTables t, int nfb, const double *__restrict__ V, const double *__restrict__ grad,
     const double *__restrict__ mu, FluxConsts fc, const int *__restrict__ nfslot, double *__restrict__ EVi,
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
     const bool act = w - kb < deg;
     const int pos = t.up.koff[w] + lanes_below(act);
     if (!act) return;
-    adj_edge<SECOND, WANTX>(t, V, grad, mu, fc, i, t.up.idx[pos], pos, EXn, ei, ej, dxb);
+    adj_edge<SECOND, WANTX, false>(t, V, grad, mu, fc, i, t.up.idx[pos], pos, EXn, ei, ej, dxb);
     store_il<W>(EVi, pos, ei);
     store_il<W>(EVj, pos, ej);
     if (SECOND && WANTX) store_il<3>(EXd, pos, dxb);
@@ -521,8 +521,8 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
     int own = i;
     asm volatile("" : "+v"(own));  // the own side is read anew for each edge
     const int j = t.up.idx[pos];
-    adj_edge<SECOND, WANTX>(t, V, grad, mu, fc, own, j, pos, EXn, ei, ej, dxb);
-    store_il<W>(EVj, pos, ej);
+    adj_edge<SECOND, WANTX, ROWS == 2>(t, V, grad, mu, fc, own, j, pos, EXn, ei, ej, dxb);
+    stream_store<W, ROWS == 2>(EVj, pos, ej);
 #pragma unroll
     for (int q = 0; q < 5; ++q) sum[q][lane] += ei[q];
     const double *X = t.X3;
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma unroll
       for (int q = 0; q < 5; ++q) sum[5 + 5 * a + q][lane] += ei[5 + q] * dx[a];
     if (WANTX) {
-      store_il<3>(EXd, pos, dxb);
+      stream_store<3, ROWS == 2>(EXd, pos, dxb);
 #pragma unroll
       for (int a = 0; a < 3; ++a) sum[20 + a][lane] -= dxb[a];
     }
@@ -577,7 +577,7 @@ __device__ __forceinline__ void add_slot(const double *ev, const double dx[3], d
 // edge pass left their sums in Vb, H and Xb), those of the lower ones are
 // gathered, and both ends' coordinates follow from the adjacency
 // rows, whose first entries are the lower neighbours.  Bound by the slots' bytes
-// (624 -> 260 us at 815k nodes, 342 with both ends' slots; 3.5 TB/s).
+// (624 -> 241 us at 815k nodes, 342 with both ends' slots).
 template <bool SECOND, bool WANTX, bool ROWS>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const double *__restrict__ grad,
                                                          const double *__restrict__ EVi,
@@ -1070,12 +1070,15 @@ int ensure_elem_tables(aerofx_ctx *c) {
   return 0;
 }
 
-// From this many 64-node slices the edge pass takes whole rows (at 562 slices
-// both products 157 us by entries, 169 by rows; 1839: 364, 352; 4292: 867, 822;
-// 14261: 2683, 2547): below that there are too few waves for the 1024 SIMDs.
-constexpr int kAdjRowSlices = 1536;
+// From this many 64-node slices the edge pass takes whole rows, and from the
+// second its streams bypass the caches.  (dR/dU)^T / both products in us, by
+// entries, by rows, by rows past the caches: at 562 slices 122 / 157, 121 / 169,
+// -; 1839: 213 / 364, 194 / 348, 210 / 348; 4292: 502 / 867, 465 / 814, 452 / 791;
+// 14261: 1494 / 2683, 1340 / 2510, 1304 / 2426.  Below, there are too few waves
+// for the 1024 SIMDs, and then the edge data still fit the caches.
+constexpr int kAdjRowSlices = 1536, kAdjStreamSlices = 3072;
 
-template <bool SECOND, bool WANTX, bool ROWS>
+template <bool SECOND, bool WANTX, int ROWS>
 static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, double *Ub, double *Xout) {
   Adjoint *a = c->adj;
   const DevTables &t = c->tab;
@@ -1090,7 +1093,7 @@ static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, dou
                        c->d_grad, a->mu, c->fc, a->nfslot, a->EVi, a->EVj, a->EXd, a->EXn, a->FV, a->FN,
                        a->Vb, a->H, a->Xb);
   // 3.
-  hipLaunchKernelGGL((k_adj_nodes<SECOND, WANTX, ROWS>), slice_grid(t.ns), b, 0, c->stream, t, c->d_grad, a->EVi, a->EVj,
+  hipLaunchKernelGGL((k_adj_nodes<SECOND, WANTX, ROWS != 0>), slice_grid(t.ns), b, 0, c->stream, t, c->d_grad, a->EVi, a->EVj,
                      a->EXd, a->FV, a->Vb, a->H, a->S, a->Xb);
   // 4.
   hipLaunchKernelGGL((k_adj_lsq<SECOND, WANTX>), slice_grid(t.ns), b, 0, c->stream, t, c->d_V, U, c->gas, a->Vb, a->H,
@@ -1119,15 +1122,18 @@ int launch_adjoint(aerofx_ctx *c, const double *U, const double *lam, double *Ub
   int rc = ensure_adjoint(c);
   // forward pass: V, gradients (recomputed), R
   if (rc || (rc = launch_residual(c, U, c->adj->R, true))) return rc;
-  const bool rows = c->tab.ns >= kAdjRowSlices;
-  if (c->p.second_order && rows)
-    return Xout ? adjoint_stages<true, true, true>(c, U, lam, Ub, Xout)
-                : adjoint_stages<true, false, true>(c, U, lam, Ub, Xout);
+  const int ns = c->tab.ns;
+  if (c->p.second_order && ns >= kAdjStreamSlices)
+    return Xout ? adjoint_stages<true, true, 2>(c, U, lam, Ub, Xout)
+                : adjoint_stages<true, false, 2>(c, U, lam, Ub, Xout);
+  if (c->p.second_order && ns >= kAdjRowSlices)
+    return Xout ? adjoint_stages<true, true, 1>(c, U, lam, Ub, Xout)
+                : adjoint_stages<true, false, 1>(c, U, lam, Ub, Xout);
   if (c->p.second_order)
-    return Xout ? adjoint_stages<true, true, false>(c, U, lam, Ub, Xout)
-                : adjoint_stages<true, false, false>(c, U, lam, Ub, Xout);
-  return Xout ? adjoint_stages<false, true, false>(c, U, lam, Ub, Xout)
-              : adjoint_stages<false, false, false>(c, U, lam, Ub, Xout);
+    return Xout ? adjoint_stages<true, true, 0>(c, U, lam, Ub, Xout)
+                : adjoint_stages<true, false, 0>(c, U, lam, Ub, Xout);
+  return Xout ? adjoint_stages<false, true, 0>(c, U, lam, Ub, Xout)
+              : adjoint_stages<false, false, 0>(c, U, lam, Ub, Xout);
 }
 
 // ---------------------------------------------------------------------------

@@ -1,6 +1,6 @@
 """The passes at the sizes where their split changes: 64-node slices (one
-short, exact, one over), the meshes on both sides of the adjoint's rule for
-whole rows (1536 slices), and rows too long for the tables in LDS (a cone with
+short, exact, one over), the meshes on both sides of the adjoint's rules for
+whole rows and streams (1536 and 3072 slices), and rows too long for the tables in LDS (a cone with
 two 301-neighbour hubs: the gradient pass gathers per entry, the viscous
 Jacobian runs its kernel per entry).
 
@@ -33,6 +33,7 @@ MESHES = {
     "cone": _cone_mesh,
     "1521 slices": lambda: M.kuhn_box(45, 45, 45, jitter=0.15, seed=3),
     "1554 slices": lambda: M.kuhn_box(45, 45, 46, jitter=0.15, seed=3),
+    "3102 slices": lambda: M.kuhn_box(57, 57, 58, jitter=0.15, seed=3),
 }
 
 
