@@ -214,7 +214,7 @@ __device__ __forceinline__ void jac_face(const DevTables &t, const double *__res
 
 // The low-Mach edges evaluate roejac6 twice inline (two waves per SIMD with ~18
 // registers spilled beat one without); the others are bound by the blocks
-// they write (assembly at 105k nodes 367 -> 137 us in FP64, 88k nodes 236 -> 88
+// they write (assembly at 105k nodes 367 -> 137 us in FP64, 69k nodes 236 -> 88
 // in FP32 with roe_jac_pair; three waves per SIMD are what the LDS admits).  A chunk that is one row of more than kBlock entries is left to
 // k_jacobian_long.
 template <class T, bool LM>

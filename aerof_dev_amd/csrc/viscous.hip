@@ -105,9 +105,10 @@ __device__ __forceinline__ double pair_swap(double v) {
   return __hiloint2double(pair_swap(__double2hiint(v)), pair_swap(__double2loint(v)));
 }
 
-// Bound by the vector cache, which takes the scattered 32-B pieces one quarter
-// wave's line at a time: the two lanes of a pair write both halves of one tet's
-// piece together, then of the other's (VISCFIG).
+// Bound by the gathers and the scattered 32-B pieces: the two lanes of a pair
+// write both halves of one tet's piece together, then of the other's, and each
+// XCD takes a contiguous range of tets, whose pieces meet in its L2 (84 -> 80 ->
+// 76 us for 1.0M tets).
 __global__ __launch_bounds__(kBlock) void k_visc_elements(int T, const int4 *__restrict__ tets,
                                                           const double *__restrict__ X4, const double *__restrict__ V,
                                                           NsConsts ns, const int4 *__restrict__ pos,
@@ -616,7 +617,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_gather(int N, const int *__rest
 //      through the element means, equal for its four vertices, a third of it.
 // An element is evaluated once per vertex instead of once per entry and per
 // diagonal block (16 times), its derivative as rank-one terms instead of five
-// full columns (88k nodes, FP32 blocks: 503 -> 157 us; 128 lanes take 29 KB of
+// full columns (69k nodes, FP32 blocks: 503 -> 157 us; 128 lanes take 29 KB of
 // LDS, five workgroups per CU).
 constexpr int kJacLanes = 128;
 constexpr int kJacRows = 16;

@@ -11,7 +11,7 @@ Steger-Warming farfield on 5 faces and a slip wall at z = 0.
 A step is one full residual evaluation (gradient pass + flux pass, 1/V
 scaling) with U resident in HBM.  value = edges / (ms per step) in Medges/s.
 
-roofline: one residual evaluation is three kernels (k_gradients,
+roofline: one residual evaluation is three kernels (k_gradients_halo,
 k_flux_edges, k_flux_nodes).  Its algorithmic bytes are 464 B/node +
 40 B/edge + 40 B/face: the gradient pass reads U, X and the LSQ factors and
 writes the gradients (232 B/node) plus an edge pair (8 B/edge); the flux pass
@@ -652,7 +652,7 @@ def main():
     achieved = whole_bytes / (kern_ms * 1e-3) / 1e9
     roofline = dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                     frac=round(achieved / HBM_PEAK_GBS, 4), traffic=load_traffic("residual_box128"),
-                    kernel="residual = k_gradients + k_flux_edges + k_flux_nodes",
+                    kernel="residual = k_gradients_halo + k_flux_edges + k_flux_nodes",
                     algorithmic_bytes=whole_bytes, ms_per_launch=round(kern_ms, 5))
     out = {
         "metric": "Medge-flux evals/s (FP64 residual, 128^3 Kuhn box)",
@@ -671,7 +671,7 @@ def main():
                    "nodes": N, "edges": E, "faces": F, "parallelism": "single GPU",
                    "gpu_rcm_s": round(t_rcm, 3), "gpu_edge_colouring_s": round(t_col, 3), "edge_colours": ncolors},
         "roofline": roofline,
-        "kernels": {"k_gradients": {"ms": round(grad_ms, 5),
+        "kernels": {"k_gradients_halo": {"ms": round(grad_ms, 5),
                                     "algorithmic_GBs": round(grad_bytes / (grad_ms * 1e-3) / 1e9, 1) if grad_ms else None},
                     "k_flux_edges+k_flux_nodes": {
                         "ms": round(edge_ms + node_ms, 5),
