@@ -508,8 +508,9 @@ int launch_tangent(aerofx_ctx *c, const double *U, const double *dU, const doubl
     if (t.E > 0)
       hipLaunchKernelGGL(k_tan_edge_normals, grid_for(t.E), dim3(kTanBlock), 0, c->stream, t, el.etrow, el.etslot,
                          (const int4 *)el.tets, dX, g->dn);
-    hipLaunchKernelGGL(k_tan_vol, grid_for(c->T), dim3(kTanBlock), 0, c->stream, c->T, (const int4 *)el.tets, t.X4, dX,
-                       g->dvol);
+    if (c->T > 0)
+      hipLaunchKernelGGL(k_tan_vol, grid_for(c->T), dim3(kTanBlock), 0, c->stream, c->T, (const int4 *)el.tets, t.X4, dX,
+                         g->dvol);
     if (t.F > 0)
       hipLaunchKernelGGL(k_tan_faces, grid_for(t.F), dim3(kTanBlock), 0, c->stream, t.F, el.faces, t.X4, dX, g->dfn);
   }
