@@ -320,7 +320,8 @@ struct aerofx_ctx {
   // slots (4 f + k), per slot the derivatives [4F][5] / [4F][3]
   int *d_face_elem = nullptr, *d_nfe_row = nullptr, *d_nfe_slot = nullptr;
   double *d_force_u = nullptr, *d_force_x = nullptr;
-  int *d_visc_pos = nullptr;   // [4T] node-slot position of element slot 4 t + j
+  // the elements by their lowest node: vertices, and node-slot positions of the vertices
+  int4 *d_visc_tets = nullptr, *d_visc_pos = nullptr;
   // device address of this GPU's static scratch array of
   // aerofx_residual_noalloc (looked up at ctx_create; null if that failed,
   // with the reason in noalloc_err)
