@@ -984,6 +984,71 @@ int check(const char *what) {
   return e == hipSuccess ? 0 : set_hip_error(e, what);
 }
 
+// The tets by their lowest node (tets, pos) from the slot lists; C: the
+// contribution buffer, which holds the slot places and counts meanwhile.
+// Waits for the result.
+int order_elements(aerofx_ctx *c, double *C, int4 *tets, int4 *pos) {
+  const int N = c->N, ns4 = 4 * c->T;
+  const ElemTables *el = c->elem;
+  int *place = (int *)C, *cnt = place + ns4;
+  const dim3 ng((unsigned)((N + 255) / 256));
+  int rc;
+  hipLaunchKernelGGL(k_slot_positions, dim3((ns4 + 255) / 256), dim3(256), 0, c->stream, ns4, el->ntslot, place);
+  hipLaunchKernelGGL(k_order_elements, ng, dim3(256), 0, c->stream, N, el->ntrow, el->ntslot, (const int4 *)el->tets,
+                     (const int4 *)place, nullptr, cnt, nullptr, nullptr);
+  if ((rc = check("element order launch"))) return rc;
+  std::vector<int> off(N);
+  hipError_t e = hipMemcpyAsync(off.data(), cnt, sizeof(int) * N, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) return set_hip_error(e, "element order counts");
+  int sum = 0;
+  for (int &o : off) {
+    const int k = o;
+    o = sum;
+    sum += k;
+  }
+  e = hipMemcpyAsync(cnt, off.data(), sizeof(int) * N, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) return set_hip_error(e, "element order offsets");
+  hipLaunchKernelGGL(k_order_elements, ng, dim3(256), 0, c->stream, N, el->ntrow, el->ntslot, (const int4 *)el->tets,
+                     (const int4 *)place, cnt, nullptr, tets, pos);
+  if ((rc = check("element order launch"))) return rc;
+  e = hipStreamSynchronize(c->stream);
+  return e == hipSuccess ? 0 : set_hip_error(e, "element order");
+}
+
+// The element contributions of the Galerkin term, their node sums and the
+// order of the element passes, allocated here, at set-up, so that no residual
+// call allocates; without the memory the per-node kernel evaluates each
+// element once per vertex instead.  The context takes them over only when the
+// order is complete: the element passes index memory by it.
+int ensure_element_order(aerofx_ctx *c) {
+  if (c->d_visc_c) return 0;
+  const size_t T = c->T;
+  void *C = nullptr, *pos = nullptr, *tets = nullptr, *g = nullptr;
+  auto release = [&] {
+    for (void *a : {C, pos, tets, g})
+      if (a) (void)hipFree(a);
+  };
+  if (hipMalloc(&C, sizeof(double) * 20 * T) != hipSuccess || hipMalloc(&pos, sizeof(int4) * T) != hipSuccess ||
+      hipMalloc(&tets, sizeof(int4) * T) != hipSuccess ||
+      hipMalloc(&g, sizeof(double) * il_count<4>(c->N)) != hipSuccess) {
+    (void)hipGetLastError();
+    release();
+    return 0;
+  }
+  if (int rc = order_elements(c, (double *)C, (int4 *)tets, (int4 *)pos)) {
+    release();
+    return rc;
+  }
+  for (void *a : {C, pos, tets, g}) c->allocs.push_back(a);
+  c->d_visc_g = (double *)g;
+  c->d_visc_c = (double *)C;
+  c->d_visc_pos = (int4 *)pos;
+  c->d_visc_tets = (int4 *)tets;
+  return 0;
+}
+
 // Domain::setNodeType priorities (DomainCore.C:618-640)
 int bc_priority(int code) {
   static const int pr[22] = {15, 16, 13, 14, 17, 11, 12, 20, 18, 19, -1, 9, 8, 10, 2, 1, 7, 4, 3, 6, 5, 0};
@@ -1175,50 +1240,7 @@ int aerofx_ctx_set_viscous(aerofx_ctx *c, const aerofx_viscous *v) {
     return set_error(AEROFX_ERR_ARG, "set_viscous: Sutherland temperature ratio must be > 0");
   int rc = ensure_elem_tables(c);
   if (rc) return rc;
-  // the element contributions of the residual [4T][5] (allocated here, at
-  // set-up, so that no residual call allocates); without the memory the
-  // per-node kernel evaluates each element once per vertex instead
-  if (!c->d_visc_c) {
-    const size_t T = c->T, N = c->N;
-    void *p = nullptr, *q = nullptr, *g = nullptr, *r = nullptr;
-    if (hipMalloc(&p, sizeof(double) * 20 * T) == hipSuccess && hipMalloc(&q, sizeof(int4) * T) == hipSuccess &&
-        hipMalloc(&r, sizeof(int4) * T) == hipSuccess &&
-        hipMalloc(&g, sizeof(double) * il_count<4>(c->N)) == hipSuccess) {
-      for (void *a : {p, q, r, g}) c->allocs.push_back(a);
-      c->d_visc_g = (double *)g;
-      c->d_visc_c = (double *)p;
-      c->d_visc_pos = (int4 *)q;
-      c->d_visc_tets = (int4 *)r;
-      // slot places and counts meanwhile in the contribution buffer
-      int *pos = (int *)p, *cnt = pos + 4 * T;
-      const int ns4 = 4 * c->T;
-      const ElemTables *el = c->elem;
-      const dim3 ng((unsigned)((N + 255) / 256));
-      hipLaunchKernelGGL(k_slot_positions, dim3((ns4 + 255) / 256), dim3(256), 0, c->stream, ns4, el->ntslot, pos);
-      hipLaunchKernelGGL(k_order_elements, ng, dim3(256), 0, c->stream, c->N, el->ntrow, el->ntslot,
-                         (const int4 *)el->tets, (const int4 *)pos, nullptr, cnt, nullptr, nullptr);
-      if ((rc = check("element order launch"))) return rc;
-      std::vector<int> off(N);
-      hipError_t e = hipMemcpyAsync(off.data(), cnt, sizeof(int) * N, hipMemcpyDeviceToHost, c->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-      int sum = 0;
-      for (int &o : off) {
-        const int k = o;
-        o = sum;
-        sum += k;
-      }
-      if (e == hipSuccess) e = hipMemcpyAsync(cnt, off.data(), sizeof(int) * N, hipMemcpyHostToDevice, c->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-      if (e != hipSuccess) return set_hip_error(e, "element order");
-      hipLaunchKernelGGL(k_order_elements, ng, dim3(256), 0, c->stream, c->N, el->ntrow, el->ntslot,
-                         (const int4 *)el->tets, (const int4 *)pos, cnt, nullptr, c->d_visc_tets, c->d_visc_pos);
-      if ((rc = check("element order launch"))) return rc;
-    } else {
-      (void)hipGetLastError();
-      for (void *a : {p, q, r})
-        if (a) (void)hipFree(a);
-    }
-  }
+  if ((rc = ensure_element_order(c))) return rc;
   // row chunks of the Jacobian pass (none if a row exceeds its limits)
   if (!c->d_visc_chunk) {
     std::vector<int> el_cnt(c->N, 0), deg(c->N, 0), chunk(1, 0);
