@@ -30,13 +30,14 @@ namespace aerofx {
 // local time step (Edge.C:87-143, Face.C:242-290, Domain.C:32-100), beta = 1
 // ---------------------------------------------------------------------------
 // min(u.n - c, 0) S through the area vector nv outward from the node: with
-// beta = 1 the wave speed 0.5 (2 u_n - 2 c) of the reference
+// beta = 1 the wave speed 0.5 (2 u_n - 2 c) of the reference.  IEEE roots and
+// division: at zero pressure c = 0 and the speed is u.n, where a root through
+// 1 / sqrt(c^2) has no value; the pass is bound by its gathers.
 __device__ __forceinline__ double inflow_speed(const Gas &g, const double V[5], const double nv[3]) {
 #pragma clang fp contract(on)
-  const double s2 = nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2];
-  const double S = s2 > 0.0 ? sqrt_from_rsq(s2, frsq(s2)) : 0.0;
-  const double c2 = g.gam * (V[4] + g.pstiff) * frcp(V[0]);
-  const double w = (V[1] * nv[0] + V[2] * nv[1] + V[3] * nv[2]) - sqrt_from_rsq(c2, frsq(c2)) * S;
+  const double S = sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]);
+  const double c = sqrt(g.gam * (V[4] + g.pstiff) / V[0]);
+  const double w = (V[1] * nv[0] + V[2] * nv[1] + V[3] * nv[2]) - c * S;
   return w < 0.0 ? w : 0.0;
 }
 
@@ -86,7 +87,7 @@ __device__ __forceinline__ int chunk_row(const int *srow, int nr, int tid) {
 
 // Entry-parallel over the whole-row chunks: a lane per adjacency entry, the
 // rows summed through LDS in entry order, so an entry's gathers are not a
-// chain of 14 (34 -> 21 us at 105k nodes).
+// chain of 14 (34 -> 22 us at 105k nodes).
 __global__ __launch_bounds__(kBlock) void k_timestep(DevTables t, const double *__restrict__ V, Gas g, double cfl,
                                                      const double *__restrict__ idtv, double viscous,
                                                      double *__restrict__ dt) {

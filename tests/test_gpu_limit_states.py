@@ -1,0 +1,48 @@
+"""States at the limit of the equations, where a reciprocal or a root of the
+kernels has the argument zero while the quantity itself is finite.
+
+The velocities are multiples of 1/16 and the density is 1, so that with
+E = |u|^2 / 2 the pressure of the conservative state comes out as exactly 0."""
+import numpy as np
+import pytest
+
+import oracle as O
+from aerof_dev_amd import FlowParams, init_state
+from aerof_dev_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+
+def _cold(n, seed):
+    """n conservative states of zero pressure and temperature."""
+    u = np.random.default_rng(seed).integers(-16, 17, size=(n, 3)) / 16.0
+    u[:, 0] += 0.03125  # not at rest
+    U = np.zeros((n, 5))
+    U[:, 0] = 1.0
+    U[:, 1:4] = u
+    U[:, 4] = 0.5 * (u[:, 0] * u[:, 0] + u[:, 1] * u[:, 1] + u[:, 2] * u[:, 2])
+    return U
+
+
+def test_timestep_of_zero_pressure(gpu):
+    """Without a sound speed the time step is the convective one (Edge.C:87-143
+    with c = 0), here on whole edges and faces of zero pressure; 1e-13 as for
+    any state."""
+    import torch
+    from aerof_dev_amd.operators import MatVecProdH1, SpaceOperator
+    m = M.box_mesh(6, jitter=0.15, seed=3)
+    p = FlowParams(mach=0.5)
+    U = init_state(p, m.X, "noise", 0.02, seed=4)
+    cold = np.flatnonzero(m.X[:, 0] < 0.5)
+    U[cold] = _cold(cold.size, 5)
+    om = O.OracleMesh(m, p)
+    V = om.residual(U)["V"]
+    assert np.all(V[cold, 4] == 0.0)
+    ref = om.timestep(V, 12.0)
+    assert np.all(np.isfinite(ref)) and np.all(ref > 0.0)
+    op = SpaceOperator(m, p)
+    dt = torch.empty(op.num_nodes, dtype=torch.float64, device=gpu)
+    MatVecProdH1(op).timestep(torch.from_numpy(U).to(gpu), 12.0, dt)
+    got = dt.cpu().numpy()
+    assert np.max(np.abs(got - ref) / ref) <= 1e-13
+    op.close()
