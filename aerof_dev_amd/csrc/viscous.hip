@@ -632,7 +632,8 @@ __global__ __launch_bounds__(kBlock) void k_visc_gather(int N, const int *__rest
 // most kJacLanes node-element slots and kJacLanes entries.
 //   1. one lane per slot evaluates its element once and leaves in LDS what its
 //      row needs: the shape gradients, the transport coefficients times the
-//      volume, the mean velocity, tau g_n and the heat flux along g_n;
+//      volume, the mean velocity, tau g_n per unit viscosity and the heat flux
+//      along g_n;
 //   2. one lane per entry (n, m) finds the slots whose element holds m and adds
 //      the derivatives with respect to m's velocity and temperature -- 20
 //      numbers -- over them in element order; the change to conservative
@@ -642,7 +643,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_gather(int N, const int *__rest
 //      through the element means, equal for its four vertices, a third of it.
 // An element is evaluated once per vertex instead of once per entry and per
 // diagonal block (16 times), its derivative as rank-one terms instead of five
-// full columns (69k nodes, FP32 blocks: 503 -> 157 us; 128 lanes take 29 KB of
+// full columns (69k nodes, FP32 blocks: 503 -> 158 us; 128 lanes take 29 KB of
 // LDS, five workgroups per CU).
 constexpr int kJacLanes = 128;
 constexpr int kJacRows = 16;
@@ -716,13 +717,20 @@ __global__ __launch_bounds__(kJacLanes) void k_visc_jacobian_rows(DevTables tb, 
     o[12] = vol * e.mu;
     o[13] = vol * e.lambda;
     o[14] = vol * e.kappa;
+    // the stress at unit viscosity along g_n: the law may be zero at the
+    // element's temperature and its derivative not (lambda is -2/3 mu, with a
+    // bulk term only at constant viscosity)
+    const double ratio = (ns.visc == 0 ? ns.bulk : 0.0) - 2.0 / 3.0;
+    const double rdiv = ratio * (e.dudxj[0][0] + e.dudxj[1][1] + e.dudxj[2][2]);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       o[15 + d] = e.ucg[d];
-      o[18 + d] = vol * (e.tij[d][0] * gn[0] + e.tij[d][1] * gn[1] + e.tij[d][2] * gn[2]);
+      double s = rdiv * gn[d];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) s += (e.dudxj[d][j] + e.dudxj[j][d]) * gn[j];
+      o[18 + d] = s;
     }
-    // d tau / d T = tau (d mu / d T) / mu: lambda follows mu unless both are constant
-    o[21] = dmu == 0.0 ? 0.0 : dmu / e.mu;
+    o[21] = vol * dmu;
     o[22] = vol * dkap * (e.dTdxj[0] * gn[0] + e.dTdxj[1] * gn[1] + e.dTdxj[2] * gn[2]);
     sid[tid] = tets[t];
     sln[tid] = ln;
@@ -766,7 +774,7 @@ __global__ __launch_bounds__(kJacLanes) void k_visc_jacobian_rows(DevTables tb, 
           for (int i = 0; i < 3; ++i) a.K[i][p] += gm[i] * mg + gn[i] * lg;
           a.K[p][p] += mu * S;
           a.E[p] += mu * S * u[p] + ugm * mg + ugn * lg;
-          a.Te[p] += 0.25 * t[p];
+          a.Te[p] += 0.25 * mu * t[p];
           a.P[p] += o[21] * t[p];
         }
         a.Q += o[14] * S;

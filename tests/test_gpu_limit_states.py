@@ -3,6 +3,9 @@ kernels has the argument zero while the quantity itself is finite.
 
 The velocities are multiples of 1/16 and the density is 1, so that with
 E = |u|^2 / 2 the pressure of the conservative state comes out as exactly 0."""
+import os
+import sys
+
 import numpy as np
 import pytest
 
@@ -11,6 +14,7 @@ from aerof_dev_amd import FlowParams, init_state
 from aerof_dev_amd import mesh as M
 
 pytestmark = pytest.mark.gpu
+sys.path.insert(0, os.path.dirname(__file__))
 
 
 def _cold(n, seed):
@@ -45,4 +49,36 @@ def test_timestep_of_zero_pressure(gpu):
     MatVecProdH1(op).timestep(torch.from_numpy(U).to(gpu), 12.0, dt)
     got = dt.cpu().numpy()
     assert np.max(np.abs(got - ref) / ref) <= 1e-13
+    op.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("viscosity", ["prandtl", "sutherland", "constant"])
+def test_viscous_jacobian_of_zero_temperature(gpu, viscosity, precision):
+    """The Galerkin blocks around elements whose mean temperature is 0: with the
+    linear law the viscosity is zero there and its derivative is not.  The
+    velocities of the cold nodes differ, so Roe's average has a sound speed."""
+    import torch
+    from aerof_dev_amd.operators import MatVecProdH1, SpaceOperator
+    from test_gpu_viscous import ns_params
+    m = M.kuhn_box(6, 5, 5, jitter=0.15, seed=3, face_codes=M.VISCOUS_CHANNEL)
+    p = ns_params(0.4, 20.0, viscosity=viscosity, bulk_viscosity=0.02)
+    U = init_state(p, m.X, "noise", 0.02, seed=14)
+    inner = np.all((m.X > m.X.min(0) + 1e-9) & (m.X < m.X.max(0) - 1e-9), axis=1)
+    tets = np.asarray(m.tets)[np.all(inner[np.asarray(m.tets)], axis=1)]
+    cold = np.unique(np.concatenate([tets[0], tets[len(tets) // 2]]))
+    U[cold] = _cold(cold.size, 6)
+    om = O.OracleMesh(m, p)
+    V = om.residual(U)["V"]
+    assert np.all(V[cold, 4] == 0.0)
+    dt = np.full(m.num_nodes, 0.05)
+    Dr, Ar = om.apply_bcs_jacobian(U, *om.jacobian(V, dt))
+    assert np.all(np.isfinite(Dr)) and np.all(np.isfinite(Ar))
+    op = SpaceOperator(m, p)
+    h1 = MatVecProdH1(op)
+    h1.evaluate(torch.from_numpy(U).to(gpu), torch.from_numpy(dt).to(gpu), precision)
+    D, A = h1.blocks()
+    tol = 1e-12 if precision == 0 else 1e-6
+    assert np.max(np.abs(D - Dr) / np.abs(Dr).max(axis=(1, 2))[:, None, None]) <= tol
+    assert np.max(np.abs(A - Ar) / (np.abs(Ar).max(axis=(2, 3))[:, :, None, None] + 1e-300)) <= tol
     op.close()
