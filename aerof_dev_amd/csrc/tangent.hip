@@ -528,8 +528,16 @@ int launch_h2_select(aerofx_ctx *c, const double *Q) {
   if (rc) return rc;
   Tangent *g = c->tan;
   const DevTables &t = c->tab;
-  if (!g->V0 && ((rc = alloc_n(c, il_count<5>(t.N), &g->V0)) || (rc = alloc_n(c, il_count<15>(t.N), &g->G0))))
-    return rc;
+  if (!g->V0) {  // both or neither
+    double *V0 = nullptr, *G0 = nullptr;
+    if ((rc = alloc_n(c, il_count<5>(t.N), &V0))) return rc;
+    if ((rc = alloc_n(c, il_count<15>(t.N), &G0))) {
+      ctx_release(c, V0);
+      return rc;
+    }
+    g->V0 = V0;
+    g->G0 = G0;
+  }
   const ResidualBufs b{g->V0, g->G0, c->d_Fm, c->d_P};
   return launch_residual_with(c, b, Q, g->S, false);
 }

@@ -61,6 +61,19 @@ def test_viscous_set_up_fails_half_way(fake_lib):
             assert _ordering_built(r["log1"]) or _ordering_built(r["log2"]), r
 
 
+@pytest.mark.parametrize("what", ["h2"])
+def test_storage_runs_out_half_way(fake_lib, what):
+    """With the n-th allocation of the call failing, its repetition allocates
+    what is missing: it may not run its kernels on a part of the storage."""
+    runs = _drive(fake_lib, what)
+    assert len(runs) >= 3
+    for r in runs:
+        assert r["first"] < 0 and "kernel " + r["kernel"] not in r["log1"], r
+        assert r["second"] == 0, r
+        use = r["log2"].index("kernel " + r["kernel"])
+        assert "hipMalloc" in r["log2"][:use], r
+
+
 # ---------------------------------------------------------------------------
 # child process: the library of AEROFX_LIB
 # ---------------------------------------------------------------------------
@@ -97,6 +110,9 @@ class _Ctx:
         v = ViscousC(100.0, 1, 0.0, 0.4, 0, 0.72, 0.0, 1.0, 0.0)
         return self.lib.aerofx_ctx_set_viscous(self.h, C.byref(v))
 
+    def select_h2(self):
+        return self.lib.aerofx_mvp_select(self.h, 2, self.ptr(self.U), None, None, 1)
+
     def residual(self):
         assert self.lib.aerofx_residual_ex(self.h, self.ptr(self.U), self.ptr(self.R), 0) == 0
         return self.log()
@@ -105,13 +121,14 @@ class _Ctx:
         self.lib.aerofx_ctx_destroy(self.h)
 
 
-def _each_failure(call):
-    """(context, first result, first log) with the n-th fallible call failing, n = 1, 2, ..."""
+def _each_failure(call, name=b""):
+    """(context, first result, first log) with the n-th call that can fail (of
+    that name) failing, n = 1, 2, ..."""
     n = 1
     while True:
         x = _Ctx()
         x.log()
-        x.lib.fake_arm(b"", C.c_long(n))
+        x.lib.fake_arm(name, C.c_long(n))
         first = call(x)
         if x.lib.fake_pending():  # fewer than n calls: the whole set-up ran
             x.lib.fake_arm(b"", C.c_long(0))
@@ -127,6 +144,14 @@ def _viscous():
             for x, first, log1 in _each_failure(_Ctx.set_viscous)]
 
 
+def _storage(call, kernel):
+    return [{"kernel": kernel, "first": first, "log1": log1, "second": call(x), "log2": x.log()}
+            for x, first, log1 in _each_failure(call, b"hipMalloc")]
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
-    print(json.dumps({"viscous": _viscous}[sys.argv[1]]()))
+    print(json.dumps({
+        "viscous": _viscous,
+        "h2": lambda: _storage(_Ctx.select_h2, "k_gradients_halo"),
+    }[sys.argv[1]]()))
