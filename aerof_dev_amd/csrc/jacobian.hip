@@ -600,11 +600,15 @@ int ensure_jacobian_storage(aerofx_ctx *c, int precision) {
     if (rc) return rc;
     c->d_fjac = (double *)p;
   }
-  if (!st[0]) {
-    int rc;
-    if ((rc = ctx_alloc(c, need_d, &st[0])) || (rc = ctx_alloc(c, need_b, &st[1])) ||
-        (rc = ctx_alloc(c, need_d, &st[2])))
-      return rc;
+  if (!st[0]) {  // all three or none
+    const size_t need[3] = {need_d, need_b, need_d};
+    void *p[3] = {nullptr, nullptr, nullptr};
+    for (int k = 0; k < 3; ++k)
+      if (int rc = ctx_alloc(c, need[k], &p[k])) {
+        while (k > 0) ctx_release(c, p[--k]);
+        return rc;
+      }
+    for (int k = 0; k < 3; ++k) st[k] = p[k];
   }
   c->d_jacD = st[0];
   c->d_jacB = st[1];

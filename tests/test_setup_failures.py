@@ -61,7 +61,7 @@ def test_viscous_set_up_fails_half_way(fake_lib):
             assert _ordering_built(r["log1"]) or _ordering_built(r["log2"]), r
 
 
-@pytest.mark.parametrize("what", ["h2"])
+@pytest.mark.parametrize("what", ["h2", "jacobian fp64", "jacobian fp32"])
 def test_storage_runs_out_half_way(fake_lib, what):
     """With the n-th allocation of the call failing, its repetition allocates
     what is missing: it may not run its kernels on a part of the storage."""
@@ -113,6 +113,9 @@ class _Ctx:
     def select_h2(self):
         return self.lib.aerofx_mvp_select(self.h, 2, self.ptr(self.U), None, None, 1)
 
+    def jacobian(self, precision):
+        return self.lib.aerofx_jacobian_setup(self.h, self.ptr(self.U), None, precision)
+
     def residual(self):
         assert self.lib.aerofx_residual_ex(self.h, self.ptr(self.U), self.ptr(self.R), 0) == 0
         return self.log()
@@ -154,4 +157,6 @@ if __name__ == "__main__":
     print(json.dumps({
         "viscous": _viscous,
         "h2": lambda: _storage(_Ctx.select_h2, "k_gradients_halo"),
+        "jacobian fp64": lambda: _storage(lambda x: x.jacobian(0), "k_jacobian"),
+        "jacobian fp32": lambda: _storage(lambda x: x.jacobian(1), "k_jacobian"),
     }[sys.argv[1]]()))
