@@ -13,6 +13,7 @@
 // sums are deterministic.
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <string>
 #include <vector>
 
@@ -1033,27 +1034,26 @@ int order_elements(aerofx_ctx *c, double *C, int4 *tets, int4 *pos) {
 int ensure_element_order(aerofx_ctx *c) {
   if (c->d_visc_c) return 0;
   const size_t T = c->T;
-  void *C = nullptr, *pos = nullptr, *tets = nullptr, *g = nullptr;
-  auto release = [&] {
-    for (void *a : {C, pos, tets, g})
-      if (a) (void)hipFree(a);
-  };
-  if (hipMalloc(&C, sizeof(double) * 20 * T) != hipSuccess || hipMalloc(&pos, sizeof(int4) * T) != hipSuccess ||
-      hipMalloc(&tets, sizeof(int4) * T) != hipSuccess ||
-      hipMalloc(&g, sizeof(double) * il_count<4>(c->N)) != hipSuccess) {
+  struct Mem {
+    void *p = nullptr;
+    ~Mem() {
+      if (p) (void)hipFree(p);
+    }
+  } C, pos, tets, g;
+  if (hipMalloc(&C.p, sizeof(double) * 20 * T) != hipSuccess || hipMalloc(&pos.p, sizeof(int4) * T) != hipSuccess ||
+      hipMalloc(&tets.p, sizeof(int4) * T) != hipSuccess ||
+      hipMalloc(&g.p, sizeof(double) * il_count<4>(c->N)) != hipSuccess) {
     (void)hipGetLastError();
-    release();
     return 0;
   }
-  if (int rc = order_elements(c, (double *)C, (int4 *)tets, (int4 *)pos)) {
-    release();
-    return rc;
-  }
-  for (void *a : {C, pos, tets, g}) c->allocs.push_back(a);
-  c->d_visc_g = (double *)g;
-  c->d_visc_c = (double *)C;
-  c->d_visc_pos = (int4 *)pos;
-  c->d_visc_tets = (int4 *)tets;
+  if (int rc = order_elements(c, (double *)C.p, (int4 *)tets.p, (int4 *)pos.p)) return rc;
+  c->allocs.reserve(c->allocs.size() + 4);
+  for (Mem *m : {&C, &pos, &tets, &g}) c->allocs.push_back(m->p);
+  c->d_visc_g = (double *)g.p;
+  c->d_visc_c = (double *)C.p;
+  c->d_visc_pos = (int4 *)pos.p;
+  c->d_visc_tets = (int4 *)tets.p;
+  for (Mem *m : {&C, &pos, &tets, &g}) m->p = nullptr;
   return 0;
 }
 
@@ -1229,9 +1229,7 @@ int refuse_viscous(aerofx_ctx *c, const char *who) {
 
 using namespace aerofx;
 
-extern "C" {
-
-int aerofx_ctx_set_viscous(aerofx_ctx *c, const aerofx_viscous *v) {
+static int set_viscous(aerofx_ctx *c, const aerofx_viscous *v) {
   if (!c) return set_error(AEROFX_ERR_ARG, "set_viscous: null context");
   if (!v) {
     c->viscous = 0;
@@ -1372,6 +1370,16 @@ int aerofx_ctx_set_viscous(aerofx_ctx *c, const aerofx_viscous *v) {
   c->ns = ns;
   c->viscous = 1;
   return AEROFX_OK;
+}
+
+extern "C" {
+
+int aerofx_ctx_set_viscous(aerofx_ctx *c, const aerofx_viscous *v) {
+  try {
+    return set_viscous(c, v);
+  } catch (std::exception &ex) {  // host memory of the tables
+    return set_error(AEROFX_ERR_NOMEM, std::string("set_viscous: ") + ex.what());
+  }
 }
 
 int aerofx_ctx_node_types(const aerofx_ctx *c, int *types) {

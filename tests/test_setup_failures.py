@@ -61,6 +61,15 @@ def test_viscous_set_up_fails_half_way(fake_lib):
             assert _ordering_built(r["log1"]) or _ordering_built(r["log2"]), r
 
 
+def test_viscous_set_up_without_host_memory(fake_lib):
+    """A failing host allocation is an error code at the C entry, not an
+    exception through it, and the next call works."""
+    runs = _drive(fake_lib, "viscous host")
+    assert len(runs) >= 20
+    for r in runs:
+        assert r["first"] == -4 and r["second"] == 0, r
+
+
 @pytest.mark.parametrize("what", ["h2", "jacobian fp64", "jacobian fp32"])
 def test_storage_runs_out_half_way(fake_lib, what):
     """With the n-th allocation of the call failing, its repetition allocates
@@ -152,10 +161,27 @@ def _storage(call, kernel):
             for x, first, log1 in _each_failure(call, b"hipMalloc")]
 
 
+def _viscous_host():
+    runs, n = [], 1
+    while True:
+        x = _Ctx()
+        x.lib.fake_arm_new(C.c_long(n))
+        first = x.set_viscous()
+        done = x.lib.fake_pending()
+        x.lib.fake_arm_new(C.c_long(0))
+        if not done:
+            runs.append({"n": n, "first": first, "second": x.set_viscous()})
+        x.close()
+        if done:
+            return runs
+        n = n + 1 if n < 40 else n + 37  # the later ones are the per-node lists
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     print(json.dumps({
         "viscous": _viscous,
+        "viscous host": _viscous_host,
         "h2": lambda: _storage(_Ctx.select_h2, "k_gradients_halo"),
         "jacobian fp64": lambda: _storage(lambda x: x.jacobian(0), "k_jacobian"),
         "jacobian fp32": lambda: _storage(lambda x: x.jacobian(1), "k_jacobian"),
