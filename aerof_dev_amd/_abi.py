@@ -38,6 +38,9 @@ AEROFX_PHYS_INVERT5_F32 = 6
 AEROFX_PHYS_ROEFLUX5 = 7
 AEROFX_PHYS_ROEJAC6_LM_SW1 = 8
 AEROFX_PHYS_ROEJAC6_LM_SW2 = 9
+AEROFX_PHYS_ROE_FLUX = 10
+AEROFX_PHYS_RECONSTRUCT = 11
+AEROFX_PHYS_ROE_JAC_PAIR = 12
 TIMER_NAMES = ("nodalGrad", "fvTerm", "fvTermNodes", "fvJac", "fluidPrecSetup", "jacApply",
                "precApply", "gramSchmidt", "feTerm", "feJac")
 

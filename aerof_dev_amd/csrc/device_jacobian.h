@@ -1,7 +1,10 @@
 // device_jacobian.h -- flux Jacobians as gfx950 device code.
 //
 //   roejac6      ROEJAC6, type 0, prec 0 or 1 (f77src/roejac6.f:1-316):
-//                0.5 |n| (A(Ug) +/- |A_roe(Ug,Ud)|), row-major 5x5
+//                0.5 |n| (A(Ug) +/- |A_roe(Ug,Ud)|), row-major 5x5; the
+//                assembly takes it with prec 1 only
+//   roe_jac_pair both prec-0 blocks of an edge from their structure, equal to
+//                roejac6's to rounding
 //   post_dVdU    VarFcnSGEuler::computedVdU + VarFcnBase::postMultiplyBydVdU
 //                (VarFcnSGEuler.h:588-603, VarFcnBase.h:383-411)
 //   wall_jac     FluxFcnSGWallEuler3D::computeJacobian (FluxFcnDescSG.C:838-886)

@@ -1,7 +1,12 @@
 // device_physics.h -- per-edge and per-face physics as gfx950 device code.
 //
-// Operation order follows the reference kernels so that, built without FMA
-// contraction, each routine reproduces the reference bit for bit:
+// reconstruct and roe_flux, below, are what the edge passes evaluate: the
+// functions of vanalbada and roeflux7 in fewer operations, equal to rounding.
+// vanalbada and roeflux7 are the statements they are held against; nothing
+// but physics_eval.hip calls them.
+//
+// Of the others the operation order follows the reference kernels so that,
+// built without FMA contraction, each reproduces the reference bit for bit:
 //   prim_from_cons  VarFcnSGEuler::conservativeToPrimitive (VarFcnSGEuler.h:307-336)
 //   va_fcn / vanalbada  RecFcn::computeVanAlbadaFcn, RecFcn::vanalbada
 //                   (RecFcn.h:269-281, 433-446; eps0 = 1e-16, RecFcn.h:47)
@@ -23,8 +28,9 @@ struct Gas {
   double gam, gam1, invgam1, pstiff;
 };
 
-// Division and square root of the flux routines: IEEE-rounded, as the
-// reference's; the Dual overloads (device_dual.h) carry derivatives.
+// Division and square root of the routines in the reference's operation
+// order: IEEE-rounded, as the reference's; the Dual overloads (device_dual.h)
+// carry derivatives.
 __device__ __forceinline__ double ddiv(double a, double b) { return a / b; }
 __device__ __forceinline__ double dsqrt(double x) { return sqrt(x); }
 
@@ -183,9 +189,10 @@ __device__ __forceinline__ Dual neg_part(Dual x) { return x.v < 0.0 ? x : Dual(0
 __device__ __forceinline__ Dual pos_part(Dual x) { return x.v > 0.0 ? x : Dual(0.0); }
 __device__ __forceinline__ Dual gabs(Dual x) { return x.v < 0.0 ? -x : x; }
 
-// The residual's Van Albada reconstruction and Roe flux: the functions of
-// vanalbada and roeflux7 (which the reverse pass differentiates; the forward
-// one takes these with T = Dual) with the fewest FP64 operations (805 -> 530 vector instructions an edge with the
+// The Van Albada reconstruction and Roe flux of the residual and, with
+// T = Dual, of its forward derivative (the reverse one differentiates
+// roeflux7's statements by hand): the functions of vanalbada and roeflux7 with
+// the fewest FP64 operations (805 -> 530 vector instructions an edge with the
 // edge pass's loads and addressing, 60 % -> 40 % of its clocks at 2.1M nodes):
 //  * the flux's sums contracted to fused multiply-adds (the gradients' and the
 //    projected slopes' keep their order), the divisions through frcp;

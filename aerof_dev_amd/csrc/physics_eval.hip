@@ -1,8 +1,11 @@
-// physics_eval.hip -- the per-edge, per-face and per-block routines that the
-// residual, Jacobian and preconditioner kernels inline (device_physics.h,
-// device_jacobian.h), evaluated one case per thread on caller arrays.  It lets
-// a test hold the device code itself against stored outputs of the
-// reference's own routines, case by case and bit for bit.
+// physics_eval.hip -- the per-edge, per-face and per-block routines of
+// device_physics.h and device_jacobian.h, evaluated one case per thread on
+// caller arrays: those that the residual, Jacobian and preconditioner kernels
+// inline (roe_flux, reconstruct, roe_jac_pair, boundflux5, roe_turkel_flux,
+// roejac6 with the low-Mach constants, invert5) and the reference's statements
+// of the first three (roeflux7, vanalbada, roejac6).  It lets a test hold the
+// device code itself against stored outputs of the reference's own routines,
+// case by case.
 #include <hip/hip_runtime.h>
 
 #include "context.h"
@@ -23,6 +26,7 @@ __global__ __launch_bounds__(kEvalBlock) void k_physics_eval(int kind, int n, Ga
   const int q = blockIdx.x * kEvalBlock + threadIdx.x;
   if (q >= n) return;
   const size_t s = (size_t)q;
+  if ((kind == AEROFX_PHYS_ROE_FLUX || kind == AEROFX_PHYS_ROE_JAC_PAIR) && d) g.pstiff = d[s];
   switch (kind) {
     case AEROFX_PHYS_ROEFLUX7: {
       double nv[3], vl[5], vr[5], f[5];
@@ -108,6 +112,40 @@ __global__ __launch_bounds__(kEvalBlock) void k_physics_eval(int kind, int n, Ga
       for (int k = 0; k < 5; ++k) out[5 * s + k] = f[k];
       break;
     }
+    case AEROFX_PHYS_ROE_FLUX: {
+      double nv[3], vl[5], vr[5], f[5];
+      for (int k = 0; k < 3; ++k) nv[k] = a[3 * s + k];
+      for (int k = 0; k < 5; ++k) {
+        vl[k] = b[5 * s + k];
+        vr[k] = c[5 * s + k];
+      }
+      roe_flux(g, nv, vl, vr, f);
+      for (int k = 0; k < 5; ++k) out[5 * s + k] = f[k];
+      break;
+    }
+    case AEROFX_PHYS_RECONSTRUCT: {
+      for (int k = 0; k < 5; ++k) {
+        double vij, vji;
+        reconstruct(scalar, a[5 * s + k], b[5 * s + k], c[5 * s + k], d[5 * s + k], vij, vji);
+        out[10 * s + k] = vij;
+        out[10 * s + 5 + k] = vji;
+      }
+      break;
+    }
+    case AEROFX_PHYS_ROE_JAC_PAIR: {
+      double nv[3], vn[5], vm[5], own[25], off[25];
+      for (int k = 0; k < 3; ++k) nv[k] = a[3 * s + k];
+      for (int k = 0; k < 5; ++k) {
+        vn[k] = b[5 * s + k];
+        vm[k] = c[5 * s + k];
+      }
+      roe_jac_pair(g, nv, vn, vm, own, off);
+      for (int k = 0; k < 25; ++k) {
+        out[50 * s + k] = own[k];
+        out[50 * s + 25 + k] = off[k];
+      }
+      break;
+    }
     default:
       break;
   }
@@ -120,15 +158,18 @@ using namespace aerofx;
 
 extern "C" int aerofx_physics_eval(int kind, int n, double scalar, const double *a, const double *b, const double *c,
                                    const double *d, double *out) {
-  if (kind < AEROFX_PHYS_ROEFLUX7 || kind > AEROFX_PHYS_ROEJAC6_LM_SW2)
+  if (kind < AEROFX_PHYS_ROEFLUX7 || kind > AEROFX_PHYS_ROE_JAC_PAIR)
     return set_error(AEROFX_ERR_ARG, "physics_eval: unknown kind");
   if (n < 0) return set_error(AEROFX_ERR_ARG, "physics_eval: n < 0");
   const bool need_bc = kind != AEROFX_PHYS_INVERT5_F64 && kind != AEROFX_PHYS_INVERT5_F32;
-  if (!a || !out || (need_bc && (!b || !c)) || ((kind == AEROFX_PHYS_VANALBADA || kind >= AEROFX_PHYS_ROEFLUX5) && !d))
+  const bool need_d = kind == AEROFX_PHYS_VANALBADA || kind == AEROFX_PHYS_RECONSTRUCT ||
+                      kind == AEROFX_PHYS_ROEFLUX5 || kind == AEROFX_PHYS_ROEJAC6_LM_SW1 ||
+                      kind == AEROFX_PHYS_ROEJAC6_LM_SW2;
+  if (!a || !out || (need_bc && (!b || !c)) || (need_d && !d))
     return set_error(AEROFX_ERR_ARG, "physics_eval: null argument");
   if (n == 0) return AEROFX_OK;
   Gas g;
-  g.gam = kind == AEROFX_PHYS_VANALBADA ? 1.4 : scalar;
+  g.gam = kind == AEROFX_PHYS_VANALBADA || kind == AEROFX_PHYS_RECONSTRUCT ? 1.4 : scalar;
   g.gam1 = g.gam - 1.0;
   g.invgam1 = 1.0 / g.gam1;
   g.pstiff = 0.0;

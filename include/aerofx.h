@@ -605,10 +605,13 @@ int aerofx_solution_read(const char *path, int step, double *tag, int n, int dim
                          double *U);
 
 /* ---- physics routines, one case per thread ----------------------------- */
-/* No counterpart in the reference: evaluates the device routines that the
- * residual, Jacobian and preconditioner kernels inline, on n cases in device
- * arrays, so that tests can compare them case by case with stored outputs of
- * the reference's routines.  Runs on the null stream and synchronises.
+/* No counterpart in the reference: evaluates device routines on n cases in
+ * device arrays, so that tests can compare them case by case with stored
+ * outputs of the reference's routines.  ROE_FLUX, RECONSTRUCT, ROE_JAC_PAIR,
+ * BOUNDFLUX5, ROEFLUX5, ROEJAC6_LM and INVERT5 are what the residual, Jacobian
+ * and preconditioner kernels inline; ROEFLUX7, VANALBADA and ROEJAC6 are the
+ * reference's statements of the first three, in its operation order.  Runs on
+ * the null stream and synchronises.
  *   AEROFX_PHYS_ROEFLUX7     ROEFLUX7 (roeflux7.f), scalar = gamma:
  *                            a normal [n][3], b V_L [n][5], c V_R [n][5] -> out [n][5]
  *   AEROFX_PHYS_BOUNDFLUX5   BOUNDFLUX5 (boundflux5.f), scalar = gamma:
@@ -628,6 +631,13 @@ int aerofx_solution_read(const char *path, int step, double *tag, int n, int dim
  *   AEROFX_PHYS_ROEJAC6_LM_SW1/2  ROEJAC6 type 1 or 2 with the low-Mach constants
  *                            (roejac6.f:130-160), scalar = gamma: a normal,
  *                            b U_g, c U_d, d [n][7] as for ROEFLUX5 -> out [n][25]
+ *   AEROFX_PHYS_ROE_FLUX     the Roe flux of the edge pass, scalar = gamma: a normal,
+ *                            b V_L, c V_R, d pstiff [n] (NULL: 0) -> out [n][5]
+ *   AEROFX_PHYS_RECONSTRUCT  the reconstruction of the edge pass, scalar = beta:
+ *                            arguments and result as VANALBADA
+ *   AEROFX_PHYS_ROE_JAC_PAIR the edge blocks of the Jacobian, scalar = gamma: a normal
+ *                            outward from n, b V_n, c V_m, d pstiff [n] (NULL: 0)
+ *                            -> out [n][50] (dF/dU_n, dF/dU_m, row-major)
  * Returns the number of singular blocks (inversions), 0, or < 0. */
 #define AEROFX_PHYS_ROEFLUX7 0
 #define AEROFX_PHYS_BOUNDFLUX5 1
@@ -639,6 +649,9 @@ int aerofx_solution_read(const char *path, int step, double *tag, int n, int dim
 #define AEROFX_PHYS_ROEFLUX5 7
 #define AEROFX_PHYS_ROEJAC6_LM_SW1 8
 #define AEROFX_PHYS_ROEJAC6_LM_SW2 9
+#define AEROFX_PHYS_ROE_FLUX 10
+#define AEROFX_PHYS_RECONSTRUCT 11
+#define AEROFX_PHYS_ROE_JAC_PAIR 12
 int aerofx_physics_eval(int kind, int n, double scalar, const double *a, const double *b,
                         const double *c, const double *d, double *out);
 

@@ -1,10 +1,9 @@
 """Nodes with more neighbours than a block holds: a cone of 300 tets around
 its axis (the apex and the base centre have 301 neighbours, more than the
-256 entries of an H1 / Jacobian block, and 301 and 300 upper edges, more
-than the 128 edges of a flux block), numbered with the two hubs in the
-middle of the node order.  Long rows go to the long-row kernels (Jacobian,
-H1 and its transpose) and are cut over several flux blocks (their flux sum
-is formed by the node pass); results match the oracle as on any mesh, the
+256 entries of an H1 / Jacobian block and the 64 of the gradient pass's LDS
+tables), numbered with the two hubs in the middle of the node order.  Long rows
+go to the long-row kernels (Jacobian, H1 and its transpose) and the gradients are
+gathered per entry; results match the oracle as on any mesh, the
 Newton history tracks the oracle's, and the batched direct solve falls back
 to one inner GMRES per right-hand side (the batched H1 apply takes nodes of
 at most 64 neighbours)."""

@@ -1,8 +1,11 @@
-"""The passes at the sizes where their split changes: 64-node slices (one
-short, exact, one over), the meshes on both sides of the adjoint's rules for
-whole rows and streams (1536 and 3072 slices), and rows too long for the tables in LDS (a cone with
+"""The derivative passes at the sizes where their split changes: 64-node slices
+(one node short, exact, two over), meshes on both sides of the adjoint's rules for
+whole rows and streams (1536 and 3072 slices; at first order the adjoint goes by
+entries on all of them), and rows too long for the tables in LDS (a cone with
 two 301-neighbour hubs: the gradient pass gathers per entry, the viscous
-Jacobian runs its kernel per entry).
+Jacobian runs its kernel per entry).  Both directions read the same tables,
+normals and gradients: test_gpu_pass_paths.py holds the residual, which reads
+them too, against the oracle at such sizes.
 
 Tangent and adjoint are the exact derivative of one residual, so <lam, dR> and
 the transposed products differ by rounding alone: each side is a sum of

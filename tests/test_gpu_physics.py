@@ -3,11 +3,13 @@ the reference's own routines (tests/golden/ref_kernels.npz, written from the
 reference's roeflux7.f, boundflux5.f, roejac6.f, RecFcn.h Van Albada and
 DenseMatrixOps.h LINPACK inverse compiled in the build container).
 
-The kernels follow those routines' operation order and are built without
-FMA contraction, with IEEE division and square root, so every case must
-match bit for bit: 400 Roe fluxes, 400 Steger-Warming farfield fluxes,
+The routines evaluated here follow those routines' operation order and are
+built without FMA contraction, with IEEE division and square root, so every
+case must match bit for bit: 400 Roe fluxes, 400 Steger-Warming farfield fluxes,
 400 x 5 Van Albada reconstructions, 2 x 400 Roe Jacobians and 400 LINPACK
-inverses in FP64 and in FP32."""
+inverses in FP64 and in FP32.  Of the Roe flux, the reconstruction and the Roe
+Jacobian the passes evaluate other, shorter statements, equal to rounding:
+test_gpu_flux_routines.py holds those against the same stored outputs."""
 import ctypes as C
 import os
 
