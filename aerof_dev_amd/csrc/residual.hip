@@ -65,6 +65,14 @@ __device__ __forceinline__ void load_x(const DevTables &t, int n, double x[3]) {
   load_il<3>(t.X3, n, x);
 }
 
+// ... from the records
+__device__ __forceinline__ void load_x4(const DevTables &t, int n, double x[3]) {
+  const double4 p = *reinterpret_cast<const double4 *>(t.X4 + 4 * (size_t)n);
+  x[0] = p.x;
+  x[1] = p.y;
+  x[2] = p.z;
+}
+
 __device__ __forceinline__ void load_lsq(const DevTables &t, int n, double L[6]) {
 #pragma unroll
   for (int q = 0; q < 6; ++q) L[q] = t.lsq6[6 * (size_t)n + q];
@@ -92,7 +100,10 @@ __device__ __forceinline__ void lsq_add(const double L[6], const double xm[3], c
   }
 }
 
-// kFromU also writes V (Vout); OUT3: gradients to ddx, ddy, ddz [N][5]
+// kFromU also writes V (Vout); OUT3: gradients to ddx, ddy, ddz [N][5].
+// Each lane walks its own row: of records (U or V [N][5], X4) a gather is one or
+// two lines, and row order and slice order cost the same to index (by slices and
+// with interleaved coordinates the pass took 176 us at 439k nodes, 112 so).
 template <int FROM, bool OUT3>
 __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double *__restrict__ W, Gas gas,
                                                       double *__restrict__ Vout, double *__restrict__ grad,
@@ -102,57 +113,45 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
   if (done && *done) return;
   if (err && blockIdx.x == 0 && threadIdx.x == 0) *err = 0;  // the flux pass follows in stream order
   const int sl = wave_slice(t);
-  if (sl >= t.ns) return;
-  const int lane = lane_id();
-  const int n = sl * kWave + lane;
-  const bool live = n < t.N;
-  const int nn = live ? n : t.N - 1;
+  const int n = sl * kWave + lane_id();
+  if (n >= t.N) return;
   double Vn[5], xn[3];
   {
     double w[5];
-    load_state<FROM>(W, nn, w);
+    load_state<FROM>(W, n, w);
     to_prim<FROM>(w, gas, Vn);
   }
-  if (Vout && live) store_il<5>(Vout, n, Vn);
-  load_x(t, nn, xn);
+  if (Vout) store_il<5>(Vout, n, Vn);
+  load_x4(t, n, xn);
   double L[6], acc[15];
-  load_lsq(t, nn, L);
+  load_lsq(t, n, L);
 #pragma unroll
   for (int q = 0; q < 15; ++q) acc[q] = 0.0;
   // Neighbours in chunks of kGradChunk: the chunk's states and coordinates
   // are requested together and the next chunk's indices are prefetched, so a
   // row costs about one memory latency per chunk.  The sums are still formed
   // one neighbour at a time in ascending order.
-  const int deg = live ? t.rowptr[n + 1] - t.rowptr[n] : 0;
-  const int k0 = t.nb.kptr[sl], kn = t.nb.kptr[sl + 1] - k0;
+  const int e0 = t.rowptr[n], e1 = t.rowptr[n + 1];
   int mi[kGradChunk];
-  auto fetch = [&](int base) {
 #pragma unroll
-    for (int k = 0; k < kGradChunk; ++k) {
-      const bool act = base + k < deg;
-      const int off = base + k < kn ? t.nb.koff[k0 + base + k] : 0;
-      const int rank = lanes_below(act);
-      mi[k] = act ? t.nb.idx[off + rank] : nn;
-    }
-  };
-  if (kn > 0) fetch(0);
-  for (int e = 0; e < kn; e += kGradChunk) {
+  for (int k = 0; k < kGradChunk; ++k) mi[k] = e0 + k < e1 ? t.adj[e0 + k] : n;
+  for (int e = e0; e < e1; e += kGradChunk) {
     double Wm[kGradChunk][5], xm[kGradChunk][3];
 #pragma unroll
     for (int k = 0; k < kGradChunk; ++k) {
       load_state<FROM>(W, mi[k], Wm[k]);
-      load_x(t, mi[k], xm[k]);
+      load_x4(t, mi[k], xm[k]);
     }
-    if (e + kGradChunk < kn) fetch(e + kGradChunk);
+#pragma unroll
+    for (int k = 0; k < kGradChunk; ++k) mi[k] = e + kGradChunk + k < e1 ? t.adj[e + kGradChunk + k] : n;
 #pragma unroll
     for (int k = 0; k < kGradChunk; ++k) {
-      if (e + k >= deg) break;
+      if (e + k >= e1) break;
       double Vm[5];
       to_prim<FROM>(Wm[k], gas, Vm);
       lsq_add(L, xm[k], xn, Vm, Vn, acc);
     }
   }
-  if (!live) return;
   if (!OUT3 && t.fs_mask && t.fs_mask[n]) {
     // DistNodalGrad::limit with failsafe tags (DistNodalGrad.C:1083-1104)
 #pragma unroll
