@@ -1123,10 +1123,11 @@ int launch_adjoint(aerofx_ctx *c, const double *U, const double *lam, double *Ub
   // forward pass: V, gradients (recomputed), R
   if (rc || (rc = launch_residual(c, U, c->adj->R, true))) return rc;
   const int ns = c->tab.ns;
-  if (c->p.second_order && ns >= kAdjStreamSlices)
+  const bool rows = c->p.second_order && row_waves(ns, kAdjRowSlices, c->max_degree);
+  if (rows && ns >= kAdjStreamSlices)
     return Xout ? adjoint_stages<true, true, 2>(c, U, lam, Ub, Xout)
                 : adjoint_stages<true, false, 2>(c, U, lam, Ub, Xout);
-  if (c->p.second_order && ns >= kAdjRowSlices)
+  if (rows)
     return Xout ? adjoint_stages<true, true, 1>(c, U, lam, Ub, Xout)
                 : adjoint_stages<true, false, 1>(c, U, lam, Ub, Xout);
   if (c->p.second_order)

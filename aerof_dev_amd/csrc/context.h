@@ -180,6 +180,17 @@ __device__ __forceinline__ int wave_slice(const DevTables &t) {
   const int nb = (t.ns + kBlock / kWave - 1) / (kBlock / kWave);
   return xcd_chunk(blockIdx.x, nb) * (kBlock / kWave) + (int)(threadIdx.x / kWave);
 }
+// Whole rows of edges per wave (flux and adjoint edge passes): from `from`
+// slices on, unless a node has so many neighbours that the pass waits for the
+// lane that takes its row.  An edge there costs some 1.5 us (flux), 3 us
+// (adjoint).  By rows and by entries, one node of 31 / 47 / 60 neighbours beside
+// 456k nodes: flux and node pass with the gradients 246 / 276 / 311 and 238 / 249
+// / 263 us, (dR/dU)^T 793 / 882 / 960 and 820 / 842 / 868; 47 / 100 / 127 / 200
+// beside 2.1M nodes: 957 / 1014 / 1067 / 1210 and 999 / 989 / 1010 / 1059, 2938 /
+// 3192 / 3382 / 3837 and 3293 / 3337 / 3383 / 3531.
+inline bool row_waves(int ns, int from, int max_degree) {
+  return ns >= from && max_degree <= (ns / 384 > 32 ? ns / 384 : 32);
+}
 inline dim3 slice_grid(int ns) { return dim3((unsigned)((ns + kBlock / kWave - 1) / (kBlock / kWave))); }
 
 // the passes' streamed data of large meshes: past the caches, which then keep

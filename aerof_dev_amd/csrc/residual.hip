@@ -756,7 +756,7 @@ int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, 
   const DevTables &t = c->tab;
   // the staged kernels evaluate ROEFLUX7 only, without the failsafe
   const bool staged = t.ngb > 0 && c->residual_kernels == AEROFX_RESIDUAL_STAGED && !c->fc.low_mach && !c->failsafe;
-  const bool rows = t.ns >= kRowWaveSlices;
+  const bool rows = row_waves(t.ns, kRowWaveSlices, c->max_degree);
   const bool all = staged || rows;  // P formed by the flux pass
   const dim3 ngrid((t.N + kBlock - 1) / kBlock), blk(kBlock);
   if (c->p.second_order) {

@@ -4,7 +4,7 @@ The gradient pass holds the different neighbours of 64 consecutive nodes in LDS:
 512 in the first batch of loads, the rest in a loop, up to 1024 (beyond, or with a
 row of more than 64 neighbours, it gathers per entry); it reads 16 neighbours'
 places at a time.  The meshes here lie on both sides of each limit.  From 6144
-slices of 64 nodes on the flux pass takes whole rows.  The residual is held
+slices of 64 nodes on the flux pass takes whole rows, unless one is too long.  The residual is held
 against the oracle to 1e-12 of each sum's magnitude, as on any mesh."""
 import os
 import sys
@@ -220,3 +220,28 @@ def test_failsafe_by_rows(gpu, large):
     assert ierr == 0 and tags[2].any()
     assert np.abs(R.cpu().numpy() - Rr).max() <= 1e-12 * np.abs(Rr).max()
     op.close()
+
+
+# ---------------------------------------------------------------------------
+# a node of more neighbours than one lane should take beside a large mesh: the
+# edge passes go by entries (a limit of 32 below 12288 slices)
+# ---------------------------------------------------------------------------
+def _beside(m, other):
+    n = m.num_nodes
+    return M.Mesh(np.vstack([m.X, other.X + 5.0]), np.vstack([m.tets, other.tets + n]).astype(np.int32),
+                  np.vstack([m.faces, other.faces + n]).astype(np.int32),
+                  np.concatenate([m.codes, other.codes]).astype(np.int32))
+
+
+@pytest.mark.parametrize("k", [31, 32])
+def test_residual_of_hub_beside_large_mesh(gpu, large, k):
+    m = _beside(large, _cone(k))
+    p = FlowParams(mach=0.5, alpha=0.05)
+    _check_residual(gpu, m, p, init_state(p, m.X, "noise", 0.005, seed=12))
+
+
+@pytest.mark.parametrize("k", [31, 32])
+def test_duality_of_hub_beside_large_mesh(gpu, k):
+    m = _beside(M.kuhn_box(45, 45, 46, jitter=0.15, seed=3), _cone(k))
+    p = FlowParams(mach=0.5, alpha=0.05)
+    _check_duality(gpu, m, p, init_state(p, m.X, "noise", 0.005, seed=12))
