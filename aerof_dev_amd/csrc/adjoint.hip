@@ -29,6 +29,8 @@
 //   6. k_adj_xgather: Xbar_i plus its tet and face slots
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "context.h"
 #include "device_dual.h"
 #include "device_sens.h"
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_mu(DevTables t, const double 
     m[k] = lam[5 * (size_t)n + k] * ic;
     s += m[k] * R[5 * (size_t)n + k];
   }
-  store_il<5>(mu, n, m);
+  store_il<5>(t.sh, mu, n, m);
   cvb[n] = -s;
 }
 
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_mu(DevTables t, const double 
 // 2. per edge
 // ---------------------------------------------------------------------------
 // A boundary-face slot: mu^T d(face flux) / d(V, face normal / 3).
-template <bool WANTX>
+template <bool WANTX, int SH>
 __device__ __forceinline__ void adj_face_slot(const DevTables &t, const double *__restrict__ V,
                                               const double *__restrict__ mu, const FluxConsts &fc,
                                               const int *__restrict__ nfslot, int q, double *__restrict__ FV,
@@ -362,8 +364,8 @@ __device__ __forceinline__ void adj_face_slot(const DevTables &t, const double *
   const int n = t.fnode[q], face = t.fidx[q];
   const int code = t.fcode[face];
   double Vn[5], m[5], nf[3];
-  load_il<5>(V, n, Vn);
-  load_il<5>(mu, n, m);
+  load_il<5>(Lay<SH>(), V, n, Vn);
+  load_il<5>(Lay<SH>(), mu, n, m);
 #pragma unroll
   for (int a = 0; a < 3; ++a) nf[a] = t.fnorm3[3 * (size_t)face + a];
 #pragma unroll 1
@@ -387,7 +389,7 @@ __device__ __forceinline__ void adj_face_slot(const DevTables &t, const double *
 // One edge (i, j) at position pos: e[0..5) = Vbar and e[5..10) = c of each end
 // (Gbar[5a+k] = c_k dx[a]: the sums form the products), dxbar, and nbar to its
 // place.
-template <bool SECOND, bool WANTX, bool NT>
+template <bool SECOND, bool WANTX, bool NT, int SH>
 __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__restrict__ V,
                                          const double *__restrict__ grad, const double *__restrict__ mu,
                                          const FluxConsts &fc, int i, int j, int pos, double *__restrict__ EXn,
@@ -395,21 +397,21 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
   double VL[5], VR[5], dV[5], g[5], di[5], dj[5];
   {
     double mj[5];
-    load_il<5>(mu, i, g);
-    load_il<5>(mu, j, mj);
+    load_il<5>(Lay<SH>(), mu, i, g);
+    load_il<5>(Lay<SH>(), mu, j, mj);
 #pragma unroll
     for (int k = 0; k < 5; ++k) g[k] -= mj[k];
   }
-  load_il<5>(V, i, VL);
-  load_il<5>(V, j, VR);
+  load_il<5>(Lay<SH>(), V, i, VL);
+  load_il<5>(Lay<SH>(), V, j, VR);
   if (SECOND) {
     double xi[3], dx[3], gi[15], gj[15];
-    load_il<3>(t.X3, i, xi);
-    load_il<3>(t.X3, j, dx);
+    load_il<3>(Lay<SH>(), t.X3, i, xi);
+    load_il<3>(Lay<SH>(), t.X3, j, dx);
 #pragma unroll
     for (int a = 0; a < 3; ++a) dx[a] -= xi[a];
-    load_il<15>(grad, i, gi);
-    load_il<15>(grad, j, gj);
+    load_il<15>(Lay<SH>(), grad, i, gi);
+    load_il<15>(Lay<SH>(), grad, j, gj);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       di[k] = dx[0] * gi[k] + dx[1] * gi[5 + k] + dx[2] * gi[10 + k];
@@ -420,12 +422,12 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
     }
   }
   double nv[3], fb[13];
-  stream_load<3, NT>(t.pnormal, pos, nv);
+  stream_load<3, NT>(Lay<SH>(), t.pnormal, pos, nv);
 #pragma unroll
   for (int d = 0; d < 13; ++d) fb[d] = 0.0;
   if (!(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2] < 1e-36))
     roeflux7_vjp(fc.gas, nv, VL, VR, g, fb, fb + 5, fb + 10);
-  if (WANTX) stream_store<3, NT>(EXn, pos, fb + 10);
+  if (WANTX) stream_store<3, NT>(Lay<SH>(), EXn, pos, fb + 10);
   if (!SECOND) {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -456,12 +458,12 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
     double h[15];
 #pragma unroll
     for (int a = 0; a < 3; ++a) dxb[a] = 0.0;
-    load_il<15>(g2, i, h);
+    load_il<15>(Lay<SH>(), g2, i, h);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
       for (int k = 0; k < 5; ++k) dxb[a] += ei[5 + k] * h[5 * a + k];
-    load_il<15>(g2, j, h);
+    load_il<15>(Lay<SH>(), g2, j, h);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -479,7 +481,7 @@ __device__ __forceinline__ void adj_edge(const DevTables &t, const double *__res
 // after the flux for dxbar rather than held across it.  ROWS 2: streams past the
 // caches, which keep the gathered node data (815k nodes, 5.6M edges: 1013 -> 530
 // us, 619 by entries, 568 by rows; the node pass 342 -> 241; 5 TB/s counted).
-template <bool SECOND, bool WANTX, int ROWS>
+template <bool SECOND, bool WANTX, int ROWS, int SH>
 __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_edges(
     DevTables t, int nfb, const double *__restrict__ V, const double *__restrict__ grad,
     const double *__restrict__ mu, FluxConsts fc, const int *__restrict__ nfslot, double *__restrict__ EVi,
@@ -488,27 +490,25 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
   constexpr int W = SECOND ? 10 : 5;
   if ((int)blockIdx.x < nfb) {
     const int q = blockIdx.x * kAdjBlock + threadIdx.x;
-    if (q < 3 * t.F) adj_face_slot<WANTX>(t, V, mu, fc, nfslot, q, FV, FN);
+    if (q < 3 * t.F) adj_face_slot<WANTX, SH>(t, V, mu, fc, nfslot, q, FV, FN);
     return;
   }
   const int nw = ROWS ? t.ns : t.nup;
   const int nb = (nw + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
   const int w = xcd_chunk(blockIdx.x - nfb, nb) * (kAdjBlock / kWave) + (int)(threadIdx.x / kWave);
   if (w >= nw) return;
-  const int sl = ROWS ? w : t.upslice[w];
-  const int kb = t.up.kptr[sl], i = sl * kWave + lane_id();
-  const int deg = i < t.N ? t.eup[i + 1] - t.eup[i] : 0;
   double ei[10], ej[10], dxb[3];
   if (!ROWS) {
-    const bool act = w - kb < deg;
-    const int pos = t.up.koff[w] + lanes_below(act);
-    if (!act) return;
-    adj_edge<SECOND, WANTX, false>(t, V, grad, mu, fc, i, t.up.idx[pos], pos, EXn, ei, ej, dxb);
-    store_il<W>(EVi, pos, ei);
-    store_il<W>(EVj, pos, ej);
-    if (SECOND && WANTX) store_il<3>(EXd, pos, dxb);
+    const UpperEntry u = upper_entry<SH>(t, w);
+    if (!u.act) return;
+    adj_edge<SECOND, WANTX, false, SH>(t, V, grad, mu, fc, u.i, t.up.idx[u.pos], u.pos, EXn, ei, ej, dxb);
+    store_il<W>(Lay<SH>(), EVi, u.pos, ei);
+    store_il<W>(Lay<SH>(), EVj, u.pos, ej);
+    if (SECOND && WANTX) store_il<3>(Lay<SH>(), EXd, u.pos, dxb);
     return;
   }
+  const int sl = w, kb = t.up.kptr[sl], i = sl * kWave + lane_id();
+  const int deg = i < t.N ? t.eup[i + 1] - t.eup[i] : 0;
   __shared__ double sums[kAdjBlock / kWave][23][kWave];
   double(*sum)[kWave] = sums[threadIdx.x / kWave];
   const int lane = lane_id(), ke = t.up.kptr[sl + 1];
@@ -521,15 +521,15 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
     int own = i;
     asm volatile("" : "+v"(own));  // the own side is read anew for each edge
     const int j = t.up.idx[pos];
-    adj_edge<SECOND, WANTX, ROWS == 2>(t, V, grad, mu, fc, own, j, pos, EXn, ei, ej, dxb);
-    stream_store<W, ROWS == 2>(EVj, pos, ej);
+    adj_edge<SECOND, WANTX, ROWS == 2, SH>(t, V, grad, mu, fc, own, j, pos, EXn, ei, ej, dxb);
+    stream_store<W, ROWS == 2>(Lay<SH>(), EVj, pos, ej);
 #pragma unroll
     for (int q = 0; q < 5; ++q) sum[q][lane] += ei[q];
     const double *X = t.X3;
     asm volatile("" : "+s"(X));
     double x[3], dx[3];
-    load_il<3>(X, own, x);
-    load_il<3>(X, j, dx);
+    load_il<3>(Lay<SH>(), X, own, x);
+    load_il<3>(Lay<SH>(), X, j, dx);
 #pragma unroll
     for (int a = 0; a < 3; ++a) dx[a] -= x[a];
 #pragma unroll
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma unroll
       for (int q = 0; q < 5; ++q) sum[5 + 5 * a + q][lane] += ei[5 + q] * dx[a];
     if (WANTX) {
-      stream_store<3, ROWS == 2>(EXd, pos, dxb);
+      stream_store<3, ROWS == 2>(Lay<SH>(), EXd, pos, dxb);
 #pragma unroll
       for (int a = 0; a < 3; ++a) sum[20 + a][lane] -= dxb[a];
     }
@@ -546,14 +546,14 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2)
   double o[15];
 #pragma unroll
   for (int q = 0; q < 5; ++q) o[q] = sum[q][lane];
-  store_il<5>(Vb, i, o);
+  store_il<5>(Lay<SH>(), Vb, i, o);
 #pragma unroll
   for (int q = 0; q < 15; ++q) o[q] = sum[5 + q][lane];
-  store_il<15>(Gb, i, o);
+  store_il<15>(Lay<SH>(), Gb, i, o);
   if (WANTX) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) o[a] = sum[20 + a][lane];
-    store_il<3>(Xb, i, o);
+    store_il<3>(Lay<SH>(), Xb, i, o);
   }
 }
 
@@ -578,7 +578,7 @@ __device__ __forceinline__ void add_slot(const double *ev, const double dx[3], d
 // gathered, and both ends' coordinates follow from the adjacency
 // rows, whose first entries are the lower neighbours.  Bound by the slots' bytes
 // (624 -> 241 us at 815k nodes, 342 with both ends' slots).
-template <bool SECOND, bool WANTX, bool ROWS>
+template <bool SECOND, bool WANTX, bool ROWS, int SH>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const double *__restrict__ grad,
                                                          const double *__restrict__ EVi,
                                                          const double *__restrict__ EVj,
@@ -594,11 +594,11 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
   double vb[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, gb[15], xb[3] = {0.0, 0.0, 0.0}, xn[3] = {0.0, 0.0, 0.0};
 #pragma unroll
   for (int q = 0; q < 15; ++q) gb[q] = 0.0;
-  if (SECOND) load_il<3>(t.X3, min(n, t.N - 1), xn);
+  if (SECOND) load_il<3>(Lay<SH>(), t.X3, min(n, t.N - 1), xn);
   if (ROWS && live) {
-    load_il<5>(Vb, n, vb);
-    load_il<15>(H, n, gb);
-    if (WANTX) load_il<3>(Xb, n, xb);
+    load_il<5>(Lay<SH>(), Vb, n, vb);
+    load_il<15>(Lay<SH>(), H, n, gb);
+    if (WANTX) load_il<3>(Lay<SH>(), Xb, n, xb);
   }
   // edges (m, n), m < n: the j-side slots
   {
@@ -610,14 +610,14 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
       if (!act) continue;
       const int pos = t.lo.idx[q];
       double ev[W], dx[3] = {0.0, 0.0, 0.0}, d[3];
-      load_il<W>(EVj, pos, ev);
+      load_il<W>(Lay<SH>(), EVj, pos, ev);
       if (SECOND) {
-        load_il<3>(t.X3, t.nb.idx[e], dx);
+        load_il<3>(Lay<SH>(), t.X3, t.nb.idx[e], dx);
 #pragma unroll
         for (int a = 0; a < 3; ++a) dx[a] = xn[a] - dx[a];
       }
       if (SECOND && WANTX) {
-        load_il<3>(EXd, pos, d);
+        load_il<3>(Lay<SH>(), EXd, pos, d);
 #pragma unroll
         for (int a = 0; a < 3; ++a) xb[a] += d[a];
       }
@@ -633,14 +633,14 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
       const int pos = t.up.koff[kb + k] + lanes_below(act);
       if (!act) continue;
       double ev[W], dx[3] = {0.0, 0.0, 0.0}, d[3];
-      load_il<W>(EVi, pos, ev);
+      load_il<W>(Lay<SH>(), EVi, pos, ev);
       if (SECOND) {
-        load_il<3>(t.X3, t.up.idx[pos], dx);
+        load_il<3>(Lay<SH>(), t.X3, t.up.idx[pos], dx);
 #pragma unroll
         for (int a = 0; a < 3; ++a) dx[a] -= xn[a];
       }
       if (SECOND && WANTX) {
-        load_il<3>(EXd, pos, d);
+        load_il<3>(Lay<SH>(), EXd, pos, d);
 #pragma unroll
         for (int a = 0; a < 3; ++a) xb[a] -= d[a];
       }
@@ -651,8 +651,8 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
   for (int q = t.frow[n]; q < t.frow[n + 1]; ++q)
 #pragma unroll
     for (int k = 0; k < 5; ++k) vb[k] += FV[5 * (size_t)q + k];
-  store_il<5>(Vb, n, vb);
-  if (WANTX) store_il<3>(Xb, n, xb);
+  store_il<5>(Lay<SH>(), Vb, n, vb);
+  if (WANTX) store_il<3>(Lay<SH>(), Xb, n, xb);
   if (!SECOND) return;
   double L[6];
 #pragma unroll
@@ -664,10 +664,10 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
 #pragma unroll
     for (int a = 0; a < 3; ++a) gb[5 * a + k] = w[a];
   }
-  store_il<15>(H, n, gb);
+  store_il<15>(Lay<SH>(), H, n, gb);
   if (WANTX) {
     double gn[15], s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    load_il<15>(grad, n, gn);
+    load_il<15>(Lay<SH>(), grad, n, gn);
     int e = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a)
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
       for (int b = a; b < 3; ++b, ++e)
 #pragma unroll
         for (int k = 0; k < 5; ++k) s[e] -= gb[5 * a + k] * gn[5 * b + k] + gb[5 * b + k] * gn[5 * a + k];
-    store_il<6>(S, n, s);
+    store_il<6>(Lay<SH>(), S, n, s);
   }
 }
 
@@ -684,7 +684,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_nodes(DevTables t, const doub
 // ---------------------------------------------------------------------------
 // Bound by the gathers of H, S, V and X (29 values an entry, where the weights of
 // both ends were formed per entry from their factors; 376 -> 229 us at 815k nodes).
-template <bool SECOND, bool WANTX>
+template <bool SECOND, bool WANTX, int SH>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double *__restrict__ V,
                                                        const double *__restrict__ U, Gas gas,
                                                        const double *__restrict__ Vb, const double *__restrict__ H,
@@ -696,12 +696,12 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double
   const bool live = n < t.N;
   const int nn = min(n, t.N - 1);
   double vb[5], Vn[5], xb[3] = {0.0, 0.0, 0.0};
-  load_il<5>(Vb, nn, vb);
-  load_il<5>(V, nn, Vn);
+  load_il<5>(Lay<SH>(), Vb, nn, vb);
+  load_il<5>(Lay<SH>(), V, nn, Vn);
   if (SECOND) {
     // sum over j of dx and of V_j - V_i: what the node's own H and S multiply
     double xn[3], sx[3] = {0.0, 0.0, 0.0}, sv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    load_il<3>(t.X3, nn, xn);
+    load_il<3>(Lay<SH>(), t.X3, nn, xn);
     const int deg = live ? t.rowptr[n + 1] - t.rowptr[n] : 0;
     const int kb = t.nb.kptr[sl], ke = t.nb.kptr[sl + 1];
     auto add = [&](const double h[15], const double s[6], const double dx[3], const double dV[5]) {
@@ -723,11 +723,11 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double
       if (!act) continue;
       const int m = t.nb.idx[pos];
       double h[15], s[6], dx[3], dV[5];
-      load_il<3>(t.X3, m, dx);
-      load_il<15>(H, m, h);
+      load_il<3>(Lay<SH>(), t.X3, m, dx);
+      load_il<15>(Lay<SH>(), H, m, h);
       if (WANTX) {
-        load_il<5>(V, m, dV);
-        load_il<6>(S, m, s);
+        load_il<5>(Lay<SH>(), V, m, dV);
+        load_il<6>(Lay<SH>(), S, m, s);
 #pragma unroll
         for (int q = 0; q < 5; ++q) {
           dV[q] -= Vn[q];
@@ -742,17 +742,17 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_lsq(DevTables t, const double
       add(h, s, dx, dV);
     }
     double h[15], s[6];
-    load_il<15>(H, nn, h);
-    if (WANTX) load_il<6>(S, nn, s);
+    load_il<15>(Lay<SH>(), H, nn, h);
+    if (WANTX) load_il<6>(Lay<SH>(), S, nn, s);
     add(h, s, sx, sv);
   }
   if (!live) return;
   if (WANTX) {
     double x[3];
-    load_il<3>(Xb, n, x);
+    load_il<3>(Lay<SH>(), Xb, n, x);
 #pragma unroll
     for (int a = 0; a < 3; ++a) x[a] += xb[a];
-    store_il<3>(Xb, n, x);
+    store_il<3>(Lay<SH>(), Xb, n, x);
   }
   if (Ub) {
     // V = (rho, u / rho, (gam - 1) (E - rho |u|^2 / 2) - gam pstiff)
@@ -794,6 +794,7 @@ __device__ __forceinline__ void add_cross(double s, const double x[3], const dou
 // before, and 282 us with each lane storing its own 96 bytes: the vector cache
 // takes a store of 64 scattered pieces one piece at a time, so they go out
 // through LDS as whole lines).
+template <int SH>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_tets(int T, const int4 *__restrict__ tets,
                                                         const int *__restrict__ tpos,
                                                         const double *__restrict__ X4,
@@ -841,7 +842,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_tets(int T, const int4 *__res
   for (int e = 0; e < 6; ++e) {
     const int a = kEnd[e][0], b = kEnd[e][1], c = kOpp[e][0], d = kOpp[e][1];
     double w[3], p[3], r[3], gp[3] = {0.0, 0.0, 0.0}, gr[3] = {0.0, 0.0, 0.0};
-    load_il<3>(EXn, ps[e], w);
+    load_il<3>(Lay<SH>(), EXn, ps[e], w);
     const double s = nd[a] < nd[b] ? 1.0 / 24.0 : -1.0 / 24.0;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -908,8 +909,6 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_faces(int F, const int *__res
 // ---------------------------------------------------------------------------
 // 6. per node: Xbar
 // ---------------------------------------------------------------------------
-typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte access at 8-byte alignment
-
 // Four lanes per node, each every fourth slot: the slot lists are read in whole
 // lines and four gathers per node are in flight (688 -> 215 us at 815k nodes, with
 // the neighbours' S moved to the pass that reads them anyway).
@@ -944,7 +943,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_xgather(DevTables t, const do
     xb[a] += __shfl_xor(xb[a], 1);
     xb[a] += __shfl_xor(xb[a], 2);
   }
-  if (n < t.N && r < 3) out[3 * (size_t)n + r] = Xb[il<3>(n, r)] + (r == 0 ? xb[0] : (r == 1 ? xb[1] : xb[2]));
+  if (n < t.N && r < 3) out[3 * (size_t)n + r] = Xb[il<3>(t.sh, n, r)] + (r == 0 ? xb[0] : (r == 1 ? xb[1] : xb[2]));
 }
 
 // edge id -> position, and the tets' edge ids to positions
@@ -1001,12 +1000,12 @@ int ensure_adjoint(aerofx_ctx *c) {
   a->ntslot = el.ntslot;
   a->nfslot = el.nfslot;
   const size_t F1 = std::max(F, 1);
-  if ((rc = alloc_n(c, il_count<10>(E), &a->EVi)) || (rc = alloc_n(c, il_count<10>(E), &a->EVj)) ||
-      (rc = alloc_n(c, il_count<3>(E), &a->EXd)) || (rc = alloc_n(c, il_count<3>(E), &a->EXn)) ||
+  if ((rc = alloc_n(c, il_count<10>(c->tab.sh, E), &a->EVi)) || (rc = alloc_n(c, il_count<10>(c->tab.sh, E), &a->EVj)) ||
+      (rc = alloc_n(c, il_count<3>(c->tab.sh, E), &a->EXd)) || (rc = alloc_n(c, il_count<3>(c->tab.sh, E), &a->EXn)) ||
       (rc = alloc_n(c, 15 * F1, &a->FV)) || (rc = alloc_n(c, 9 * F1, &a->FN)) ||
-      (rc = alloc_n(c, il_count<5>(N), &a->mu)) || (rc = alloc_n(c, (size_t)N, &a->cvb)) ||
-      (rc = alloc_n(c, il_count<5>(N), &a->Vb)) || (rc = alloc_n(c, il_count<15>(N), &a->H)) ||
-      (rc = alloc_n(c, il_count<3>(N), &a->Xb)) || (rc = alloc_n(c, il_count<6>(N), &a->S)) ||
+      (rc = alloc_n(c, il_count<5>(c->tab.sh, N), &a->mu)) || (rc = alloc_n(c, (size_t)N, &a->cvb)) ||
+      (rc = alloc_n(c, il_count<5>(c->tab.sh, N), &a->Vb)) || (rc = alloc_n(c, il_count<15>(c->tab.sh, N), &a->H)) ||
+      (rc = alloc_n(c, il_count<3>(c->tab.sh, N), &a->Xb)) || (rc = alloc_n(c, il_count<6>(c->tab.sh, N), &a->S)) ||
       (rc = alloc_n(c, 5 * (size_t)N, &a->R)) || (rc = alloc_n(c, 12 * (size_t)std::max(T, 1), &a->TX)) ||
       (rc = alloc_n(c, 9 * F1, &a->FX)) || (rc = alloc_n(c, (size_t)F + 1, &a->Jf)) ||
       (rc = upload_vec(c, c->tet_edges, &a->tpos))) {
@@ -1078,7 +1077,7 @@ int ensure_elem_tables(aerofx_ctx *c) {
 // for the 1024 SIMDs, and then the edge data still fit the caches.
 constexpr int kAdjRowSlices = 1536, kAdjStreamSlices = 3072;
 
-template <bool SECOND, bool WANTX, int ROWS>
+template <bool SECOND, bool WANTX, int ROWS, int SH>
 static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, double *Ub, double *Xout) {
   Adjoint *a = c->adj;
   const DevTables &t = c->tab;
@@ -1089,14 +1088,14 @@ static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, dou
   const int nfb = (3 * t.F + kAdjBlock - 1) / kAdjBlock;
   const int nb = ((ROWS ? t.ns : t.nup) + kAdjBlock / kWave - 1) / (kAdjBlock / kWave);
   if (nfb + nb)
-    hipLaunchKernelGGL((k_adj_edges<SECOND, WANTX, ROWS>), dim3((unsigned)(nfb + nb)), b, 0, c->stream, t, nfb, c->d_V,
+    hipLaunchKernelGGL((k_adj_edges<SECOND, WANTX, ROWS, SH>), dim3((unsigned)(nfb + nb)), b, 0, c->stream, t, nfb, c->d_V,
                        c->d_grad, a->mu, c->fc, a->nfslot, a->EVi, a->EVj, a->EXd, a->EXn, a->FV, a->FN,
                        a->Vb, a->H, a->Xb);
   // 3.
-  hipLaunchKernelGGL((k_adj_nodes<SECOND, WANTX, ROWS != 0>), slice_grid(t.ns), b, 0, c->stream, t, c->d_grad, a->EVi, a->EVj,
+  hipLaunchKernelGGL((k_adj_nodes<SECOND, WANTX, ROWS != 0, SH>), slice_grid(t.ns), b, 0, c->stream, t, c->d_grad, a->EVi, a->EVj,
                      a->EXd, a->FV, a->Vb, a->H, a->S, a->Xb);
   // 4.
-  hipLaunchKernelGGL((k_adj_lsq<SECOND, WANTX>), slice_grid(t.ns), b, 0, c->stream, t, c->d_V, U, c->gas, a->Vb, a->H,
+  hipLaunchKernelGGL((k_adj_lsq<SECOND, WANTX, SH>), slice_grid(t.ns), b, 0, c->stream, t, c->d_V, U, c->gas, a->Vb, a->H,
                      a->S, Ub, a->Xb);
   int rc;
   // the Navier-Stokes Galerkin term (its element derivative, transposed)
@@ -1104,7 +1103,7 @@ static int adjoint_stages(aerofx_ctx *c, const double *U, const double *lam, dou
   if (WANTX) {
     // 5.
     if (c->T > 0)
-      hipLaunchKernelGGL(k_adj_tets, grid_for(c->T), b, 0, c->stream, c->T, (const int4 *)a->tets, a->tpos, t.X4,
+      hipLaunchKernelGGL(k_adj_tets<SH>, grid_for(c->T), b, 0, c->stream, c->T, (const int4 *)a->tets, a->tpos, t.X4,
                          a->cvb, a->EXn, a->TX);
     // the Navier-Stokes Galerkin term's coordinate derivative, per element
     if (c->T > 0 && (rc = launch_visc_adjoint_x(c, lam, a->TX))) return rc;
@@ -1122,19 +1121,19 @@ int launch_adjoint(aerofx_ctx *c, const double *U, const double *lam, double *Ub
   int rc = ensure_adjoint(c);
   // forward pass: V, gradients (recomputed), R
   if (rc || (rc = launch_residual(c, U, c->adj->R, true))) return rc;
-  const int ns = c->tab.ns;
-  const bool rows = c->p.second_order && row_waves(ns, kAdjRowSlices, c->max_degree);
-  if (rows && ns >= kAdjStreamSlices)
-    return Xout ? adjoint_stages<true, true, 2>(c, U, lam, Ub, Xout)
-                : adjoint_stages<true, false, 2>(c, U, lam, Ub, Xout);
-  if (rows)
-    return Xout ? adjoint_stages<true, true, 1>(c, U, lam, Ub, Xout)
-                : adjoint_stages<true, false, 1>(c, U, lam, Ub, Xout);
-  if (c->p.second_order)
-    return Xout ? adjoint_stages<true, true, 0>(c, U, lam, Ub, Xout)
-                : adjoint_stages<true, false, 0>(c, U, lam, Ub, Xout);
-  return Xout ? adjoint_stages<false, true, 0>(c, U, lam, Ub, Xout)
-              : adjoint_stages<false, false, 0>(c, U, lam, Ub, Xout);
+  const DevTables &t = c->tab;
+  const bool second = c->p.second_order != 0, rows = second && t.sh && row_waves(t.ns, kAdjRowSlices, c->max_degree);
+  auto stages = [&](auto wantx) {
+    constexpr bool X = decltype(wantx)::value;
+    const auto f = rows && t.ns >= kAdjStreamSlices ? adjoint_stages<true, X, 2, kGroupShift>
+                   : rows                           ? adjoint_stages<true, X, 1, kGroupShift>
+                   : second && t.sh                 ? adjoint_stages<true, X, 0, kGroupShift>
+                   : second                         ? adjoint_stages<true, X, 0, 0>
+                   : t.sh                           ? adjoint_stages<false, X, 0, kGroupShift>
+                                                    : adjoint_stages<false, X, 0, 0>;
+    return f(c, U, lam, Ub, Xout);
+  };
+  return Xout ? stages(std::true_type()) : stages(std::false_type());
 }
 
 // ---------------------------------------------------------------------------
@@ -1143,7 +1142,7 @@ int launch_adjoint(aerofx_ctx *c, const double *U, const double *lam, double *Ub
 // pressure force on the wall projected on d)
 // ---------------------------------------------------------------------------
 // per face: J_f, and the coordinate derivative of J_f (9 slots)
-__global__ __launch_bounds__(kAdjBlock) void k_lift_faces(int F, const int *__restrict__ faces,
+__global__ __launch_bounds__(kAdjBlock) void k_lift_faces(int F, int sh, const int *__restrict__ faces,
                                                           const int *__restrict__ fcode,
                                                           const double *__restrict__ fnorm3,
                                                           const double *__restrict__ X4,
@@ -1159,7 +1158,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_lift_faces(int F, const int *__re
 #pragma unroll
   for (int v = 0; v < 3; ++v) {
     nd[v] = faces[3 * (size_t)f + v];
-    psum += V[il<5>(nd[v], 4)];
+    psum += V[il<5>(sh, nd[v], 4)];
   }
   if (!wall) psum = 0.0;
   const double *nv = fnorm3 + 3 * (size_t)f;
@@ -1272,7 +1271,7 @@ extern "C" int aerofx_wall_force(aerofx_ctx *ctx, const double *U, const double 
   const DevTables &t = ctx->tab;
   if ((rc = launch_primitive_il(ctx, U))) return rc;
   if (ctx->F > 0) {
-    hipLaunchKernelGGL(k_lift_faces, grid_for(ctx->F), dim3(kAdjBlock), 0, ctx->stream, ctx->F, a->faces, t.fcode,
+    hipLaunchKernelGGL(k_lift_faces, grid_for(ctx->F), dim3(kAdjBlock), 0, ctx->stream, ctx->F, t.sh, a->faces, t.fcode,
                        t.fnorm3, t.X4, ctx->d_V, dir[0], dir[1], dir[2], a->Jf, dJdX ? a->FX : nullptr);
     // the viscous stress on the wall faces (PostFcnNS::computeForce)
     if ((rc = launch_visc_force(ctx, dir, a->Jf, dJdU || dJdX))) return rc;

@@ -60,17 +60,61 @@ inline size_t blk64_count(size_t nblocks) { return (nblocks + 63) / 64 * 64 * 25
 // accesses per load and wave, which took 85 % of the flux pass's clocks; from
 // the planes it takes about 28 over the neighbours of 64 consecutive nodes in
 // RCM order (flux and node pass at 2.1M nodes 864 -> 727 us).
+// The groups have 1 << sh items: 64 (sh = kGroupShift), or one (sh = 0), plain
+// records, 15 and 3 fields padded to whole lines, where the numbering scatters
+// a node's neighbours: the planes of an item that no lane beside reads cost a
+// line each (DevTables::sh).  The passes that gather most are instantiated for
+// either, the others read the shift.
+constexpr int kGroupShift = 6;
+// One layout fixed at compile time (kGroupShift or 0), for the passes that are
+// instantiated for each; where a layout is read from the tables it is the int.
+template <int SH>
+struct Lay {};
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte access at 8-byte alignment
 template <int W>
-__host__ __device__ __forceinline__ size_t il(size_t n, int k) {
-  const size_t g = (n >> 6) * (64 * W), l = n & 63;
-  return k < (W & ~1) ? g + (k >> 1) * 128 + 2 * l + (k & 1) : g + (W - 1) * 64 + l;
+constexpr int record_size() {
+  return W == 15 ? 16 : (W == 3 ? 4 : W);
 }
 template <int W>
-inline size_t il_count(size_t n) {
-  return (n + 63) / 64 * 64 * W;
+__host__ __device__ __forceinline__ size_t il_group(int sh, size_t n) {
+  return (n >> sh) * (sh ? 64 * W : record_size<W>());
 }
 template <int W>
-__device__ __forceinline__ void load_il(const double *__restrict__ p, int n, double v[W]) {
+__host__ __device__ __forceinline__ size_t il(int sh, size_t n, int k) {
+  const size_t g = il_group<W>(sh, n), l = n & ((1u << sh) - 1);
+  return k < (W & ~1) ? g + ((size_t)(k >> 1) << (sh + 1)) + 2 * l + (k & 1) : g + ((size_t)(W - 1) << sh) + l;
+}
+template <int W>
+inline size_t il_count(int sh, size_t n) {
+  return sh ? (n + 63) / 64 * 64 * W : n * record_size<W>();
+}
+template <int W>
+__device__ __forceinline__ void load_il(int sh, const double *__restrict__ p, int n, double v[W]) {
+  const double *q = p + il_group<W>(sh, n);
+  const int l = n & ((1 << sh) - 1);
+#pragma unroll
+  for (int k = 0; k < W / 2; ++k) {
+    const double2u a = *reinterpret_cast<const double2u *>(q + (k << (sh + 1)) + 2 * l);
+    v[2 * k] = a.x;
+    v[2 * k + 1] = a.y;
+  }
+  if (W & 1) v[W - 1] = q[((W - 1) << sh) + l];
+}
+template <int W>
+__device__ __forceinline__ void store_il(int sh, double *__restrict__ p, int n, const double v[W]) {
+  double *q = p + il_group<W>(sh, n);
+  const int l = n & ((1 << sh) - 1);
+#pragma unroll
+  for (int k = 0; k < W / 2; ++k) {
+    const double2u a = {v[2 * k], v[2 * k + 1]};
+    *reinterpret_cast<double2u *>(q + (k << (sh + 1)) + 2 * l) = a;
+  }
+  if (W & 1) q[((W - 1) << sh) + l] = v[W - 1];
+}
+
+template <int W, int SH>
+__device__ __forceinline__ void load_il(Lay<SH>, const double *__restrict__ p, int n, double v[W]) {
+  if constexpr (SH == 0) return load_il<W>(0, p, n, v);
   const double *q = p + ((size_t)n >> 6) * (64 * W);
   const int l = n & 63;
 #pragma unroll
@@ -81,8 +125,9 @@ __device__ __forceinline__ void load_il(const double *__restrict__ p, int n, dou
   }
   if (W & 1) v[W - 1] = q[(W - 1) * 64 + l];
 }
-template <int W>
-__device__ __forceinline__ void store_il(double *__restrict__ p, int n, const double v[W]) {
+template <int W, int SH>
+__device__ __forceinline__ void store_il(Lay<SH>, double *__restrict__ p, int n, const double v[W]) {
+  if constexpr (SH == 0) return store_il<W>(0, p, n, v);
   double *q = p + ((size_t)n >> 6) * (64 * W);
   const int l = n & 63;
 #pragma unroll
@@ -114,6 +159,7 @@ constexpr int kHaloRow = 64;  // bounds the padding of the places
 struct DevTables {
   int N, E, F;
   int ns;                // 64-node slices
+  int sh;                // group size of the interleaved arrays, 1 << sh items
   const double *X4;      // [N][4] coordinates padded to 32 B
   const double *X3;      // il<3>: coordinates
   const int *fs_mask;    // [N] failsafe first-order nodes (gradients zeroed), or null
@@ -142,8 +188,9 @@ struct DevTables {
   int halo_cap, halo_pairs;
   const int *halo;
   const uint32_t *hloc;
-  int nup;               // (slice, k) pairs of up
-  const int *upslice;    // [nup] their slices
+  int nup;               // waves of the passes by entries: (slice, k) pairs of up, or with records 64 edges each
+  const int *upslice;    // [nup] the pairs' slices (with records null)
+  const int *uprow;      // [E] row of each position (with records, else null)
   const int *pedge;      // [E] edge id at each position
   const double *pnormal; // il<3> over positions: dual-face area vectors
   const int *eup;        // [N+1] first edge whose lower node is i
@@ -191,6 +238,31 @@ __device__ __forceinline__ int wave_slice(const DevTables &t) {
 inline bool row_waves(int ns, int from, int max_degree) {
   return ns >= from && max_degree <= (ns / 384 > 32 ? ns / 384 : 32);
 }
+// The edge of this lane in wave w of a pass by entries (t.nup waves): row, place
+// in the edge storage and whether there is one.  A wave takes the k-th upper edges
+// of a slice; with records (SH = 0) 64 consecutive places, since a scattered
+// numbering leaves half of a slice's k-th places empty (its nodes have from 0 to
+// all neighbours above them).
+struct UpperEntry {
+  int i = 0, pos = 0;
+  bool act = false;
+};
+template <int SH>
+__device__ __forceinline__ UpperEntry upper_entry(const DevTables &t, int w) {
+  UpperEntry u;
+  if (SH == 0) {
+    const int at = w * kWave + lane_id();
+    u.act = at < t.E;
+    u.pos = u.act ? at : t.E - 1;
+    u.i = t.uprow[u.pos];
+  } else {
+    const int sl = t.upslice[w];
+    u.i = sl * kWave + lane_id();
+    u.act = u.i < t.N && w - t.up.kptr[sl] < t.eup[min(u.i, t.N - 1) + 1] - t.eup[min(u.i, t.N - 1)];
+    u.pos = t.up.koff[w] + lanes_below(u.act);
+  }
+  return u;
+}
 inline dim3 slice_grid(int ns) { return dim3((unsigned)((ns + kBlock / kWave - 1) / (kBlock / kWave))); }
 
 // the passes' streamed data of large meshes: past the caches, which then keep
@@ -198,9 +270,10 @@ inline dim3 slice_grid(int ns) { return dim3((unsigned)((ns + kBlock / kWave - 1
 // after it 212 -> 205; at 275k nodes the fluxes would miss the cache instead:
 // 106 -> 109 us)
 typedef double nt_double2 __attribute__((ext_vector_type(2)));
-template <int W, bool NT>
-__device__ __forceinline__ void stream_load(const double *__restrict__ p, int n, double v[W]) {
-  if (!NT) return load_il<W>(p, n, v);
+template <int W, bool NT, int SH>
+__device__ __forceinline__ void stream_load(Lay<SH> lay, const double *__restrict__ p, int n, double v[W]) {
+  static_assert(!NT || SH == kGroupShift, "records share lines between stores");
+  if (!NT) return load_il<W>(lay, p, n, v);
   const double *q = p + ((size_t)n >> 6) * (64 * W);
   const int l = n & 63;
 #pragma unroll
@@ -211,9 +284,10 @@ __device__ __forceinline__ void stream_load(const double *__restrict__ p, int n,
   }
   if (W & 1) v[W - 1] = __builtin_nontemporal_load(q + (W - 1) * 64 + l);
 }
-template <int W, bool NT>
-__device__ __forceinline__ void stream_store(double *__restrict__ p, int n, const double v[W]) {
-  if (!NT) return store_il<W>(p, n, v);
+template <int W, bool NT, int SH>
+__device__ __forceinline__ void stream_store(Lay<SH> lay, double *__restrict__ p, int n, const double v[W]) {
+  static_assert(!NT || SH == kGroupShift, "records share lines between stores");
+  if (!NT) return store_il<W>(lay, p, n, v);
   double *q = p + ((size_t)n >> 6) * (64 * W);
   const int l = n & 63;
 #pragma unroll
@@ -227,8 +301,8 @@ __device__ __forceinline__ void stream_store(double *__restrict__ p, int n, cons
 // s -= (LOWER: edge positions in rows.idx) or += (upper edges: the entries'
 // own places) the fluxes of this lane's row, in row order; four entries'
 // loads in flight together.
-template <bool LOWER>
-__device__ __forceinline__ void add_slots(const RowSlices &rows, int sl, int deg, const double *__restrict__ Fm,
+template <bool LOWER, int SH>
+__device__ __forceinline__ void add_slots(Lay<SH> lay, const RowSlices &rows, int sl, int deg, const double *__restrict__ Fm,
                                           double s[5]) {
   constexpr int B = 4;
   const int kb = rows.kptr[sl], kn = rows.kptr[sl + 1] - kb;
@@ -243,7 +317,7 @@ __device__ __forceinline__ void add_slots(const RowSlices &rows, int sl, int deg
     }
     double v[B][5];
 #pragma unroll
-    for (int u = 0; u < B; ++u) load_il<5>(Fm, pos[u], v[u]);
+    for (int u = 0; u < B; ++u) load_il<5>(lay, Fm, pos[u], v[u]);
 #pragma unroll
     for (int u = 0; u < B; ++u)
       if (k0 + u < deg) {

@@ -239,6 +239,35 @@ int slice_halos(int N, const HostSlices &h, const std::vector<int> &rowptr, int 
   return most;
 }
 
+// Whether the gathers of the passes find less than half of what a line holds:
+// the different groups of eight consecutive nodes (a line of a plane of the
+// interleaved arrays) that the slices' entries name, per entry.  A box, channel
+// or RCM order has 0.04 to 0.07, nodes shuffled within windows of 256 / 1024 /
+// 65536 0.24 / 0.44 / 0.96.  At 1.0M nodes interleaved against records in us,
+// residual 771 / 1028 / 1501 and 756 / 819 / 1011, (dR/dU)^T 2298 / 2906 / 5246
+// and 2302 / 2508 / 2945 (in file order 432 and 629, 1373 and 2013); at 69k
+// nodes within 256 / 1024 65 / 77 and 70 / 75, 204 / 240 and 204 / 216; at 4.9k,
+// all shuffled (0.56), 33 and 35, 135 and 117: below 256 slices there is little
+// between them.
+constexpr double kScatteredLines = 0.25;
+constexpr int kScatteredSlices = 256;
+bool scattered(int N, const HostSlices &h) {
+  const int ns = (int)h.kptr.size() - 1;
+  if (ns < kScatteredSlices) return false;
+  std::vector<int> stamp((size_t)N / 8 + 1, -1);
+  size_t lines = 0;
+  for (int s = 0; s < ns; ++s) {
+    const int e0 = h.kptr[s] < (int)h.koff.size() ? h.koff[h.kptr[s]] : (int)h.idx.size();
+    const int e1 = h.kptr[s + 1] < (int)h.koff.size() ? h.koff[h.kptr[s + 1]] : (int)h.idx.size();
+    for (int e = e0; e < e1; ++e)
+      if (stamp[h.idx[e] / 8] != s) {
+        stamp[h.idx[e] / 8] = s;
+        ++lines;
+      }
+  }
+  return lines > kScatteredLines * h.idx.size();
+}
+
 int upload_slices(aerofx_ctx *c, const HostSlices &h, RowSlices *r) {
   int rc;
   if ((rc = upload(c, h.kptr, &r->kptr)) || (rc = upload(c, h.koff, &r->koff)) ||
@@ -249,22 +278,22 @@ int upload_slices(aerofx_ctx *c, const HostSlices &h, RowSlices *r) {
 
 // interleaved copy of a table of three doubles per item (items taken at
 // perm, or in order), rows of `ld` doubles
-__global__ __launch_bounds__(kBlock) void k_interleave3(int n, const int *__restrict__ perm,
+__global__ __launch_bounds__(kBlock) void k_interleave3(int n, int sh, const int *__restrict__ perm,
                                                         const double *__restrict__ src, int ld,
                                                         double *__restrict__ dst) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   const size_t q = (size_t)(perm ? perm[i] : i) * ld;
 #pragma unroll
-  for (int d = 0; d < 3; ++d) dst[il<3>(i, d)] = src[q + d];
+  for (int d = 0; d < 3; ++d) dst[il<3>(sh, i, d)] = src[q + d];
 }
 
 int interleave3(aerofx_ctx *c, int n, const int *perm, const double *src, int ld, const double **out) {
   void *p = nullptr;
-  int rc = ctx_alloc(c, sizeof(double) * il_count<3>(n), &p);
+  int rc = ctx_alloc(c, sizeof(double) * il_count<3>(c->tab.sh, n), &p);
   if (rc) return rc;
   if (n > 0)
-    hipLaunchKernelGGL(k_interleave3, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, 0, n, perm, src, ld,
+    hipLaunchKernelGGL(k_interleave3, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, 0, n, c->tab.sh, perm, src, ld,
                        static_cast<double *>(p));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_hip_error(e, "interleave launch");
@@ -451,17 +480,16 @@ int aerofx_ctx_create(const aerofx_mesh *m, const aerofx_params *p, aerofx_ctx *
     std::vector<int> halo;
     std::vector<uint32_t> hloc;
     int halo_cap = 0;
+    bool records = false;
     std::future<HostSlices> nb_task = std::async(std::launch::async, [&] {
       HostSlices h = slice_rows(N, rowptr, adj, nullptr);
-      halo_cap = slice_halos(N, h, rowptr, c->max_degree, halo, hloc);
+      records = scattered(N, h);
+      if (!records) halo_cap = slice_halos(N, h, rowptr, c->max_degree, halo, hloc);
       return h;
     });
     const HostSlices hup = slice_rows(N, eup, jcol, &epos);
     for (int q = 0; q < E; ++q) lpos[q] = epos[ledge[q]];
     const HostSlices hlo = slice_rows(N, lrow, lpos, nullptr);
-    std::vector<int> upslice(hup.koff.size());
-    for (int sl = 0; sl + 1 < (int)hup.kptr.size(); ++sl)
-      std::fill(upslice.begin() + hup.kptr[sl], upslice.begin() + hup.kptr[sl + 1], sl);
     std::vector<int> pedge(E);
     for (int l = 0; l < E; ++l) pedge[epos[l]] = l;
     for (int n = 0; n < N; ++n)
@@ -490,6 +518,16 @@ int aerofx_ctx_create(const aerofx_mesh *m, const aerofx_params *p, aerofx_ctx *
     t.N = N;
     t.E = E;
     t.F = F;
+    t.sh = records ? 0 : kGroupShift;
+    std::vector<int> upslice, uprow;
+    if (t.sh) {
+      upslice.resize(hup.koff.size());
+      for (int sl = 0; sl + 1 < (int)hup.kptr.size(); ++sl)
+        std::fill(upslice.begin() + hup.kptr[sl], upslice.begin() + hup.kptr[sl + 1], sl);
+    } else {
+      uprow.resize(E);
+      for (int p = 0; p < E; ++p) uprow[p] = eij[pedge[p]].x;
+    }
     if ((rc = upload(c, X4, &t.X4)) || (rc = upload(c, lsq6, &t.lsq6)) || (rc = upload(c, invcv, &t.invcv)) || (rc = upload(c, c->cv, &t.cv)) ||
         (rc = upload(c, gchunk, &t.gchunk)) || (rc = upload(c, glong, &t.glong)) || (rc = upload(c, rowptr, &t.rowptr)) ||
         (rc = upload(c, adj, &t.adj)) || (rc = upload(c, eid, &t.eidx)) || (rc = upload(c, mirror, &t.mirror)) || (rc = upload(c, eup, &t.eup)) ||
@@ -498,7 +536,7 @@ int aerofx_ctx_create(const aerofx_mesh *m, const aerofx_params *p, aerofx_ctx *
         (rc = upload(c, frow, &t.frow)) || (rc = upload(c, fidx, &t.fidx)) || (rc = upload(c, fcode, &t.fcode)) ||
         (rc = upload(c, fnorm3, &t.fnorm3)) || (rc = upload(c, c->fnorm, &t.fnorm)) ||
         (rc = upload(c, fnode, &t.fnode)) || (rc = upload(c, pedge, &t.pedge)) ||
-        (rc = upload(c, upslice, &t.upslice)) ||
+        (rc = upload(c, upslice, &t.upslice)) || (rc = upload(c, uprow, &t.uprow)) ||
         (halo_cap && ((rc = upload(c, halo, &t.halo)) || (rc = upload(c, hloc, &t.hloc)))) ||
         (rc = upload_slices(c, hup, &t.up)) || (rc = upload_slices(c, hlo, &t.lo)) ||
         (rc = upload_slices(c, hnb, &t.nb)) || (rc = interleave3(c, N, nullptr, t.X4, 4, &t.X3)) ||
@@ -516,11 +554,11 @@ int aerofx_ctx_create(const aerofx_mesh *m, const aerofx_params *p, aerofx_ctx *
     t.ns = (N + 63) / 64;
     t.halo_cap = halo_cap;
     t.halo_pairs = (c->max_degree + 1) / 2;
-    t.nup = (int)hup.koff.size();
+    t.nup = t.sh ? (int)hup.koff.size() : (E + 63) / 64;
     void *pv = nullptr;
-    const std::pair<double **, size_t> bufs[] = {{&c->d_V, il_count<5>(N)},     {&c->d_grad, il_count<15>(N)},
-                                                 {&c->d_Fm, il_count<5>(E)},    {&c->d_P, il_count<5>(N)},
-                                                 {&c->d_Ff, 15 * (size_t)F},    {&c->d_dt, 5 * (size_t)N}};
+    const std::pair<double **, size_t> bufs[] = {{&c->d_V, il_count<5>(t.sh, N)}, {&c->d_grad, il_count<15>(t.sh, N)},
+                                                 {&c->d_Fm, il_count<5>(t.sh, E)}, {&c->d_P, il_count<5>(t.sh, N)},
+                                                 {&c->d_Ff, 15 * (size_t)F},       {&c->d_dt, 5 * (size_t)N}};
     for (const auto &b : bufs) {
       if ((rc = ctx_alloc(c, sizeof(double) * b.second, &pv))) { destroy(c); return rc; }
       *b.first = static_cast<double *>(pv);
@@ -704,9 +742,9 @@ int aerofx_residual_noalloc(aerofx_ctx *c, const double *U, double *R, int flags
   // never more than kNoAllocSlackBytes beyond it
   const size_t need = 2 * align256(5 * sizeof(double) * (size_t)c->N) + align256(16 * sizeof(double) * (size_t)c->N) +
                       align256(5 * sizeof(double) * (size_t)c->E);
-  const size_t oV = 0, oG = align256(sizeof(double) * il_count<5>(c->N));
-  const size_t oP = oG + align256(sizeof(double) * il_count<15>(c->N));
-  const size_t oF = oP + align256(sizeof(double) * il_count<5>(c->N));
+  const size_t oV = 0, oG = align256(sizeof(double) * il_count<5>(c->tab.sh, c->N));
+  const size_t oP = oG + align256(sizeof(double) * il_count<15>(c->tab.sh, c->N));
+  const size_t oF = oP + align256(sizeof(double) * il_count<5>(c->tab.sh, c->N));
   if (need > kNoAllocScratchBytes)
     return set_error(AEROFX_ERR_ARG, "residual_noalloc: the mesh (" + std::to_string(c->N) + " nodes, " +
                                          std::to_string(c->E) + " edges) needs " + std::to_string(need) +

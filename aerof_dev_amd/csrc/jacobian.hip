@@ -49,8 +49,8 @@ __device__ __forceinline__ double timestep_entry(const DevTables &t, const doubl
   const double sg = n < m ? 1.0 : -1.0;
   const double nv[3] = {sg * nl[0], sg * nl[1], sg * nl[2]};
   double Vn[5], Vm[5], Vmid[5];
-  load_il<5>(V, n, Vn);
-  load_il<5>(V, m, Vm);
+  load_il<5>(t.sh, V, n, Vn);
+  load_il<5>(t.sh, V, m, Vm);
 #pragma unroll
   for (int k = 0; k < 5; ++k) Vmid[k] = 0.5 * (Vn[k] + Vm[k]);
   return inflow_speed(g, Vmid, nv);
@@ -65,7 +65,7 @@ __device__ __forceinline__ void timestep_node(const DevTables &t, const double *
   const int q0 = t.frow[n], q1 = t.frow[n + 1];
   if (q0 < q1) {
     double Vn[5];
-    load_il<5>(V, n, Vn);
+    load_il<5>(t.sh, V, n, Vn);
     for (int q = q0; q < q1; ++q) {
       const double *nf = t.fnorm + 3 * (size_t)t.fidx[q];
       const double nv[3] = {nf[0], nf[1], nf[2]};
@@ -153,8 +153,8 @@ __device__ __forceinline__ void jac_entry(const DevTables &t, const double *__re
     return;
   }
   double Vn[5], Vm[5];
-  load_il<5>(V, n, Vn);
-  load_il<5>(V, m, Vm);
+  load_il<5>(t.sh, V, n, Vn);
+  load_il<5>(t.sh, V, m, Vm);
   const double voln = t.invcv[n];
   double length = 1.0;
   if (LM) {
@@ -202,7 +202,7 @@ __device__ __forceinline__ void jac_face(const DevTables &t, const double *__res
   const int code = t.fcode[face];
   const double nv[3] = {t.fnorm3[3 * (size_t)face], t.fnorm3[3 * (size_t)face + 1], t.fnorm3[3 * (size_t)face + 2]};
   double Vn[5], jac[25];
-  load_il<5>(V, n, Vn);
+  load_il<5>(t.sh, V, n, Vn);
   if (is_wall_code(code)) {
     wall_jac(fc.gas, nv, 0.0, Vn, jac);
   } else {

@@ -43,10 +43,10 @@ constexpr int kGradChunk = 8;
 // ---------------------------------------------------------------------------
 // where a state comes from: U or V as [N][5], or the interleaved V
 enum { kFromU = 0, kFromV = 1, kFromVil = 2 };
-template <int FROM>
-__device__ __forceinline__ void load_state(const double *__restrict__ W, int n, double w[5]) {
+template <int FROM, class L>
+__device__ __forceinline__ void load_state(L lay, const double *__restrict__ W, int n, double w[5]) {
   if (FROM == kFromVil) {
-    load_il<5>(W, n, w);
+    load_il<5>(lay, W, n, w);
   } else {
 #pragma unroll
     for (int k = 0; k < 5; ++k) w[k] = W[5 * (size_t)n + k];
@@ -61,8 +61,9 @@ __device__ __forceinline__ void to_prim(const double w[5], const Gas &gas, doubl
     for (int k = 0; k < 5; ++k) v[k] = w[k];
   }
 }
-__device__ __forceinline__ void load_x(const DevTables &t, int n, double x[3]) {
-  load_il<3>(t.X3, n, x);
+template <class L>
+__device__ __forceinline__ void load_x(L lay, const DevTables &t, int n, double x[3]) {
+  load_il<3>(lay, t.X3, n, x);
 }
 
 // ... from the records
@@ -118,10 +119,10 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
   double Vn[5], xn[3];
   {
     double w[5];
-    load_state<FROM>(W, n, w);
+    load_state<FROM>(t.sh, W, n, w);
     to_prim<FROM>(w, gas, Vn);
   }
-  if (Vout) store_il<5>(Vout, n, Vn);
+  if (Vout) store_il<5>(t.sh, Vout, n, Vn);
   load_x4(t, n, xn);
   double L[6], acc[15];
   load_lsq(t, n, L);
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
     double Wm[kGradChunk][5], xm[kGradChunk][3];
 #pragma unroll
     for (int k = 0; k < kGradChunk; ++k) {
-      load_state<FROM>(W, mi[k], Wm[k]);
+      load_state<FROM>(t.sh, W, mi[k], Wm[k]);
       load_x4(t, mi[k], xm[k]);
     }
 #pragma unroll
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
     for (int q = 0; q < 15; ++q) acc[q] = 0.0;
   }
   if (!OUT3) {
-    store_il<15>(grad, n, acc);
+    store_il<15>(t.sh, grad, n, acc);
   } else {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -194,8 +195,8 @@ struct HaloLoad {
                                           const int m[kHaloBatch]) {
 #pragma unroll
     for (int r = 0; r < kHaloBatch; ++r) {
-      load_state<FROM>(U, m[r], w[r]);
-      load_x(t, m[r], x[r]);
+      load_state<FROM>(Lay<kGroupShift>(), U, m[r], w[r]);
+      load_x(Lay<kGroupShift>(), t, m[r], x[r]);
     }
   }
   // pair q of halo node h to sp[q * cap + h]: (V0, V1) (V2, V3) (V4, X0) (X1, X2)
@@ -229,8 +230,8 @@ struct HaloRow {
   template <int FROM>
   __device__ __forceinline__ void request(const DevTables &t, const double *__restrict__ U, int sl) {
     const int nn = min(sl * kWave + lane_id(), t.N - 1);
-    load_state<FROM>(U, nn, w);
-    load_x(t, nn, xn);
+    load_state<FROM>(Lay<kGroupShift>(), U, nn, w);
+    load_x(Lay<kGroupShift>(), t, nn, xn);
     load_lsq(t, nn, L);
     deg = t.rowptr[nn + 1] - t.rowptr[nn];
     places(t, sl, 0);
@@ -270,7 +271,7 @@ __device__ __forceinline__ void halo_sums(const DevTables &t, const double2 *sp,
 #pragma unroll
   for (int d = 0; d < 3; ++d)
 #pragma unroll
-    for (int q = V0; q < V1; ++q) grad[il<15>(n, 5 * d + q)] = acc[5 * d + q];
+    for (int q = V0; q < V1; ++q) grad[il<15>(kGroupShift, n, 5 * d + q)] = acc[5 * d + q];
 }
 
 // The workgroups b, b + 8, ... take turns over the b % 8-th part of the slices
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(kHaloThreads) void k_gradients_halo(DevTables t, co
     const int n = sl * kWave + lane_id();
     if (n < t.N) {
       if ((int)threadIdx.x < kWave) {
-        if (Vout) store_il<5>(Vout, n, Vn);
+        if (Vout) store_il<5>(Lay<kGroupShift>(), Vout, n, Vn);
         halo_sums<0, 3>(t, sp, cur, Vn, sl, n, grad);
       } else {
         halo_sums<3, 5>(t, sp, cur, Vn, sl, n, grad);
@@ -379,13 +380,14 @@ __device__ __forceinline__ void edge_flux(const FluxConsts &fc, const double Vi[
 }
 
 // flux of boundary-face slot q (a face of node fnode[q]) into Ff[q]
+template <int SH>
 __device__ __forceinline__ void face_slot_flux(const DevTables &t, const double *__restrict__ V, const FluxConsts &fc,
                                                int q, double *__restrict__ Ff) {
   const int n = t.fnode[q], face = t.fidx[q];
   const int code = t.fcode[face];
   const double nv[3] = {t.fnorm3[3 * (size_t)face], t.fnorm3[3 * (size_t)face + 1], t.fnorm3[3 * (size_t)face + 2]};
   double Vn[5], fl[5];
-  load_state<kFromVil>(V, n, Vn);
+  load_state<kFromVil>(Lay<SH>(), V, n, Vn);
   if (is_wall_code(code)) {
     wallflux(nv, 0.0, Vn, fl);
   } else {
@@ -399,7 +401,7 @@ __device__ __forceinline__ void face_slot_flux(const DevTables &t, const double 
 // ALL: a wave per slice, lane r takes the upper edges of its node in turn
 // (node data in registers, P summed here); otherwise a wave per (slice, k)
 // pair.  The first nfb blocks take the boundary-face slots.
-template <bool SECOND, bool LM, bool ALL>
+template <bool SECOND, bool LM, bool ALL, int SH>
 __global__ __launch_bounds__(kBlock) void k_flux_edges(DevTables t, int nfb, const double *__restrict__ V,
                                                        const double *__restrict__ grad, FluxConsts fc,
                                                        double *__restrict__ Fm, double *__restrict__ P,
@@ -408,36 +410,38 @@ __global__ __launch_bounds__(kBlock) void k_flux_edges(DevTables t, int nfb, con
   if (done && *done) return;
   if ((int)blockIdx.x < nfb) {
     const int q = blockIdx.x * kBlock + (int)threadIdx.x;
-    if (q < 3 * t.F) face_slot_flux(t, V, fc, q, Ff);
+    if (q < 3 * t.F) face_slot_flux<SH>(t, V, fc, q, Ff);
     return;
   }
   const int nw = ALL ? t.ns : t.nup;
   const int nb = (nw + kBlock / kWave - 1) / (kBlock / kWave);
   const int w = xcd_chunk(blockIdx.x - nfb, nb) * (kBlock / kWave) + (int)(threadIdx.x / kWave);
   if (w >= nw) return;
-  const int sl = ALL ? w : t.upslice[w];
-  const int kb = t.up.kptr[sl], ke = t.up.kptr[sl + 1];
   const int lane = lane_id();
-  const int i = sl * kWave + lane;
-  const bool live = i < t.N;
-  const int ii = live ? i : t.N - 1;
-  const int deg = live ? t.eup[i + 1] - t.eup[i] : 0;
+  // (upper_entry's edge, with the own state requested before its place is known)
+  constexpr bool places = !ALL && SH == 0;
+  const int at = w * kWave + lane, sl = ALL ? w : (places ? 0 : t.upslice[w]);
+  const int kb = places ? 0 : t.up.kptr[sl], ke = ALL ? t.up.kptr[sl + 1] : 0;
+  const int i = places ? t.uprow[min(at, t.E - 1)] : sl * kWave + lane;
+  const bool live = places ? at < t.E : i < t.N;
+  const int ii = places || live ? i : t.N - 1;
+  const int deg = !places && live ? t.eup[i + 1] - t.eup[i] : 0;
   double Vi[5], xi[3] = {0.0, 0.0, 0.0}, gi[15];
-  load_state<kFromVil>(V, ii, Vi);
-  if (SECOND || LM) load_x(t, ii, xi);
-  if (SECOND) load_il<15>(grad, ii, gi);
+  load_state<kFromVil>(Lay<SH>(), V, ii, Vi);
+  if (SECOND || LM) load_x(Lay<SH>(), t, ii, xi);
+  if (SECOND) load_il<15>(Lay<SH>(), grad, ii, gi);
   double p[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   for (int kk = ALL ? kb : w; kk < (ALL ? ke : w + 1); ++kk) {
-    const bool act = kk - kb < deg;
-    const int pos = t.up.koff[kk] + lanes_below(act);
+    const bool act = places ? live : kk - kb < deg;
+    const int pos = places ? at : t.up.koff[kk] + lanes_below(act);
     if (!act) continue;
     const int j = t.up.idx[pos];
     double Vj[5], xj[3] = {0.0, 0.0, 0.0}, gj[15];
-    load_state<kFromVil>(V, j, Vj);
-    if (SECOND || LM) load_x(t, j, xj);
-    if (SECOND) load_il<15>(grad, j, gj);
+    load_state<kFromVil>(Lay<SH>(), V, j, Vj);
+    if (SECOND || LM) load_x(Lay<SH>(), t, j, xj);
+    if (SECOND) load_il<15>(Lay<SH>(), grad, j, gj);
     double nv[3];
-    stream_load<3, ALL>(t.pnormal, pos, nv);
+    stream_load<3, ALL>(Lay<SH>(), t.pnormal, pos, nv);
     double f[5];
     bool bi, bj;
     edge_flux<SECOND, LM>(fc, Vi, xi, gi, Vj, xj, gj, nv, f, bi, bj);
@@ -448,18 +452,21 @@ __global__ __launch_bounds__(kBlock) void k_flux_edges(DevTables t, int nfb, con
         if (bj) tag0[j] = 1;
       }
     }
-    stream_store<5, ALL>(Fm, pos, f);
+    stream_store<5, ALL>(Lay<SH>(), Fm, pos, f);
 #pragma unroll
     for (int k = 0; k < 5; ++k) p[k] += f[k];
   }
-  if (ALL && live) store_il<5>(P, i, p);
+  if (ALL && live) store_il<5>(Lay<SH>(), P, i, p);
 }
 
 __global__ __launch_bounds__(kBlock) void k_face_flux(DevTables t, const double *__restrict__ V, FluxConsts fc,
                                                       double *__restrict__ Ff, const int *__restrict__ done) {
   if (done && *done) return;
   const int q = blockIdx.x * kBlock + (int)threadIdx.x;
-  if (q < 3 * t.F) face_slot_flux(t, V, fc, q, Ff);
+  if (q < 3 * t.F) {
+    if (t.sh) face_slot_flux<kGroupShift>(t, V, fc, q, Ff);
+    else face_slot_flux<0>(t, V, fc, q, Ff);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -515,7 +522,7 @@ __global__ __launch_bounds__(kGradStrip) void k_gradients_staged(DevTables t, co
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
     Vn[k] = sv[k * kGradHalo + hn];
-    Vout[il<5>(n, k)] = Vn[k];
+    Vout[il<5>(t.sh, n, k)] = Vn[k];
   }
   const double xn[3] = {sv[5 * kGradHalo + hn], sv[6 * kGradHalo + hn], sv[7 * kGradHalo + hn]};
   double L[6], acc[15];
@@ -531,7 +538,7 @@ __global__ __launch_bounds__(kGradStrip) void k_gradients_staged(DevTables t, co
     for (int q = 0; q < 5; ++q) Vm[q] = sv[q * kGradHalo + hm];
     lsq_add(L, xm, xn, Vm, Vn, acc);
   }
-  store_il<15>(grad, n, acc);
+  store_il<15>(t.sh, grad, n, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -578,7 +585,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
   for (int r = 0; r < PV; ++r) {
     const int q = tid + r * kFluxStrip;
     const int h = q / 5, f = q - 5 * h;
-    rv[r] = q < 5 * H ? V[il<5>(sidx[min(h, H - 1)], f)] : 0.0;
+    rv[r] = q < 5 * H ? V[il<5>(t.sh, sidx[min(h, H - 1)], f)] : 0.0;
   }
   if (SECOND) {
 #pragma unroll
@@ -589,7 +596,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
 #pragma unroll
     for (int r = 0; r < PG; ++r) {
       const int q = tid + r * kFluxStrip;
-      rg[r] = q < 16 * H && (q & 15) < 15 ? grad[il<15>(sidx[min(q >> 4, H - 1)], q & 15)] : 0.0;
+      rg[r] = q < 16 * H && (q & 15) < 15 ? grad[il<15>(t.sh, sidx[min(q >> 4, H - 1)], q & 15)] : 0.0;
     }
   }
 #pragma unroll
@@ -624,7 +631,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
       Vj[k] = sj[k];
     }
     double nv[3];
-    load_il<3>(t.pnormal, t.epos[l], nv);
+    load_il<3>(t.sh, t.pnormal, t.epos[l], nv);
     bool bi, bj;
     edge_flux<SECOND, false>(fc, Vi, si + 5, si + 8, Vj, sj + 5, sj + 8, nv, f, bi, bj);
     if (bi || bj) atomicAdd(err, (int)bi + (int)bj);
@@ -634,7 +641,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
 #pragma unroll
   for (int k = 0; k < 5; ++k) sf[k * FS + tid] = f[k];
   __syncthreads();
-  if (tid < ne) store_il<5>(Fm, t.epos[l0 + tid], f);
+  if (tid < ne) store_il<5>(t.sh, Fm, t.epos[l0 + tid], f);
   const int nr = r1 - r0;
   for (int idx = tid; idx < nr * 5; idx += kFluxStrip) {
     const int rr = idx / 5, q = idx - 5 * rr;
@@ -642,7 +649,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
     const int eb = t.eup[r] - l0, eend = t.eup[r + 1] - l0;
     double s = 0.0;
     for (int e = eb; e < eend; ++e) s += sf[q * FS + e];
-    P[il<5>(r, q)] = s;
+    P[il<5>(t.sh, r, q)] = s;
   }
 }
 
@@ -654,6 +661,7 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
 // contributions (momentum and energy), added before the 1/V scaling.
 // host_err (or null): pinned copy of the error count of the finished flux
 // pass, so a synchronous caller needs no copy of its own.
+template <int SH>
 __global__ __launch_bounds__(kBlock) void k_flux_nodes(DevTables t, const double *__restrict__ Fm,
                                                        const double *__restrict__ P, const double *__restrict__ Ff,
                                                        int scale, const double *__restrict__ vg,
@@ -668,17 +676,17 @@ __global__ __launch_bounds__(kBlock) void k_flux_nodes(DevTables t, const double
   const int n = sl * kWave + lane;
   const bool live = n < t.N;
   double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  add_slots<true>(t.lo, sl, live ? t.lrow[n + 1] - t.lrow[n] : 0, Fm, s);
+  add_slots<true>(Lay<SH>(), t.lo, sl, live ? t.lrow[n + 1] - t.lrow[n] : 0, Fm, s);
   if (P) {
     if (live) {
       double p[5];
-      load_il<5>(P, n, p);
+      load_il<5>(Lay<SH>(), P, n, p);
 #pragma unroll
       for (int k = 0; k < 5; ++k) s[k] += p[k];
     }
   } else {
     double p[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    add_slots<false>(t.up, sl, live ? t.eup[n + 1] - t.eup[n] : 0, Fm, p);
+    add_slots<false>(Lay<SH>(), t.up, sl, live ? t.eup[n + 1] - t.eup[n] : 0, Fm, p);
 #pragma unroll
     for (int k = 0; k < 5; ++k) s[k] += p[k];
   }
@@ -688,7 +696,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_nodes(DevTables t, const double
     for (int k = 0; k < 5; ++k) s[k] += Ff[5 * (size_t)q + k];
   if (vg) {
     double g[4];
-    load_il<4>(vg, n, g);
+    load_il<4>(Lay<SH>(), vg, n, g);
 #pragma unroll
     for (int k = 0; k < 4; ++k) s[1 + k] += g[k];
   }
@@ -699,7 +707,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_nodes(DevTables t, const double
 
 // V = V(U), as [N][5] (IL false) or interleaved; clears *err (or null)
 template <bool IL>
-__global__ __launch_bounds__(kBlock) void k_primitive(int N, const double *__restrict__ U, Gas g,
+__global__ __launch_bounds__(kBlock) void k_primitive(int N, int sh, const double *__restrict__ U, Gas g,
                                                       double *__restrict__ V, int *__restrict__ err,
                                                       const int *__restrict__ done) {
   if (done && *done) return;
@@ -711,7 +719,7 @@ __global__ __launch_bounds__(kBlock) void k_primitive(int N, const double *__res
   for (int k = 0; k < 5; ++k) u[k] = U[5 * (size_t)n + k];
   prim_from_cons(u, g, v);
 #pragma unroll
-  for (int k = 0; k < 5; ++k) V[IL ? il<5>(n, k) : 5 * (size_t)n + k] = v[k];
+  for (int k = 0; k < 5; ++k) V[IL ? il<5>(sh, n, k) : 5 * (size_t)n + k] = v[k];
 }
 
 __global__ void k_zero_int(int *p, int n, const int *done) {
@@ -743,12 +751,11 @@ static void launch_flux_edges(aerofx_ctx *c, const ResidualBufs &b, bool all, co
   const int nfb = (3 * t.F + kBlock - 1) / kBlock;
   const dim3 grid(nfb + slice_grid(all ? t.ns : t.nup).x);
   if (grid.x == 0) return;
-  if (all)
-    hipLaunchKernelGGL((k_flux_edges<SECOND, LM, true>), grid, dim3(kBlock), 0, c->stream, t, nfb, b.V, b.grad, c->fc,
-                       b.Fm, b.P, c->d_Ff, c->d_err, b.tag0, done);
-  else
-    hipLaunchKernelGGL((k_flux_edges<SECOND, LM, false>), grid, dim3(kBlock), 0, c->stream, t, nfb, b.V, b.grad,
-                       c->fc, b.Fm, b.P, c->d_Ff, c->d_err, b.tag0, done);
+  const auto k = all    ? k_flux_edges<SECOND, LM, true, kGroupShift>
+                 : t.sh ? k_flux_edges<SECOND, LM, false, kGroupShift>
+                        : k_flux_edges<SECOND, LM, false, 0>;
+  hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, c->stream, t, nfb, b.V, b.grad, c->fc, b.Fm, b.P, c->d_Ff, c->d_err,
+                     b.tag0, done);
 }
 
 int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, double *R, bool scale,
@@ -756,7 +763,7 @@ int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, 
   const DevTables &t = c->tab;
   // the staged kernels evaluate ROEFLUX7 only, without the failsafe
   const bool staged = t.ngb > 0 && c->residual_kernels == AEROFX_RESIDUAL_STAGED && !c->fc.low_mach && !c->failsafe;
-  const bool rows = row_waves(t.ns, kRowWaveSlices, c->max_degree);
+  const bool rows = t.sh && row_waves(t.ns, kRowWaveSlices, c->max_degree);
   const bool all = staged || rows;  // P formed by the flux pass
   const dim3 ngrid((t.N + kBlock - 1) / kBlock), blk(kBlock);
   if (c->p.second_order) {
@@ -772,7 +779,7 @@ int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, 
                          b.grad, nullptr, nullptr, nullptr, c->d_err, done);
     }
   } else {
-    hipLaunchKernelGGL(k_primitive<true>, ngrid, blk, 0, c->stream, t.N, U, c->gas, b.V, c->d_err, done);
+    hipLaunchKernelGGL(k_primitive<true>, ngrid, blk, 0, c->stream, t.N, t.sh, U, c->gas, b.V, c->d_err, done);
   }
   {
     ProfScope ps(c, AEROFX_TIMER_FV_TERM);
@@ -806,8 +813,9 @@ int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, 
   }
   {
     ProfScope ps(c, AEROFX_TIMER_FV_NODES);
-    hipLaunchKernelGGL(k_flux_nodes, slice_grid(t.ns), blk, 0, c->stream, t, b.Fm, all ? b.P : nullptr, c->d_Ff,
-                       scale ? 1 : 0, fold ? c->d_visc_g : nullptr, c->d_err, host_err, R, done);
+    hipLaunchKernelGGL(t.sh ? k_flux_nodes<kGroupShift> : k_flux_nodes<0>, slice_grid(t.ns), blk, 0, c->stream, t,
+                       b.Fm, all ? b.P : nullptr, c->d_Ff, scale ? 1 : 0, fold ? c->d_visc_g : nullptr, c->d_err,
+                       host_err, R, done);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_hip_error(e, "residual launch");
@@ -887,15 +895,15 @@ int launch_gradients_v(aerofx_ctx *c, const double *V, double *ddx, double *ddy,
 }
 
 int launch_primitive(aerofx_ctx *c, const double *U, double *V) {
-  hipLaunchKernelGGL(k_primitive<false>, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N, U,
-                     c->gas, V, nullptr, nullptr);
+  hipLaunchKernelGGL(k_primitive<false>, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N, c->tab.sh,
+                     U, c->gas, V, nullptr, nullptr);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_hip_error(e, "primitive launch");
 }
 
 int launch_primitive_il(aerofx_ctx *c, const double *U) {
-  hipLaunchKernelGGL(k_primitive<true>, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N, U,
-                     c->gas, c->d_V, nullptr, nullptr);
+  hipLaunchKernelGGL(k_primitive<true>, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N, c->tab.sh,
+                     U, c->gas, c->d_V, nullptr, nullptr);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_hip_error(e, "primitive launch");
 }

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_edge_normals(DevTables t, con
   }
 #pragma unroll
   for (int a = 0; a < 3; ++a) acc[a] *= 1.0 / 24.0;
-  store_il<3>(dn, pos, acc);
+  store_il<3>(t.sh, dn, pos, acc);
 }
 
 // a quarter of each tet's volume derivative (ElemTet::computeVolume,
@@ -212,7 +212,7 @@ __device__ __forceinline__ void load_v(const double *__restrict__ U, const doubl
 
 // dV alone; with the mesh fixed the gradients are linear in V, so theirs are
 // the gradients of dV (launch_gradients_il)
-__global__ __launch_bounds__(kTanBlock) void k_tan_dv(int N, const double *__restrict__ U,
+__global__ __launch_bounds__(kTanBlock) void k_tan_dv(int N, int sh, const double *__restrict__ U,
                                                       const double *__restrict__ dU, Gas gas,
                                                       double *__restrict__ dV, const int *__restrict__ done) {
   if (done && *done) return;
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_dv(int N, const double *__res
   Dual v[5];
   load_v(U, dU, n, gas, v);
   const double d[5] = {v[0].d, v[1].d, v[2].d, v[3].d, v[4].d};
-  store_il<5>(dV, n, d);
+  store_il<5>(sh, dV, n, d);
 }
 
 // the derivative of the gradients with the mesh moving: g solves M g = b with the
@@ -229,6 +229,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_dv(int N, const double *__res
 //   dg = M^-1 (db - dM g) = M^-1 sum ddx (dV - dx . g) + dx (ddV - ddx . g):
 // one sweep over the neighbours, and the weights of the gradient pass (linear in
 // dx) apply M^-1.
+template <int SH>
 __global__ __launch_bounds__(kTanBlock) void k_tan_grad(DevTables t, const double *__restrict__ V,
                                                         const double *__restrict__ grad,
                                                         const double *__restrict__ dV,
@@ -238,10 +239,10 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_grad(DevTables t, const doubl
   const int n = sl * kWave + lane_id(), nn = min(n, t.N - 1);
   const int deg = n < t.N ? t.rowptr[n + 1] - t.rowptr[n] : 0;
   double vn[5], wn[5], gn[15], xn[3], yn[3], acc[15];
-  load_il<5>(V, nn, vn);
-  load_il<5>(dV, nn, wn);
-  load_il<15>(grad, nn, gn);
-  load_il<3>(t.X3, nn, xn);
+  load_il<5>(Lay<SH>(), V, nn, vn);
+  load_il<5>(Lay<SH>(), dV, nn, wn);
+  load_il<15>(Lay<SH>(), grad, nn, gn);
+  load_il<3>(Lay<SH>(), t.X3, nn, xn);
 #pragma unroll
   for (int a = 0; a < 3; ++a) yn[a] = dX[3 * (size_t)nn + a];
 #pragma unroll
@@ -253,9 +254,9 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_grad(DevTables t, const doubl
     if (!act) continue;
     const int m = t.nb.idx[pos];
     double vm[5], wm[5], dx[3], dy[3];
-    load_il<5>(V, m, vm);
-    load_il<5>(dV, m, wm);
-    load_il<3>(t.X3, m, dx);
+    load_il<5>(Lay<SH>(), V, m, vm);
+    load_il<5>(Lay<SH>(), dV, m, wm);
+    load_il<3>(Lay<SH>(), t.X3, m, dx);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       dy[a] = dX[3 * (size_t)m + a] - yn[a];
@@ -280,7 +281,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_grad(DevTables t, const doubl
 #pragma unroll
     for (int a = 0; a < 3; ++a) acc[5 * a + q] = w[a];
   }
-  store_il<15>(dG, n, acc);
+  store_il<15>(Lay<SH>(), dG, n, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_grad(DevTables t, const doubl
 // Bound by the gathers of both ends' 46 values (44 us at 104k nodes; selection,
 // time step and two products there 512 -> 296 us, with the flux's derivative by
 // position and summed as the residual's).
-template <bool SECOND, bool MOVE>
+template <bool SECOND, bool MOVE, int SH>
 __global__ __launch_bounds__(kTanBlock) void k_tan_flux(DevTables t, int nfb, const double *__restrict__ V,
                                                         const double *__restrict__ grad,
                                                         const double *__restrict__ dV,
@@ -308,8 +309,8 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_flux(DevTables t, int nfb, co
     if (q >= 3 * t.F) return;
     const int n = t.fnode[q], face = t.fidx[q];
     double v[5], dv[5];
-    load_il<5>(V, n, v);
-    load_il<5>(dV, n, dv);
+    load_il<5>(Lay<SH>(), V, n, v);
+    load_il<5>(Lay<SH>(), dV, n, dv);
     Dual Vn[5], nv[3], fl[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) Vn[k] = Dual(v[k], dv[k]);
@@ -325,36 +326,34 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_flux(DevTables t, int nfb, co
   const int nb = (t.nup + kTanBlock / kWave - 1) / (kTanBlock / kWave);
   const int w = xcd_chunk(blockIdx.x - nfb, nb) * (kTanBlock / kWave) + (int)(threadIdx.x / kWave);
   if (w >= t.nup) return;
-  const int sl = t.upslice[w];
-  const int i = sl * kWave + lane_id();
-  const bool act = i < t.N && w - t.up.kptr[sl] < t.eup[min(i, t.N - 1) + 1] - t.eup[min(i, t.N - 1)];
-  const int pos = t.up.koff[w] + lanes_below(act);
-  if (!act) return;
+  const UpperEntry u = upper_entry<SH>(t, w);
+  if (!u.act) return;
+  const int i = u.i, pos = u.pos;
   const int j = t.up.idx[pos];
   Dual Vi[5], Vj[5], Vij[5], Vji[5];
   {
     double a[5], b[5];
-    load_il<5>(V, i, a);
-    load_il<5>(dV, i, b);
+    load_il<5>(Lay<SH>(), V, i, a);
+    load_il<5>(Lay<SH>(), dV, i, b);
 #pragma unroll
     for (int k = 0; k < 5; ++k) Vi[k] = Dual(a[k], b[k]);
-    load_il<5>(V, j, a);
-    load_il<5>(dV, j, b);
+    load_il<5>(Lay<SH>(), V, j, a);
+    load_il<5>(Lay<SH>(), dV, j, b);
 #pragma unroll
     for (int k = 0; k < 5; ++k) Vj[k] = Dual(a[k], b[k]);
   }
   if (SECOND) {
     double xi[3], xj[3], gi[15], gj[15], hi[15], hj[15];
-    load_il<3>(t.X3, i, xi);
-    load_il<3>(t.X3, j, xj);
+    load_il<3>(Lay<SH>(), t.X3, i, xi);
+    load_il<3>(Lay<SH>(), t.X3, j, xj);
     Dual dx[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a)
       dx[a] = Dual(xj[a] - xi[a], MOVE ? dX[3 * (size_t)j + a] - dX[3 * (size_t)i + a] : 0.0);
-    load_il<15>(grad, i, gi);
-    load_il<15>(dG, i, hi);
-    load_il<15>(grad, j, gj);
-    load_il<15>(dG, j, hj);
+    load_il<15>(Lay<SH>(), grad, i, gi);
+    load_il<15>(Lay<SH>(), dG, i, hi);
+    load_il<15>(Lay<SH>(), grad, j, gj);
+    load_il<15>(Lay<SH>(), dG, j, hj);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       const Dual ddVij = dx[0] * Dual(gi[k], hi[k]) + dx[1] * Dual(gi[5 + k], hi[5 + k]) +
@@ -371,20 +370,20 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_flux(DevTables t, int nfb, co
     }
   }
   double n0[3], n1[3] = {0.0, 0.0, 0.0};
-  load_il<3>(t.pnormal, pos, n0);
-  if (MOVE) load_il<3>(dn, pos, n1);
+  load_il<3>(Lay<SH>(), t.pnormal, pos, n0);
+  if (MOVE) load_il<3>(Lay<SH>(), dn, pos, n1);
   const Dual nv[3] = {Dual(n0[0], n1[0]), Dual(n0[1], n1[1]), Dual(n0[2], n1[2])};
   Dual f[5];
   if (n0[0] * n0[0] + n0[1] * n0[1] + n0[2] * n0[2] >= 1e-36) roe_flux(fc.gas, nv, Vij, Vji, f);
   const double d[5] = {f[0].d, f[1].d, f[2].d, f[3].d, f[4].d};
-  store_il<5>(dF, pos, d);
+  store_il<5>(Lay<SH>(), dF, pos, d);
 }
 
 // ---------------------------------------------------------------------------
 // 5. per node: dS and dR (+ p / dt, the backward-Euler time term of the exact
 //    product, when dt is given)
 // ---------------------------------------------------------------------------
-template <bool MOVE>
+template <bool MOVE, int SH>
 __global__ __launch_bounds__(kTanBlock) void k_tan_nodes(DevTables t, const double *__restrict__ S,
                                                          const int *__restrict__ ntrow,
                                                          const int *__restrict__ ntslot,
@@ -399,8 +398,8 @@ __global__ __launch_bounds__(kTanBlock) void k_tan_nodes(DevTables t, const doub
   const int n = sl * kWave + lane_id();
   const bool live = n < t.N;
   double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  add_slots<false>(t.up, sl, live ? t.eup[n + 1] - t.eup[n] : 0, dF, s);
-  add_slots<true>(t.lo, sl, live ? t.lrow[n + 1] - t.lrow[n] : 0, dF, s);
+  add_slots<false>(Lay<SH>(), t.up, sl, live ? t.eup[n + 1] - t.eup[n] : 0, dF, s);
+  add_slots<true>(Lay<SH>(), t.lo, sl, live ? t.lrow[n + 1] - t.lrow[n] : 0, dF, s);
   if (!live) return;
   for (int q = t.frow[n]; q < t.frow[n + 1]; ++q)
 #pragma unroll
@@ -438,10 +437,10 @@ int ensure_tangent(aerofx_ctx *c) {
   if (rc) return rc;
   Tangent *g = new Tangent();
   const size_t N = c->N, E = c->E, F = std::max(c->F, 1);
-  if ((rc = alloc_n(c, 5 * N, &g->S)) || (rc = alloc_n(c, il_count<5>(N), &g->dV)) ||
-      (rc = alloc_n(c, il_count<15>(N), &g->dG)) || (rc = alloc_n(c, il_count<3>(E), &g->dn)) ||
+  if ((rc = alloc_n(c, 5 * N, &g->S)) || (rc = alloc_n(c, il_count<5>(c->tab.sh, N), &g->dV)) ||
+      (rc = alloc_n(c, il_count<15>(c->tab.sh, N), &g->dG)) || (rc = alloc_n(c, il_count<3>(c->tab.sh, E), &g->dn)) ||
       (rc = alloc_n(c, (size_t)c->T, &g->dvol)) || (rc = alloc_n(c, 3 * F, &g->dfn)) ||
-      (rc = alloc_n(c, il_count<5>(E), &g->dF)) || (rc = alloc_n(c, 15 * F, &g->dFf))) {
+      (rc = alloc_n(c, il_count<5>(c->tab.sh, E), &g->dF)) || (rc = alloc_n(c, 15 * F, &g->dFf))) {
     delete g;
     return rc;
   }
@@ -457,9 +456,10 @@ void launch_flux(aerofx_ctx *c, const double *V, const double *G, const double *
   const DevTables &t = c->tab;
   const int nfb = (3 * t.F + kTanBlock - 1) / kTanBlock;
   const unsigned nb = (unsigned)((t.nup + kTanBlock / kWave - 1) / (kTanBlock / kWave));
+  const auto k = t.sh ? k_tan_flux<SECOND, MOVE, kGroupShift> : k_tan_flux<SECOND, MOVE, 0>;
   if (nfb + nb)
-    hipLaunchKernelGGL((k_tan_flux<SECOND, MOVE>), dim3(nfb + nb), dim3(kTanBlock), 0, c->stream, t, nfb, V, G, g->dV,
-                       g->dG, dX, g->dn, g->dfn, c->fc, g->dF, g->dFf, done);
+    hipLaunchKernelGGL(k, dim3(nfb + nb), dim3(kTanBlock), 0, c->stream, t, nfb, V, G, g->dV, g->dG, dX, g->dn, g->dfn,
+                       c->fc, g->dF, g->dFf, done);
 }
 
 // stages 3 to 5 about the state U with its V and gradients G
@@ -469,9 +469,10 @@ int launch_stages(aerofx_ctx *c, const double *U, const double *V, const double 
   const ElemTables &el = *c->elem;
   const DevTables &t = c->tab;
   const bool second = c->p.second_order != 0;
-  hipLaunchKernelGGL(k_tan_dv, grid_for(t.N), dim3(kTanBlock), 0, c->stream, t.N, U, dU, c->gas, g->dV, done);
+  hipLaunchKernelGGL(k_tan_dv, grid_for(t.N), dim3(kTanBlock), 0, c->stream, t.N, t.sh, U, dU, c->gas, g->dV, done);
   if (second && dX) {
-    hipLaunchKernelGGL(k_tan_grad, slice_grid(t.ns), dim3(kTanBlock), 0, c->stream, t, V, G, g->dV, dX, g->dG);
+    hipLaunchKernelGGL(t.sh ? k_tan_grad<kGroupShift> : k_tan_grad<0>, slice_grid(t.ns), dim3(kTanBlock), 0,
+                       c->stream, t, V, G, g->dV, dX, g->dG);
   } else if (second) {
     if (int rc = launch_gradients_il(c, g->dV, g->dG, done)) return rc;
   }
@@ -483,12 +484,15 @@ int launch_stages(aerofx_ctx *c, const double *U, const double *V, const double 
     launch_flux<false, true>(c, V, G, dX, done);
   else
     launch_flux<false, false>(c, V, G, nullptr, done);
-  if (dX)
-    hipLaunchKernelGGL(k_tan_nodes<true>, slice_grid(t.ns), dim3(kTanBlock), 0, c->stream, t, g->S, el.ntrow, el.ntslot,
-                       g->dvol, g->dF, g->dFf, nullptr, nullptr, dR, done);
-  else
-    hipLaunchKernelGGL(k_tan_nodes<false>, slice_grid(t.ns), dim3(kTanBlock), 0, c->stream, t, g->S, nullptr, nullptr,
-                       nullptr, g->dF, g->dFf, dU, dt, dR, done);
+  if (dX) {
+    const auto k = t.sh ? k_tan_nodes<true, kGroupShift> : k_tan_nodes<true, 0>;
+    hipLaunchKernelGGL(k, slice_grid(t.ns), dim3(kTanBlock), 0, c->stream, t, g->S, el.ntrow, el.ntslot, g->dvol, g->dF,
+                       g->dFf, nullptr, nullptr, dR, done);
+  } else {
+    const auto k = t.sh ? k_tan_nodes<false, kGroupShift> : k_tan_nodes<false, 0>;
+    hipLaunchKernelGGL(k, slice_grid(t.ns), dim3(kTanBlock), 0, c->stream, t, g->S, nullptr, nullptr, nullptr, g->dF,
+                       g->dFf, dU, dt, dR, done);
+  }
   // the Navier-Stokes Galerkin term
   return launch_visc_tangent(c, V, dU, dX, dR, done);
 }
@@ -530,8 +534,8 @@ int launch_h2_select(aerofx_ctx *c, const double *Q) {
   const DevTables &t = c->tab;
   if (!g->V0) {  // both or neither
     double *V0 = nullptr, *G0 = nullptr;
-    if ((rc = alloc_n(c, il_count<5>(t.N), &V0))) return rc;
-    if ((rc = alloc_n(c, il_count<15>(t.N), &G0))) {
+    if ((rc = alloc_n(c, il_count<5>(c->tab.sh, t.N), &V0))) return rc;
+    if ((rc = alloc_n(c, il_count<15>(c->tab.sh, t.N), &G0))) {
       ctx_release(c, V0);
       return rc;
     }

@@ -28,7 +28,7 @@ namespace {
 
 constexpr int kLocalEdge[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
 
-__device__ __forceinline__ void load_element(const int4 *__restrict__ tets, const double *__restrict__ X4,
+__device__ __forceinline__ void load_element(int sh, const int4 *__restrict__ tets, const double *__restrict__ X4,
                                              const double *__restrict__ V, int t, double x[4][3], double v[4][5]) {
   const int4 nd = tets[t];
   const int id[4] = {nd.x, nd.y, nd.z, nd.w};
@@ -38,7 +38,7 @@ __device__ __forceinline__ void load_element(const int4 *__restrict__ tets, cons
     x[k][0] = p.x;
     x[k][1] = p.y;
     x[k][2] = p.z;
-    load_il<5>(V, id[k], v[k]);
+    load_il<5>(sh, V, id[k], v[k]);
   }
 }
 
@@ -64,7 +64,7 @@ __device__ __forceinline__ double pick4(const double a[4], int k) {
 __global__ __launch_bounds__(kBlock) void k_visc_residual(int N, const int *__restrict__ ntrow,
                                                           const int *__restrict__ ntslot,
                                                           const int4 *__restrict__ tets, const double *__restrict__ X4,
-                                                          const double *__restrict__ V,
+                                                          const double *__restrict__ V, int sh,
                                                           const double *__restrict__ invcv, NsConsts ns, int scale,
                                                           double *__restrict__ R, const int *__restrict__ done) {
   if (done && *done) return;
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_residual(int N, const int *__re
   for (int s = ntrow[n]; s < ntrow[n + 1]; ++s) {
     const int slot = ntslot[s], t = slot >> 2, loc = slot & 3;
     double x[4][3], v[4][5], g[4][3];
-    load_element(tets, X4, V, t, x, v);
+    load_element(sh, tets, X4, V, t, x, v);
     const double vol = p1_gradients(x, g);
     NsElem e;
     ns_element(ns, g, v, e);
@@ -136,14 +136,14 @@ __device__ __forceinline__ double pair_swap(double v) {
 // XCD takes a contiguous range of tets, whose pieces meet in its L2 (84 -> 80 ->
 // 76 us for 1.0M tets, and 72 with them ordered by lowest node).
 __global__ __launch_bounds__(kBlock) void k_visc_elements(int T, const int4 *__restrict__ tets,
-                                                          const double *__restrict__ X4, const double *__restrict__ V,
+                                                          const double *__restrict__ X4, const double *__restrict__ V, int sh,
                                                           NsConsts ns, const int4 *__restrict__ pos,
                                                           double *__restrict__ C, const int *__restrict__ done) {
   if (done && *done) return;
   const int ti = xcd_chunk(blockIdx.x, (T + kBlock - 1) / kBlock) * kBlock + (int)threadIdx.x;
   const int t = min(ti, T - 1);  // a lane past the last tet only helps its pair
   double x[4][3], v[4][5], g[4][3];
-  load_element(tets, X4, V, t, x, v);
+  load_element(sh, tets, X4, V, t, x, v);
   const double vol = p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_elements(int T, const int4 *__r
 // slots share a line.  One lane per node and five records per slot touched a
 // line per lane and load: the node pass of the residual took 85 us at 179k
 // nodes.
-__global__ __launch_bounds__(kBlock) void k_visc_sum(int N, const int *__restrict__ ntrow,
+__global__ __launch_bounds__(kBlock) void k_visc_sum(int N, int sh, const int *__restrict__ ntrow,
                                                      const double *__restrict__ C, double *__restrict__ G,
                                                      const int *__restrict__ done) {
   if (done && *done) return;
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_sum(int N, const int *__restric
   double acc = 0.0;
 #pragma unroll 8
   for (int s = ntrow[n]; s < s1; ++s) acc += C[4 * (size_t)s + k];
-  G[il<4>(n, k)] = acc;
+  G[il<4>(sh, n, k)] = acc;
 }
 
 // Transposed element pass: each element once, C[pos[4 t + k]] = vol (d r /
@@ -190,14 +190,14 @@ __global__ __launch_bounds__(kBlock) void k_visc_sum(int N, const int *__restric
 // transposed product.
 __global__ __launch_bounds__(kBlock) void k_visc_adj_elements(int T, const int4 *__restrict__ tets,
                                                               const double *__restrict__ X4,
-                                                              const double *__restrict__ V,
+                                                              const double *__restrict__ V, int sh,
                                                               const double *__restrict__ lam,
                                                               const double *__restrict__ invcv, NsConsts ns,
                                                               const int4 *__restrict__ pos, double *__restrict__ C) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= T) return;
   double x[4][3], v[4][5], g[4][3];
-  load_element(tets, X4, V, t, x, v);
+  load_element(sh, tets, X4, V, t, x, v);
   const double vol = p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -317,14 +317,14 @@ __device__ __forceinline__ void ns_shape_contrib(const NsElem &e, const double v
 // d x_a[d] (added to the element's other geometry terms before the node
 // gather of the adjoint)
 __global__ __launch_bounds__(kBlock) void k_visc_adj_x(int T, const int4 *__restrict__ tets,
-                                                       const double *__restrict__ X4, const double *__restrict__ V,
+                                                       const double *__restrict__ X4, const double *__restrict__ V, int sh,
                                                        const double *__restrict__ lam,
                                                        const double *__restrict__ invcv, NsConsts ns,
                                                        double *__restrict__ TX) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= T) return;
   double x[4][3], v[4][5], g[4][3];
-  load_element(tets, X4, V, t, x, v);
+  load_element(sh, tets, X4, V, t, x, v);
   p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_adj_x(int T, const int4 *__rest
 // to C[pos[4 t + j]]; k_visc_gather then adds the node sums (/ V).
 __global__ __launch_bounds__(kBlock) void k_visc_tan_elements(int T, const int4 *__restrict__ tets,
                                                               const double *__restrict__ X4,
-                                                              const double *__restrict__ V,
+                                                              const double *__restrict__ V, int sh,
                                                               const double *__restrict__ dU,
                                                               const double *__restrict__ dX, NsConsts ns,
                                                               const int4 *__restrict__ pos, double *__restrict__ C,
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_tan_elements(int T, const int4 
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= T) return;
   double x[4][3], v[4][5], g[4][3];
-  load_element(tets, X4, V, t, x, v);
+  load_element(sh, tets, X4, V, t, x, v);
   const double vol = p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_force(int F, const int *__restr
                                                        const double *__restrict__ fnorm,
                                                        const int *__restrict__ face_elem,
                                                        const int4 *__restrict__ tets, const double *__restrict__ X4,
-                                                       const double *__restrict__ V, NsConsts ns, double d0, double d1,
+                                                       const double *__restrict__ V, int sh, NsConsts ns, double d0, double d1,
                                                        double d2, double *__restrict__ Jf, double *__restrict__ FU,
                                                        double *__restrict__ FX) {
   const int f = blockIdx.x * kBlock + threadIdx.x;
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_force(int F, const int *__restr
   const int t = face_elem[f];
   if (t < 0 || !is_wall_code(fcode[f])) return;
   double x[4][3], v[4][5], g[4][3];
-  load_element(tets, X4, V, t, x, v);
+  load_element(sh, tets, X4, V, t, x, v);
   p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -703,7 +703,7 @@ __global__ __launch_bounds__(kJacLanes) void k_visc_jacobian_rows(DevTables tb, 
   if (tid < nslots) {
     const int slot = ntslot[s0 + tid], t = slot >> 2, ln = slot & 3;
     double x[4][3], v[4][5], g[4][3];
-    load_element(tets, tb.X4, V, t, x, v);
+    load_element(tb.sh, tets, tb.X4, V, t, x, v);
     const double vol = p1_gradients(x, g);
     NsElem e;
     ns_element(ns, g, v, e);
@@ -782,7 +782,7 @@ __global__ __launch_bounds__(kJacLanes) void k_visc_jacobian_rows(DevTables tb, 
         a.Qm += o[21] * (u[0] * t[0] + u[1] * t[1] + u[2] * t[2]) + o[22];
       }
     double Vm[5];
-    load_il<5>(V, m, Vm);
+    load_il<5>(tb.sh, V, m, Vm);
     visc_block_add(ns, a, Vm, tb.invcv[n], B + blk64_base(e0 + tid));
   }
   __syncthreads();
@@ -807,7 +807,7 @@ __global__ __launch_bounds__(kJacLanes) void k_visc_jacobian_rows(DevTables tb, 
 #pragma unroll
     for (int k = 0; k < kAccF; ++k) p[k] = sdiag[tid * kAccF + k];
     double Vn[5];
-    load_il<5>(V, n, Vn);
+    load_il<5>(tb.sh, V, n, Vn);
     visc_block_add(ns, d, Vn, tb.invcv[n], D + blk64_base(n));
   }
 }
@@ -848,7 +848,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_jacobian(DevTables tb, const in
       const int a = kLocalEdge[le][0], b = kLocalEdge[le][1];
       const int ln = id[a] == n ? a : b, lm = id[a] == n ? b : a;
       double x[4][3], v[4][5], g[4][3];
-      load_element(tets, tb.X4, V, t, x, v);
+      load_element(tb.sh, tets, tb.X4, V, t, x, v);
       const double vol = p1_gradients(x, g);
       NsElem el;
       ns_element(ns, g, v, el);
@@ -868,7 +868,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_jacobian(DevTables tb, const in
     for (int s = ntrow[n]; s < ntrow[n + 1]; ++s) {
       const int slot = ntslot[s], t = slot >> 2, loc = slot & 3;
       double x[4][3], v[4][5], g[4][3];
-      load_element(tets, tb.X4, V, t, x, v);
+      load_element(tb.sh, tets, tb.X4, V, t, x, v);
       const double vol = p1_gradients(x, g);
       NsElem el;
       ns_element(ns, g, v, el);
@@ -890,7 +890,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_jacobian(DevTables tb, const in
 // the element's mean state (Vmid summed in vertex order, times 1/4)
 __global__ __launch_bounds__(kBlock) void k_visc_idtv(int N, const int *__restrict__ ntrow,
                                                       const int *__restrict__ ntslot, const int4 *__restrict__ tets,
-                                                      const double *__restrict__ X4, const double *__restrict__ V,
+                                                      const double *__restrict__ X4, const double *__restrict__ V, int sh,
                                                       NsConsts ns, double *__restrict__ idtv) {
   const int n = blockIdx.x * kBlock + threadIdx.x;
   if (n >= N) return;
@@ -898,7 +898,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_idtv(int N, const int *__restri
   for (int s = ntrow[n]; s < ntrow[n + 1]; ++s) {
     const int slot = ntslot[s], t = slot >> 2, loc = slot & 3;
     double x[4][3], v[4][5], g[4][3];
-    load_element(tets, X4, V, t, x, v);
+    load_element(sh, tets, X4, V, t, x, v);
     double Vmid[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) Vmid[k] = (((0.0 + v[0][k]) + v[1][k]) + v[2][k]) + v[3][k];
@@ -1042,7 +1042,7 @@ int ensure_element_order(aerofx_ctx *c) {
   } C, pos, tets, g;
   if (hipMalloc(&C.p, sizeof(double) * 20 * T) != hipSuccess || hipMalloc(&pos.p, sizeof(int4) * T) != hipSuccess ||
       hipMalloc(&tets.p, sizeof(int4) * T) != hipSuccess ||
-      hipMalloc(&g.p, sizeof(double) * il_count<4>(c->N)) != hipSuccess) {
+      hipMalloc(&g.p, sizeof(double) * il_count<4>(c->tab.sh, c->N)) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
@@ -1069,14 +1069,14 @@ int launch_visc_elements(aerofx_ctx *c, const double *V, const int *done) {
   const ElemTables *el = c->elem;
   ProfScope ps(c, AEROFX_TIMER_FE_TERM);
   hipLaunchKernelGGL(k_visc_elements, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     c->d_visc_tets, c->tab.X4, V, c->ns, c->d_visc_pos, c->d_visc_c, done);
+                     c->d_visc_tets, c->tab.X4, V, c->tab.sh, c->ns, c->d_visc_pos, c->d_visc_c, done);
   return check("viscous element launch");
 }
 
 int launch_visc_sum(aerofx_ctx *c, const int *done) {
   ProfScope ps(c, AEROFX_TIMER_FE_TERM);
   hipLaunchKernelGGL(k_visc_sum, dim3((unsigned)((4 * (size_t)c->N + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->stream, c->N,
-                     c->elem->ntrow, c->d_visc_c, c->d_visc_g, done);
+                     c->tab.sh, c->elem->ntrow, c->d_visc_c, c->d_visc_g, done);
   return check("viscous sum launch");
 }
 
@@ -1086,7 +1086,7 @@ int launch_visc_residual(aerofx_ctx *c, const double *V, double *R, bool scale, 
   const ElemTables *el = c->elem;
   ProfScope ps(c, AEROFX_TIMER_FE_TERM);
   hipLaunchKernelGGL(k_visc_residual, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
-                     el->ntrow, el->ntslot, (const int4 *)el->tets, c->tab.X4, V, c->tab.invcv, c->ns,
+                     el->ntrow, el->ntslot, (const int4 *)el->tets, c->tab.X4, V, c->tab.sh, c->tab.invcv, c->ns,
                      scale ? 1 : 0, R, done);
   return check("viscous residual launch");
 }
@@ -1133,7 +1133,7 @@ int launch_visc_adjoint(aerofx_ctx *c, const double *lam, double *Ub) {
   if (!c->d_visc_c) return set_error(AEROFX_ERR_STATE, "adjoint: the viscous contribution buffer is missing");
   const ElemTables *el = c->elem;
   hipLaunchKernelGGL(k_visc_adj_elements, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     c->d_visc_tets, c->tab.X4, c->d_V, lam, c->tab.invcv, c->ns,
+                     c->d_visc_tets, c->tab.X4, c->d_V, c->tab.sh, lam, c->tab.invcv, c->ns,
                      c->d_visc_pos, c->d_visc_c);
   hipLaunchKernelGGL(k_visc_gather, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
                      el->ntrow, c->d_visc_c, c->tab.invcv, 0, Ub, nullptr);
@@ -1146,7 +1146,7 @@ int launch_visc_tangent(aerofx_ctx *c, const double *V, const double *dU, const 
   if (!c->d_visc_c) return set_error(AEROFX_ERR_STATE, "tangent: the viscous contribution buffer is missing");
   const ElemTables *el = c->elem;
   hipLaunchKernelGGL(k_visc_tan_elements, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     c->d_visc_tets, c->tab.X4, V, dU, dX, c->ns, c->d_visc_pos, c->d_visc_c,
+                     c->d_visc_tets, c->tab.X4, V, c->tab.sh, dU, dX, c->ns, c->d_visc_pos, c->d_visc_c,
                      done);
   hipLaunchKernelGGL(k_visc_gather, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
                      el->ntrow, c->d_visc_c, c->tab.invcv, 1, dR, done);
@@ -1157,7 +1157,7 @@ int launch_visc_adjoint_x(aerofx_ctx *c, const double *lam, double *TX) {
   if (!c->viscous) return 0;
   const ElemTables *el = c->elem;
   hipLaunchKernelGGL(k_visc_adj_x, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     (const int4 *)el->tets, c->tab.X4, c->d_V, lam, c->tab.invcv, c->ns, TX);
+                     (const int4 *)el->tets, c->tab.X4, c->d_V, c->tab.sh, lam, c->tab.invcv, c->ns, TX);
   return check("viscous shape adjoint launch");
 }
 
@@ -1165,7 +1165,7 @@ int launch_visc_force(aerofx_ctx *c, const double dir[3], double *Jf, bool deriv
   if (!c->viscous || !c->F) return 0;
   const ElemTables *el = c->elem;
   hipLaunchKernelGGL(k_visc_force, dim3((c->F + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->F, el->faces,
-                     c->tab.fcode, c->tab.fnorm, c->d_face_elem, (const int4 *)el->tets, c->tab.X4, c->d_V, c->ns,
+                     c->tab.fcode, c->tab.fnorm, c->d_face_elem, (const int4 *)el->tets, c->tab.X4, c->d_V, c->tab.sh, c->ns,
                      dir[0], dir[1], dir[2], Jf, derivs ? c->d_force_u : nullptr, derivs ? c->d_force_x : nullptr);
   return check("viscous force launch");
 }
@@ -1215,7 +1215,7 @@ int launch_visc_idtv(aerofx_ctx *c, double **idtv) {
   }
   const ElemTables *el = c->elem;
   hipLaunchKernelGGL(k_visc_idtv, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N, el->ntrow,
-                     el->ntslot, (const int4 *)el->tets, c->tab.X4, c->d_V, c->ns, c->d_idtv);
+                     el->ntslot, (const int4 *)el->tets, c->tab.X4, c->d_V, c->tab.sh, c->ns, c->d_idtv);
   *idtv = c->d_idtv;
   return check("viscous time-step launch");
 }

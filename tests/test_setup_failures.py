@@ -83,16 +83,24 @@ def test_storage_runs_out_half_way(fake_lib, what):
         assert "hipMalloc" in r["log2"][:use], r
 
 
+def test_layout_by_numbering(fake_lib):
+    """Records (the gradient pass gathers per entry) for nodes in random order from
+    256 slices of 64 on, interleaved arrays (the gradient pass through LDS)
+    otherwise."""
+    assert _drive(fake_lib, "layout") == [["25 box", "k_gradients_halo"], ["25 shuffled", "k_gradients"],
+                                          ["24 shuffled", "k_gradients_halo"]]
+
+
 # ---------------------------------------------------------------------------
 # child process: the library of AEROFX_LIB
 # ---------------------------------------------------------------------------
 class _Ctx:
-    def __init__(self, viscous=False):
+    def __init__(self, mesh=None):
         import numpy as np
         from aerof_dev_amd import FlowParams, init_state
         from aerof_dev_amd import mesh as M
         from aerof_dev_amd._abi import Mesh as CMesh, c_double_p, c_int_p, lib
-        m = M.kuhn_box(4, 3, 3, jitter=0.1, seed=3, face_codes=M.VISCOUS_CHANNEL)
+        m = mesh or M.kuhn_box(4, 3, 3, jitter=0.1, seed=3, face_codes=M.VISCOUS_CHANNEL)
         p = FlowParams(mach=0.4)
         self.lib = lib()
         self.a = [np.ascontiguousarray(m.X), np.ascontiguousarray(m.tets, dtype=np.int32),
@@ -156,6 +164,22 @@ def _viscous():
             for x, first, log1 in _each_failure(_Ctx.set_viscous)]
 
 
+def _layout():
+    import numpy as np
+    from aerof_dev_amd import mesh as M
+    out = []
+    for n, shuffled in ((25, False), (25, True), (24, True)):  # 17576, 15625 nodes: 275 and 245 slices
+        m = M.kuhn_box(n, n, n)
+        if shuffled:
+            m = M.renumber(m, np.random.default_rng(1).permutation(m.num_nodes).astype(np.int32))
+        x = _Ctx(m)
+        x.log()
+        gradients = [e for e in x.residual() if e.startswith("kernel k_gradients")]
+        out.append([f"{n} {'shuffled' if shuffled else 'box'}", gradients[0].split()[1]])
+        x.close()
+    return out
+
+
 def _storage(call, kernel):
     return [{"kernel": kernel, "first": first, "log1": log1, "second": call(x), "log2": x.log()}
             for x, first, log1 in _each_failure(call, b"hipMalloc")]
@@ -180,6 +204,7 @@ def _viscous_host():
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     print(json.dumps({
+        "layout": _layout,
         "viscous": _viscous,
         "viscous host": _viscous_host,
         "h2": lambda: _storage(_Ctx.select_h2, "k_gradients_halo"),
