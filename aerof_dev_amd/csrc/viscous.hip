@@ -28,7 +28,8 @@ namespace {
 
 constexpr int kLocalEdge[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
 
-__device__ __forceinline__ void load_element(int sh, const int4 *__restrict__ tets, const double *__restrict__ X4,
+template <class L>
+__device__ __forceinline__ void load_element(L lay, const int4 *__restrict__ tets, const double *__restrict__ X4,
                                              const double *__restrict__ V, int t, double x[4][3], double v[4][5]) {
   const int4 nd = tets[t];
   const int id[4] = {nd.x, nd.y, nd.z, nd.w};
@@ -38,7 +39,7 @@ __device__ __forceinline__ void load_element(int sh, const int4 *__restrict__ te
     x[k][0] = p.x;
     x[k][1] = p.y;
     x[k][2] = p.z;
-    load_il<5>(sh, V, id[k], v[k]);
+    load_il<5>(lay, V, id[k], v[k]);
   }
 }
 
@@ -135,15 +136,16 @@ __device__ __forceinline__ double pair_swap(double v) {
 // write both halves of one tet's piece together, then of the other's, and each
 // XCD takes a contiguous range of tets, whose pieces meet in its L2 (84 -> 80 ->
 // 76 us for 1.0M tets, and 72 with them ordered by lowest node).
+template <int SH>
 __global__ __launch_bounds__(kBlock) void k_visc_elements(int T, const int4 *__restrict__ tets,
-                                                          const double *__restrict__ X4, const double *__restrict__ V, int sh,
+                                                          const double *__restrict__ X4, const double *__restrict__ V,
                                                           NsConsts ns, const int4 *__restrict__ pos,
                                                           double *__restrict__ C, const int *__restrict__ done) {
   if (done && *done) return;
   const int ti = xcd_chunk(blockIdx.x, (T + kBlock - 1) / kBlock) * kBlock + (int)threadIdx.x;
   const int t = min(ti, T - 1);  // a lane past the last tet only helps its pair
   double x[4][3], v[4][5], g[4][3];
-  load_element(sh, tets, X4, V, t, x, v);
+  load_element(Lay<SH>(), tets, X4, V, t, x, v);
   const double vol = p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -188,16 +190,17 @@ __global__ __launch_bounds__(kBlock) void k_visc_sum(int N, int sh, const int *_
 // d U_k)^T w with w[j][m] = sum_i g_i[j] lambda_i[m] / V_i (the residual of
 // vertex i carries 1/V_i); k_visc_gather then adds the node sums to the
 // transposed product.
+template <int SH>
 __global__ __launch_bounds__(kBlock) void k_visc_adj_elements(int T, const int4 *__restrict__ tets,
                                                               const double *__restrict__ X4,
-                                                              const double *__restrict__ V, int sh,
+                                                              const double *__restrict__ V,
                                                               const double *__restrict__ lam,
                                                               const double *__restrict__ invcv, NsConsts ns,
                                                               const int4 *__restrict__ pos, double *__restrict__ C) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= T) return;
   double x[4][3], v[4][5], g[4][3];
-  load_element(sh, tets, X4, V, t, x, v);
+  load_element(Lay<SH>(), tets, X4, V, t, x, v);
   const double vol = p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -316,15 +319,16 @@ __device__ __forceinline__ void ns_shape_contrib(const NsElem &e, const double v
 // Adjoint of the shape part: TX[t][3 a + d] += sum_j lam_j / V_j . d c_j /
 // d x_a[d] (added to the element's other geometry terms before the node
 // gather of the adjoint)
+template <int SH>
 __global__ __launch_bounds__(kBlock) void k_visc_adj_x(int T, const int4 *__restrict__ tets,
-                                                       const double *__restrict__ X4, const double *__restrict__ V, int sh,
+                                                       const double *__restrict__ X4, const double *__restrict__ V,
                                                        const double *__restrict__ lam,
                                                        const double *__restrict__ invcv, NsConsts ns,
                                                        double *__restrict__ TX) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= T) return;
   double x[4][3], v[4][5], g[4][3];
-  load_element(sh, tets, X4, V, t, x, v);
+  load_element(Lay<SH>(), tets, X4, V, t, x, v);
   p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -358,9 +362,10 @@ __global__ __launch_bounds__(kBlock) void k_visc_adj_x(int T, const int4 *__rest
 // Forward element pass of the state derivative: each element once,
 // dr = sum_k (d r / d U_k) dU_k and its vertex contributions vol (dr . g_j)
 // to C[pos[4 t + j]]; k_visc_gather then adds the node sums (/ V).
+template <int SH>
 __global__ __launch_bounds__(kBlock) void k_visc_tan_elements(int T, const int4 *__restrict__ tets,
                                                               const double *__restrict__ X4,
-                                                              const double *__restrict__ V, int sh,
+                                                              const double *__restrict__ V,
                                                               const double *__restrict__ dU,
                                                               const double *__restrict__ dX, NsConsts ns,
                                                               const int4 *__restrict__ pos, double *__restrict__ C,
@@ -369,7 +374,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_tan_elements(int T, const int4 
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= T) return;
   double x[4][3], v[4][5], g[4][3];
-  load_element(sh, tets, X4, V, t, x, v);
+  load_element(Lay<SH>(), tets, X4, V, t, x, v);
   const double vol = p1_gradients(x, g);
   NsElem e;
   ns_element(ns, g, v, e);
@@ -1068,8 +1073,9 @@ int bc_priority(int code) {
 int launch_visc_elements(aerofx_ctx *c, const double *V, const int *done) {
   const ElemTables *el = c->elem;
   ProfScope ps(c, AEROFX_TIMER_FE_TERM);
-  hipLaunchKernelGGL(k_visc_elements, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     c->d_visc_tets, c->tab.X4, V, c->tab.sh, c->ns, c->d_visc_pos, c->d_visc_c, done);
+  const auto k = c->tab.sh ? k_visc_elements<kGroupShift> : k_visc_elements<0>;
+  hipLaunchKernelGGL(k, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
+                     c->d_visc_tets, c->tab.X4, V, c->ns, c->d_visc_pos, c->d_visc_c, done);
   return check("viscous element launch");
 }
 
@@ -1132,9 +1138,9 @@ int launch_visc_adjoint(aerofx_ctx *c, const double *lam, double *Ub) {
   if (!c->viscous) return 0;
   if (!c->d_visc_c) return set_error(AEROFX_ERR_STATE, "adjoint: the viscous contribution buffer is missing");
   const ElemTables *el = c->elem;
-  hipLaunchKernelGGL(k_visc_adj_elements, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     c->d_visc_tets, c->tab.X4, c->d_V, c->tab.sh, lam, c->tab.invcv, c->ns,
-                     c->d_visc_pos, c->d_visc_c);
+  const auto k = c->tab.sh ? k_visc_adj_elements<kGroupShift> : k_visc_adj_elements<0>;
+  hipLaunchKernelGGL(k, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
+                     c->d_visc_tets, c->tab.X4, c->d_V, lam, c->tab.invcv, c->ns, c->d_visc_pos, c->d_visc_c);
   hipLaunchKernelGGL(k_visc_gather, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
                      el->ntrow, c->d_visc_c, c->tab.invcv, 0, Ub, nullptr);
   return check("viscous adjoint launch");
@@ -1145,9 +1151,9 @@ int launch_visc_tangent(aerofx_ctx *c, const double *V, const double *dU, const 
   if (!c->viscous || (!dU && !dX)) return 0;
   if (!c->d_visc_c) return set_error(AEROFX_ERR_STATE, "tangent: the viscous contribution buffer is missing");
   const ElemTables *el = c->elem;
-  hipLaunchKernelGGL(k_visc_tan_elements, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     c->d_visc_tets, c->tab.X4, V, c->tab.sh, dU, dX, c->ns, c->d_visc_pos, c->d_visc_c,
-                     done);
+  const auto k = c->tab.sh ? k_visc_tan_elements<kGroupShift> : k_visc_tan_elements<0>;
+  hipLaunchKernelGGL(k, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
+                     c->d_visc_tets, c->tab.X4, V, dU, dX, c->ns, c->d_visc_pos, c->d_visc_c, done);
   hipLaunchKernelGGL(k_visc_gather, dim3((c->N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->N,
                      el->ntrow, c->d_visc_c, c->tab.invcv, 1, dR, done);
   return check("viscous tangent launch");
@@ -1156,8 +1162,9 @@ int launch_visc_tangent(aerofx_ctx *c, const double *V, const double *dU, const 
 int launch_visc_adjoint_x(aerofx_ctx *c, const double *lam, double *TX) {
   if (!c->viscous) return 0;
   const ElemTables *el = c->elem;
-  hipLaunchKernelGGL(k_visc_adj_x, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
-                     (const int4 *)el->tets, c->tab.X4, c->d_V, c->tab.sh, lam, c->tab.invcv, c->ns, TX);
+  const auto k = c->tab.sh ? k_visc_adj_x<kGroupShift> : k_visc_adj_x<0>;
+  hipLaunchKernelGGL(k, dim3((c->T + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->T,
+                     (const int4 *)el->tets, c->tab.X4, c->d_V, lam, c->tab.invcv, c->ns, TX);
   return check("viscous shape adjoint launch");
 }
 
