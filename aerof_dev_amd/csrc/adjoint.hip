@@ -67,11 +67,8 @@ struct Adjoint {
 namespace {
 
 constexpr int kAdjBlock = 256;
-// ElemTet edge -> (end, end) table (ElemTetCore.C:19-21) and the edge's opposite
-// vertices (c, d): in a tet the median dual face of edge (a, b), from a to b, is
-// (c - d) x (a + b - c - d) / 24
+// ElemTet edge -> (end, end) table (ElemTetCore.C:19-21)
 constexpr int kEnd[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
-constexpr int kOpp[6][2] = {{3, 2}, {1, 3}, {2, 1}, {3, 0}, {0, 2}, {1, 0}};
 
 __device__ __forceinline__ double seed(int dir, int k) { return dir == k ? 1.0 : 0.0; }
 

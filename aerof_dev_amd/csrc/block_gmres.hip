@@ -760,8 +760,9 @@ __global__ void k_colnorm_reduce(const double *__restrict__ partial, double *__r
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+constexpr int kDotsWaves = 4;  // waves per workgroup of k_tsg_dots: they share LDS
+
 struct TsgShape {
-  int waves_dots = 4;    // waves per workgroup of k_tsg_dots (fixed: they share LDS)
   int waves_update = 4;  // waves per workgroup of k_tsg_update
   bool tuned = false;
 };
@@ -822,7 +823,7 @@ BlockSolver *get_block(aerofx_ctx *c, int m, int *rc);
 // out[b] = V_b^T W (and out2[b] = V_b^T W2 when W2 is given), b < nb
 void tsg_dots(BlockSolver *s, int nb, const double *V, const double *W, double *out, const double *W2 = nullptr,
               double *out2 = nullptr) {
-  const dim3 grid(s->nchunks), block(256);
+  const dim3 grid(s->nchunks), block(kDotsWaves * 64);
 #define TSG_DOTS(TWO, NBM)                                                                                     \
   hipLaunchKernelGGL((k_tsg_dots<TWO, NBM>), grid, block, 0, s->stream, s->npad, s->chunk_rows, s->m + 1, nb, V, \
                      s->npad * kS, W, W2, s->partial, s->partial2)
@@ -1016,8 +1017,7 @@ void autotune(aerofx_ctx *c, BlockSolver *s) {
   int kb = 0;
   for (int k = 1; k < 4; ++k)
     if (best[k] < best[kb]) kb = k;
-  c->blk_tune[0] = s->shape.waves_dots;
-  c->blk_tune[1] = s->shape.waves_update = cand_u[kb];
+  c->blk_tune = s->shape.waves_update = cand_u[kb];
   s->shape.tuned = true;
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
@@ -1118,9 +1118,8 @@ BlockSolver *get_block(aerofx_ctx *c, int m, int *rc) {
   double *vecs[6] = {s->W, s->Z, s->R, s->X, s->B, s->T};
   for (double *p : vecs) (void)hipMemsetAsync(p, 0, blk * sizeof(double), s->stream);
   (void)hipMemsetAsync(s->Hbar, 0, (size_t)(m + 1) * m * kTile * sizeof(double), s->stream);
-  if (c->blk_tune[0] > 0) {
-    s->shape.waves_dots = c->blk_tune[0];
-    s->shape.waves_update = c->blk_tune[1];
+  if (c->blk_tune > 0) {
+    s->shape.waves_update = c->blk_tune;
     s->shape.tuned = true;
   }
   c->blk = s;
@@ -1288,7 +1287,7 @@ extern "C" int aerofx_block_gmres(aerofx_ctx *c, int nrhs, const double *Bv, dou
   if (e != hipSuccess) return set_hip_error(e, "block_gmres finish");
   st->cycles = cycle;
   st->res_max = worst;
-  st->tune_waves_dots = s->shape.waves_dots;
+  st->tune_waves_dots = kDotsWaves;
   st->tune_waves_update = s->shape.waves_update;
   st->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return AEROFX_OK;

@@ -150,7 +150,8 @@ __device__ __forceinline__ int lanes_below(bool active) {
   return __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u));
 }
 
-// 64 B of LDS per halo node: five workgroups per CU at 512 nodes
+// 64 B of LDS per halo node: 512 nodes (about a slice's in RCM or row order)
+// leave room for five workgroups per CU, of which registers let four run
 constexpr int kHaloCap = 1024;
 constexpr int kHaloRow = 64;  // bounds the padding of the places
 
@@ -443,7 +444,7 @@ struct aerofx_ctx {
   aerofx::Ilu *ilu = nullptr;
   aerofx::FgWork *fgm = nullptr;  // flexible GMRES workspace (fgmres.hip)
   aerofx::BlockSolver *blk = nullptr;
-  int blk_tune[2] = {0, 0};  // autotuned waves per workgroup of the block GEMMs
+  int blk_tune = 0;  // autotuned waves per workgroup of the block update, 0: not yet
   // per-kernel timers (the reference's Timer buckets, Timer.h:12-15)
   bool prof = false;
   struct Pending {

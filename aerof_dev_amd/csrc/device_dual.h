@@ -59,8 +59,4 @@ __device__ __forceinline__ Dual gsqrt(Dual x) {
   return Dual(s, 0.5 * x.d / s);
 }
 
-// the quotient and square root the Roe flux uses (ddiv / dsqrt for double)
-__device__ __forceinline__ Dual ddiv(Dual a, Dual b) { return a / b; }
-__device__ __forceinline__ Dual dsqrt(Dual x) { return gsqrt(x); }
-
 }  // namespace aerofx

@@ -29,8 +29,7 @@ struct Gas {
 };
 
 // Division and square root of the routines in the reference's operation
-// order: IEEE-rounded, as the reference's; the Dual overloads (device_dual.h)
-// carry derivatives.
+// order: IEEE-rounded, as the reference's.
 __device__ __forceinline__ double ddiv(double a, double b) { return a / b; }
 __device__ __forceinline__ double dsqrt(double x) { return sqrt(x); }
 

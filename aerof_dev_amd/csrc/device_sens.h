@@ -9,6 +9,12 @@
 
 namespace aerofx {
 
+// The vertices (c, d) opposite to a tet's edge (a, b), in the order that makes
+// the tet's part of the median dual face, from a to b,
+// (c - d) x (a + b - c - d) / 24 (ElemTet edge and face tables,
+// ElemTetCore.C:19-21)
+constexpr int kOpp[6][2] = {{3, 2}, {1, 3}, {2, 1}, {3, 0}, {0, 2}, {1, 0}};
+
 // LSQ weights W(dx; L) (computeLocalWeightsLeastSquares, SubDomain.C:137-159)
 // in the gradient pass's operation order; linear in dx: W = M^-1 dx with the
 // moments M.

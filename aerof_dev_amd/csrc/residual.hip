@@ -9,7 +9,7 @@
 //     the reference's LSQ edge loop (SubDomain.C:137-159, 297-374) with the
 //     same per-node addition order.  The pass also writes V = V(U), which
 //     later passes gather, interleaved.
-//  2. k_flux_edges each edge flux once (MUSCL + Van Albada + ROEFLUX7,
+//  2. k_flux_edges each edge flux once (MUSCL + Van Albada + Roe's flux,
 //     Edge.C:372-439), a wave per 64 lower nodes i: lane r takes the edges of
 //     node i in turn, so its state, coordinates and gradients stay in
 //     registers and the +f contributions P_i are summed in edge order (large
@@ -175,14 +175,14 @@ __global__ __launch_bounds__(kBlock) void k_gradients(DevTables t, const double 
 // in RCM or row order, runs of consecutive ids).  Each node of the halo is
 // loaded once, by consecutive lanes, and the entries read LDS: 16-B pairs,
 // consecutive lanes on consecutive nodes.  The pass is bound by the loads in
-// flight, which LDS limits (64 B a halo node: five workgroups per CU): two
+// flight: four workgroups per CU (by LDS, 64 B a halo node, five): two
 // waves share the halo and split the variables, the workgroups stay for
 // several slices and request the next one's data before they compute, and the
 // tables are padded to one length per slice, so those requests depend on one
 // earlier load only.  The sums are k_gradients', term for term.  At 2.1M nodes
-// 245 us, 275k nodes 35 us (k_gradients with record gathers 296 and 46;
-// without the overlap 266 + 28 for a pass that converts U first, with one wave
-// per slice 366 + 28).
+// 266 us (kernel trace), at 275k 37, with U -> V in the same pass; k_gradients
+// takes 252 and 34 from plain records of V, and a conversion of U before it 28
+// at 2.1M.  Without the overlap 266 + 28, with one wave per slice 366 + 28.
 constexpr int kHaloWaves = 2;
 constexpr int kHaloThreads = kWave * kHaloWaves;
 constexpr int kHaloBatch = 4;   // halo nodes a lane has in flight
@@ -544,11 +544,16 @@ __global__ __launch_bounds__(kGradStrip) void k_gradients_staged(DevTables t, co
 // ---------------------------------------------------------------------------
 // 2'. edge fluxes with the strip's node data staged in LDS.  A block covers
 //     the edges of consecutive rows (lower nodes) [r0, r1); the rows and the
-//     upper ends of their edges (ascending ids) are loaded once, field by
-//     field with consecutive lanes on consecutive doubles of a record
-//     (V: 5, X: 3 of 4, gradients: 15 of 16), so the loads coalesce.  Lane k
-//     computes edge l0 + k from LDS exactly as the per-lane kernel does; the
-//     fluxes go through the same LDS for the per-row sums P.
+//     upper ends of their edges (ascending ids) are loaded once, consecutive
+//     lanes taking consecutive fields of a node.  With plain records those
+//     are consecutive doubles; in the interleaved layout a field's pair lies
+//     in a plane of its own, so a load touches a line per two fields and the
+//     lines are shared by the lanes of neighbouring nodes.  Lane k computes
+//     edge l0 + k from LDS exactly as the per-lane kernel does; the fluxes go
+//     through the same LDS for the per-row sums P.  Boundary faces take a
+//     launch of their own (k_face_flux).  An option, not the default: it
+//     measures 158 us a second-order residual at 275k nodes and 1155 at 2.1M,
+//     against 131 and 923 of the passes above (on plain records 182 and 1236).
 // ---------------------------------------------------------------------------
 template <bool SECOND>
 __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const double *__restrict__ V,
@@ -574,9 +579,9 @@ __global__ __launch_bounds__(kFluxStrip) void k_flux_staged(DevTables t, const d
   const int tid = threadIdx.x;
   for (int h = tid; h < H; h += kFluxStrip) sidx[h] = t.fhalo[hr.x + h];
   __syncthreads();
-  // all of a lane's staging loads are in flight together: consecutive lanes
-  // take consecutive doubles of the records (V: 5, X: 3 of 4, gradients: 15
-  // of 16), so the loads coalesce, and a block waits one memory latency
+  // all of a lane's staging loads are in flight together (consecutive lanes on
+  // consecutive fields: V 5, X 3 of 4, gradients 15 of 16), so a block waits
+  // one memory latency
   constexpr int PV = (5 * HS + kFluxStrip - 1) / kFluxStrip;
   constexpr int PX = (4 * HS + kFluxStrip - 1) / kFluxStrip;
   constexpr int PG = (16 * HS + kFluxStrip - 1) / kFluxStrip;
@@ -761,7 +766,7 @@ static void launch_flux_edges(aerofx_ctx *c, const ResidualBufs &b, bool all, co
 int launch_residual_with(aerofx_ctx *c, const ResidualBufs &b, const double *U, double *R, bool scale,
                          const int *done, int *host_err) {
   const DevTables &t = c->tab;
-  // the staged kernels evaluate ROEFLUX7 only, without the failsafe
+  // the staged kernels evaluate Roe's flux only, without the failsafe
   const bool staged = t.ngb > 0 && c->residual_kernels == AEROFX_RESIDUAL_STAGED && !c->fc.low_mach && !c->failsafe;
   const bool rows = t.sh && row_waves(t.ns, kRowWaveSlices, c->max_degree);
   const bool all = staged || rows;  // P formed by the flux pass

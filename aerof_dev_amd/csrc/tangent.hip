@@ -54,10 +54,6 @@ void free_tangent(aerofx_ctx *c) {
 namespace {
 
 constexpr int kTanBlock = 256;
-// the vertices opposite to a tet's edge, in the order that makes the dual-face
-// area vector from the edge's first to its second end (c - d) x (a + b - c - d) / 24
-// (ElemTet edge and face tables, ElemTetCore.C:19-21)
-constexpr int kOpp[6][2] = {{3, 2}, {1, 3}, {2, 1}, {3, 0}, {0, 2}, {1, 0}};
 
 __device__ __forceinline__ Dual coord(const double *__restrict__ X4, const double *__restrict__ dX, int n, int a) {
   return Dual(X4[4 * (size_t)n + a], dX ? dX[3 * (size_t)n + a] : 0.0);

@@ -433,7 +433,8 @@ typedef struct {
   int converged;
   double res_max;        /* max_k ||b_k - A x_k|| / ||b_k|| (FP64 operator) */
   double seconds;
-  int tune_waves_dots, tune_waves_update;  /* autotuned launch shapes */
+  int tune_waves_dots;   /* waves per workgroup of the block products: fixed at 4 */
+  int tune_waves_update; /* of the block updates: autotuned */
 } aerofx_block_stats;
 /* Block GMRES(m) for nrhs <= 16 systems A x_k = b_k with the operators of
  * the last aerofx_jacobian_setup (which must be FP64, precision 0): H1 with
